@@ -436,7 +436,7 @@ class Mamba2Block:
         w_out = self._weights(u.dtype)[1]
         if save_for_backward and state is not None:
             raise ValueError("backward through a window that continues a carried state is not supported")
-        if block_post_proj_supported(y, w_out) and y.numel() // self.d_inner >= 8192:
+        if block_post_proj_supported(y, w_out):
             # gate, norm and out-projection as one kernel: the normalised rows never reach memory (the backward pass
             # needs them for one weight gradient only, and has its post stage write them on the way: yn=None)
             out = block_post_proj(y, zxbcdt, self.norm_w, w_out, self.H, self.P, self.N, self.G, self.eps)
@@ -482,10 +482,11 @@ class Mamba2Block:
 
     def _project(self, u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) -> torch.Tensor:
         """u . weight^T in the activation dtype: the library's kernel where it takes the shape (bf16, in_features 128
-        or 256, a tall u), else the BLAS behind torch."""
+        or 256, a tall u), else the BLAS behind torch.  Measured crossovers in us, library against BLAS: 256 -> 648
+        at 2 048 rows 6.7 / 6.7, 16 384 rows 14.6 / 24.9; 256 -> 256 at 8 192 rows 7.0 / 6.6, 16 384 rows 7.9 / 8.2."""
         w = weight.to(u.dtype)
         u = u.contiguous()
-        if block_proj_supported(u, w) and u.numel() // u.shape[-1] >= 16384:
+        if block_proj_supported(u, w) and u.numel() // u.shape[-1] >= (2048 if w.shape[0] > 256 else 16384):
             return block_proj(u, w.contiguous(), pad_rows=pad_rows)
         return torch.matmul(u, w.t()).contiguous()
 

@@ -23,7 +23,7 @@ namespace {
 constexpr int kProjWaves = 8;         // waves per workgroup: two per SIMD, 256 registers each
 constexpr int kProjBlockCols = 160;   // most output columns per workgroup (their rows of w stay in LDS)
 constexpr int kProjChunk = 32;        // output columns per MFMA tile
-constexpr int kProjTiles = 8;         // tiles of 32 rows per wave
+constexpr int kProjTiles = 8;         // most tiles of 32 rows per wave
 
 // CH: 32-column chunks of the widest block of columns (1..5; a block takes CH or CH - 1 chunks, and its last chunk
 // may hold fewer columns than it covers).  The chunk count is a template parameter and every store goes out without a condition -- a
@@ -32,7 +32,7 @@ constexpr int kProjTiles = 8;         // tiles of 32 rows per wave
 // store counted does the compiler wait for a tile's rows of u by their exact position in that order.  With a loop of
 // unknown length or a guarded store in between it waits for everything outstanding -- the next tile's rows, requested
 // a moment ago, and the last stores -- and the tile's loads, products and stores ran one after the other.
-template <int KS, int CH>  // K = 16 * KS
+template <int KS, int CH, int TILES>  // K = 16 * KS; TILES: tiles of 32 rows per wave
 __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf16 *__restrict__ u,
                                                                       const __bf16 *__restrict__ w,
                                                                       __bf16 *__restrict__ out, long long M, int N,
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
     const long long rg = (long long)(within / col_blocks) * 8 + xcd;
     const int n0 = cb * block_cols;                 // this workgroup's first column
     const int ncols = cb == col_blocks - 1 ? N - n0 : block_cols;  // a multiple of 8; the last block takes the rest
-    const long long row0 = rg * kProjTiles * (32LL * kProjWaves);
+    const long long row0 = rg * TILES * (32LL * kProjWaves);
     if (row0 >= M) return;  // the grid is padded to whole rounds of XCDs
 
     {   // rows n0 .. n0 + 32 * CH - 1 of w, all requested before the first is written to LDS (rows past N repeat the
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
     const int r = lane & 31, half = lane >> 5;
     unsigned char *tile = otile[wave];
     // the workgroup's rows of `out` as a range-checked buffer: 2 048 rows of at most ldo elements
-    const __amdgpu_buffer_rsrc_t obuf = make_buffer(out + (size_t)row0 * ldo, (unsigned)min((long long)kProjTiles * 32 * kProjWaves, M - row0) * (unsigned)ldo * 2u);
+    const __amdgpu_buffer_rsrc_t obuf = make_buffer(out + (size_t)row0 * ldo, (unsigned)min((long long)TILES * 32 * kProjWaves, M - row0) * (unsigned)ldo * 2u);
     auto tile_row0 = [&](int t) { return row0 + (long long)t * (32 * kProjWaves) + wave * 32; };
     // this lane's part of its row of u: K elements 16 ks + 8 half .. + 7 for every K step (rows past M repeat the
     // last row; they are never stored)
@@ -156,11 +156,11 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
     Frag<__bf16> ua[KS], ub[KS];
     load_rows(0, ua);
 #pragma unroll
-    for (int t = 0; t < kProjTiles; t += 2) {
-        load_rows(t + 1, ub);
+    for (int t = 0; t < TILES; t += 2) {
+        if (t + 1 < TILES) load_rows(t + 1, ub);
         tile_product(t, ua);
-        if (t + 2 < kProjTiles) load_rows(t + 2, ua);
-        tile_product(t + 1, ub);
+        if (t + 2 < TILES) load_rows(t + 2, ua);
+        if (t + 1 < TILES) tile_product(t + 1, ub);
     }
 }
 
@@ -181,14 +181,18 @@ constexpr int kPostProjMaxCols = 256;
 template <int KS, int CH>  // K = 16 * KS inner channels, CH chunks of 32 output columns
 __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     const __bf16 *__restrict__ y, const __bf16 *__restrict__ zxbcdt, const float *__restrict__ norm_w, float eps,
-    const __bf16 *__restrict__ w, __bf16 *__restrict__ out, long long M, int N, int ld_z, int ldo, int tiles) {
+    const __bf16 *__restrict__ w, __bf16 *__restrict__ out, long long M, int N, int ld_z, int ldo, int tiles, int col_blocks) {
     constexpr int K = 16 * KS, NTHR = 64 * kProjWaves, PPR = K / 8;  // 16-byte pieces per row of w
     constexpr int ROWB = K * 2 + 16;  // a staged row of w: 16 bytes of padding shift the banks from row to row
     constexpr int kTileRowB = 64 * 2 + 16;
     __shared__ __attribute__((aligned(16))) unsigned char wsm[CH * kProjChunk * ROWB];
     __shared__ __attribute__((aligned(16))) unsigned char otile[kProjWaves][16 * kTileRowB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const long long row0 = (long long)blockIdx.x * tiles * (32LL * kProjWaves);  // tiles: 32-row tiles per wave, 1 .. kProjTiles
+    // (the column blocks of a range of rows are consecutive workgroups of one XCD, as in block_proj_kernel)
+    const int xcd = blockIdx.x % 8, within = blockIdx.x / 8;
+    const int n0 = (within % col_blocks) * (CH * kProjChunk);  // this workgroup's first column
+    const long long row0 = ((long long)(within / col_blocks) * 8 + xcd) * tiles * (32LL * kProjWaves);  // tiles: 32-row tiles per wave, 1 .. kProjTiles
+    if (row0 >= M) return;  // the grid is padded to whole rounds of XCDs
     const int r = lane & 31, half = lane >> 5;
     // this lane's K elements are 16 ks + 8 half .. + 7 for every K step
     auto tile_row0 = [&](int t) { return row0 + (long long)t * (32 * kProjWaves) + wave * 32; };
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
         for (int i = 0; i < FILL; ++i) {
             const int p = min(tid + i * NTHR, PIECES - 1);
             const int row = p / PPR, piece = p % PPR;
-            const Pack8<__bf16> q = Pack8<__bf16>::load(w + (size_t)min(row, N - 1) * K + piece * 8);
+            const Pack8<__bf16> q = Pack8<__bf16>::load(w + (size_t)min(n0 + row, N - 1) * K + piece * 8);
             const float4 na = *reinterpret_cast<const float4 *>(norm_w + piece * 8);
             const float4 nb = *reinterpret_cast<const float4 *>(norm_w + piece * 8 + 4);
             uint4 o;
@@ -227,7 +231,6 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
         }
     }
     __syncthreads();
-    if (row0 >= M) return;
     unsigned char *tile = otile[wave];
     const __amdgpu_buffer_rsrc_t obuf = make_buffer(out + (size_t)row0 * ldo, (unsigned)min((long long)tiles * 32 * kProjWaves, M - row0) * (unsigned)ldo * 2u);
     const float inv_k = 1.f / (float)K;
@@ -297,10 +300,10 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int pass = 0; pass < 2; ++pass) {
-                    const int trw = pass * 8 + (lane >> 3), row = rh * 16 + trw, col = c0 * kProjChunk + (lane & 7) * 8;
+                    const int trw = pass * 8 + (lane >> 3), row = rh * 16 + trw, lcol = c0 * kProjChunk + (lane & 7) * 8, col = n0 + lcol;
                     const u32x4 q = *reinterpret_cast<const u32x4 *>(tile + trw * kTileRowB + (lane & 7) * 16);
                     const u32x4 v = (pass & 1) ? u32x4{q.z, q.w, q.x, q.y} : q;  // (halves swapped in rows 8 .. 15)
-                    const bool ok = m0 + row < M && col < N;
+                    const bool ok = m0 + row < M && lcol < CH * kProjChunk && col < N;
                     const unsigned off = ((trow + (unsigned)row) * (unsigned)ldo + (unsigned)col) * 2u;
                     __builtin_amdgcn_raw_buffer_store_b128(v, obuf, ok ? off : kBufferDropOffset, 0, 0);
                 }
@@ -333,13 +336,52 @@ static void proj_col_blocks(int out_features, int *col_blocks, int *block_cols) 
     }
 }
 
+// How the product is cut over workgroups: the columns in blocks, the rows in ranges of 256 times 1, 2, 4 or 8 tiles per
+// wave.  A compute unit holds one workgroup, so what counts is rounds of workgroups times the time of one.  Long
+// ranges pay the fill of w once for many rows, but at 16 384 rows (256 -> 648) eight tiles leave 40 workgroups for 256
+// compute units: 40.4 us, 14.6 with two tiles on blocks of 96 columns.  Times of a workgroup in us, alone on its compute
+// unit, fitted to sweeps of rows 512 .. 524 288 times columns 256 and 648 (the choice is within 6 % of the best of each):
+// one tile 4.5 + 0.5 per 32 columns, two 9 + 1.4, four 18 + 1.4, eight 34 + 1.6.
+static hipError_t proj_split(long long rows, int out_features, int *col_blocks, int *block_cols, int *tiles) {
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = device_cu_count(dev, &cus);
+    if (e != hipSuccess) return e;
+    constexpr float kFixed[4] = {4.5f, 9.f, 18.f, 34.f}, kPerChunk[4] = {0.5f, 1.4f, 1.4f, 1.6f};
+    float best = 0.f;
+    for (int cut = 0; cut < 5; ++cut) {
+        int cb, bc;
+        proj_col_blocks(out_features, &cb, &bc);
+        if (cut > 0) {  // blocks of 128, 96, 64, 32 columns: more workgroups where rows are few
+            const int narrow = kProjChunk * (5 - cut);
+            if (narrow >= bc) continue;
+            bc = narrow;
+            cb = (out_features + bc - 1) / bc;
+        }
+        const int chunks = (std::max(bc, out_features - (cb - 1) * bc) + kProjChunk - 1) / kProjChunk;
+        for (int k = 0; k < 4; ++k) {
+            const long long per_group = 32LL * kProjWaves << k;
+            const long long groups = (rows + per_group - 1) / per_group * cb;
+            const float cost = (float)((groups + cus - 1) / cus) * (kFixed[k] + kPerChunk[k] * (float)chunks);
+            if (best == 0.f || cost < best) {
+                best = cost;
+                *col_blocks = cb;
+                *block_cols = bc;
+                *tiles = 1 << k;
+            }
+        }
+    }
+    return hipSuccess;
+}
+
 hipError_t launch_block_proj(long long rows, int in_features, int out_features, int out_ld, const void *u, const void *w,
                              void *out, hipStream_t st) {
     if (!block_proj_supported(rows, in_features, out_features) || out_ld < out_features || out_ld % 8 != 0)
         return hipErrorInvalidValue;
-    int col_blocks, block_cols;
-    proj_col_blocks(out_features, &col_blocks, &block_cols);
-    const long long rows_per_group = 32LL * kProjWaves * kProjTiles;
+    int col_blocks, block_cols, tiles;
+    hipError_t e = proj_split(rows, out_features, &col_blocks, &block_cols, &tiles);
+    if (e != hipSuccess) return e;
+    const long long rows_per_group = 32LL * kProjWaves * tiles;
     const long long groups = ((rows + rows_per_group - 1) / rows_per_group + 7) / 8 * 8 * col_blocks;
     if (groups > 0x7fffffffLL || out_features - (col_blocks - 1) * block_cols > kProjBlockCols ||
         out_features - (col_blocks - 1) * block_cols <= 0)
@@ -350,13 +392,15 @@ hipError_t launch_block_proj(long long rows, int in_features, int out_features, 
     // the chunks of 32 columns the widest block takes
     const int widest = std::max(block_cols, out_features - (col_blocks - 1) * block_cols);
     const int ch = (widest + kProjChunk - 1) / kProjChunk;
-#define SSD_PROJ_CASE(KSv, CHv)                                                                                        \
-    if (in_features == 16 * KSv && ch == CHv) {                                                                        \
-        block_proj_kernel<KSv, CHv><<<grid, block, 0, st>>>(uu, ww, oo, rows, out_features, out_ld, col_blocks, block_cols); \
+#define SSD_PROJ_CASE(KSv, CHv, Tv)                                                                                    \
+    if (in_features == 16 * KSv && ch == CHv && tiles == Tv) {                                                         \
+        block_proj_kernel<KSv, CHv, Tv><<<grid, block, 0, st>>>(uu, ww, oo, rows, out_features, out_ld, col_blocks, block_cols); \
         return hipGetLastError();                                                                                      \
     }
-    SSD_PROJ_CASE(8, 1) SSD_PROJ_CASE(8, 2) SSD_PROJ_CASE(8, 3) SSD_PROJ_CASE(8, 4) SSD_PROJ_CASE(8, 5)
-    SSD_PROJ_CASE(16, 1) SSD_PROJ_CASE(16, 2) SSD_PROJ_CASE(16, 3) SSD_PROJ_CASE(16, 4) SSD_PROJ_CASE(16, 5)
+#define SSD_PROJ_TILES(KSv, CHv) SSD_PROJ_CASE(KSv, CHv, 1) SSD_PROJ_CASE(KSv, CHv, 2) SSD_PROJ_CASE(KSv, CHv, 4) SSD_PROJ_CASE(KSv, CHv, 8)
+    SSD_PROJ_TILES(8, 1) SSD_PROJ_TILES(8, 2) SSD_PROJ_TILES(8, 3) SSD_PROJ_TILES(8, 4) SSD_PROJ_TILES(8, 5)
+    SSD_PROJ_TILES(16, 1) SSD_PROJ_TILES(16, 2) SSD_PROJ_TILES(16, 3) SSD_PROJ_TILES(16, 4) SSD_PROJ_TILES(16, 5)
+#undef SSD_PROJ_TILES
 #undef SSD_PROJ_CASE
     return hipErrorInvalidValue;
 }
@@ -381,16 +425,22 @@ hipError_t launch_block_post_proj(const BlockShape &s, const void *y, const void
     if (e != hipSuccess) return e;
     const long long per_tile = 32LL * kProjWaves;
     const int tiles = (int)std::max<long long>(1, std::min<long long>(kProjTiles, rows / (per_tile * cus)));
+    // Where one tile per wave still leaves compute units idle, the columns are cut too, in up to eight blocks of 32 (each
+    // gates its rows anew; staging w and the products shrink): 16 384 rows, 256 -> 256, in us with 1, 2, 4, 8 blocks:
+    // 20.7, 17.5, 17.0, 26.3 (256 workgroups are a round); 8 192 rows 19.6, 16.4, 15.7, 14.1.
+    int col_blocks = 1;
+    const int chunks = (out_features + kProjChunk - 1) / kProjChunk;
+    while (col_blocks < 8 && 2 * col_blocks <= chunks && (rows + per_tile - 1) / per_tile * (2 * col_blocks) <= cus) col_blocks *= 2;
     const long long rows_per_group = per_tile * tiles;
-    const long long groups = (rows + rows_per_group - 1) / rows_per_group;
+    const long long groups = ((rows + rows_per_group - 1) / rows_per_group + 7) / 8 * 8 * col_blocks;
     if (groups > 0x7fffffffLL || (unsigned long long)rows_per_group * out_ld * 2 > 0x7fffffffULL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)groups), block(64 * kProjWaves);
     const __bf16 *yy = static_cast<const __bf16 *>(y), *zz = static_cast<const __bf16 *>(zxbcdt), *ww = static_cast<const __bf16 *>(w);
     __bf16 *oo = static_cast<__bf16 *>(out);
-    const int ch = (out_features + kProjChunk - 1) / kProjChunk;
+    const int ch = (chunks + col_blocks - 1) / col_blocks;
 #define SSD_POST_PROJ_CASE(KSv, CHv)                                                                                   \
     if (K == 16 * KSv && ch == CHv) {                                                                                  \
-        block_post_proj_kernel<KSv, CHv><<<grid, block, 0, st>>>(yy, zz, norm_w, eps, ww, oo, rows, out_features, s.ld, out_ld, tiles); \
+        block_post_proj_kernel<KSv, CHv><<<grid, block, 0, st>>>(yy, zz, norm_w, eps, ww, oo, rows, out_features, s.ld, out_ld, tiles, col_blocks); \
         return hipGetLastError();                                                                                      \
     }
     SSD_POST_PROJ_CASE(8, 1) SSD_POST_PROJ_CASE(8, 2) SSD_POST_PROJ_CASE(8, 3) SSD_POST_PROJ_CASE(8, 4)
