@@ -269,6 +269,43 @@ def test_decay_gradient_between_far_anchors(w):
     assert (got["dA"].double() - total).abs().max().item() <= 1e-5 * scale
 
 
+@pytest.mark.parametrize("w", [
+    Workload("bwd_segments_two_tiles", 2, 65, 8, 32, 64, 1, 64, dtype="bf16", init_std=0.5),          # 2 segments of a tile
+    Workload("bwd_segments_one_tile_each", 1, 64 * 6 + 1, 8, 32, 64, 1, 128, dtype="bf16", init_std=0.5),
+    Workload("bwd_segments_ragged", 12, 64 * 23 + 31, 8, 32, 64, 1, 64, dtype="bf16", init_std=0.5),  # the last is shorter
+    Workload("bwd_segments_wide", 40, 64 * 13, 8, 32, 64, 1, 64, dtype="bf16", init_std=0.5),
+    Workload("bwd_segments_narrow_state", 3, 64 * 9 + 7, 8, 32, 32, 1, 64, dtype="bf16", init_std=0.5),
+    Workload("bwd_segments_three_groups", 2, 64 * 5 + 63, 24, 32, 64, 3, 64, dtype="bf16", init_std=0.5),
+    Workload("bwd_segments_strong_decay", 4, 64 * 17 - 1, 8, 32, 64, 1, 64, dtype="bf16", a_log_range=(0.01, 64.0),
+             dt_law="mixture", x_law="student-t3"),
+], ids=lambda w: w.name)
+@pytest.mark.parametrize("carried", [True, False])
+def test_gradients_on_segments_of_the_sequence(w, carried):
+    """Few sequences run on segments of several tiles, or one, that start from states of their own: restarts on every tile
+    border around the segments', a row that restarts at once (whatever its initial state holds), with and without carried
+    states, one to three groups of eight heads, both widths of the transposed scans."""
+    dev = make_inputs(w, seed=8, device="cuda")
+    m = (np.random.default_rng(3).random((w.batch, w.seqlen)) < 0.004).astype(np.uint8)
+    m[0] = 0
+    if w.batch > 1:
+        m[1, 63::64] = 1
+        m[1, 0] = 1
+        m[-1, 64::64] = 1
+    g = torch.Generator(device="cuda").manual_seed(5)
+    dy = torch.randn(dev["x"].shape, generator=g, device="cuda").to(torch.bfloat16)
+    dfin = torch.randn(w.batch, w.nheads, w.headdim, w.dstate, generator=g, device="cuda") if carried else None
+    init = dev["init"] if carried else None
+    got = ssd_chunk_scan_backward(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], dy, chunk=w.chunk,
+                                  initial_states=init, dfinal_states=dfin, need_dinitial_states=True,
+                                  reset=torch.from_numpy(m).cuda())
+    ref = bwd.ssd_backward_sequential(np64(dev["x"]), np64(dev["dt"]), np64(dev["A"]), np64(dev["B"]), np64(dev["C"]),
+                                      np64(dev["D"]), np64(init), np64(dy), np64(dfin), reset=m)
+    for k_out, k_ref in (("dx", "dx"), ("ddt", "ddt"), ("dB", "dB"), ("dC", "dC"), ("dinitial_states", "dinit")):
+        check(got[k_out], ref[k_ref], torch.bfloat16, f"{w.name} {k_out}")
+    check(got["dA"], ref["dA"], torch.bfloat16, f"{w.name} dA", ref["dA_scale"])
+    check(got["dD"], ref["dD"], torch.bfloat16, f"{w.name} dD", ref["dD_scale"])
+
+
 def test_restarts_on_the_one_pass_adjoint_scan():
     """Enough bf16 sequences for the adjoint recurrence to take the one-pass kernel: rows against the oracle."""
     w = Workload("bwd_reset_onepass", 96, 200, 8, 32, 64, 1, 128, dtype="bf16")

@@ -9,7 +9,9 @@
 #include <cstdlib>
 #include <cstring>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "ssd_launch.h"
 
@@ -182,7 +184,8 @@ int run_staged(const ssd::ScanShape &s, int dtype, const void *x, const void *dt
 // array), the gathered operands (reversed ones padded to whole chunks) and the scans' float outputs.
 struct BwdWorkspace {
     size_t scan_off, states2, dy_rev, x_rev, c_rev_g, b_rev_g, c_rev_h, b_fwd_h, r_rev, yb_rev, yc, gfin, gfin_t, ffin_t,
-        init_t, dfin_t, e1, dd, u, parts, anchor, da_part, dt_parts, a_parts, total;
+        init_t, dfin_t, e1, dd, u, parts, anchor, da_part, dt_parts, a_parts, seg_fwd, seg_adj, seg_fwd_t, seg_adj_t, seg_decay,
+        total;
 };
 
 // Which kernels a backward pass of a given shape runs on (a function of shape and dtype only: the workspace is laid
@@ -193,6 +196,7 @@ struct BwdPlan {
     bool sum_on_chip;   // ... on its transposed kinds, which sum dB and dC over a group's heads themselves
     bool rows_in_scan;  // the adjoint scan with the row products in its epilogue (writes dx; no float r)
     int anchor_stride;  // tiles between two meetings of the transposed scans' states (the decay gradient's anchors)
+    int seg_tiles;      // the three scans on segments of that many tiles (0: not cut)
 };
 
 // The decay gradient is anchored where the two transposed scans' states meet; between two anchors it sums the
@@ -201,6 +205,30 @@ struct BwdPlan {
 // of the pass's time); in bf16 mode, where the gradient is rounded to 8 bits, runs of 512 steps stay three orders of
 // magnitude below that rounding.
 constexpr int kBf16AnchorStride = 8;
+
+// Tiles per segment of the three scans where one workgroup per eight heads and sequence leaves compute units idle (0: not
+// cut), by estimated microseconds: uncut, 30 + 18.5 per tile; cut, every round of 256 workgroups costs 60 (the prologues
+// of five launches: the states-only passes, the entering states, the scans) and 19.5 per tile below the 96 workgroups
+// from which the transposed scans are wide, 27 to 37 from there to 256.  Measured at eight heads of 32, state 64
+// (sequences x steps, as chosen here / uncut / the general path they took before): 32 x 2 048 219 / 555 / 631, 4 x 4 096
+// 111 / 1 048 / 216, 64 x 2 048 365 / 594 / 792, 16 x 8 192 363 / 2 154 / 1 197, 1 x 146 59 / 78 / 92; uncut as chosen:
+// 52 x 153 94 (cut 91) / 115.
+int bwd_segment_tiles(const ssd::ScanShape &s) {
+    const double groups = (double)s.B * s.H / 8;
+    double best = 30.0 + 18.5 * s.nc;
+    int tiles = 0;
+    for (int S = 2; S <= s.nc && groups * (S - 1) < 512; ++S) {  // (more than two rounds are never the fastest)
+        const int t = (s.nc + S - 1) / S;
+        const double W = groups * ((s.nc + t - 1) / t);
+        const double per_tile = W < 96 ? 19.5 : 27.0 + 10.0 * std::min(1.0, (W - 96) / 160);
+        const double cost = std::ceil(W / 256) * (60.0 + per_tile * t);
+        if (cost < best) {
+            best = cost;
+            tiles = t;
+        }
+    }
+    return tiles;
+}
 
 BwdPlan plan_bwd(const ssd::ScanShape &s, const ssd::ScanShape &sT, int dtype) {
     const int inner = dtype == SSD_DTYPE_F32 ? SSD_DTYPE_F32 : SSD_DTYPE_BF16_Y32;  // the scans write float y
@@ -218,9 +246,20 @@ BwdPlan plan_bwd(const ssd::ScanShape &s, const ssd::ScanShape &sT, int dtype) {
     p.sum_on_chip = inner != SSD_DTYPE_F32 && ssd::transposed_scan_supported(sT, s.G) &&
                     (int64_t)s.B * (s.H / 8) * (s.N / 32) >= kOnePassMinWorkgroups;
     p.fast_r = one_pass(s);  // (the padded length does not enter)
+    // Fewer sequences: the same kinds, on segments where that is faster.  The anchors stay at every tile there, as on the
+    // general path these shapes took before: the dA of a few sequences has fewer terms to average over, and with anchors
+    // eight tiles apart its error against float64 was four to ten times the general path's (4 x 1 000 steps 1.3e-4
+    // against 2.1e-5 of its norm; 1.4e-5 with one at every tile).
+    const bool few = !p.fast_r;
+    p.seg_tiles = 0;
+    if (few && inner != SSD_DTYPE_F32 && s.Q == 64 && ssd::transposed_scan_supported(sT, s.G) &&
+        ssd::adjoint_rows_scan_supported(s) && ssd::fused_scan_waves(s, inner) == 8) {
+        p.sum_on_chip = p.fast_r = true;
+        p.seg_tiles = bwd_segment_tiles(s);
+    }
     p.fast_t = p.sum_on_chip || one_pass(sT);
     p.rows_in_scan = p.sum_on_chip && p.fast_r && ssd::adjoint_rows_scan_supported(s);
-    p.anchor_stride = (p.rows_in_scan && ssd::bwd_ddt_anchor_stride_supported(s, (s.N + 31) / 32)) ? kBf16AnchorStride : 1;
+    p.anchor_stride = (p.rows_in_scan && !few && ssd::bwd_ddt_anchor_stride_supported(s, (s.N + 31) / 32)) ? kBf16AnchorStride : 1;
     return p;
 }
 
@@ -265,6 +304,14 @@ BwdWorkspace carve_bwd(const ssd::ScanShape &s, const ssd::ScanShape &sT, int el
     // dt and A once per part of a head, for the transposed scans of a state scanned in parts
     w.dt_parts = take_if(sT.H > s.H, BL * sT.H * elem_bytes);
     w.a_parts = take_if(sT.H > s.H, (size_t)sT.H * sizeof(float));
+    // on segments: what each adds to the forward and the adjoint state, the states entering each (transposed; the
+    // adjoint's also in place of what it adds), the segments' decays
+    const size_t segs = plan.seg_tiles > 0 ? (size_t)((s.nc + plan.seg_tiles - 1) / plan.seg_tiles) : 0;
+    w.seg_fwd = take(segs * st);
+    w.seg_adj = take(segs * st);
+    w.seg_fwd_t = take(segs * st);
+    w.seg_adj_t = take(segs * st);
+    w.seg_decay = take(2 * segs * s.B * s.H * sizeof(float));
     w.total = off;
     return w;
 }
@@ -590,11 +637,29 @@ int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const voi
         }
     }
     const float *init_t = nullptr, *dfin_t = nullptr;
-    if (initial_states != nullptr) {
+    const float *adj_init = dfinal_states;  // what the adjoint scan starts from
+    if (plan.seg_tiles > 0) {
+        ssd::ScanShape f = s, fa = sR;
+        f.seg_tiles = fa.seg_tiles = sR.seg_tiles = sTR.seg_tiles = sT.seg_tiles = plan.seg_tiles;
+        fa.mode = 1;
+        fa.dt_len = s.L;
+        float *decay_f = atf(w.seg_decay), *decay_a = decay_f + (size_t)s.B * ssd::scan_segments(f) * s.H;
+        BWD_LAUNCH(ssd::launch_segment_states(f, false, x, dt, A, Bm, reset, atf(w.seg_fwd), decay_f, st), "segment states");
+        BWD_LAUNCH(ssd::launch_segment_states(fa, true, dy, dt, A, Cm, reset, atf(w.seg_adj), decay_a, st),
+                   "segment states (adjoint)");
+        BWD_LAUNCH(ssd::launch_segment_entries(f, atf(w.seg_fwd), decay_f, initial_states, reset, atf(w.seg_fwd_t), atf(w.seg_adj),
+                                               decay_a, dfinal_states, atf(w.seg_adj_t), st),
+                   "segment entries");
+        adj_init = atf(w.seg_adj);
+    }
+    // (on segments the transposed initial states are the first segments' entering states)
+    if (plan.seg_tiles > 0 && initial_states != nullptr) init_t = atf(w.seg_fwd_t);
+    else if (initial_states != nullptr) {
         BWD_LAUNCH(ssd::launch_transpose_state(initial_states, atf(w.init_t), (long long)s.B * s.H, s.P, s.N, st), "transpose");
         init_t = atf(w.init_t);
     }
-    if (dfinal_states != nullptr) {
+    if (plan.seg_tiles > 0 && dfinal_states != nullptr) dfin_t = atf(w.seg_adj_t);
+    else if (dfinal_states != nullptr) {
         BWD_LAUNCH(ssd::launch_transpose_state(dfinal_states, atf(w.dfin_t), (long long)s.B * s.H, s.P, s.N, st), "transpose");
         dfin_t = atf(w.dfin_t);
     }
@@ -623,7 +688,7 @@ int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const voi
         ssd::ScanShape f = sR;
         f.mode = 1;
         f.dt_len = s.L;
-        BWD_LAUNCH(ssd::launch_adjoint_rows_scan(f, dy, dt, A, Cm, Bm, D, x, dfinal_states, reset, dx, atf(w.gfin), atf(w.e1), st),
+        BWD_LAUNCH(ssd::launch_adjoint_rows_scan(f, dy, dt, A, Cm, Bm, D, x, adj_init, reset, dx, atf(w.gfin), atf(w.e1), st),
                    "adjoint scan with row products");
     } else if (int rc = fast_r ? scan(sR, true, dy, Cm, Bm, dfinal_states, 1, at(w.r_rev), atf(w.gfin), states, false, 0)
                         : scan(sR, false, at(w.dy_rev), at(w.c_rev_g), at(w.b_rev_g), dfinal_states, 1, at(w.r_rev),
@@ -641,24 +706,32 @@ int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const voi
         an.other_tiles = states;
         an.out = reinterpret_cast<double *>(base + w.anchor);
         an.stride = keep.stride = plan.anchor_stride;
+        const float *ff_init = init_t, *fa_init = dfin_t;  // what the two scans start from
+        if (plan.seg_tiles > 0) {
+            ff_init = atf(w.seg_fwd_t);
+            fa_init = atf(w.seg_adj_t);
+            an.other_init_segs = ssd::scan_segments(ff);
+        }
         if (ssd::transposed_scan_anchors_in_adjoint(sT)) {
-            BWD_LAUNCH(ssd::launch_transposed_scan(ff, false, Bm, dt, A, x, dy, Cm, init_t, reset, dC, atf(w.ffin_t), states,
+            BWD_LAUNCH(ssd::launch_transposed_scan(ff, false, Bm, dt, A, x, dy, Cm, ff_init, reset, dC, atf(w.ffin_t), states,
                                                    atf(w.parts), keep, st),
                        "transposed forward scan");
             an.other_final = atf(w.ffin_t);
+            an.no_init = dfinal_states == nullptr;
             an.other_init = init_t;
-            BWD_LAUNCH(ssd::launch_transposed_scan(fa, true, Cm, dt, A, dy, x, nullptr, dfin_t, reset, dB, nullptr, nullptr,
+            BWD_LAUNCH(ssd::launch_transposed_scan(fa, true, Cm, dt, A, dy, x, nullptr, fa_init, reset, dB, nullptr, nullptr,
                                                    nullptr, an, st),
                        "transposed adjoint scan");
         } else {
             // (the adjoint scan's tile c starts where forward tile nc - c ends)
             an.phase = keep.phase = s.nc % plan.anchor_stride;
-            BWD_LAUNCH(ssd::launch_transposed_scan(fa, true, Cm, dt, A, dy, x, nullptr, dfin_t, reset, dB, atf(w.gfin_t),
+            BWD_LAUNCH(ssd::launch_transposed_scan(fa, true, Cm, dt, A, dy, x, nullptr, fa_init, reset, dB, atf(w.gfin_t),
                                                    states, nullptr, keep, st),
                        "transposed adjoint scan");
             an.other_final = atf(w.gfin_t);
+            an.no_init = initial_states == nullptr;
             an.other_init = dfin_t;
-            BWD_LAUNCH(ssd::launch_transposed_scan(ff, false, Bm, dt, A, x, dy, Cm, init_t, reset, dC, nullptr, nullptr,
+            BWD_LAUNCH(ssd::launch_transposed_scan(ff, false, Bm, dt, A, x, dy, Cm, ff_init, reset, dC, nullptr, nullptr,
                                                    atf(w.parts), an, st),
                        "transposed forward scan");
         }

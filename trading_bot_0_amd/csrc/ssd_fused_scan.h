@@ -151,6 +151,8 @@ constexpr size_t fused_scan_lds_bytes(int N, int Q, int waves) {
 // holds a head's whole row).  With r_t the recurrence's output it writes dx_t = dt_t r_t + D x_t (x being the
 // scan's x operand, dy) instead of r, and per (b, t, h) the pair (aux_t . r_t, aux_t . x_t) -- aux is the forward's
 // x, so these are e1 = x . r and dd = dy . x -- into seg_decay as float2 [B, L, H].
+// KIND 8: KIND 2 for the reversed-adjoint recurrence.  Kinds 3 to 7 walk segments as well (s.seg_tiles), each from a
+// state of its own in `init` [B, S, H, P, N].
 // LDS of a workgroup of the transposed scans: a B and a C tile per wave (eight waves), the shared x tile and
 // second-operand tile, the per-wave tables, and a [Q][33] float tile per wave for the heads' outputs (summed in a
 // fixed order when the workgroup writes them out, so that results do not depend on timing).
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
     const float *init, const unsigned char *__restrict__ reset, TO *__restrict__ y, float *final_states,
     float *tile_states, float *seg_decay, const __bf16 *__restrict__ aux, ScanShape s, ScanAnchors an) {
     using T = __bf16;
-    constexpr bool ADJ = KIND == 1 || KIND == 4 || KIND == 5 || KIND == 7, STATES_ONLY = KIND == 2;
+    constexpr bool ADJ = KIND == 1 || KIND == 4 || KIND == 5 || KIND == 7 || KIND == 8, STATES_ONLY = KIND == 2 || KIND == 8;
     constexpr bool TR = KIND == 3 || KIND == 4 || KIND == 6 || KIND == 7;
     constexpr bool TR_FWD = KIND == 3 || KIND == 6, TR_ADJ = KIND == 4 || KIND == 7;
     constexpr int SL = (KIND == 6 || KIND == 7) ? 2 : 1;  // 32-column slices of x (and of the state) per wave
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
     // leave it in LDS in the accumulator's own layout, every wave reads the three from there: 12 matrix instructions
     // per tile and workgroup instead of 96, for 12 KB of LDS and a second barrier per tile (behind the first block's
     // readout, where the scores are first needed).
-    constexpr bool kSharedScores = !TR && KIND != 2 && WAVES == 8 && QB == 2 && NK <= 4;
+    constexpr bool kSharedScores = !TR && !STATES_ONLY && WAVES == 8 && QB == 2 && NK <= 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[SL == 2 ? wide_transposed_scan_lds_bytes(Q)
                                                                         : TR ? transposed_scan_lds_bytes(Q)
                                                                              : fused_scan_lds_bytes(N, Q, WAVES) + (kSharedScores ? 3 * 32 * 32 * 4 : 0)];  // (kind 5 uses one set of the two)
@@ -536,7 +538,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
         // (the other scan kept the states entering its tiles phase, phase + stride, ..: anchor_here says which j meet one)
         const int kept = s.nc > an.phase ? (s.nc - 1 - an.phase) / an.stride + 1 : 1;
         const size_t bh = tiles ? ((size_t)b * kept + (zero ? 0 : (s.nc - j - an.phase) / an.stride)) * s.H + h
-                                : (size_t)b * s.H + h;
+                                : (size_t)b * (j == s.nc ? an.other_init_segs : 1) * s.H + h;
         return (zero ? an.other_tiles : g) + (bh * s.P + pb * 32 + (lane0 & 31)) * N + 4 * (lane0 >> 5);
     };
     // one slice at a time, so that at most one slice of the other scan's state is held in registers
@@ -567,19 +569,22 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
     };
     if constexpr (ANCH) {
         if (an.out != nullptr) {
-            bool zero0;
-            const float *g0 = adjoint_state(0, zero0);
-            zero0 = zero0 || init == nullptr;  // no initial state: a zero anchor
+            // (where a segment ends the anchor is the next segment's: it starts with that state)
+            if (c_first == 0 || anchor_here(c_first)) {
+                bool zero0;
+                const float *g0 = adjoint_state(c_first, zero0);
+                zero0 = zero0 || (c_first == 0 && (init == nullptr || an.no_init));  // no initial state: a zero anchor
 #pragma unroll
-            for (int sl = 0; sl < SL; ++sl) {
-                float4 gq[NB][4];
-                load_other(g0, sl, gq);
-                write_anchor(0, sl, gq, zero0);
+                for (int sl = 0; sl < SL; ++sl) {
+                    float4 gq[NB][4];
+                    load_other(g0, sl, gq);
+                    write_anchor(c_first, sl, gq, zero0);
+                }
             }
         }
     }
 
-    float seg_total = 1.f;  // product of the tiles' decays (KIND 2)
+    float seg_total = 1.f;  // product of the tiles' decays (states only)
     // one tile; `set` (a compile-time 0 or 1) is the set of LDS tiles it uses; false when the scan ends inside it
     auto tile = [&](const int c, auto set) -> bool {
         constexpr int SET = decltype(set)::value;
@@ -1022,6 +1027,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
         // (the forward's last tile of a segment other than the last, or of a call that asks for no final state: nobody
         // reads the state it leaves)
         if (KIND == 0 && c + 1 == c_end && !(final_states != nullptr && seg == S - 1)) return false;
+        if ((TR || ROWS) && c + 1 == c_end && c_end < s.nc) return false;
         if (!kEarlyPrefetch && c + 1 < c_end) prefetch(c + 1);
         // the other scan's state where this tile ends: the first slice in flight during phase 2, the second (two
         // slices per wave leave no registers to hold both) requested after it
@@ -1144,7 +1150,7 @@ static hipError_t fused_launch(const ScanShape &s, const void *x, const void *dt
                                const void *Cm, const float *D, const float *init, const unsigned char *reset, void *y,
                                float *final_states, float *tile_states, hipStream_t st) {
     const int units = (s.H / s.G) * (s.P / 32);
-    const int segments = s.seg_tiles > 0 ? (s.nc + s.seg_tiles - 1) / s.seg_tiles : 1;
+    const int segments = scan_segments(s);
     const int grid = s.B * s.G * (units / WAVES) * segments;
     const __bf16 *xx = static_cast<const __bf16 *>(x), *dd = static_cast<const __bf16 *>(dt);
     const __bf16 *bb = static_cast<const __bf16 *>(Bm), *cc = static_cast<const __bf16 *>(Cm);
@@ -1164,17 +1170,18 @@ static hipError_t fused_launch(const ScanShape &s, const void *x, const void *dt
     return hipGetLastError();
 }
 
-// States only (KIND 2): per segment, the state it leaves behind from `init` ([B,S,H,P,N] or NULL = zero) into
-// seg_states [B,S,H,P,N] and its total decay into seg_decay [B,S,H].
-template <int NK, int QB, int WAVES>
+// States only (KIND 2, or 8 for the reversed-adjoint recurrence): per segment, the state it leaves behind from `init`
+// ([B,S,H,P,N] or NULL = zero) into seg_states [B,S,H,P,N] and its total decay into seg_decay [B,S,H].
+template <int NK, int QB, int WAVES, int KIND = 2>
 static hipError_t fused_launch_states(const ScanShape &s, const void *x, const void *dt, const float *A, const void *Bm,
                                       const float *init, const unsigned char *reset, float *seg_states, float *seg_decay,
                                       hipStream_t st) {
+    static_assert(KIND == 2 || KIND == 8, "the kinds that write states only");
     const int units = (s.H / s.G) * (s.P / 32);
-    const int segments = s.seg_tiles > 0 ? (s.nc + s.seg_tiles - 1) / s.seg_tiles : 1;
+    const int segments = scan_segments(s);
     const int grid = s.B * s.G * (units / WAVES) * segments;
     const __bf16 *bb = static_cast<const __bf16 *>(Bm);
-    fused_scan_kernel<__bf16, NK, QB, WAVES, 2><<<dim3(grid), dim3(64 * WAVES), 0, st>>>(
+    fused_scan_kernel<__bf16, NK, QB, WAVES, KIND><<<dim3(grid), dim3(64 * WAVES), 0, st>>>(
         static_cast<const __bf16 *>(x), static_cast<const __bf16 *>(dt), A, bb, bb, nullptr, init, reset, nullptr, seg_states,
         nullptr, seg_decay, nullptr, s, ScanAnchors{});
     return hipGetLastError();
@@ -1190,11 +1197,12 @@ static hipError_t fused_launch_transposed(const ScanShape &s, const void *x, con
                                           const void *Cm, const void *aux, const float *init, const unsigned char *reset,
                                           void *out, float *final_states, float *tile_states, float *parts,
                                           const ScanAnchors &an, hipStream_t st) {
-    if (s.N != 32 || s.G != s.H || s.x_groups <= 0 || s.H != 8 * s.x_groups || s.P % 32 != 0 || s.seg_tiles != 0)
+    if (s.N != 32 || s.G != s.H || s.x_groups <= 0 || s.H != 8 * s.x_groups || s.P % 32 != 0 ||
+        (s.seg_tiles != 0 && init == nullptr))
         return hipErrorInvalidValue;
     constexpr bool kWide = KIND == 6 || KIND == 7;  // both slices of a 64-wide state in one wave
     if (kWide && s.P != 64) return hipErrorInvalidValue;
-    const int grid = s.B * (s.H / 8) * (kWide ? 1 : s.P / 32);
+    const int grid = s.B * (s.H / 8) * (kWide ? 1 : s.P / 32) * scan_segments(s);
     fused_scan_kernel<TO, 2, kOnePassTile / 32, 8, KIND><<<dim3(grid), dim3(512), 0, st>>>(
         static_cast<const __bf16 *>(x), static_cast<const __bf16 *>(dt), A, static_cast<const __bf16 *>(Bm),
         static_cast<const __bf16 *>(Cm), nullptr, init, reset, static_cast<TO *>(out), final_states, tile_states, parts,
@@ -1210,10 +1218,10 @@ static hipError_t fused_launch_adjoint_rows(const ScanShape &s, const void *x, c
                                             const unsigned char *reset, void *dx, float *final_states, float *pairs,
                                             hipStream_t st) {
     const int units = (s.H / s.G) * (s.P / 32);
-    if (s.P != 32 || units % 8 != 0 || s.seg_tiles != 0 || s.x_groups != 0 || s.N != 16 * NK || aux == nullptr ||
+    if (s.P != 32 || units % 8 != 0 || (s.seg_tiles != 0 && init == nullptr) || s.x_groups != 0 || s.N != 16 * NK || aux == nullptr ||
         pairs == nullptr)
         return hipErrorInvalidValue;
-    const int grid = s.B * s.G * (units / 8);
+    const int grid = s.B * s.G * (units / 8) * scan_segments(s);
     fused_scan_kernel<__bf16, NK, kOnePassTile / 32, 8, 5><<<dim3(grid), dim3(512), 0, st>>>(
         static_cast<const __bf16 *>(x), static_cast<const __bf16 *>(dt), A, static_cast<const __bf16 *>(Bm),
         static_cast<const __bf16 *>(Cm), D, init, reset, static_cast<__bf16 *>(dx), final_states, nullptr, pairs,

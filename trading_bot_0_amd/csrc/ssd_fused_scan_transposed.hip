@@ -13,7 +13,7 @@ namespace {
 // a 64-wide state with both slices in one wave where that still leaves enough workgroups for the chip
 bool wide(const ScanShape &sT) {
     constexpr int kWideMinWorkgroups = 96;
-    return sT.P == 64 && (long long)sT.B * (sT.H / 8) >= kWideMinWorkgroups;
+    return sT.P == 64 && (long long)sT.B * (sT.H / 8) * scan_segments(sT) >= kWideMinWorkgroups;
 }
 }  // namespace
 

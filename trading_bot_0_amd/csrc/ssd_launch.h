@@ -29,6 +29,9 @@ struct ScanShape {
     const unsigned char *fresh = nullptr;
 };
 
+// How many segments a sequence of s.nc tiles is cut into (1 = not cut)
+inline int scan_segments(const ScanShape &s) { return s.seg_tiles > 0 ? (s.nc + s.seg_tiles - 1) / s.seg_tiles : 1; }
+
 struct StepShape {
     int B, H, P, N, G;
 };
@@ -174,6 +177,8 @@ struct ScanAnchors {
     const float *other_tiles = nullptr, *other_final = nullptr, *other_init = nullptr;
     double *out = nullptr;
     int stride = 1, phase = 0;
+    int other_init_segs = 1;  // other_init is the first of that many states per batch row, [B, segs, H, P, N]
+    bool no_init = false;  // on segments, which all have a state of their own: the sequence has no initial state
 };
 bool transposed_scan_anchors_in_adjoint(const ScanShape &sT);
 bool transposed_scan_supported(const ScanShape &sT, int x_groups);
@@ -181,6 +186,20 @@ hipError_t launch_transposed_scan(const ScanShape &sT, bool adjoint, const void 
                                   const void *Bm, const void *Cm, const void *aux, const float *init,
                                   const unsigned char *reset, void *out, float *final_states, float *tile_states,
                                   float *parts, const ScanAnchors &an, hipStream_t stream);
+
+// For the backward pass on segments (s: the forward shape, seg_tiles set, L padded to whole tiles and dt_len the true
+// length for the adjoint): from x | B (forward) or dy | C (adjoint), what every segment but the last adds to the state
+// from zero, seg_states [B, S, H, P, N], and its total decay, seg_decay [B, S, H].
+hipError_t launch_segment_states(const ScanShape &s, bool adjoint, const void *x, const void *dt, const float *A,
+                                 const void *Bm, const unsigned char *reset, float *seg_states, float *seg_decay,
+                                 hipStream_t stream);
+// The states entering every segment, from the above: enter[0] = init (zero if NULL, or where the forward's `fresh` mask
+// [B, L] restarts the sequence before its first step), enter[j+1] = decay[j] enter[j] + states[j], for the forward and
+// the adjoint recurrence in one launch.  Written with the state transposed, [B, S, H, N, P]; the adjoint's also as it
+// is, in place of adj_states.
+hipError_t launch_segment_entries(const ScanShape &s, const float *fwd_states, const float *fwd_decay, const float *fwd_init,
+                                  const unsigned char *fresh, float *fwd_enter_t, float *adj_states, const float *adj_decay,
+                                  const float *adj_init, float *adj_enter_t, hipStream_t stream);
 
 // The backward pass's reversed-adjoint scan with the row products in its epilogue (bf16, headdim 32, heads per
 // group a multiple of eight, dstate 32 or 64).  sR is the forward shape with L padded to whole tiles, mode 1 and
