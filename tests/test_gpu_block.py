@@ -421,6 +421,40 @@ def test_block_step_as_one_launch(cfg, dtype):
         conv_ref = np64(st_f.conv)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cfg", [(256, 8, 32, 64, 1, 4, 257), (128, 8, 16, 64, 1, 3, 259), (256, 8, 16, 64, 1, 2, 300),
+                                 (128, 16, 16, 64, 1, 4, 66), (256, 8, 32, 64, 2, 4, 258), (128, 8, 32, 64, 4, 3, 1)])
+def test_block_step_for_many_streams(cfg, dtype):
+    """A 64-wide state: one stream per workgroup up to as many streams as compute units, two above (an odd count leaves one
+    alone), and the kernel for more rows of w_in than the overlapped one takes; two steps against the stage kernels, which
+    round at the same points (bars as in test_block_step_as_one_launch), and the last streams against the oracle."""
+    d_model, H, P, N, G, K, Bsz = cfg
+    b = Mamba2Block(d_model=d_model, nheads=H, headdim=P, dstate=N, ngroups=G, d_conv=K, seed=9)
+    g = torch.Generator().manual_seed(33)
+    C = H * P + 2 * G * N
+    conv0 = torch.randn(Bsz, K - 1, C, generator=g).to(dtype).cuda()
+    ssm0 = torch.randn(Bsz, H, P, N, generator=g).cuda()
+    us = torch.randn(2, Bsz, d_model, generator=g).to(dtype).cuda()
+    st_f, st_s = b.new_state(Bsz, dtype=dtype), b.new_state(Bsz, dtype=dtype)
+    for st in (st_f, st_s):
+        st.conv.copy_(conv0)
+        st.ssm.state.copy_(ssm0)
+    last = slice(max(0, Bsz - 3), Bsz)
+    ref, _, ssm_ref = blk.block_forward(np64(us[0][last]).reshape(-1, 1, d_model), oracle_params(b), conv_state=np64(conv0[last]),
+                                        ssm_state=np64(ssm0[last]))
+    for i in range(2):
+        out_f = b.step(us[i], st_f)
+        out_s = b.step(us[i], st_s, fused=False)
+        torch.cuda.synchronize()
+        assert st_f.ssm.initialized and st_s.ssm.initialized
+        assert rel_err(out_f, np64(out_s)) <= (1e-4 if dtype == torch.float32 else 5e-2), f"step {i}"
+        assert rel_err(st_f.ssm.state, np64(st_s.ssm.state)) <= (1e-5 if dtype == torch.float32 else 1e-2), f"step {i}: state"
+        assert rel_err(st_f.conv, np64(st_s.conv)) <= (1e-5 if dtype == torch.float32 else 2.0 ** -7 * 6), f"step {i}: conv"
+        if i == 0:
+            assert rel_err(out_f[last], ref[:, 0]) <= (1e-3 if dtype == torch.float32 else 1e-1)
+            assert rel_err(st_f.ssm.state[last], ssm_ref) <= (1e-3 if dtype == torch.float32 else 1e-1)
+
+
 def test_block_step_as_one_launch_refuses_what_it_does_not_take():
     b = Mamba2Block(d_model=64, nheads=8, headdim=32, dstate=64, seed=1)
     st = b.new_state(2, dtype=torch.float32)

@@ -191,8 +191,10 @@ def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups,
     return out
 
 
-# batches up to which one workgroup per stream (each reading both weight matrices whole) beats the stage kernels
-FUSED_STEP_MAX_BATCH = 64
+# batches up to which the one-launch step (each workgroup reading both weight matrices whole) beats the stage kernels and the
+# BLAS.  Eager, d_model 256, bf16 / float32 in us: 512 streams 21 / 24 against 104 / 104 (the host's issue of six launches),
+# 1 024 streams 41 / 48; replayed as a graph 22 / 25 against 32 / 39, and 42 / 50 against 44 / 49.
+FUSED_STEP_MAX_BATCH = 1024
 
 
 def block_step_supported(u_t: torch.Tensor, d_inner: int, dstate: int) -> bool:
@@ -526,8 +528,10 @@ class Mamba2Block:
         if fused is None:
             fused = u_t.shape[0] <= FUSED_STEP_MAX_BATCH and block_step_supported(u_t, self.d_inner, self.N)
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
-            return block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
-                              self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
+            out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
+                             self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
+            state.ssm.initialized = True    # as `SsdStreamState.step` leaves it
+            return out
         zxbcdt = torch.matmul(u_t, w_in.t()).unsqueeze(1).contiguous()
         x, Bm, Cm, dt, _ = block_pre(zxbcdt, self.conv_w, self.conv_b, self.dt_bias, self.H, self.P, self.N,
                                      self.G, conv_state=state.conv, conv_state_out=state.conv)  # in place
