@@ -163,6 +163,26 @@ def test_post_scan_with_out_projection_in_one_kernel(shape, padded):
     assert (np.abs(o - two) <= 2 * (1.05 * 2.0 ** -8 * mag + 2.0 ** -8 * np.abs(ref)) + 1e-30).all()
 
 
+@pytest.mark.parametrize("rows,n", [(2517, 648), (16385, 648), (33000, 648), (67423, 648), (131073, 648), (300007, 648),
+                                    (65537, 256), (180001, 72)])
+def test_projections_do_not_depend_on_how_rows_and_columns_are_cut(rows, n):
+    """A row's product is the same bits whatever ranges of rows and blocks of columns the row count makes the two kernels
+    choose: the rows around the ends of ranges, as a batch of their own, against the whole."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    u = torch.randn(rows, 256, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(n, 256, generator=g, device="cuda") / 16).to(torch.bfloat16)
+    pick = torch.unique(torch.tensor([r for e in (0, 256, 512, 1024, 2048, rows // 256 * 256, rows) for r in range(e - 3, e + 3)
+                                      if 0 <= r < rows], device="cuda"))
+    assert torch.equal(block_proj(u, w)[pick], block_proj(u[pick], w))
+    if n <= 256:
+        H, P, N, G = 8, 32, 64, 1
+        y = torch.randn(1, rows, H, P, generator=g, device="cuda").to(torch.bfloat16)
+        z = torch.randn(1, rows, 2 * H * P + 2 * G * N + H, generator=g, device="cuda").to(torch.bfloat16)
+        nw = torch.rand(H * P, generator=g, device="cuda") + 0.5
+        whole = block_post_proj(y, z, nw, w, H, P, N, G)
+        assert torch.equal(whole[:, pick], block_post_proj(y[:, pick], z[:, pick], nw, w, H, P, N, G))
+
+
 @pytest.mark.parametrize("rows,k,n", [(300, 256, 648), (4099, 256, 256), (2049, 128, 168), (33, 256, 8), (5000, 256, 768)])
 def test_projection_into_padded_rows(rows, k, n):
     """pad_rows: the same numbers as the dense call, bit for bit, in rows a multiple of 64 elements apart; columns

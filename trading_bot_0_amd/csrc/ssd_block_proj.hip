@@ -340,8 +340,9 @@ static void proj_col_blocks(int out_features, int *col_blocks, int *block_cols) 
 // wave.  A compute unit holds one workgroup, so what counts is rounds of workgroups times the time of one.  Long
 // ranges pay the fill of w once for many rows, but at 16 384 rows (256 -> 648) eight tiles leave 40 workgroups for 256
 // compute units: 40.4 us, 14.6 with two tiles on blocks of 96 columns.  Times of a workgroup in us, alone on its compute
-// unit, fitted to sweeps of rows 512 .. 524 288 times columns 256 and 648 (the choice is within 6 % of the best of each):
-// one tile 4.5 + 0.5 per 32 columns, two 9 + 1.4, four 18 + 1.4, eight 34 + 1.6.
+// unit, fitted to sweeps of rows 512 .. 524 288 times columns 256 and 648: one tile 4.5 + 0.5 per 32 columns, two 9 + 1.4,
+// four 18 + 1.4, eight 34 + 1.6.  Rounds are counted per XCD: counted over the whole chip, 67 423 rows took one tile
+// per wave and a round more on one XCD in eight (256 -> 648 71 us, 47 as chosen now; 50 000 rows 45.7, 33.2).
 static hipError_t proj_split(long long rows, int out_features, int *col_blocks, int *block_cols, int *tiles) {
     int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -361,8 +362,10 @@ static hipError_t proj_split(long long rows, int out_features, int *col_blocks, 
         const int chunks = (std::max(bc, out_features - (cb - 1) * bc) + kProjChunk - 1) / kProjChunk;
         for (int k = 0; k < 4; ++k) {
             const long long per_group = 32LL * kProjWaves << k;
-            const long long groups = (rows + per_group - 1) / per_group * cb;
-            const float cost = (float)((groups + cus - 1) / cus) * (kFixed[k] + kPerChunk[k] * (float)chunks);
+            // (the column blocks of a range of rows stay on one of the 8 XCDs: its workgroups against its compute units)
+            const long long per_xcd = ((rows + per_group - 1) / per_group + 7) / 8 * cb;
+            const int xcd_cus = std::max(1, cus / 8);
+            const float cost = (float)((per_xcd + xcd_cus - 1) / xcd_cus) * (kFixed[k] + kPerChunk[k] * (float)chunks);
             if (best == 0.f || cost < best) {
                 best = cost;
                 *col_blocks = cb;
@@ -417,14 +420,15 @@ hipError_t launch_block_post_proj(const BlockShape &s, const void *y, const void
     if (!block_post_proj_supported(s, out_features) || out_ld < out_features || out_ld % 8 != 0) return hipErrorInvalidValue;
     const int K = s.H * s.P;
     const long long rows = (long long)s.B * s.L;
-    // rows per workgroup: up to kProjTiles tiles of 32 rows per wave, fewer when that would leave CUs without a
-    // workgroup (each workgroup stages all of w, as much as 256 of its rows, so more than one tile where rows allow)
+    // rows per workgroup: as many tiles of 32 rows per wave, up to kProjTiles, as make one round of workgroups (each
+    // workgroup stages all of w, as much as 256 of its rows; rounded down instead, 67 423 rows were two rounds of one tile:
+    // 44 us against 36 with two, 180 001 rows 79 against 61)
     int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = device_cu_count(dev, &cus);
     if (e != hipSuccess) return e;
     const long long per_tile = 32LL * kProjWaves;
-    const int tiles = (int)std::max<long long>(1, std::min<long long>(kProjTiles, rows / (per_tile * cus)));
+    const int tiles = (int)std::max<long long>(1, std::min<long long>(kProjTiles, (rows + per_tile * cus - 1) / (per_tile * cus)));
     // Where one tile per wave still leaves compute units idle, the columns are cut too, in up to eight blocks of 32 (each
     // gates its rows anew; staging w and the products shrink): 16 384 rows, 256 -> 256, in us with 1, 2, 4, 8 blocks:
     // 20.7, 17.5, 17.0, 26.3 (256 workgroups are a round); 8 192 rows 19.6, 16.4, 15.7, 14.1.
