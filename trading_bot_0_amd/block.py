@@ -116,17 +116,16 @@ def block_pre(zxbcdt, conv_w, conv_b, dt_bias, nheads, headdim, dstate, ngroups,
     ssd._require(dt_bias, "dt_bias", (H,), torch.float32)
     if conv_state is not None:
         ssd._require(conv_state, "conv_state", (Bsz, d_conv - 1, C), dtype)
-    dev = zxbcdt.device
-    x = torch.empty((Bsz, L, H, P), dtype=dtype, device=dev)
-    Bm = torch.empty((Bsz, L, G, N), dtype=dtype, device=dev)
-    Cm = torch.empty((Bsz, L, G, N), dtype=dtype, device=dev)
-    dt = torch.empty((Bsz, L, H), dtype=dtype, device=dev)
+    x = zxbcdt.new_empty((Bsz, L, H, P))
+    Bm = zxbcdt.new_empty((Bsz, L, G, N))
+    Cm = zxbcdt.new_empty((Bsz, L, G, N))
+    dt = zxbcdt.new_empty((Bsz, L, H))
     new_state = None
     if conv_state_out is not None:
         ssd._require(conv_state_out, "conv_state_out", (Bsz, d_conv - 1, C), dtype)
         new_state, return_conv_state = conv_state_out, True
     elif return_conv_state:
-        new_state = torch.empty((Bsz, d_conv - 1, C), dtype=dtype, device=dev)
+        new_state = zxbcdt.new_empty((Bsz, d_conv - 1, C))
     if reset is not None:
         if reset.dtype == torch.bool:
             reset = reset.view(torch.uint8)
@@ -183,7 +182,7 @@ def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups,
     ssd._require(norm_w, "norm_w", (H * P,), torch.float32)
     if weight.dim() != 2 or weight.shape[1] != H * P or not weight.is_contiguous():
         raise ValueError(f"weight must be contiguous [out_features, {H * P}], got {tuple(weight.shape)}")
-    out = torch.empty((Bsz, L, weight.shape[0]), dtype=torch.bfloat16, device=zxbcdt.device)
+    out = zxbcdt.new_empty((Bsz, L, weight.shape[0]))
     dims = SsdBlockDims(Bsz, L, H, P, N, G, 4, ld)
     ssd._check(lib, lib.ssd_block_post_proj_fwd(byref(dims), ssd.SSD_DTYPE_BF16, y.data_ptr(), zxbcdt.data_ptr(),
                                                 norm_w.data_ptr(), c_float(eps), weight.data_ptr(), weight.shape[0], 0,
@@ -229,7 +228,7 @@ def block_step(u_t, w_in, conv_w, conv_b, dt_bias, A, D, norm_w, w_out, conv_sta
     ssd._require(conv_state, "conv_state", (Bsz, d_conv - 1, C), dtype)
     ssd._require(ssm_state, "ssm_state", (Bsz, H, P, N), torch.float32)
     if out is None:
-        out = torch.empty((Bsz, d_model), dtype=dtype, device=u_t.device)
+        out = u_t.new_empty((Bsz, d_model))
     else:
         ssd._require(out, "out", (Bsz, d_model), dtype)
     dims = SsdBlockDims(Bsz, 1, H, P, N, G, d_conv, 0)
@@ -272,8 +271,8 @@ def block_post_bwd(y, zxbcdt, norm_w, dout, dzxbcdt, nheads, headdim, dstate, ng
     ssd._require(y, "y", (Bsz, L, H, P), y.dtype)
     ssd._require(dout, "dout", (Bsz, L, H * P), dtype)
     ssd._require(norm_w, "norm_w", (H * P,), torch.float32)
-    dy = torch.empty((Bsz, L, H, P), dtype=dtype, device=zxbcdt.device)
-    dnorm_w = torch.empty(H * P, dtype=torch.float32, device=zxbcdt.device)
+    dy = zxbcdt.new_empty((Bsz, L, H, P))
+    dnorm_w = zxbcdt.new_empty(H * P, dtype=torch.float32)
     if workspace is None:
         workspace = block_bwd_workspace(Bsz, L, H, P, N, G, d_conv, dtype, zxbcdt.device)
     dims = SsdBlockDims(Bsz, L, H, P, N, G, d_conv, ld)
@@ -314,13 +313,12 @@ def block_pre_bwd(zxbcdt, conv_w, conv_b, dt_bias, dx, dB, dC, ddt, dzxbcdt, nhe
         if reset.dtype == torch.bool:
             reset = reset.view(torch.uint8)
         ssd._require(reset, "reset", (Bsz, L), torch.uint8)
-    dev = zxbcdt.device
-    dconv_w = torch.empty((C, d_conv), dtype=torch.float32, device=dev)
-    dconv_b = torch.empty(C, dtype=torch.float32, device=dev)
-    ddt_bias = torch.empty(H, dtype=torch.float32, device=dev)
-    dstate = torch.empty((Bsz, d_conv - 1, C), dtype=dtype, device=dev) if need_dconv_state else None
+    dconv_w = zxbcdt.new_empty((C, d_conv), dtype=torch.float32)
+    dconv_b = zxbcdt.new_empty(C, dtype=torch.float32)
+    ddt_bias = zxbcdt.new_empty(H, dtype=torch.float32)
+    dstate = zxbcdt.new_empty((Bsz, d_conv - 1, C)) if need_dconv_state else None
     if workspace is None:
-        workspace = block_bwd_workspace(Bsz, L, H, P, N, G, d_conv, dtype, dev)
+        workspace = block_bwd_workspace(Bsz, L, H, P, N, G, d_conv, dtype, zxbcdt.device)
     dims = SsdBlockDims(Bsz, L, H, P, N, G, d_conv, ld)
     ssd._check(lib, lib.ssd_block_pre_bwd(byref(dims), code, zxbcdt.data_ptr(), conv_w.data_ptr(), conv_b.data_ptr(),
                                           dt_bias.data_ptr(), ssd._ptr(conv_state), ssd._ptr(reset), dx.data_ptr(),
@@ -352,7 +350,7 @@ def block_proj(u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) ->
     rows = u.numel() // u.shape[-1]
     width = weight.shape[0]
     ld = (width + 63) // 64 * 64 if pad_rows else width
-    out = torch.empty(u.shape[:-1] + (ld,), dtype=torch.bfloat16, device=u.device)
+    out = u.new_empty(u.shape[:-1] + (ld,))
     ssd._check(lib, lib.ssd_block_proj_fwd(rows, u.shape[-1], width, ld, ssd.SSD_DTYPE_BF16, u.data_ptr(),
                                            weight.data_ptr(), out.data_ptr(), ssd._stream_ptr(u)))
     return out[..., :width] if ld != width else out
@@ -460,6 +458,7 @@ class Mamba2Block:
         act = u.dtype
         E = in_proj_width(self.H, self.P, self.N, self.G)
         w_in, w_out = self._weights(act)
+        A = self.A
         dout2 = dout.reshape(Bsz * L, self.d_model)
         dyn = self._project(dout2, self._out_proj_transposed(act)).view(Bsz, L, self.d_inner)
         # (a forward that ran gate, norm and out-projection as one kernel kept no normalised rows: post_bwd writes them)
@@ -472,7 +471,7 @@ class Mamba2Block:
         dy, dnorm_w = block_post_bwd(y, zxbcdt, self.norm_w, dyn, dzx, self.H, self.P, self.N, self.G, self.eps, workspace=ws,
                                      d_conv=self.d_conv, yn_out=yn_new)
         dout_proj = _weight_gradient(dout2, (yn if yn is not None else yn_new).reshape(Bsz * L, self.d_inner))
-        g = ssd.ssd_chunk_scan_backward(x, dt, self.A, Bm, Cm, self.D, dy, chunk=self.chunk, reset=reset)
+        g = ssd.ssd_chunk_scan_backward(x, dt, A, Bm, Cm, self.D, dy, chunk=self.chunk, reset=reset)
         dconv_w, dconv_b, ddt_bias, _ = block_pre_bwd(zxbcdt, self.conv_w, self.conv_b, self.dt_bias, g["dx"], g["dB"],
                                                       g["dC"], g["ddt"], dzx, self.H, self.P, self.N, self.G, reset=reset,
                                                       workspace=ws)
@@ -480,15 +479,16 @@ class Mamba2Block:
         du = torch.matmul(dz2, w_in).view(Bsz, L, self.d_model)
         din_proj = _weight_gradient(dz2, u.reshape(Bsz * L, self.d_model))
         return dict(du=du, din_proj=din_proj, dconv_w=dconv_w, dconv_b=dconv_b, ddt_bias=ddt_bias, dA=g["dA"],
-                    dA_log=g["dA"] * self.A, dD=g["dD"], dnorm_w=dnorm_w, dout_proj=dout_proj)
+                    dA_log=g["dA"] * A, dD=g["dD"], dnorm_w=dnorm_w, dout_proj=dout_proj)
 
     def _project(self, u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) -> torch.Tensor:
         """u . weight^T in the activation dtype: the library's kernel where it takes the shape (bf16, in_features 128
-        or 256, a tall u), else the BLAS behind torch.  Measured crossovers in us, library against BLAS: 256 -> 648
-        at 2 048 rows 6.7 / 6.7, 16 384 rows 14.6 / 24.9; 256 -> 256 at 8 192 rows 7.0 / 6.6, 16 384 rows 7.9 / 8.2."""
+        or 256), else the BLAS behind torch.  In us of the GPU, library against BLAS: 256 -> 648 at 2 048 rows 6.7 / 6.7, 16 384
+        rows 14.6 / 24.9; 256 -> 256 at 8 192 rows 7.0 / 6.6, 16 384 rows 7.9 / 8.2; and of the host's time to issue it 8
+        against 20, which is what counts at few rows."""
         w = weight.to(u.dtype)
         u = u.contiguous()
-        if block_proj_supported(u, w) and u.numel() // u.shape[-1] >= (2048 if w.shape[0] > 256 else 16384):
+        if block_proj_supported(u, w):
             return block_proj(u, w.contiguous(), pad_rows=pad_rows)
         return torch.matmul(u, w.t()).contiguous()
 
