@@ -275,6 +275,16 @@ int ssd_block_pre_reset_fwd(const ssd_block_dims *dims, int dtype, const void *z
 int ssd_block_proj_fwd(int64_t rows, int64_t in_features, int64_t out_features, int64_t out_ld, int dtype, const void *u,
                        const void *w, void *out, void *hip_stream);
 
+/* Weight gradient of a projection: out [a_features, b_features] (float32) = sum over rows of a[r]^T b[r], with
+ * a [rows, a_features] (rows a_ld elements apart: 0 = a_features, else at least that and a multiple of 8) and
+ * b [rows, b_features], bfloat16 (dtype 1), float32 accumulation in a fixed order; for out = u . w^T it is dw with
+ * a = dout and b = u.  a_features must be a multiple of 8 (at most 8 192) and b_features 128 or 256
+ * (SSD_ERR_UNSUPPORTED otherwise: use the caller's BLAS).  workspace: ssd_block_wgrad_workspace_bytes (may be 0 bytes, and
+ * workspace NULL then). */
+int ssd_block_wgrad_workspace_bytes(int64_t rows, int64_t a_features, int64_t b_features, size_t *out_bytes);
+int ssd_block_wgrad(int64_t rows, int64_t a_features, int64_t b_features, int64_t a_ld, int dtype, const void *a,
+                    const void *b, float *out, void *workspace, size_t workspace_bytes, void *hip_stream);
+
 /* out [B,L,H*P] = rmsnorm(y * silu(z)) * norm_w over the H*P channels of a timestep (z from zxbcdt). */
 int ssd_block_post_fwd(const ssd_block_dims *dims, int dtype, const void *y, const void *zxbcdt,
                        const float *norm_w, float eps, void *out, void *hip_stream);

@@ -239,3 +239,26 @@ def test_weight_gradient_slabs_against_float64(rows, e, ld, d):
     err = (np.abs(got.double().cpu().numpy() - ref) / scale).max()
     assert err <= 1e-3, f"{err:.3e}"
     assert torch.equal(got, _weight_gradient(a, bm)), "the same bits on a second run"
+
+
+@pytest.mark.parametrize("rows,E,ld,D", [(1, 648, 704, 256), (63, 256, 256, 256), (64, 8, 8, 128), (257, 648, 648, 256), (300, 264, 320, 128),
+                                         (4097, 648, 704, 256), (16384, 256, 256, 256), (72828, 648, 704, 256), (72829, 128, 136, 128)])
+def test_weight_gradient_of_a_projection(rows, E, ld, D):
+    """a^T b against float64, for row counts around a step of 64 rows, a split and the longest float32 sum, widths that leave the
+    last block of 128 outputs part or nearly all empty, and padded rows whose padding holds NaN.  Bound: products of bf16 are
+    exact in float32; no float32 sum is longer than 4 096 rows, whose rounding errors of random sign come to sqrt(4 096) 2^-24
+    = 2^-18 of the terms' magnitudes."""
+    from trading_bot_0_amd.block import block_wgrad
+    g = torch.Generator(device="cuda").manual_seed(rows + E)
+    buf = torch.full((rows, ld), float("nan"), dtype=torch.bfloat16, device="cuda")
+    buf[:, :E] = torch.randn(rows, E, generator=g, device="cuda").to(torch.bfloat16)
+    a, b = buf[:, :E], torch.randn(rows, D, generator=g, device="cuda").to(torch.bfloat16)
+    out = block_wgrad(a, b)
+    assert out.shape == (E, D) and out.dtype == torch.float32
+    ref = a.double().t().contiguous() @ b.double()
+    mag = a.double().abs().t().contiguous() @ b.double().abs()
+    over = (out.double() - ref).abs() - 2.0 ** -18 * mag
+    assert torch.isfinite(out).all() and over.max().item() <= 0, f"over the bound by {over.max().item():.3e}"
+    assert torch.equal(out, block_wgrad(a, b))
+    with pytest.raises(ValueError):
+        block_wgrad(a, b[:, : D - 8].contiguous())

@@ -35,6 +35,8 @@ def _lib():
         lib.ssd_block_pre_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, P, P, P, P, P, P, P, P]
         lib.ssd_block_post_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, P]
         lib.ssd_block_proj_fwd.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int, P, P, P, P]
+        lib.ssd_block_wgrad_workspace_bytes.argtypes = [c_int64, c_int64, c_int64, POINTER(c_size_t)]
+        lib.ssd_block_wgrad.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int, P, P, P, P, c_size_t, P]
         lib.ssd_block_post_proj_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, c_int64, c_int64, P, P]
         lib.ssd_block_post_proj_fwd.restype = c_int
         lib.ssd_block_step_fwd.argtypes = [POINTER(SsdBlockDims), c_int, c_int64, P, P, P, P, P, P, P, P, c_float, P, P, P, P, P]
@@ -54,9 +56,35 @@ def _lib():
     return lib
 
 
+def block_wgrad_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether `block_wgrad` takes these tensors (else the caller's BLAS does it)."""
+    return (a.is_cuda and a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16 and b.shape[1] in (128, 256)
+            and a.shape[1] % 8 == 0 and 0 < a.shape[1] <= 8192 and 0 < a.shape[0] < 2 ** 31 and a.stride(1) == 1
+            and a.stride(0) % 8 == 0 and a.stride(0) >= a.shape[1] and a.data_ptr() % 16 == 0 and b.is_contiguous()
+            and b.data_ptr() % 16 == 0)
+
+
+def block_wgrad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a^T b [E,D] in float32, summed over the rows of a [rows,E] (rows dense or evenly padded) and b [rows,D], bf16: the
+    weight gradient of a projection (a = the gradient of its output, b = its input)."""
+    lib = _lib()
+    if a.dim() != 2 or b.dim() != 2 or a.shape[0] != b.shape[0] or a.device != b.device or not block_wgrad_supported(a, b):
+        raise ValueError(f"block_wgrad does not take {tuple(a.shape)} {a.dtype} (strides {a.stride()}) and {tuple(b.shape)} {b.dtype}")
+    rows, E, D = a.shape[0], a.shape[1], b.shape[1]
+    need = c_size_t(0)
+    ssd._check(lib, lib.ssd_block_wgrad_workspace_bytes(rows, E, D, byref(need)))
+    ws = a.new_empty(need.value, dtype=torch.uint8) if need.value else None
+    out = a.new_empty((E, D), dtype=torch.float32)
+    ssd._check(lib, lib.ssd_block_wgrad(rows, E, D, a.stride(0), ssd.SSD_DTYPE_BF16, a.data_ptr(), b.data_ptr(), out.data_ptr(),
+                                        ssd._ptr(ws), need.value, ssd._stream_ptr(a)))
+    return out
+
+
 def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T b in float32 for tall a [rows, E] (its rows may be a view into wider ones) and b [rows, D]: a sum over all
-    rows of the batch and the sequence.  As one GEMM the BLAS behind torch sees a contraction hundreds of thousands
+    rows of the batch and the sequence.  bf16 with D 128 or 256 runs on the library's kernel (72 828 rows, 648 x 256 outputs:
+    59 us, the BLAS 151), except where the rows make 64 slabs or more for the BLAS behind torch (262 144 rows: 200, 150), as
+    everything else does: as one GEMM the BLAS behind torch sees a contraction hundreds of thousands
     long against outputs a few hundred wide and runs it at a fifth of its rate, so the rows are cut into equal slabs,
     multiplied as one batched GEMM with float32 outputs, and the slabs' products added in order (measured on MI355X,
     524 288 rows: 648 x 256 outputs 1 333 -> 232 us, 256 x 256 outputs 1 059 -> 129 us; the float32 partial products also
@@ -65,6 +93,8 @@ def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     slabs = 1
     while slabs < 128 and rows % (2 * slabs) == 0 and rows // (2 * slabs) >= 4096:
         slabs *= 2
+    if slabs < 64 and block_wgrad_supported(a, b):
+        return block_wgrad(a, b)
     if slabs == 1 or a.dtype == torch.float32:
         return torch.matmul(a.t(), b).float()
     a3 = a.unflatten(0, (slabs, rows // slabs))

@@ -966,6 +966,47 @@ int ssd_block_proj_fwd(int64_t rows, int64_t in_features, int64_t out_features, 
     return e == hipSuccess ? SSD_OK : hip_fail(e, "block projection launch");
 }
 
+static int check_wgrad(int64_t rows, int64_t a_features, int64_t b_features) {
+    if (rows <= 0 || a_features <= 0 || b_features <= 0)
+        return fail(SSD_ERR_INVALID, "ssd: weight gradient sizes must be positive, got %lld rows of %lld and %lld", (long long)rows,
+                    (long long)a_features, (long long)b_features);
+    if (a_features > 0x7fffffff || b_features > 0x7fffffff ||
+        !ssd::block_wgrad_supported(rows, (int)a_features, (int)b_features))
+        return fail(SSD_ERR_UNSUPPORTED,
+                    "ssd: the weight gradient needs a_features a multiple of 8 up to 8192, b_features 128 or 256 and fewer than "
+                    "2^31 rows, got %lld, %lld and %lld",
+                    (long long)a_features, (long long)b_features, (long long)rows);
+    return SSD_OK;
+}
+
+int ssd_block_wgrad_workspace_bytes(int64_t rows, int64_t a_features, int64_t b_features, size_t *out_bytes) {
+    if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
+    if (int rc = check_wgrad(rows, a_features, b_features)) return rc;
+    *out_bytes = ssd::block_wgrad_workspace_bytes(rows, (int)a_features, (int)b_features);
+    return SSD_OK;
+}
+
+int ssd_block_wgrad(int64_t rows, int64_t a_features, int64_t b_features, int64_t a_ld, int dtype, const void *a, const void *b,
+                    float *out, void *workspace, size_t workspace_bytes, void *hip_stream) {
+    if (dtype != SSD_DTYPE_BF16)
+        return fail(SSD_ERR_UNSUPPORTED, "ssd: the weight gradient takes dtype 1 (bfloat16), got %d", dtype);
+    if (int rc = check_wgrad(rows, a_features, b_features)) return rc;
+    if (a_ld == 0) a_ld = a_features;
+    if (a_ld < a_features || a_ld > 0x7fffffff || a_ld % 8 != 0)
+        return fail(SSD_ERR_INVALID, "ssd: a_ld must be 0 or at least a_features (%lld) and a multiple of 8, got %lld",
+                    (long long)a_features, (long long)a_ld);
+    REQUIRE_PTR(a);
+    REQUIRE_PTR(b);
+    REQUIRE_PTR(out);
+    OPTIONAL_PTR(workspace);
+    const size_t need = ssd::block_wgrad_workspace_bytes(rows, (int)a_features, (int)b_features);
+    if (workspace_bytes < need || (need > 0 && workspace == nullptr))
+        return fail(SSD_ERR_WORKSPACE, "ssd: weight gradient workspace has %zu bytes, %zu needed", workspace_bytes, need);
+    hipError_t e = ssd::launch_block_wgrad(rows, (int)a_features, (int)b_features, (int)a_ld, a, b, out, workspace,
+                                           (hipStream_t)hip_stream);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "weight gradient launch");
+}
+
 int ssd_block_bwd_workspace_bytes(const ssd_block_dims *dims, int dtype, size_t *out_bytes) {
     if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
     ssd::BlockShape s;

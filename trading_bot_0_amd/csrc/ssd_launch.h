@@ -129,6 +129,12 @@ bool block_supported(const BlockShape &s);
 bool block_proj_supported(long long rows, int in_features, int out_features);
 hipError_t launch_block_proj(long long rows, int in_features, int out_features, int out_ld, const void *u, const void *w,
                              void *out, hipStream_t st);
+// The projections' weight gradients: out [E, N] (float32) = a^T b over all rows, a [rows, E] (rows lda elements apart, a
+// multiple of 8) and b [rows, N] in bf16; E a multiple of 8, N 128 or 256.  workspace: the partial sums.
+bool block_wgrad_supported(long long rows, int E, int N);
+size_t block_wgrad_workspace_bytes(long long rows, int E, int N);
+hipError_t launch_block_wgrad(long long rows, int E, int N, int lda, const void *a, const void *b, float *out, void *workspace,
+                              hipStream_t st);
 hipError_t launch_block_pre(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w,
                             const float *conv_b, const float *dt_bias, const void *state_in, void *state_out,
                             const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t stream);
