@@ -4,8 +4,9 @@ encoder block sits in `patch_trunk` (`trading_bots/src/torch/model/trading_model
 `trading_bots/src/torch/model/blocks/gqa.rs:82-109`), with the conv's streaming state carried next to the SSM
 state the way the reference's `StreamState` carries its encoder memory (`trading_model.rs:56-75`).
 
-The two projections are torch matmuls (plain GEMMs); everything between them runs in libssd_hip: the pre-scan
-and post-scan kernels bound here and the scan / step of `ssd.py`.
+Everything runs in libssd_hip -- the projections, the pre-scan and post-scan kernels and the weight gradients bound here, the
+scan / step of `ssd.py` -- but the products its kernels do not take (float32, other widths; the gradient of the block's
+input), which are torch matmuls.
 """
 from __future__ import annotations
 
@@ -480,7 +481,7 @@ class Mamba2Block:
 
     def backward(self, ctx: dict, dout: torch.Tensor) -> dict:
         """Gradients of sum(out * dout) with respect to the input and every parameter, from the tensors `forward`
-        kept: two GEMMs per projection (torch), the library's post, scan and pre backward kernels between them.
+        kept: two products per projection, the library's post, scan and pre backward kernels between them.
         Returns du [B,L,d_model] and float32 din_proj, dconv_w, dconv_b, ddt_bias, dA, dA_log, dD, dnorm_w, dout_proj."""
         u, zxbcdt, y, yn, reset = ctx["u"], ctx["zxbcdt"], ctx["y"], ctx["yn"], ctx["reset"]
         x, Bm, Cm, dt = ctx["x"], ctx["Bm"], ctx["Cm"], ctx["dt"]

