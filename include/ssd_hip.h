@@ -294,8 +294,8 @@ int ssd_block_post_fwd(const ssd_block_dims *dims, int dtype, const void *y, con
  * never reach memory (the reference's counterpart is the output linear layer of its temporal mixer,
  * trading_bots/src/torch/model/blocks/gqa.rs:82-109).  bfloat16 only (dtype 1: y, zxbcdt, w and out bf16, float32
  * accumulation), H*P 128 or 256, out_features a multiple of 8 up to 256; SSD_ERR_UNSUPPORTED otherwise (run the two
- * stages).  Rounding differs from the two stages' by where it happens: the gated row and the weights times norm_w
- * are rounded to bf16 once each, the row's rsqrt factor is applied to the float32 sums. */
+ * stages).  The normalised row is rounded to bf16 once in front of the product, where ssd_block_post_fwd rounds what it
+ * stores; the two differ in the order in which a row's squares are added up. */
 int ssd_block_post_proj_fwd(const ssd_block_dims *dims, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
                             float eps, const void *w, int64_t out_features, int64_t out_ld, void *out, void *hip_stream);
 

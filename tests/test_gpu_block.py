@@ -133,7 +133,7 @@ def test_stages_take_padded_rows(shape, dtype):
 @pytest.mark.parametrize("padded", [False, True])
 def test_post_scan_with_out_projection_in_one_kernel(shape, padded):
     """rmsnorm(y silu(z)) norm_w . w^T as one kernel against the float64 value of the same bf16 inputs.  The kernel
-    rounds the gated row and the weights times norm_w to bf16 once each and the sum once more on the way out, so
+    rounds the normalised row to bf16 once and the sum once more on the way out, so
     every element lies within 2^-8 of the sum of its terms' magnitudes plus one bf16 rounding of itself -- a bound
     on rounding alone; a misplaced row, channel or factor is off by the terms' 2-norm, an order of magnitude more.
     Ragged row counts (rows past the last tile), column counts off the chunks of 32, rows of whole lines."""
@@ -161,6 +161,30 @@ def test_post_scan_with_out_projection_in_one_kernel(shape, padded):
     # and next to the two stages run one after the other (their bf16 roundings fall elsewhere, within the same bound)
     two = np64(block_proj(block_post(y, z, p["norm_w"], H, P, N, G), w)).reshape(Bsz * L, dm)
     assert (np.abs(o - two) <= 2 * (1.05 * 2.0 ** -8 * mag + 2.0 ** -8 * np.abs(ref)) + 1e-30).all()
+
+
+@pytest.mark.parametrize("rows,di", [(300, 256), (300, 128), (16384, 256), (140001, 256)])
+def test_fused_out_projection_rounds_the_row_as_the_post_stage_does(rows, di):
+    """Weights that are the identity matrix show the normalised rows that the product was formed from: bit for bit the
+    post stage's (one rounding, of v * rstd * norm_w), but for the two orders in which a row's squares are added up.  Those differ
+    by at most 256 float32 roundings, i.e. 2^-16 of the factor, and move an element to the neighbouring bf16 value only where it
+    lies that close to the middle between two: under 2^-7 of the elements.  With weights of any kind the error
+    against float64 is then the two stages' (1.22 times that with the norm's scale rounded once more, at scales spread by 0.2)."""
+    H, P, N, G = 8, di // 8, 64, 1
+    g = torch.Generator(device="cuda").manual_seed(rows + di)
+    y = torch.randn(1, rows, H, P, generator=g, device="cuda").to(torch.bfloat16)
+    z = torch.randn(1, rows, 2 * di + 2 * G * N + H, generator=g, device="cuda").to(torch.bfloat16)
+    nw = 1 + 0.2 * torch.randn(di, generator=g, device="cuda")
+    rows_post = block_post(y, z, nw, H, P, N, G)
+    rows_fused = block_post_proj(y, z, nw, torch.eye(di, device="cuda").to(torch.bfloat16), H, P, N, G)
+    off = (rows_fused.float() - rows_post.float()).abs()
+    assert (off <= 2.0 ** -7 * rows_post.float().abs()).all() and (off > 0).float().mean().item() <= 2.0 ** -7
+    w = (torch.randn(256, di, generator=g, device="cuda") / di ** 0.5).to(torch.bfloat16)
+    v = y.double().view(1, rows, di) * torch.nn.functional.silu(z[..., :di].double())
+    exact = (v * torch.rsqrt((v * v).mean(-1, keepdim=True) + 1e-5) * nw.double()) @ w.double().t().contiguous()
+    err = lambda o: ((o.double() - exact).norm() / exact.norm()).item()
+    one, two = err(block_post_proj(y, z, nw, w, H, P, N, G)), err(block_proj(rows_post, w))
+    assert one <= 1.02 * two, f"{one:.3e} against the two stages' {two:.3e}"
 
 
 @pytest.mark.parametrize("rows,n", [(2517, 648), (16385, 648), (33000, 648), (67423, 648), (131073, 648), (300007, 648),

@@ -170,11 +170,14 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
 // yn[m, k] = v[m, k] rsqrt(mean_k v[m, k]^2 + eps) norm_w[k], v = y silu(z) -- the normalised row never reaches
 // memory (it would be written by one kernel and read back by the next: two thirds of the bytes of a row's y and z).
 // A row of the inner width K (128 or 256 channels) is exactly the MFMA's K axis, which a lane pair (r, r + 32) holds
-// entirely in its operand fragments: the prologue turns a tile's rows of y and z into fragments of bf16(v) and the
-// pair's sum of squares; the norm's weights are folded into the staged matrix (w[n, k] norm_w[k], rounded to bf16)
-// and the row's rsqrt factor scales the accumulators, whose lanes hold one row each.  One workgroup takes all
-// out_features (at most 256) columns, so that the prologue runs once per row: its rows of w fill 132 KB of LDS, and a
-// wave's output tile covers 16 rows at a time to fit beside them.
+// entirely in registers: the prologue forms a tile's v in float32, the pair's sum of squares and then fragments of
+// bf16(yn), the only rounding in front of the product and the one block_post makes when it stores the row (with the norm's
+// weights folded into w instead, which rounds the weights once more, the result's error against float64 was 2.88e-3 where
+// it is 2.35e-3, at scales spread by 0.2 around one; 256 -> 256 in us, folded / here: 16 384 rows 17.5 / 16.7, 131 072 rows
+// 42 / 45, 524 288 rows 176 / 176).  v takes the registers of the pieces of y and z it is formed from; the norm's weights are
+// in LDS.  A workgroup takes all out_features (at most 256) columns where rows are many, so that the prologue runs once
+// per row: its rows of w fill 132 KB of LDS, and a wave's output tile covers 16 rows at a time to fit beside them; where rows
+// are few the columns are cut as well and each block of columns gates its rows anew (launch_block_post_proj).
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kPostProjMaxCols = 256;
 
@@ -187,6 +190,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     constexpr int kTileRowB = 64 * 2 + 16;
     __shared__ __attribute__((aligned(16))) unsigned char wsm[CH * kProjChunk * ROWB];
     __shared__ __attribute__((aligned(16))) unsigned char otile[kProjWaves][16 * kTileRowB];
+    __shared__ __attribute__((aligned(16))) float nw_s[K];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // (the column blocks of a range of rows are consecutive workgroups of one XCD, as in block_proj_kernel)
     const int xcd = blockIdx.x % 8, within = blockIdx.x / 8;
@@ -212,55 +216,64 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
         for (int ks = 0; ks < KS; ++ks) zq[ks] = *reinterpret_cast<const uint4 *>(zr + 16 * ks);
     };
     load_y(0);  // in flight while w is staged
-    {   // rows 0 .. 32 CH - 1 of w times norm_w, rounded to bf16 (rows past N repeat the last one: never stored)
+    const float nw_q = norm_w[min(tid, K - 1)];
+    {   // rows n0 .. n0 + 32 CH - 1 of w (rows past N repeat the last one: never stored)
         constexpr int PIECES = CH * kProjChunk * PPR;
         constexpr int FILL = (PIECES + NTHR - 1) / NTHR;
 #pragma unroll 4
         for (int i = 0; i < FILL; ++i) {
             const int p = min(tid + i * NTHR, PIECES - 1);
             const int row = p / PPR, piece = p % PPR;
-            const Pack8<__bf16> q = Pack8<__bf16>::load(w + (size_t)min(n0 + row, N - 1) * K + piece * 8);
-            const float4 na = *reinterpret_cast<const float4 *>(norm_w + piece * 8);
-            const float4 nb = *reinterpret_cast<const float4 *>(norm_w + piece * 8 + 4);
-            uint4 o;
-            o.x = pack_bf16x2(q.get(0) * na.x, q.get(1) * na.y);
-            o.y = pack_bf16x2(q.get(2) * na.z, q.get(3) * na.w);
-            o.z = pack_bf16x2(q.get(4) * nb.x, q.get(5) * nb.y);
-            o.w = pack_bf16x2(q.get(6) * nb.z, q.get(7) * nb.w);
-            *reinterpret_cast<uint4 *>(wsm + row * ROWB + piece * 16) = o;
+            *reinterpret_cast<uint4 *>(wsm + row * ROWB + piece * 16) =
+                *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + row, N - 1) * K + piece * 8);
         }
     }
+    if (tid < K) nw_s[tid] = nw_q;
     __syncthreads();
     unsigned char *tile = otile[wave];
     const __amdgpu_buffer_rsrc_t obuf = make_buffer(out + (size_t)row0 * ldo, (unsigned)min((long long)tiles * 32 * kProjWaves, M - row0) * (unsigned)ldo * 2u);
     const float inv_k = 1.f / (float)K;
 #pragma unroll 1
     for (int t = 0; t < tiles; ++t) {
-        // ---- prologue: this tile's rows of y and z -> fragments of bf16(y silu(z)) and the rows' rsqrt factor ----
+        // ---- prologue: this tile's rows of y and z -> fragments of the normalised rows ----
         load_z(t);
-        Frag<__bf16> uf[KS];
+        float v[KS][8];
         float ss = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const Pack8<__bf16> yy{yq[ks]}, zz{zq[ks]};
-            float v[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                v[i] = yy.get(i) * silu(zz.get(i));
-                ss += v[i] * v[i];
+                v[ks][i] = yy.get(i) * silu(zz.get(i));
+                ss += v[ks][i] * v[ks][i];
             }
-            uint4 o;
-            o.x = pack_bf16x2(v[0], v[1]);
-            o.y = pack_bf16x2(v[2], v[3]);
-            o.z = pack_bf16x2(v[4], v[5]);
-            o.w = pack_bf16x2(v[6], v[7]);
-            uf[ks].v = __builtin_bit_cast(bf16x8, o);
         }
         ss += __shfl_xor(ss, 32, 64);
         const float rstd = rsqrtf(ss * inv_k + eps);
+        Frag<__bf16> uf[KS];
+        int nw0 = 8 * half;
+        asm volatile("" : "+v"(nw0));  // (read per tile: hoisted out of the loop the weights would take 128 registers)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const float4 na = *reinterpret_cast<const float4 *>(nw_s + nw0 + 16 * ks);
+            const float4 nb = *reinterpret_cast<const float4 *>(nw_s + nw0 + 16 * ks + 4);
+            uint4 o;
+            o.x = pack_bf16x2(v[ks][0] * rstd * na.x, v[ks][1] * rstd * na.y);
+            o.y = pack_bf16x2(v[ks][2] * rstd * na.z, v[ks][3] * rstd * na.w);
+            o.z = pack_bf16x2(v[ks][4] * rstd * nb.x, v[ks][5] * rstd * nb.y);
+            o.w = pack_bf16x2(v[ks][6] * rstd * nb.z, v[ks][7] * rstd * nb.w);
+            // (formed here: left alone, the compiler reads all of the weights ahead and forms the fragments behind the next
+            // rows' requests, 91 spilled registers)
+            asm volatile("" : "+v"(o.x), "+v"(o.y), "+v"(o.z), "+v"(o.w));
+            uf[ks].v = __builtin_bit_cast(bf16x8, o);
+        }
         // the next tile's rows of y: requested before this tile's products and stores (loads and stores complete in
         // order per wave: requested behind the stores they would wait for those to reach memory)
         if (t + 1 < tiles) load_y(t + 1);
+        else {  // (named here, the pieces need no registers from their use above to this point)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) yq[ks] = make_uint4(0, 0, 0, 0);
+        }
         const unsigned trow = (unsigned)(t * (32 * kProjWaves) + wave * 32);
         const long long m0 = tile_row0(t);
 #pragma unroll
@@ -281,7 +294,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
                     acc[sub] = mma32(wf0, uf[ks], acc[sub]);
                     acc_odd = mma32(wf1, uf[ks + 1], acc_odd);
                 }
-                acc[sub] = (acc[sub] + acc_odd) * rstd;
+                acc[sub] = acc[sub] + acc_odd;
             }
             // acc[sub][4 vg + i] = out[m0 + r, 32 (c0 + sub) + 8 vg + 4 half + i]; the wave's tile holds 16 rows, so
             // the rows go out in two halves (rows r < 16, then the others)
