@@ -499,6 +499,45 @@ def test_block_step_for_many_streams(cfg, dtype):
             assert rel_err(st_f.ssm.state[last], ssm_ref) <= (1e-3 if dtype == torch.float32 else 1e-1)
 
 
+def _at_offset(t, elements):
+    """The same values, contiguous, starting that many elements into a flat buffer."""
+    flat = torch.zeros(t.numel() + elements, dtype=t.dtype, device=t.device)
+    flat[elements:] = t.reshape(-1)
+    return flat[elements:].view(t.shape)
+
+
+@pytest.mark.parametrize("rows", [(2, 30), (1, 9000), (3, 5500)])
+def test_block_takes_inputs_that_start_anywhere_in_a_buffer(rows):
+    """u and dout that are not aligned to 16 bytes (the library's kernels load 16 bytes at a time): the products that read them
+    run on the BLAS, everything behind is as for aligned ones.  Between the two in-projections, whose sums run in other
+    orders, elements of zxbcdt differ by a bf16 rounding now and then, which travels through the block: the block tests' bar."""
+    b = Mamba2Block(d_model=256, nheads=8, headdim=32, dstate=64, seed=4)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    u = torch.randn(*rows, 256, generator=g, device="cuda").to(torch.bfloat16)
+    dout = torch.randn(*rows, 256, generator=g, device="cuda").to(torch.bfloat16)
+    ref, ctx = b.forward(u, save_for_backward=True)
+    ref_g = b.backward(ctx, dout)
+    for off in (1, 4):
+        out, ctx = b.forward(_at_offset(u, off), save_for_backward=True)
+        assert rel_err(out, np64(ref)) <= 1e-1
+        got = b.backward(ctx, _at_offset(dout, off))
+        for k, v in got.items():
+            assert (v.double() - ref_g[k].double()).norm() <= 1e-1 * ref_g[k].double().norm(), k
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_block_step_takes_inputs_that_start_anywhere_in_a_buffer(dtype):
+    """The same for a step of more streams than compute units, and for weights that are views (the step's stage kernels and the
+    BLAS take any address; bars as in test_block_step_as_one_launch)."""
+    b = Mamba2Block(d_model=256, nheads=8, headdim=32, dstate=64, seed=4)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    u = torch.randn(70, 256, generator=g, device="cuda").to(dtype)
+    ref = b.step(u, b.new_state(70, dtype=dtype))
+    assert rel_err(b.step(_at_offset(u, 1), b.new_state(70, dtype=dtype)), np64(ref)) <= (1e-4 if dtype == torch.float32 else 5e-2)
+    b.in_proj, b.out_proj = _at_offset(b.in_proj, 1), _at_offset(b.out_proj, 1)
+    assert rel_err(b.step(u, b.new_state(70, dtype=dtype)), np64(ref)) <= (1e-4 if dtype == torch.float32 else 5e-2)
+
+
 def test_block_step_as_one_launch_refuses_what_it_does_not_take():
     b = Mamba2Block(d_model=64, nheads=8, headdim=32, dstate=64, seed=1)
     st = b.new_state(2, dtype=torch.float32)

@@ -192,10 +192,16 @@ def block_post(y, zxbcdt, norm_w, nheads, headdim, dstate, ngroups, eps=1e-5):
     return out
 
 
+def _aligned(*tensors: torch.Tensor) -> bool:
+    """Whether the kernels' 16-byte loads can read these contiguous tensors (one that starts elsewhere in a flat buffer goes to
+    the BLAS, which takes any address)."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def block_post_proj_supported(y: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `block_post_proj` takes these tensors (else `block_post`, then the projection)."""
     return (y.is_cuda and y.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2
-            and weight.shape[1] in (128, 256) and weight.shape[0] % 8 == 0 and weight.shape[0] <= 256)
+            and weight.shape[1] in (128, 256) and weight.shape[0] % 8 == 0 and weight.shape[0] <= 256 and _aligned(y, weight))
 
 
 def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups, eps=1e-5):
@@ -230,7 +236,7 @@ FUSED_STEP_MAX_BATCH = 1024
 def block_step_supported(u_t: torch.Tensor, d_inner: int, dstate: int) -> bool:
     """Whether `block_step` takes this step (else the stage kernels, one launch each)."""
     return (u_t.is_cuda and u_t.dtype in (torch.bfloat16, torch.float32) and u_t.dim() == 2
-            and u_t.shape[1] in (128, 256) and d_inner in (128, 256) and dstate % 16 == 0)
+            and u_t.shape[1] in (128, 256) and d_inner in (128, 256) and dstate % 16 == 0 and _aligned(u_t))
 
 
 def block_step(u_t, w_in, conv_w, conv_b, dt_bias, A, D, norm_w, w_out, conv_state, ssm_state, nheads, headdim, dstate,
@@ -363,7 +369,7 @@ def block_pre_bwd(zxbcdt, conv_w, conv_b, dt_bias, dx, dB, dC, ddt, dzxbcdt, nhe
 def block_proj_supported(u: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `block_proj` takes this product (else the caller's BLAS does it)."""
     return (u.is_cuda and u.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and u.shape[-1] in (128, 256)
-            and weight.shape[0] % 8 == 0 and u.numel() > 0)
+            and weight.shape[0] % 8 == 0 and u.numel() > 0 and _aligned(u, weight))
 
 
 def block_proj(u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) -> torch.Tensor:
@@ -517,10 +523,10 @@ class Mamba2Block:
         or 256), else the BLAS behind torch.  In us of the GPU, library against BLAS: 256 -> 648 at 2 048 rows 6.7 / 6.7, 16 384
         rows 14.6 / 24.9; 256 -> 256 at 8 192 rows 7.0 / 6.6, 16 384 rows 7.9 / 8.2; and of the host's time to issue it 8
         against 20, which is what counts at few rows."""
-        w = weight.to(u.dtype)
+        w = weight.to(u.dtype).contiguous()
         u = u.contiguous()
         if block_proj_supported(u, w):
-            return block_proj(u, w.contiguous(), pad_rows=pad_rows)
+            return block_proj(u, w, pad_rows=pad_rows)
         return torch.matmul(u, w.t()).contiguous()
 
     def _weights(self, dtype: torch.dtype):
@@ -557,7 +563,8 @@ class Mamba2Block:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         w_in, w_out = self._weights(u_t.dtype)
         if fused is None:
-            fused = u_t.shape[0] <= FUSED_STEP_MAX_BATCH and block_step_supported(u_t, self.d_inner, self.N)
+            fused = (u_t.shape[0] <= FUSED_STEP_MAX_BATCH and _aligned(w_in, w_out)
+                     and block_step_supported(u_t.contiguous(), self.d_inner, self.N))
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
             out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
                              self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
