@@ -538,6 +538,17 @@ def test_block_step_takes_inputs_that_start_anywhere_in_a_buffer(dtype):
     assert rel_err(b.step(u, b.new_state(70, dtype=dtype)), np64(ref)) <= (1e-4 if dtype == torch.float32 else 5e-2)
 
 
+@pytest.mark.parametrize("batch", [3, 70])
+def test_block_step_of_more_channels_than_one_launch_holds(batch):
+    """32 groups of a 128-wide state: the one-launch step's vectors (in-projection, conv, state rows) come to 71 KB of LDS, and
+    it takes 64; the step runs on the stage kernels."""
+    b = Mamba2Block(d_model=128, nheads=32, headdim=8, dstate=128, ngroups=32, seed=2)
+    u = torch.randn(batch, 128, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").to(torch.bfloat16)
+    with pytest.raises(SsdError):
+        b.step(u, b.new_state(batch), fused=True)
+    assert torch.equal(b.step(u, b.new_state(batch)), b.step(u, b.new_state(batch), fused=False))
+
+
 def test_block_step_as_one_launch_refuses_what_it_does_not_take():
     b = Mamba2Block(d_model=64, nheads=8, headdim=32, dstate=64, seed=1)
     st = b.new_state(2, dtype=torch.float32)

@@ -10,6 +10,7 @@ input), which are torch matmuls.
 """
 from __future__ import annotations
 
+import functools
 import math
 from ctypes import POINTER, Structure, byref, c_float, c_int, c_int64, c_size_t, c_void_p
 from dataclasses import dataclass
@@ -231,6 +232,15 @@ def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups,
 # BLAS.  Eager, d_model 256, bf16 / float32 in us: 512 streams 21 / 24 against 104 / 104 (the host's issue of six launches),
 # 1 024 streams 41 / 48; replayed as a graph 22 / 25 against 32 / 39, and 42 / 50 against 44 / 49.
 FUSED_STEP_MAX_BATCH = 1024
+
+
+@functools.lru_cache(maxsize=64)
+def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
+    """The largest batch whose step is taken as one launch (0: the launch's vectors, as the library lays them out, do not fit the
+    64 KB of LDS that it asks for)."""
+    d_inner, E = nheads * headdim, in_proj_width(nheads, headdim, dstate, ngroups)
+    vectors = d_model + E + (E - d_inner - nheads) + (nheads + 3) // 4 * 4 + d_inner + 16
+    return FUSED_STEP_MAX_BATCH if 4 * vectors <= 64 * 1024 else 0
 
 
 def block_step_supported(u_t: torch.Tensor, d_inner: int, dstate: int) -> bool:
@@ -563,7 +573,7 @@ class Mamba2Block:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         w_in, w_out = self._weights(u_t.dtype)
         if fused is None:
-            fused = (u_t.shape[0] <= FUSED_STEP_MAX_BATCH and _aligned(w_in, w_out)
+            fused = (u_t.shape[0] <= _step_max_batch(self.d_model, self.H, self.P, self.N, self.G) and _aligned(w_in, w_out)
                      and block_step_supported(u_t.contiguous(), self.d_inner, self.N))
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
             out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
