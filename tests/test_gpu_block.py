@@ -549,6 +549,21 @@ def test_block_step_of_more_channels_than_one_launch_holds(batch):
     assert torch.equal(b.step(u, b.new_state(batch)), b.step(u, b.new_state(batch), fused=False))
 
 
+@pytest.mark.parametrize("state,groups,limit", [(64, 1, 1024), (32, 1, 256), (128, 1, 256), (64, 2, 256)])
+def test_block_step_route_by_batch_and_kernel(state, groups, limit, monkeypatch):
+    """Up to which batch a step is one launch: by the kernel that runs for the shape (776 rows of w_in with two groups of 64)."""
+    b = Mamba2Block(d_model=256, nheads=8, headdim=32, dstate=state, ngroups=groups, seed=2)
+    u = torch.randn(limit + 1, 256, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").to(torch.bfloat16)
+    from trading_bot_0_amd import block as module
+    calls, launch = [], module.block_step
+    monkeypatch.setattr(module, "block_step", lambda *a, **k: calls.append(a[0].shape[0]) or launch(*a, **k))
+    for batch, fused in ((limit, True), (limit + 1, False)):
+        out = b.step(u[:batch], b.new_state(batch))
+        assert calls == ([limit] if fused else []), f"{batch} streams"
+        assert torch.equal(out, b.step(u[:batch], b.new_state(batch), fused=fused))
+        calls.clear()
+
+
 def test_block_step_as_one_launch_refuses_what_it_does_not_take():
     b = Mamba2Block(d_model=64, nheads=8, headdim=32, dstate=64, seed=1)
     st = b.new_state(2, dtype=torch.float32)

@@ -229,18 +229,26 @@ def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups,
 
 
 # batches up to which the one-launch step (each workgroup reading both weight matrices whole) beats the stage kernels and the
-# BLAS.  Eager, d_model 256, bf16 / float32 in us: 512 streams 21 / 24 against 104 / 104 (the host's issue of six launches),
-# 1 024 streams 41 / 48; replayed as a graph 22 / 25 against 32 / 39, and 42 / 50 against 44 / 49.
+# BLAS, in us with d_model 256, bf16 / float32, against those.  The overlapped kernel (64-wide state, at most 768 rows of w_in):
+# eager 512 streams 21 / 24 against 92 / 92 (the host's issue of six launches), 1 024 40 / 48; replayed by `graphed_step` 512
+# streams 25 / 28 against 36 / 41, 1 024 43 / 49 against 47 / 53.
 FUSED_STEP_MAX_BATCH = 1024
+# ... and the kernel for other shapes: one round of workgroups.  Replayed, 256 streams: state 32 21 / 24 against 35 / 88, state 128
+# 30 / 32 against 43 / 100, two groups of 64 24 / 27 against 36 / 91; 384 streams 34 / 36 against 29 / 33, 47 / 50 against 41 / 46,
+# 38 / 41 against 32 / 37; 1 024 65 / 70 against 38 / 43, 94 / 99 against 69 / 75, 77 / 82 against 49 / 55.  (Eager, where the
+# stage kernels cost 92, it would win up to some 768; a step captured by the caller is not known to be one.)
+FUSED_STEP_MAX_BATCH_OTHER = 256
 
 
 @functools.lru_cache(maxsize=64)
 def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
-    """The largest batch whose step is taken as one launch (0: the launch's vectors, as the library lays them out, do not fit the
-    64 KB of LDS that it asks for)."""
+    """The largest batch whose step is taken as one launch, by the kernel that the library runs for the shape (0: the launch's
+    vectors, as it lays them out, do not fit the 64 KB of LDS that it asks for)."""
     d_inner, E = nheads * headdim, in_proj_width(nheads, headdim, dstate, ngroups)
     vectors = d_model + E + (E - d_inner - nheads) + (nheads + 3) // 4 * 4 + d_inner + 16
-    return FUSED_STEP_MAX_BATCH if 4 * vectors <= 64 * 1024 else 0
+    if 4 * vectors > 64 * 1024:
+        return 0
+    return FUSED_STEP_MAX_BATCH if dstate == 64 and E <= 768 else FUSED_STEP_MAX_BATCH_OTHER
 
 
 def block_step_supported(u_t: torch.Tensor, d_inner: int, dstate: int) -> bool:
@@ -567,8 +575,8 @@ class Mamba2Block:
 
     def step(self, u_t: torch.Tensor, state: Mamba2StreamState, fused: Optional[bool] = None) -> torch.Tensor:
         """One timestep for every stream: u_t [B,d_model] -> [B,d_model]; advances `state` in place.  `fused`: run the
-        step as one launch (default: for batches up to FUSED_STEP_MAX_BATCH of shapes the fused kernel takes) or as the
-        stage kernels with the projections on the BLAS behind torch."""
+        step as one launch (default: where the fused kernel takes the shape, up to 1 024 or 256 streams) or as the stage kernels
+        with the projections on the BLAS behind torch."""
         if u_t.dim() != 2 or u_t.shape[1] != self.d_model:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         w_in, w_out = self._weights(u_t.dtype)
