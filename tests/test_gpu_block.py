@@ -207,6 +207,17 @@ def test_projections_do_not_depend_on_how_rows_and_columns_are_cut(rows, n):
         assert torch.equal(whole[:, pick], block_post_proj(y[:, pick], z[:, pick], nw, w, H, P, N, G))
 
 
+@pytest.mark.parametrize("rows,n", [(16385, 648), (107479, 64), (76265, 384), (393246, 144)])
+def test_projections_of_128_channels_do_not_depend_on_how_they_are_cut(rows, n):
+    """The same for u of 128 channels, whose cuts have prices of their own (one, two, four and eight tiles per wave)."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    u = torch.randn(rows, 128, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(n, 128, generator=g, device="cuda") / 16).to(torch.bfloat16)
+    pick = torch.unique(torch.tensor([r for e in (0, 256, 512, 1024, 2048, rows // 256 * 256, rows) for r in range(e - 3, e + 3)
+                                      if 0 <= r < rows], device="cuda"))
+    assert torch.equal(block_proj(u, w)[pick], block_proj(u[pick], w))
+
+
 @pytest.mark.parametrize("rows,k,n", [(300, 256, 648), (4099, 256, 256), (2049, 128, 168), (33, 256, 8), (5000, 256, 768)])
 def test_projection_into_padded_rows(rows, k, n):
     """pad_rows: the same numbers as the dense call, bit for bit, in rows a multiple of 64 elements apart; columns

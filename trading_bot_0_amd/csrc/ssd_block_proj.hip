@@ -352,17 +352,23 @@ static void proj_col_blocks(int out_features, int *col_blocks, int *block_cols) 
 // How the product is cut over workgroups: the columns in blocks, the rows in ranges of 256 times 1, 2, 4 or 8 tiles per
 // wave.  A compute unit holds one workgroup, so what counts is rounds of workgroups times the time of one.  Long
 // ranges pay the fill of w once for many rows, but at 16 384 rows (256 -> 648) eight tiles leave 40 workgroups for 256
-// compute units: 40.4 us, 14.6 with two tiles on blocks of 96 columns.  Times of a workgroup in us, alone on its compute
-// unit, fitted to sweeps of rows 512 .. 524 288 times columns 256 and 648: one tile 4.5 + 0.5 per 32 columns, two 9 + 1.4,
-// four 18 + 1.4, eight 34 + 1.6.  Rounds are counted per XCD: counted over the whole chip, 67 423 rows took one tile
-// per wave and a round more on one XCD in eight (256 -> 648 71 us, 47 as chosen now; 50 000 rows 45.7, 33.2).
-static hipError_t proj_split(long long rows, int out_features, int *col_blocks, int *block_cols, int *tiles) {
+// compute units: 40.5 us, 15.1 with two tiles on blocks of 96 columns.  A workgroup is priced at kFixed + kPerChunk per 32
+// columns, for each width of u and number of tiles; the prices (in about us, but no workgroup's times) are those whose choice
+// came out best over 242 pairs of rows (300 .. 524 288) and columns (64 .. 1 120) with every cut timed; on 90 further pairs the
+// choice is 1.4 % (256) and 1.9 % (128) slower than the best cut on average, and than eight tiles on the widest blocks by 7 %
+// at most.  Of two cuts at one price the longer range is taken.  Rounds are counted per XCD: counted over the whole chip, 67 423 rows (256 -> 648) took
+// one tile and a round more on one XCD in eight (71 us, 45.5 with eight tiles, as chosen now; 50 000 rows 45.7, 33.0).
+static hipError_t proj_split(long long rows, int in_features, int out_features, int *col_blocks, int *block_cols, int *tiles) {
     int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = device_cu_count(dev, &cus);
     if (e != hipSuccess) return e;
-    constexpr float kFixed[4] = {4.5f, 9.f, 18.f, 34.f}, kPerChunk[4] = {0.5f, 1.4f, 1.4f, 1.6f};
-    float best = 0.f;
+    constexpr double kFixed[2][4] = {{4.5, 7.82, 17.79, 38.65}, {5.95, 6.45, 17.61, 24.59}};  // in_features 128, 256
+    constexpr double kPerChunk[2][4] = {{0.5, 1.41, 1.4, 1.8}, {0.21, 1.72, 0.68, 2.34}};
+    constexpr double kSame = 1e-9;
+    const int wide = in_features == 256 ? 1 : 0;
+    double best = 0.;
+    *tiles = 0;
     for (int cut = 0; cut < 5; ++cut) {
         int cb, bc;
         proj_col_blocks(out_features, &cb, &bc);
@@ -378,8 +384,8 @@ static hipError_t proj_split(long long rows, int out_features, int *col_blocks, 
             // (the column blocks of a range of rows stay on one of the 8 XCDs: its workgroups against its compute units)
             const long long per_xcd = ((rows + per_group - 1) / per_group + 7) / 8 * cb;
             const int xcd_cus = std::max(1, cus / 8);
-            const float cost = (float)((per_xcd + xcd_cus - 1) / xcd_cus) * (kFixed[k] + kPerChunk[k] * (float)chunks);
-            if (best == 0.f || cost < best) {
+            const double cost = (double)((per_xcd + xcd_cus - 1) / xcd_cus) * (kFixed[wide][k] + kPerChunk[wide][k] * chunks);
+            if (*tiles == 0 || cost < best - kSame || (cost < best + kSame && (1 << k) > *tiles)) {
                 best = cost;
                 *col_blocks = cb;
                 *block_cols = bc;
@@ -395,7 +401,7 @@ hipError_t launch_block_proj(long long rows, int in_features, int out_features, 
     if (!block_proj_supported(rows, in_features, out_features) || out_ld < out_features || out_ld % 8 != 0)
         return hipErrorInvalidValue;
     int col_blocks, block_cols, tiles;
-    hipError_t e = proj_split(rows, out_features, &col_blocks, &block_cols, &tiles);
+    hipError_t e = proj_split(rows, in_features, out_features, &col_blocks, &block_cols, &tiles);
     if (e != hipSuccess) return e;
     const long long rows_per_group = 32LL * kProjWaves * tiles;
     const long long groups = ((rows + rows_per_group - 1) / rows_per_group + 7) / 8 * 8 * col_blocks;
