@@ -244,7 +244,7 @@ def test_weight_gradient_slabs_against_float64(rows, e, ld, d):
 @pytest.mark.parametrize("rows,E,ld,D", [(1, 648, 704, 256), (63, 256, 256, 256), (64, 8, 8, 128), (257, 648, 648, 256), (300, 264, 320, 128),
                                          (4097, 648, 704, 256), (16384, 256, 256, 256), (72828, 648, 704, 256), (72829, 128, 136, 128)])
 def test_weight_gradient_of_a_projection(rows, E, ld, D):
-    """a^T b against float64, for row counts around a step of 64 rows, a split and the longest float32 sum, widths that leave the
+    """a^T b against float64, for row counts around a step of 64 rows and a split, widths that leave the
     last block of 128 outputs part or nearly all empty, and padded rows whose padding holds NaN.  Bound: products of bf16 are
     exact in float32; no float32 sum is longer than 4 096 rows, whose rounding errors of random sign come to sqrt(4 096) 2^-24
     = 2^-18 of the terms' magnitudes."""
@@ -262,3 +262,22 @@ def test_weight_gradient_of_a_projection(rows, E, ld, D):
     assert torch.equal(out, block_wgrad(a, b))
     with pytest.raises(ValueError):
         block_wgrad(a, b[:, : D - 8].contiguous())
+
+
+@pytest.mark.parametrize("rows,E,ld,D", [(32768, 4224, 4224, 128), (33280, 4224, 4224, 128), (33217, 4224, 4288, 256), (66048, 4224, 4224, 128),
+                                         (199374, 648, 704, 256)])
+def test_weight_gradient_over_more_rows_than_one_float32_sum(rows, E, ld, D):
+    """Splits of 64 and 65 steps of 64 rows (the second sum begins with the 65th), a last step of one row, of 129 steps (two
+    sums moved to the totals), and the six blocks of a projection at 78: bound and inputs as above."""
+    from trading_bot_0_amd.block import block_wgrad
+    g = torch.Generator(device="cuda").manual_seed(rows + E)
+    buf = torch.full((rows, ld), float("nan"), dtype=torch.bfloat16, device="cuda")
+    buf[:, :E] = torch.randn(rows, E, generator=g, device="cuda").to(torch.bfloat16)
+    a, b = buf[:, :E], torch.randn(rows, D, generator=g, device="cuda").to(torch.bfloat16)
+    out = block_wgrad(a, b)
+    b64 = b.double()
+    for e0 in range(0, E, 1024):    # (a piece of the float64 operand at a time)
+        a64 = a[:, e0 : e0 + 1024].double().t().contiguous()
+        over = (out[e0 : e0 + 1024].double() - a64 @ b64).abs() - 2.0 ** -18 * (a64.abs() @ b64.abs())
+        assert torch.isfinite(over).all() and over.max().item() <= 0, f"over the bound by {over.max().item():.3e}"
+    assert torch.equal(out, block_wgrad(a, b))
