@@ -281,3 +281,22 @@ def test_weight_gradient_over_more_rows_than_one_float32_sum(rows, E, ld, D):
         over = (out[e0 : e0 + 1024].double() - a64 @ b64).abs() - 2.0 ** -18 * (a64.abs() @ b64.abs())
         assert torch.isfinite(over).all() and over.max().item() <= 0, f"over the bound by {over.max().item():.3e}"
     assert torch.equal(out, block_wgrad(a, b))
+
+
+@pytest.mark.parametrize("rows,E,D,library", [(131104, 648, 256, True), (262144, 648, 256, False), (131056, 392, 256, True),
+                                              (131072, 392, 256, False), (65552, 72, 256, True), (131072, 72, 256, False),
+                                              (131072, 72, 128, True), (32764, 1160, 256, True), (32768, 1160, 256, False),
+                                              (8191, 2184, 128, True), (8192, 2184, 128, False), (4099, 4368, 128, False)])
+def test_weight_gradient_route_by_slabs_and_width(rows, E, D, library, monkeypatch):
+    """Which of the two a row count and a width take, either side of each line, and that the two agree: float32 sums, or where
+    the rows make one slab for the BLAS its bf16 result (2^-8)."""
+    from trading_bot_0_amd import block as module
+    calls, launch = [], module.block_wgrad
+    monkeypatch.setattr(module, "block_wgrad", lambda a, b: calls.append(a.shape) or launch(a, b))
+    g = torch.Generator(device="cuda").manual_seed(rows + E)
+    a = torch.randn(rows, E, generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(rows, D, generator=g, device="cuda").to(torch.bfloat16)
+    out = module._weight_gradient(a, b)
+    assert bool(calls) == library and out.dtype == torch.float32
+    ref = launch(a, b)
+    assert (out - ref).norm() <= (1e-5 if library or rows % 2 == 0 else 2.0 ** -8) * ref.norm()

@@ -82,11 +82,23 @@ def block_wgrad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _wgrad_slab_limit(E: int, D: int) -> int:
+    """The number of slabs from which the BLAS runs a weight gradient of E x D outputs at least as fast as `block_wgrad`: the more
+    slabs the rows make the more of the chip its batched products fill, and the library's kernel reads b again for every 128
+    of the E.  In us, library against BLAS, D 256: E 648, 32 slabs 173 / 258 (245 760 rows), 64 slabs 190 / 122 (262 144); E 392,
+    16 slabs 57 / 79, 32 slabs 57 / 51 (131 072); E 128, 16 slabs 39 / 60, 32 slabs 39 / 35; E 1 160, 4 slabs 60 / 99 (49 156), 16 slabs
+    300 / 279 (262 160) and E 1 288, 8 slabs 417 / 335; E 2 184, one slab 234 / 294 (72 829), 4 slabs 143 / 117; E 4 368, one 467 / 353.
+    Both sides measured at E of 72 to 4 368, both D and 1 to 128 slabs."""
+    if E > 896:
+        return 8 if E <= 1792 else 2 if E <= 2304 else 0
+    return 32 if 384 < E <= 512 or (E <= 128 and D == 256) else 64
+
+
 def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T b in float32 for tall a [rows, E] (its rows may be a view into wider ones) and b [rows, D]: a sum over all
     rows of the batch and the sequence.  bf16 with D 128 or 256 runs on the library's kernel (72 828 rows, 648 x 256 outputs:
-    59 us, the BLAS 151), except where the rows make 64 slabs or more for the BLAS behind torch (262 144 rows: 200, 150), as
-    everything else does: as one GEMM the BLAS behind torch sees a contraction hundreds of thousands
+    59 us, the BLAS 151), except where the rows make enough slabs for the BLAS behind torch (`_wgrad_slab_limit`); there, and for
+    everything else: as one GEMM the BLAS behind torch sees a contraction hundreds of thousands
     long against outputs a few hundred wide and runs it at a fifth of its rate, so the rows are cut into equal slabs,
     multiplied as one batched GEMM with float32 outputs, and the slabs' products added in order (measured on MI355X,
     524 288 rows: 648 x 256 outputs 1 333 -> 232 us, 256 x 256 outputs 1 059 -> 129 us; the float32 partial products also
@@ -95,7 +107,7 @@ def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     slabs = 1
     while slabs < 128 and rows % (2 * slabs) == 0 and rows // (2 * slabs) >= 4096:
         slabs *= 2
-    if slabs < 64 and block_wgrad_supported(a, b):
+    if slabs < _wgrad_slab_limit(a.shape[1], b.shape[1]) and block_wgrad_supported(a, b):
         return block_wgrad(a, b)
     if slabs == 1 or a.dtype == torch.float32:
         return torch.matmul(a.t(), b).float()
