@@ -10,7 +10,6 @@ input), which are torch matmuls.
 """
 from __future__ import annotations
 
-import functools
 import math
 from ctypes import POINTER, Structure, byref, c_float, c_int, c_int64, c_size_t, c_void_p
 from dataclasses import dataclass
@@ -205,16 +204,12 @@ def block_post(y, zxbcdt, norm_w, nheads, headdim, dstate, ngroups, eps=1e-5):
     return out
 
 
-def _aligned(*tensors: torch.Tensor) -> bool:
-    """Whether the kernels' 16-byte loads can read these contiguous tensors (one that starts elsewhere in a flat buffer goes to
-    the BLAS, which takes any address)."""
-    return all(t.data_ptr() % 16 == 0 for t in tensors)
-
-
 def block_post_proj_supported(y: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether `block_post_proj` takes these tensors (else `block_post`, then the projection)."""
+    """Whether `block_post_proj` takes these tensors (else `block_post`, then the projection).  (The addresses: the kernels load 16
+    bytes at a time, and a tensor that starts elsewhere in a flat buffer goes to the BLAS, which takes any.)"""
     return (y.is_cuda and y.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2
-            and weight.shape[1] in (128, 256) and weight.shape[0] % 8 == 0 and weight.shape[0] <= 256 and _aligned(y, weight))
+            and weight.shape[1] in (128, 256) and weight.shape[0] % 8 == 0 and weight.shape[0] <= 256
+            and (y.data_ptr() | weight.data_ptr()) % 16 == 0)
 
 
 def block_post_proj(y, zxbcdt, norm_w, weight, nheads, headdim, dstate, ngroups, eps=1e-5):
@@ -252,7 +247,6 @@ FUSED_STEP_MAX_BATCH = 1024
 FUSED_STEP_MAX_BATCH_OTHER = 256
 
 
-@functools.lru_cache(maxsize=64)
 def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
     """The largest batch whose step is taken as one launch, by the kernel that the library runs for the shape (0: the launch's
     vectors, as it lays them out, do not fit the 64 KB of LDS that it asks for)."""
@@ -266,7 +260,7 @@ def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroup
 def block_step_supported(u_t: torch.Tensor, d_inner: int, dstate: int) -> bool:
     """Whether `block_step` takes this step (else the stage kernels, one launch each)."""
     return (u_t.is_cuda and u_t.dtype in (torch.bfloat16, torch.float32) and u_t.dim() == 2
-            and u_t.shape[1] in (128, 256) and d_inner in (128, 256) and dstate % 16 == 0 and _aligned(u_t))
+            and u_t.shape[1] in (128, 256) and d_inner in (128, 256) and dstate % 16 == 0 and u_t.data_ptr() % 16 == 0)
 
 
 def block_step(u_t, w_in, conv_w, conv_b, dt_bias, A, D, norm_w, w_out, conv_state, ssm_state, nheads, headdim, dstate,
@@ -399,7 +393,7 @@ def block_pre_bwd(zxbcdt, conv_w, conv_b, dt_bias, dx, dB, dC, ddt, dzxbcdt, nhe
 def block_proj_supported(u: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `block_proj` takes this product (else the caller's BLAS does it)."""
     return (u.is_cuda and u.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and u.shape[-1] in (128, 256)
-            and weight.shape[0] % 8 == 0 and u.numel() > 0 and _aligned(u, weight))
+            and weight.shape[0] % 8 == 0 and u.numel() > 0 and (u.data_ptr() | weight.data_ptr()) % 16 == 0)
 
 
 def block_proj(u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) -> torch.Tensor:
@@ -565,8 +559,10 @@ class Mamba2Block:
         key = (dtype, self.in_proj._version, self.out_proj._version, self.in_proj.data_ptr(), self.out_proj.data_ptr())
         cached = getattr(self, "_weights_cache", None)
         if cached is None or cached[0] != key:
-            w_out = self.out_proj.to(dtype).contiguous()
-            cached = (key, self.in_proj.to(dtype).contiguous(), w_out, w_out.t().contiguous())
+            w_in, w_out = self.in_proj.to(dtype).contiguous(), self.out_proj.to(dtype).contiguous()
+            # (with them: the batch up to which a step is one launch, whose kernel reads both 16 bytes at a time)
+            limit = _step_max_batch(self.d_model, self.H, self.P, self.N, self.G) if (w_in.data_ptr() | w_out.data_ptr()) % 16 == 0 else 0
+            cached = (key, w_in, w_out, w_out.t().contiguous(), limit)
             self._weights_cache = cached
         return cached[1], cached[2]
 
@@ -593,8 +589,7 @@ class Mamba2Block:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         w_in, w_out = self._weights(u_t.dtype)
         if fused is None:
-            fused = (u_t.shape[0] <= _step_max_batch(self.d_model, self.H, self.P, self.N, self.G) and _aligned(w_in, w_out)
-                     and block_step_supported(u_t.contiguous(), self.d_inner, self.N))
+            fused = u_t.shape[0] <= self._weights_cache[4] and block_step_supported(u_t, self.d_inner, self.N)
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
             out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
                              self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
