@@ -307,8 +307,9 @@ int ssd_block_post_proj_fwd(const ssd_block_dims *dims, int dtype, const void *y
  * [d_model, H*P] in the activation type (dtype 0: float32, 1: bfloat16), conv_w [C,d_conv], conv_b [C], dt_bias [H],
  * A [H], D [H] or NULL, norm_w [H*P] float32; conv_state [B,d_conv-1,C] (activation type) and ssm_state [B,H,P,N]
  * (float32) advance in place; out [B,d_model].  d_model and H*P must each be 128 or 256 and dstate a multiple of 16
- * (SSD_ERR_UNSUPPORTED otherwise: run the stages).  A workgroup per stream reads both weight matrices whole, so the
- * call is meant for small batches (up to a few dozen streams); large ones are faster through the stage kernels. */
+ * (SSD_ERR_UNSUPPORTED otherwise: run the stages).  A workgroup of one stream, or two, reads both weight matrices whole, so the
+ * call is meant for small batches: up to 1 024 streams with dstate 64 and at most 768 rows of w_in, 256 otherwise; larger ones
+ * are faster through the stage kernels. */
 int ssd_block_step_fwd(const ssd_block_dims *dims, int dtype, int64_t d_model, const void *u, const void *w_in,
                        const float *conv_w, const float *conv_b, const float *dt_bias, const float *A, const float *D,
                        const float *norm_w, float eps, const void *w_out, void *conv_state, float *ssm_state, void *out,

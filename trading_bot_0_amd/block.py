@@ -5,8 +5,8 @@ encoder block sits in `patch_trunk` (`trading_bots/src/torch/model/trading_model
 state the way the reference's `StreamState` carries its encoder memory (`trading_model.rs:56-75`).
 
 Everything runs in libssd_hip -- the projections, the pre-scan and post-scan kernels and the weight gradients bound here, the
-scan / step of `ssd.py` -- but the products its kernels do not take (float32, other widths; the gradient of the block's
-input), which are torch matmuls.
+scan / step of `ssd.py` -- but the products its kernels do not take (float32, other widths and addresses, weight gradients of
+many rows or wide; the gradient of the block's input), which are torch matmuls.
 """
 from __future__ import annotations
 
@@ -499,7 +499,9 @@ class Mamba2Block:
             raise ValueError("backward through a window that continues a carried state is not supported")
         if block_post_proj_supported(y, w_out):
             # gate, norm and out-projection as one kernel: the normalised rows never reach memory (the backward pass
-            # needs them for one weight gradient only, and has its post stage write them on the way: yn=None)
+            # needs them for one weight gradient only, and has its post stage write them on the way: yn=None).  Of few rows it
+            # saves the host's time, not the GPU's (256 -> 256 in us, one kernel / two, and called one by one: 512 rows 13.3 / 7.1
+            # and 13 / 30, 8 191 rows 14.8 / 11.0 and 15 / 29)
             out = block_post_proj(y, zxbcdt, self.norm_w, w_out, self.H, self.P, self.N, self.G, self.eps)
             yn = None
         else:
@@ -544,9 +546,9 @@ class Mamba2Block:
 
     def _project(self, u: torch.Tensor, weight: torch.Tensor, pad_rows: bool = False) -> torch.Tensor:
         """u . weight^T in the activation dtype: the library's kernel where it takes the shape (bf16, in_features 128
-        or 256), else the BLAS behind torch.  In us of the GPU, library against BLAS: 256 -> 648 at 2 048 rows 6.7 / 6.7, 16 384
-        rows 14.6 / 24.9; 256 -> 256 at 8 192 rows 7.0 / 6.6, 16 384 rows 7.9 / 8.2; and of the host's time to issue it 8
-        against 20, which is what counts at few rows."""
+        or 256), else the BLAS behind torch.  In us of the GPU, library against BLAS: 256 -> 648 at 512 rows 6.4 / 4.7, 2 048 rows
+        6.5 / 6.7, 16 383 rows 14.6 / 24.2; 256 -> 256 at 512 rows 6.1 / 4.2, 8 192 rows 6.7 / 6.5, 16 383 rows 7.6 / 7.8; and of the
+        host's time to issue it 8 against 19, which is what counts at few rows unless the caller replays a graph."""
         w = weight.to(u.dtype).contiguous()
         u = u.contiguous()
         if block_proj_supported(u, w):

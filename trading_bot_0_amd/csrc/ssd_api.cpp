@@ -212,7 +212,8 @@ constexpr int kBf16AnchorStride = 8;
 // from which the transposed scans are wide, 27 to 37 from there to 256.  Measured at eight heads of 32, state 64
 // (sequences x steps, as chosen here / uncut / the general path they took before): 32 x 2 048 219 / 555 / 631, 4 x 4 096
 // 111 / 1 048 / 216, 64 x 2 048 365 / 594 / 792, 16 x 8 192 363 / 2 154 / 1 197, 1 x 146 59 / 78 / 92; uncut as chosen:
-// 52 x 153 94 (cut 91) / 115.
+// 52 x 153 94 (cut 91) / 115.  (256 compute units are a constant here: the workspace is laid out by the segments, and the
+// gradients' last bits, which depend on where a sequence is cut, do not depend on the device.)
 int bwd_segment_tiles(const ssd::ScanShape &s) {
     const double groups = (double)s.B * s.H / 8;
     double best = 30.0 + 18.5 * s.nc;

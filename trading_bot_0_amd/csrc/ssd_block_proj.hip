@@ -2,8 +2,8 @@
 // columns) and a small weight matrix, bf16 in and out, float32 accumulation (gfx950).
 //
 // With K of a few hundred the product is bound by memory, not by the matrix cores: u is read once, out written once
-// (0.95 GB for 524 288 rows, 256 -> 648).  A workgroup owns a block of at most 160 output columns and a range of
-// rows: it puts its rows of w into LDS once (84 KB), and from then on its eight waves run without a barrier -- each
+// (0.95 GB for 524 288 rows, 256 -> 648).  A workgroup owns a block of at most 160 output columns and a range of 256 to
+// 2 048 rows (proj_split): it puts its rows of w into LDS once (84 KB at most), and from then on its eight waves run without a barrier -- each
 // takes tiles of 32 rows, loads its rows of u straight into MFMA operand fragments (u and w are both contiguous
 // along K, so a lane's eight K elements are one 16-byte load; the next tile's rows are in flight during this
 // tile's products), and walks the block's columns in chunks of 32 with the w fragments read from LDS.  The MFMA's
@@ -25,8 +25,9 @@ constexpr int kProjBlockCols = 160;   // most output columns per workgroup (thei
 constexpr int kProjChunk = 32;        // output columns per MFMA tile
 constexpr int kProjTiles = 8;         // most tiles of 32 rows per wave
 
-// CH: 32-column chunks of the widest block of columns (1..5; a block takes CH or CH - 1 chunks, and its last chunk
-// may hold fewer columns than it covers).  The chunk count is a template parameter and every store goes out without a condition -- a
+// CH: 32-column chunks of the widest block of columns (1..5; a block walks CH chunks, or CH - 1 where those cover it, and the
+// chunks past its columns -- several, where a last narrow block is left: 648 columns in blocks of 128 leave 8 -- are
+// multiplied and not stored).  The chunk count is a template parameter and every store goes out without a condition -- a
 // buffer store whose offset is put out of range for rows past M and columns past the block, which the hardware then
 // drops -- because loads and stores share one counter per wave, in order: only in straight-line code with every
 // store counted does the compiler wait for a tile's rows of u by their exact position in that order.  With a loop of
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
 
     const int r = lane & 31, half = lane >> 5;
     unsigned char *tile = otile[wave];
-    // the workgroup's rows of `out` as a range-checked buffer: 2 048 rows of at most ldo elements
+    // the workgroup's rows of `out` as a range-checked buffer: up to 2 048 rows of at most ldo elements
     const __amdgpu_buffer_rsrc_t obuf = make_buffer(out + (size_t)row0 * ldo, (unsigned)min((long long)TILES * 32 * kProjWaves, M - row0) * (unsigned)ldo * 2u);
     auto tile_row0 = [&](int t) { return row0 + (long long)t * (32 * kProjWaves) + wave * 32; };
     // this lane's part of its row of u: K elements 16 ks + 8 half .. + 7 for every K step (rows past M repeat the

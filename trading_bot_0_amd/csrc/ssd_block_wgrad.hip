@@ -12,8 +12,10 @@
 // Against the BLAS, whose batched products over equal slabs of rows need a row count with a power of two in it (any other
 // ran as one product with a bf16 result at a fifth of the rate), in us, BLAS / here: 648 x 256 outputs at 16 384 rows 38 / 26,
 // 72 828 rows 151 / 59, 131 072 rows 130 / 103, 199 374 rows 388 / 155, 262 144 rows 150 / 200, 524 288 rows 300 / 415; 256 x 256
-// at the same rows 36 / 22, 83 / 35, 51 / 45, 360 / 58, 85 / 93, 120 / 167: the caller keeps the BLAS for the largest that it cuts into 64
-// slabs or more.  There this kernel waits for memory with 48 KB per compute unit in flight: two steps ahead take 72
+// at the same rows 36 / 22, 83 / 35, 51 / 45, 360 / 58, 85 / 93, 120 / 167: the caller keeps the BLAS for row counts that it cuts
+// into many slabs, 64 and more at these widths and fewer at wide E (b is read again for every 128 of it, and above 1 024 a round of
+// splits no longer fills the chip: E 2 184 at 131 056 rows 204 / 410).  At the largest this kernel waits for memory with 48 KB per
+// compute unit in flight: two steps ahead take 72
 // registers more than there are (spilled: 477), and four waves with all registers leave the reads of LDS uncovered (824).
 #include "ssd_fused_scan.h"
 
@@ -157,7 +159,8 @@ struct WgradPlan {
     long long split_rows;
 };
 
-// Splits: one round of workgroups (a compute unit holds one), whole XCDs, none below kWgradMinRows rows.
+// Splits: one round of workgroups (a compute unit holds one), whole XCDs, none below kWgradMinRows rows.  (256 compute units are
+// a constant here: the workspace is laid out by the splits, and the order of the sums, so the bits, do not depend on the device.)
 WgradPlan wgrad_plan(long long rows, int E) {
     WgradPlan p;
     p.blocks = (E + kWgradCols - 1) / kWgradCols;
