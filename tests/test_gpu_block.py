@@ -605,3 +605,35 @@ def test_graphed_step_equals_the_eager_step_on_every_replay():
         assert torch.equal(out_g, out_e), f"replay {i}: output"
         assert torch.equal(st_g.conv, st_e.conv) and torch.equal(st_g.ssm.state, st_e.ssm.state), f"replay {i}: state"
         _ = (prefix.float() * 2).sum().item()      # eager work and a synchronisation between the replays
+
+
+@pytest.mark.parametrize("batch,state,own", [(4, 64, False), (70, 64, False), (70, 64, True), (200, 32, True), (300, 32, False)])
+def test_captured_step_reads_a_changed_decay(batch, state, own):
+    """A_log modified in place between the replays of a captured step (of `graphed_step`, or of a graph of the caller's of more
+    than 64 streams): every replay, before and after an eager step has formed A anew, is the eager step bit for bit."""
+    blk = Mamba2Block(d_model=256, nheads=8, headdim=32, dstate=state, seed=3)
+    bars = torch.randn(5, batch, 256, generator=torch.Generator(device="cuda").manual_seed(5), device="cuda").to(torch.bfloat16)
+    st_e, st_g = blk.new_state(batch), blk.new_state(batch)
+    if own:
+        u = torch.zeros(batch, 256, dtype=torch.bfloat16, device="cuda")
+        blk.step(u, blk.new_state(batch))
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = blk.step(u, st_g)
+
+        def step(bar):
+            u.copy_(bar)
+            graph.replay()
+            return out
+    else:
+        step = blk.graphed_step(st_g)
+    for i in range(bars.shape[0]):
+        if i % 2 == 1:
+            blk.A_log.add_(0.3)
+        out_g = step(bars[i]).clone()
+        torch.cuda.synchronize()
+        out_e = blk.step(bars[i], st_e)
+        torch.cuda.synchronize()
+        assert torch.equal(out_g, out_e) and torch.equal(st_g.ssm.state, st_e.ssm.state), f"replay {i}"
+        _ = (bars.float() * 2).sum().item()        # eager work and a synchronisation between the replays

@@ -245,6 +245,8 @@ FUSED_STEP_MAX_BATCH = 1024
 # 38 / 41 against 32 / 37; 1 024 65 / 70 against 38 / 43, 94 / 99 against 69 / 75, 77 / 82 against 49 / 55.  (Eager, where the
 # stage kernels cost 92, it would win up to some 768; a step captured by the caller is not known to be one.)
 FUSED_STEP_MAX_BATCH_OTHER = 256
+# batches up to which a step that a caller captures keeps the A formed before (above, a captured step forms it at every replay)
+STEP_CACHED_A_MAX_BATCH = 64
 
 
 def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
@@ -574,9 +576,12 @@ class Mamba2Block:
         self._weights(dtype)
         return self._weights_cache[3]
 
+    def _A_key(self):
+        return (self.A_log._version, self.A_log.data_ptr())
+
     def _A_cached(self) -> torch.Tensor:
         """-exp(A_log), computed once per version of A_log (a launch of its own otherwise, per step)."""
-        key = (self.A_log._version, self.A_log.data_ptr())
+        key = self._A_key()
         cached = getattr(self, "_A_cache", None)
         if cached is None or cached[0] != key:
             cached = (key, -torch.exp(self.A_log))
@@ -593,16 +598,21 @@ class Mamba2Block:
         if fused is None:
             fused = u_t.shape[0] <= self._weights_cache[4] and block_step_supported(u_t, self.d_inner, self.N)
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
-            out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self._A_cached(), self.D,
-                             self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
-            state.ssm.initialized = True    # as `SsdStreamState.step` leaves it
-            return out
+            # (a captured step of more streams forms A at every replay, as one of stage kernels does)
+            fresh = u_t.shape[0] > STEP_CACHED_A_MAX_BATCH and torch.cuda.is_current_stream_capturing()
+            return self._one_launch_step(u_t.contiguous(), state, w_in, w_out, self.A if fresh else self._A_cached())
         zxbcdt = torch.matmul(u_t, w_in.t()).unsqueeze(1).contiguous()
         x, Bm, Cm, dt, _ = block_pre(zxbcdt, self.conv_w, self.conv_b, self.dt_bias, self.H, self.P, self.N,
                                      self.G, conv_state=state.conv, conv_state_out=state.conv)  # in place
         y = state.ssm.step(x[:, 0], dt[:, 0], self.A, Bm[:, 0], Cm[:, 0], self.D)
         yn = block_post(y.unsqueeze(1), zxbcdt, self.norm_w, self.H, self.P, self.N, self.G, self.eps)
         return torch.matmul(yn[:, 0], w_out.t())
+
+    def _one_launch_step(self, u_t, state: Mamba2StreamState, w_in, w_out, A) -> torch.Tensor:
+        out = block_step(u_t, w_in, self.conv_w, self.conv_b, self.dt_bias, A, self.D, self.norm_w, w_out, state.conv,
+                         state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
+        state.ssm.initialized = True    # as `SsdStreamState.step` leaves it
+        return out
 
     def graphed_step(self, state: Mamba2StreamState, dtype: torch.dtype = torch.bfloat16) -> "GraphedBlockStep":
         """`step` for `state`'s streams captured once in a HIP graph and replayed per bar: at a few streams a step
@@ -616,7 +626,8 @@ class GraphedBlockStep:
     """A captured `Mamba2Block.step` over fixed buffers.  Calling it copies the bar's input into the captured input
     buffer, replays the graph and returns the captured output buffer (overwritten by the next call).  The state it
     was built for advances in place, as with `step`; the block's parameters are read at replay time, except the
-    projection matrices, whose activation-dtype copies are made at capture."""
+    projection matrices, whose activation-dtype copies are made at capture.  (A = -exp(A_log) of a step captured as one launch is
+    a buffer of the graph's own, filled again when A_log has been modified.)"""
 
     def __init__(self, block: Mamba2Block, state: Mamba2StreamState, dtype: torch.dtype):
         batch = state.conv.shape[0]
@@ -624,19 +635,32 @@ class GraphedBlockStep:
         self.u = torch.zeros((batch, block.d_model), dtype=dtype, device=dev)
         # what the warm-up steps below do to the state is undone afterwards
         conv_keep, ssm_keep = state.conv.clone(), state.ssm.state.clone()
+        self.block, self.A = block, None
+        self.weights = block._weights(dtype)    # (kept: the graph reads these copies, whatever becomes of the block's)
+
+        def step():
+            if self.A is None:
+                return block.step(self.u, state, fused=False)
+            return block._one_launch_step(self.u, state, *self.weights, self.A)
+
+        if batch <= block._weights_cache[4] and block_step_supported(self.u, block.d_inner, block.N):
+            self.A, self.A_key = block.A, block._A_key()
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
         with torch.cuda.stream(side):
             for _ in range(2):  # library handles, kernel modules and the weights' copies exist before the capture
-                block.step(self.u, state)
+                step()
         torch.cuda.current_stream(dev).wait_stream(side)
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
-            self.out = block.step(self.u, state)
+            self.out = step()
         state.conv.copy_(conv_keep)
         state.ssm.state.copy_(ssm_keep)
 
     def __call__(self, u_t: torch.Tensor) -> torch.Tensor:
         self.u.copy_(u_t)
+        if self.A is not None and self.A_key != self.block._A_key():
+            self.A.copy_(self.block.A)
+            self.A_key = self.block._A_key()
         self.graph.replay()
         return self.out
