@@ -249,12 +249,13 @@ FUSED_STEP_MAX_BATCH_OTHER = 256
 STEP_CACHED_A_MAX_BATCH = 64
 
 
-def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
-    """The largest batch whose step is taken as one launch, by the kernel that the library runs for the shape (0: the launch's
-    vectors, as it lays them out, do not fit the 64 KB of LDS that it asks for)."""
+def _step_max_batch(dtype: torch.dtype, d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
+    """The largest batch whose step is taken as one launch, by the kernel that the library runs for the shape (0: it takes none,
+    or the launch's vectors, as it lays them out, do not fit the 64 KB of LDS that it asks for)."""
     d_inner, E = nheads * headdim, in_proj_width(nheads, headdim, dstate, ngroups)
     vectors = d_model + E + (E - d_inner - nheads) + (nheads + 3) // 4 * 4 + d_inner + 16
-    if 4 * vectors > 64 * 1024:
+    if (dtype not in (torch.bfloat16, torch.float32) or d_model not in (128, 256) or d_inner not in (128, 256) or dstate % 16
+            or 4 * vectors > 64 * 1024):
         return 0
     return FUSED_STEP_MAX_BATCH if dstate == 64 and E <= 768 else FUSED_STEP_MAX_BATCH_OTHER
 
@@ -565,7 +566,9 @@ class Mamba2Block:
         if cached is None or cached[0] != key:
             w_in, w_out = self.in_proj.to(dtype).contiguous(), self.out_proj.to(dtype).contiguous()
             # (with them: the batch up to which a step is one launch, whose kernel reads both 16 bytes at a time)
-            limit = _step_max_batch(self.d_model, self.H, self.P, self.N, self.G) if (w_in.data_ptr() | w_out.data_ptr()) % 16 == 0 else 0
+            limit = _step_max_batch(dtype, self.d_model, self.H, self.P, self.N, self.G)
+            if (w_in.data_ptr() | w_out.data_ptr()) % 16:
+                limit = 0
             cached = (key, w_in, w_out, w_out.t().contiguous(), limit)
             self._weights_cache = cached
         return cached[1], cached[2]
@@ -576,12 +579,9 @@ class Mamba2Block:
         self._weights(dtype)
         return self._weights_cache[3]
 
-    def _A_key(self):
-        return (self.A_log._version, self.A_log.data_ptr())
-
     def _A_cached(self) -> torch.Tensor:
         """-exp(A_log), computed once per version of A_log (a launch of its own otherwise, per step)."""
-        key = self._A_key()
+        key = (self.A_log._version, self.A_log.data_ptr())
         cached = getattr(self, "_A_cache", None)
         if cached is None or cached[0] != key:
             cached = (key, -torch.exp(self.A_log))
@@ -594,25 +594,23 @@ class Mamba2Block:
         with the projections on the BLAS behind torch."""
         if u_t.dim() != 2 or u_t.shape[1] != self.d_model:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
+        batch = u_t.shape[0]
         w_in, w_out = self._weights(u_t.dtype)
         if fused is None:
-            fused = u_t.shape[0] <= self._weights_cache[4] and block_step_supported(u_t, self.d_inner, self.N)
+            fused = batch <= self._weights_cache[4] and u_t.is_cuda and u_t.data_ptr() % 16 == 0
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
             # (a captured step of more streams forms A at every replay, as one of stage kernels does)
-            fresh = u_t.shape[0] > STEP_CACHED_A_MAX_BATCH and torch.cuda.is_current_stream_capturing()
-            return self._one_launch_step(u_t.contiguous(), state, w_in, w_out, self.A if fresh else self._A_cached())
+            fresh = batch > STEP_CACHED_A_MAX_BATCH and torch.cuda.is_current_stream_capturing()
+            out = block_step(u_t.contiguous(), w_in, self.conv_w, self.conv_b, self.dt_bias, self.A if fresh else self._A_cached(),
+                             self.D, self.norm_w, w_out, state.conv, state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
+            state.ssm.initialized = True    # as `SsdStreamState.step` leaves it
+            return out
         zxbcdt = torch.matmul(u_t, w_in.t()).unsqueeze(1).contiguous()
         x, Bm, Cm, dt, _ = block_pre(zxbcdt, self.conv_w, self.conv_b, self.dt_bias, self.H, self.P, self.N,
                                      self.G, conv_state=state.conv, conv_state_out=state.conv)  # in place
         y = state.ssm.step(x[:, 0], dt[:, 0], self.A, Bm[:, 0], Cm[:, 0], self.D)
         yn = block_post(y.unsqueeze(1), zxbcdt, self.norm_w, self.H, self.P, self.N, self.G, self.eps)
         return torch.matmul(yn[:, 0], w_out.t())
-
-    def _one_launch_step(self, u_t, state: Mamba2StreamState, w_in, w_out, A) -> torch.Tensor:
-        out = block_step(u_t, w_in, self.conv_w, self.conv_b, self.dt_bias, A, self.D, self.norm_w, w_out, state.conv,
-                         state.ssm.state, self.H, self.P, self.N, self.G, self.eps)
-        state.ssm.initialized = True    # as `SsdStreamState.step` leaves it
-        return out
 
     def graphed_step(self, state: Mamba2StreamState, dtype: torch.dtype = torch.bfloat16) -> "GraphedBlockStep":
         """`step` for `state`'s streams captured once in a HIP graph and replayed per bar: at a few streams a step
@@ -641,10 +639,12 @@ class GraphedBlockStep:
         def step():
             if self.A is None:
                 return block.step(self.u, state, fused=False)
-            return block._one_launch_step(self.u, state, *self.weights, self.A)
+            state.ssm.initialized = True
+            return block_step(self.u, self.weights[0], block.conv_w, block.conv_b, block.dt_bias, self.A, block.D, block.norm_w,
+                              self.weights[1], state.conv, state.ssm.state, block.H, block.P, block.N, block.G, block.eps)
 
         if batch <= block._weights_cache[4] and block_step_supported(self.u, block.d_inner, block.N):
-            self.A, self.A_key = block.A, block._A_key()
+            self.A, self.A_key = block.A, (block.A_log._version, block.A_log.data_ptr())
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
         with torch.cuda.stream(side):
@@ -659,8 +659,10 @@ class GraphedBlockStep:
 
     def __call__(self, u_t: torch.Tensor) -> torch.Tensor:
         self.u.copy_(u_t)
-        if self.A is not None and self.A_key != self.block._A_key():
-            self.A.copy_(self.block.A)
-            self.A_key = self.block._A_key()
+        if self.A is not None:
+            key = (self.block.A_log._version, self.block.A_log.data_ptr())
+            if key != self.A_key:
+                self.A.copy_(self.block.A)
+                self.A_key = key
         self.graph.replay()
         return self.out
