@@ -153,6 +153,24 @@ def dims(**kw):
     return ssd.SsdDims(*[d[k] for k in ("batch", "seqlen", "nheads", "headdim", "dstate", "ngroups", "chunk")])
 
 
+@pytest.mark.parametrize("layout", [dict(nheads=8, dstate=64), dict(nheads=8, dstate=32), dict(nheads=24, dstate=64, ngroups=3)])
+def test_backward_workspace_of_few_sequences_holds_smaller_calls(lib, layout):
+    """Where the backward pass runs on segments, what it asks for grows with the batch and with the length, although the number
+    of segments does not: a workspace sized for the largest call of a program holds the others.  (From 96 groups of eight heads on
+    the pass runs on other kernels, which ask for less.)"""
+    def need(batch, seqlen):
+        out = c_size_t(0)
+        d = ssd.SsdDims(batch, seqlen, layout["nheads"], 32, layout["dstate"], layout.get("ngroups", 1), 64)
+        assert lib.ssd_chunk_scan_bwd_workspace_bytes(byref(d), 1, byref(out)) == 0
+        return out.value
+
+    most = 95 * 8 // layout["nheads"]
+    lengths = (1, 64, 65, 129, 320, 512, 1000, 2048, 3000, 4096, 8191, 16384)
+    sizes = [[need(batch, seqlen) for batch in range(1, most + 1)] for seqlen in lengths]
+    assert all(a <= b for row in sizes for a, b in zip(row, row[1:])), "a larger batch asks for less"
+    assert all(a <= b for col in zip(*sizes) for a, b in zip(col, col[1:])), "a longer sequence asks for less"
+
+
 def test_workspace_bytes_formula(lib):
     out = c_size_t(0)
     assert lib.ssd_workspace_bytes(byref(dims()), byref(out)) == 0

@@ -197,6 +197,7 @@ struct BwdPlan {
     bool rows_in_scan;  // the adjoint scan with the row products in its epilogue (writes dx; no float r)
     int anchor_stride;  // tiles between two meetings of the transposed scans' states (the decay gradient's anchors)
     int seg_tiles;      // the three scans on segments of that many tiles (0: not cut)
+    int seg_groups;     // segments times groups of eight heads that the workspace holds
 };
 
 // The decay gradient is anchored where the two transposed scans' states meet; between two anchors it sums the
@@ -214,13 +215,16 @@ constexpr int kBf16AnchorStride = 8;
 // 111 / 1 048 / 216, 64 x 2 048 365 / 594 / 792, 16 x 8 192 363 / 2 154 / 1 197, 1 x 146 59 / 78 / 92; uncut as chosen:
 // 52 x 153 94 (cut 91) / 115.  (256 compute units are a constant here: the workspace is laid out by the segments, and the
 // gradients' last bits, which depend on where a sequence is cut, do not depend on the device.)
+constexpr int kBwdMaxSegmentGroups = 511;  // (two rounds of workgroups, which never are the fastest, would be 512)
+
 int bwd_segment_tiles(const ssd::ScanShape &s) {
     const double groups = (double)s.B * s.H / 8;
     double best = 30.0 + 18.5 * s.nc;
     int tiles = 0;
-    for (int S = 2; S <= s.nc && groups * (S - 1) < 512; ++S) {  // (more than two rounds are never the fastest)
+    for (int S = 2; S <= s.nc && groups * (S - 1) <= kBwdMaxSegmentGroups; ++S) {
         const int t = (s.nc + S - 1) / S;
         const double W = groups * ((s.nc + t - 1) / t);
+        if (W > kBwdMaxSegmentGroups) continue;
         const double per_tile = W < 96 ? 19.5 : 27.0 + 10.0 * std::min(1.0, (W - 96) / 160);
         const double cost = std::ceil(W / 256) * (60.0 + per_tile * t);
         if (cost < best) {
@@ -252,11 +256,14 @@ BwdPlan plan_bwd(const ssd::ScanShape &s, const ssd::ScanShape &sT, int dtype) {
     // eight tiles apart its error against float64 was four to ten times the general path's (4 x 1 000 steps 1.3e-4
     // against 2.1e-5 of its norm; 1.4e-5 with one at every tile).
     const bool few = !p.fast_r;
-    p.seg_tiles = 0;
+    p.seg_tiles = p.seg_groups = 0;
     if (few && inner != SSD_DTYPE_F32 && s.Q == 64 && ssd::transposed_scan_supported(sT, s.G) &&
         ssd::adjoint_rows_scan_supported(s) && ssd::fused_scan_waves(s, inner) == 8) {
         p.sum_on_chip = p.fast_r = true;
         p.seg_tiles = bwd_segment_tiles(s);
+        // (sized by a bound that grows with batch and length, also where a shape is not cut: the number of segments does not, and
+        // a workspace sized for the largest of a program's batches has to hold the smaller ones)
+        p.seg_groups = (int)std::min<int64_t>(kBwdMaxSegmentGroups, (int64_t)s.B * (s.H / 8) * s.nc);
     }
     p.fast_t = p.sum_on_chip || one_pass(sT);
     p.rows_in_scan = p.sum_on_chip && p.fast_r && ssd::adjoint_rows_scan_supported(s);
@@ -307,12 +314,12 @@ BwdWorkspace carve_bwd(const ssd::ScanShape &s, const ssd::ScanShape &sT, int el
     w.a_parts = take_if(sT.H > s.H, (size_t)sT.H * sizeof(float));
     // on segments: what each adds to the forward and the adjoint state, the states entering each (transposed; the
     // adjoint's also in place of what it adds), the segments' decays
-    const size_t segs = plan.seg_tiles > 0 ? (size_t)((s.nc + plan.seg_tiles - 1) / plan.seg_tiles) : 0;
-    w.seg_fwd = take(segs * st);
-    w.seg_adj = take(segs * st);
-    w.seg_fwd_t = take(segs * st);
-    w.seg_adj_t = take(segs * st);
-    w.seg_decay = take(2 * segs * s.B * s.H * sizeof(float));
+    const size_t seg_st = (size_t)plan.seg_groups * 8 * s.P * s.N * sizeof(float);
+    w.seg_fwd = take(seg_st);
+    w.seg_adj = take(seg_st);
+    w.seg_fwd_t = take(seg_st);
+    w.seg_adj_t = take(seg_st);
+    w.seg_decay = take((size_t)2 * plan.seg_groups * 8 * sizeof(float));
     w.total = off;
     return w;
 }
