@@ -558,9 +558,9 @@ class Mamba2Block:
             return block_proj(u, w, pad_rows=pad_rows)
         return torch.matmul(u, w.t()).contiguous()
 
-    def _weights(self, dtype: torch.dtype):
-        """The two projection matrices in the activation dtype, converted once per dtype (and again when a master
-        copy has been modified in place)."""
+    def _converted(self, dtype: torch.dtype):
+        """(key, in_proj, out_proj, out_proj^T, step limit) in the activation dtype, converted once per dtype (and again when a
+        master copy has been modified in place)."""
         key = (dtype, self.in_proj._version, self.out_proj._version, self.in_proj.data_ptr(), self.out_proj.data_ptr())
         cached = getattr(self, "_weights_cache", None)
         if cached is None or cached[0] != key:
@@ -571,13 +571,16 @@ class Mamba2Block:
                 limit = 0
             cached = (key, w_in, w_out, w_out.t().contiguous(), limit)
             self._weights_cache = cached
-        return cached[1], cached[2]
+        return cached
+
+    def _weights(self, dtype: torch.dtype):
+        """The two projection matrices in the activation dtype."""
+        return self._converted(dtype)[1:3]
 
     def _out_proj_transposed(self, dtype: torch.dtype) -> torch.Tensor:
         """out_proj^T [d_inner, d_model] in the activation dtype (the backward's dyn = dout . out_proj is then a
         product of the forward's form, which the library's projection kernel takes), cached with the others."""
-        self._weights(dtype)
-        return self._weights_cache[3]
+        return self._converted(dtype)[3]
 
     def _A_cached(self) -> torch.Tensor:
         """-exp(A_log), computed once per version of A_log (a launch of its own otherwise, per step)."""
@@ -595,9 +598,9 @@ class Mamba2Block:
         if u_t.dim() != 2 or u_t.shape[1] != self.d_model:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         batch = u_t.shape[0]
-        w_in, w_out = self._weights(u_t.dtype)
+        _, w_in, w_out, _, limit = self._converted(u_t.dtype)
         if fused is None:
-            fused = batch <= self._weights_cache[4] and u_t.is_cuda and u_t.data_ptr() % 16 == 0
+            fused = batch <= limit and u_t.is_cuda and u_t.data_ptr() % 16 == 0
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches
             # (a captured step of more streams forms A at every replay, as one of stage kernels does)
             fresh = batch > STEP_CACHED_A_MAX_BATCH and torch.cuda.is_current_stream_capturing()
@@ -643,7 +646,7 @@ class GraphedBlockStep:
             return block_step(self.u, self.weights[0], block.conv_w, block.conv_b, block.dt_bias, self.A, block.D, block.norm_w,
                               self.weights[1], state.conv, state.ssm.state, block.H, block.P, block.N, block.G, block.eps)
 
-        if batch <= block._weights_cache[4] and block_step_supported(self.u, block.d_inner, block.N):
+        if batch <= block._converted(dtype)[4] and block_step_supported(self.u, block.d_inner, block.N):
             self.A, self.A_key = block.A, (block.A_log._version, block.A_log.data_ptr())
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
