@@ -249,13 +249,15 @@ FUSED_STEP_MAX_BATCH_OTHER = 256
 STEP_CACHED_A_MAX_BATCH = 64
 
 
-def _step_max_batch(dtype: torch.dtype, d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
+_STEP_DTYPES = (torch.bfloat16, torch.float32)
+
+
+def _step_max_batch(d_model: int, nheads: int, headdim: int, dstate: int, ngroups: int) -> int:
     """The largest batch whose step is taken as one launch, by the kernel that the library runs for the shape (0: it takes none,
     or the launch's vectors, as it lays them out, do not fit the 64 KB of LDS that it asks for)."""
     d_inner, E = nheads * headdim, in_proj_width(nheads, headdim, dstate, ngroups)
     vectors = d_model + E + (E - d_inner - nheads) + (nheads + 3) // 4 * 4 + d_inner + 16
-    if (dtype not in (torch.bfloat16, torch.float32) or d_model not in (128, 256) or d_inner not in (128, 256) or dstate % 16
-            or 4 * vectors > 64 * 1024):
+    if d_model not in (128, 256) or d_inner not in (128, 256) or dstate % 16 or 4 * vectors > 64 * 1024:
         return 0
     return FUSED_STEP_MAX_BATCH if dstate == 64 and E <= 768 else FUSED_STEP_MAX_BATCH_OTHER
 
@@ -449,6 +451,7 @@ class Mamba2Block:
         self.d_conv, self.chunk, self.eps = d_conv, chunk, eps
         self.d_inner = nheads * headdim
         self.conv_dim = self.d_inner + 2 * ngroups * dstate
+        self._step_limit = _step_max_batch(d_model, nheads, headdim, dstate, ngroups)
         E = in_proj_width(nheads, headdim, dstate, ngroups)
         g = torch.Generator(device="cpu")
         g.manual_seed(seed)
@@ -566,9 +569,7 @@ class Mamba2Block:
         if cached is None or cached[0] != key:
             w_in, w_out = self.in_proj.to(dtype).contiguous(), self.out_proj.to(dtype).contiguous()
             # (with them: the batch up to which a step is one launch, whose kernel reads both 16 bytes at a time)
-            limit = _step_max_batch(dtype, self.d_model, self.H, self.P, self.N, self.G)
-            if (w_in.data_ptr() | w_out.data_ptr()) % 16:
-                limit = 0
+            limit = self._step_limit if dtype in _STEP_DTYPES and (w_in.data_ptr() | w_out.data_ptr()) % 16 == 0 else 0
             cached = (key, w_in, w_out, w_out.t().contiguous(), limit)
             self._weights_cache = cached
         return cached
