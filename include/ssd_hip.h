@@ -79,7 +79,8 @@ char *ssd_get_and_reset_last_err(void);
 /* Bytes of scratch ssd_chunk_scan_fwd needs for these dims.  The reference lets ATen allocate
  * op temporaries; a capturable op cannot, so the caller owns the buffer (the Rust side would
  * hold it as a Tensor::empty, cf. the persistent rollout buffers at
- * trading_bots/src/torch/train/trainer.rs:622-944). */
+ * trading_bots/src/torch/train/trainer.rs:622-944).  (A float32 forward that runs on the staged kernels uses chunks of 64
+ * steps, and runs faster, if the workspace has room for them: what this function names for dims with chunk 64, where that is more.) */
 int ssd_workspace_bytes(const ssd_dims *dims, size_t *out_bytes);
 
 /* Whole forward: stages 1-4 on one stream.  Fills y and, when non-NULL, final_states.

@@ -1,0 +1,113 @@
+"""The staged forward in two or three launches (stages 2 and 4 work out the decays themselves; stage 4 runs the recurrence over
+the chunks where they are few) at the edges of its dispatch, against the float64 sequential oracle and against the stages
+called one by one, which share the same arithmetic up to the order of float32 sums."""
+import pytest
+import torch
+
+from trading_bot_0_amd import ssd, ssd_chunk_scan
+from trading_bot_0_amd.synthetic import Workload, make_inputs
+
+from _util import assert_close, check_y, np64, oracle_scan, to_dev
+from oracle import c_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+# (batch, seqlen, heads, headdim, dstate, groups, chunk): one chunk; a batch of the recurrence and one over (2, 3, 4, 5 chunks);
+# the last chunk of one step; heads of 8, 24 and 64; every state width; more chunks than are folded (33), than one round of the
+# separate recurrence holds (65) and a run of it that is cut short (18); more tiles, and more bytes, than are folded
+SHAPES = [(1, 1, 1, 8, 16, 1, 32), (3, 70, 4, 24, 16, 1, 128), (2, 129, 2, 64, 128, 1, 64), (2, 161, 8, 32, 64, 1, 32),
+          (2, 320, 4, 16, 32, 2, 64), (1, 130, 3, 40, 128, 3, 128), (2, 33 * 32, 2, 16, 16, 1, 32), (1, 65 * 32 - 5, 2, 32, 64, 1, 32),
+          (2, 18 * 64 - 63, 2, 8, 64, 2, 64), (70, 8 * 64, 8, 16, 16, 1, 64), (3, 256 * 3 + 1, 16, 64, 128, 2, 256),
+          (3, 290, 8, 32, 64, 1, 128)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_against_the_oracle(shape, dtype):
+    B, L, H, P, N, G, Q = shape
+    if dtype == "f32" and P * N * Q > 64 * 128 * 64:
+        Q = 64   # (float32 tiles of the largest head sizes do not fit the LDS)
+    w = Workload("staged", B, L, H, P, N, G, Q, dtype=dtype, init_std=0.5)
+    cpu = make_inputs(w, seed=L)
+    dev = to_dev(cpu)
+    g = torch.Generator().manual_seed(L)
+    mask = torch.rand(B, L, generator=g) < 0.02
+    mask[0, 0] = True                                   # a row whose initial state is not read ...
+    dev["init"][0] = float("nan")                       # ... whatever it holds
+    cpu["init"][0] = 0.0
+    yr, fr = c_oracle_reset(cpu, mask)
+    finals = []
+
+    def call(yd):
+        y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=Q, initial_states=dev["init"],
+                              reset=mask.cuda(), y_dtype=yd)
+        finals.append(f)
+        return y
+
+    check_y(call, yr, w.torch_dtype, f"{shape} y")
+    assert_close(finals[0], fr, w.torch_dtype, f"{shape} final")
+    y0, f0 = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=Q, initial_states=dev["init"],
+                            reset=mask.cuda(), return_final_states=False)
+    assert f0 is None and torch.equal(y0, call(None))   # (a final state that is not asked for changes nothing)
+
+
+def c_oracle_reset(cpu, mask):
+    """Row by row and episode by episode through the sequential oracle."""
+    import numpy as np
+
+    x, dt, A, Bm, Cm, D, init = (np64(cpu[k]) for k in ("x", "dt", "A", "B", "C", "D", "init"))
+    Bsz, L = mask.shape
+    y, fin = np.zeros_like(x), np.zeros((Bsz,) + init.shape[1:])
+    for b in range(Bsz):
+        cuts = [0] + [t for t in range(1, L) if mask[b, t]] + [L]
+        state = init[b:b + 1] * 0.0 if mask[b, 0] else init[b:b + 1]
+        for t0, t1 in zip(cuts, cuts[1:]):
+            yb, state = c_oracle.ssd_sequential_c(x[b:b + 1, t0:t1].copy(), dt[b:b + 1, t0:t1].copy(), A, Bm[b:b + 1, t0:t1].copy(),
+                                                  Cm[b:b + 1, t0:t1].copy(), D, state.copy(), nthreads=1)
+            y[b, t0:t1] = yb[0]
+            last = state
+            state = np.zeros_like(state)
+        fin[b] = last[0]
+    return y, fin
+
+
+@pytest.mark.parametrize("seqlen", [100, 400, 2000])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_final_state_written_over_the_initial_state(seqlen, dtype):
+    """A stream's prefix that continues a state in place: the same buffer as initial and final state, at lengths whose separate
+    buffers would take the recurrence inside stage 4."""
+    w = Workload("inplace", 3, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
+    cpu = make_inputs(w, seed=3)
+    dev = to_dev(cpu)
+    yr, fr = oracle_scan(cpu)
+    for _ in range(4):
+        state = dev["init"].clone()
+        y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=128, initial_states=state,
+                              final_out=state, y_dtype=torch.float32)
+        assert f.data_ptr() == state.data_ptr()
+        assert_close(y, yr, w.torch_dtype, "y")
+        assert_close(state, fr, w.torch_dtype, "final")
+
+
+@pytest.mark.parametrize("nc", [1, 7, 8, 9, 15, 17, 63, 64, 65, 129, 200])
+def test_state_passing_runs(nc):
+    """The recurrence over the chunks in parallel runs: numbers of chunks around the runs' lengths and whole rounds, in place and
+    not, against float64 (float32 sums of terms that decay: 1e-5 of the largest is four times what it shows)."""
+    g = torch.Generator().manual_seed(nc)
+    B, H, P, N, Q = 2, 3, 8, 16, 32
+    S = torch.randn(B, nc, H, P, N, generator=g)
+    init = torch.randn(B, H, P, N, generator=g)
+    dt = torch.rand(B, nc * Q, H, generator=g) * 0.05
+    A = -torch.rand(H, generator=g) - 0.1
+    dtcs = ssd.chunk_cumsum(dt.cuda(), A.cuda(), Q)
+    dec = torch.exp2((dtcs[:, :, :, 0, -1].double() + dtcs[:, :, :, 1, -1].double()).cpu())   # [B,H,nc]
+    st, ref = init.double(), []
+    for c in range(nc):
+        ref.append(st)
+        st = dec[:, :, c, None, None] * st + S[:, c].double()
+    ref = torch.stack(ref, 1)
+    for in_place in (False, True):
+        prev, fin = ssd.state_passing(S.cuda(), dtcs, init.cuda(), in_place=in_place)
+        assert (prev.cpu().double() - ref).abs().max() <= 1e-5 * ref.abs().max()
+        assert (fin.cpu().double() - st).abs().max() <= 1e-5 * st.abs().max()

@@ -124,6 +124,19 @@ Workspace carve(const ssd::ScanShape &s) {
     return w;
 }
 
+// The chunk the staged forward runs on.  In float32 a chunk's scores cost a quarter of the time they take in bf16 as states would:
+// chunks of 64 instead of the caller's 128 (8 heads of 32, state 64: 3 x 300 steps 21 -> 17 us, 10 x 3 000 102 -> 86, 60 x 300
+// 76 -> 61, 5 x 1 500 as fast), where the scratch holds their states: ssd_workspace_bytes of the caller's own chunk does not, that
+// of chunk 64 does.  (Wider states go the other way: heads of 64, state 128,
+// 4 x 2 000 172 -> 219.)
+ssd::ScanShape staged_shape(const ssd::ScanShape &s, int dtype, size_t scratch_bytes) {
+    ssd::ScanShape f = s;
+    f.Q = 64;
+    f.nc = (s.L + 63) / 64;
+    if (dtype != SSD_DTYPE_F32 || s.Q <= 64 || s.P * s.N > 2048 || (int64_t)f.B * f.nc * f.H > 0x7fffffff) return s;
+    return carve(f).total <= scratch_bytes ? f : s;
+}
+
 bool takes_one_pass(const ssd::ScanShape &s, int dtype) {
     int segments;
     return ssd::fused_scan_plan(s, dtype, &segments) == 1;
@@ -156,10 +169,61 @@ int static_scratch_address(void **out) {
     return SSD_OK;
 }
 
+// Whether stage 4 also runs the recurrence over the chunks, in place of a launch of its own that reads and writes every chunk's
+// state: every tile then reads the states of all chunks before its own, so it pays while those reads stay small.  Measured, folded
+// against separate (us of the GPU): 8 heads of 32, state 64, 3 x 300 steps 13.1 / 16, 8 x 2 048 (64 MB of reads) 24.1 / 30.3, 20 x 1 000
+// 29.2 / 37.2, 4 x 4 096 (134 MB) 31.7 / 29.9; 4 heads of 16, state 16, 20 x 2 000 (32 chunks) 31.2 / 32.6, 100 x 1 000 (6 400 tiles)
+// 66.2 / 62.5; 16 heads of 64, state 128, 4 x 2 000 (67 MB) 51.7 / 59.5, 2 x 4 000 (134 MB) 62.2 / 57.4.
+constexpr int kFoldMaxChunks = 32, kFoldMaxTiles = 4096;
+constexpr int64_t kFoldMaxBytes = (int64_t)72 << 20;
+
+bool fold_states(const ssd::ScanShape &s) {
+    const int64_t tiles = (int64_t)s.B * s.H * s.nc;
+    return s.nc <= kFoldMaxChunks && tiles <= kFoldMaxTiles && tiles * (s.nc / 2) * s.P * s.N * 4 <= kFoldMaxBytes;
+}
+
+// The forward in two or three launches, stages 2 and 4 working out the decays themselves (short batches are bound by launches,
+// each some 4 us of the host and a start, a trip to memory and a drain of the chip; four launches -> as here, back to back: 4 heads
+// of 16, 4 x 256 steps, float32 24.7 -> 18.5 us, 8 heads of 32, state 64, bf16, 3 x 300 24.4 -> 18.6, 8 x 2 048 34.6 -> 23.2, 2 x 9 000
+// 45.2 -> 35.2; 16 heads of 64, state 128, 2 x 500 35.4 -> 23.9, 4 x 4 000 100 -> 96.  Batches of 512 sequences and more, whose stages 2
+// and 3 were one kernel that spills its registers: 4 heads of 16, bf16, 150 x 3 000 158 -> 109, float32 300 x 300 68 -> 63,
+// 500 x 500 135 -> 138).  keep_prev: the states entering the
+// chunks are wanted in `states`.
+int run_staged_own(const ssd::ScanShape &s, int dtype, const void *x, const void *dt, const float *A, const void *Bm, const void *Cm,
+                   const float *D, const float *initial_states, const uint8_t *reset, void *y, float *final_states, float *alpha_end,
+                   float *states, hipStream_t st, bool keep_prev) {
+    ssd::ScanShape sp = s;
+    sp.fresh = reset;
+    ssd::OwnDecays own;
+    own.dt = dt;
+    own.A = A;
+    own.reset = reset;
+    own.alpha_end = alpha_end;
+    hipError_t e = ssd::launch_chunk_state_own(s, dtype, x, Bm, own, states, st);
+    if (e != hipSuccess) return hip_fail(e, "chunk_state launch");
+    // Every tile of a sequence reads its initial state, so a final state written over it (as a stream's prefix does that
+    // continues a state in place) would reach tiles that have not read it yet: those calls take the separate stage 3.
+    const size_t state_floats = (size_t)s.B * s.H * s.P * s.N;
+    const bool in_place = initial_states != nullptr && final_states != nullptr && initial_states < final_states + state_floats &&
+                          final_states < initial_states + state_floats;
+    own.fold = !keep_prev && !in_place && fold_states(s);
+    own.init = initial_states;
+    own.final_states = final_states;
+    if (!own.fold) {
+        e = ssd::launch_state_passing(sp, states, alpha_end, 1, initial_states, states, final_states, st);  // in place
+        if (e != hipSuccess) return hip_fail(e, "state_passing launch");
+    }
+    e = ssd::launch_chunk_scan_own(sp, dtype, x, Bm, Cm, own, states, D, y, st);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "chunk_scan launch");
+}
+
 // Stages 1-4 one after the other.  mode as for launch_chunk_cumsum (0 = the forward's decays and weights).
 int run_staged(const ssd::ScanShape &s, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
                const void *Cm, const float *D, const float *initial_states, const uint8_t *reset, int mode, void *y,
-               float *final_states, float *dtcs, float *states, hipStream_t st, int dt_len = 0) {
+               float *final_states, float *dtcs, float *states, hipStream_t st, int dt_len = 0,
+               bool keep_prev = false) {
+    if (mode == 0 && ssd::own_decays_supported(s, dtype == SSD_DTYPE_F32 ? 4 : 2))
+        return run_staged_own(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, dtcs, states, st, keep_prev);
     hipError_t e = ssd::launch_chunk_cumsum(s, dtype, dt, A, reset, dtcs, st, mode, dt_len);
     if (e != hipSuccess) return hip_fail(e, "chunk_cumsum launch");
     ssd::ScanShape sp = s;  // for the kernels that read the initial state
@@ -171,7 +235,7 @@ int run_staged(const ssd::ScanShape &s, int dtype, const void *x, const void *dt
     } else {
         e = ssd::launch_chunk_state(s, dtype, x, Bm, dtcs, states, st);
         if (e != hipSuccess) return hip_fail(e, "chunk_state launch");
-        e = ssd::launch_state_passing(sp, states, dtcs, initial_states, states, final_states, st);  // in place
+        e = ssd::launch_state_passing(sp, states, dtcs + s.Q - 1, 4 * s.Q, initial_states, states, final_states, st);  // in place
         if (e != hipSuccess) return hip_fail(e, "state_passing launch");
     }
     e = ssd::launch_chunk_scan(s, dtype, x, Bm, Cm, dtcs, states, D, y, st);
@@ -419,7 +483,7 @@ int ssd_state_passing_fwd(const ssd_dims *dims, const float *chunk_states, const
     REQUIRE_PTR(prev_states);
     OPTIONAL_PTR(initial_states);
     OPTIONAL_PTR(final_states);
-    hipError_t e = ssd::launch_state_passing(s, chunk_states, dtcs, initial_states, prev_states, final_states,
+    hipError_t e = ssd::launch_state_passing(s, chunk_states, dtcs + s.Q - 1, 4 * s.Q, initial_states, prev_states, final_states,
                                              (hipStream_t)hip_stream);
     return e == hipSuccess ? SSD_OK : hip_fail(e, "state_passing launch");
 }
@@ -464,15 +528,12 @@ size_t scan_scratch_bytes(const ssd::ScanShape &s, int dtype) {
     return carve(s).total;
 }
 
-// The forward proper, arguments checked: the way the plan says for this shape, with `workspace` (carve(s).total bytes,
-// or anything at all when scan_scratch_bytes says the shape needs none) as scratch.
+// The forward proper, arguments checked: the way the plan says for this shape, with `workspace` (carve(s).total bytes or
+// more, or anything at all when scan_scratch_bytes says the shape needs none) as scratch.
 static int scan_forward(const ssd::ScanShape &s, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
                         const void *Cm, const float *D, const float *initial_states, const uint8_t *reset, void *y,
-                        float *final_states, void *workspace, hipStream_t st) {
-    const Workspace w = carve(s);
+                        float *final_states, void *workspace, size_t workspace_bytes, hipStream_t st) {
     char *base = static_cast<char *>(workspace);
-    float *dtcs = reinterpret_cast<float *>(base + w.dtcs_off);
-    float *states = reinterpret_cast<float *>(base + w.st_off);
     // One batch of sequences, the way the plan says.  The workspace is carved for the whole batch and so holds any
     // part of it.
     auto forward = [&](const ssd::ScanShape &part, const void *px, const void *pdt, const void *pb, const void *pc,
@@ -494,7 +555,10 @@ static int scan_forward(const ssd::ScanShape &s, int dtype, const void *x, const
                                                  seg_states, seg_decay, st);
             return e == hipSuccess ? SSD_OK : hip_fail(e, "segmented one-pass scan launch");
         }
-        return run_staged(part, dtype, px, pdt, A, pb, pc, D, pinit, preset, 0, py, pfinal, dtcs, states, st);
+        const ssd::ScanShape on = staged_shape(part, dtype, workspace_bytes);
+        const Workspace w = carve(on);
+        return run_staged(on, dtype, px, pdt, A, pb, pc, D, pinit, preset, 0, py, pfinal, reinterpret_cast<float *>(base + w.dtcs_off),
+                          reinterpret_cast<float *>(base + w.st_off), st);
     };
     // A batch that fills the chip some whole number of times and a bit: the whole rounds run as one launch of the
     // one-pass kernel, the rest as a batch of its own (cut into segments or staged, as the plan says for it) -- a
@@ -543,7 +607,7 @@ int ssd_chunk_scan_reset_fwd(const ssd_dims *dims, int dtype, const void *x, con
     const Workspace w = carve(s);
     if (workspace_bytes < w.total)
         return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, w.total);
-    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, workspace,
+    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, workspace, workspace_bytes,
                         (hipStream_t)hip_stream);
 }
 
@@ -561,7 +625,7 @@ int ssd_chunk_scan_noalloc_fwd(const ssd_dims *dims, int dtype, const void *x, c
     SSD_SCAN_POINTER_CHECKS;
     void *scratch = nullptr;
     if (int rc = static_scratch_address(&scratch)) return rc;
-    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch,
+    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, kStaticScratchBytes,
                         (hipStream_t)hip_stream);
 }
 
@@ -685,7 +749,7 @@ int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const voi
                                                      keep_states ? sstates : nullptr);
             return err == hipSuccess ? SSD_OK : hip_fail(err, "one-pass scan launch (backward)");
         }
-        return run_staged(shape, inner, sx, sdt, sA, sb, sc, nullptr, sinit, reset, mode, sy, sfinal, dtcs, sstates, st, s.L);
+        return run_staged(shape, inner, sx, sdt, sA, sb, sc, nullptr, sinit, reset, mode, sy, sfinal, dtcs, sstates, st, s.L, true);
     };
     if (sT.H > s.H) {
         BWD_LAUNCH(ssd::launch_replicate_columns(el, dt, at(w.dt_parts), (long long)s.B * s.L, s.H, sT.H / s.H, st), "dt per part");

@@ -27,6 +27,8 @@
 // Persistent and software-pipelined like stage 2: the next tile's B, x, entering state and
 // alpha rows sit in registers while the current tile's MFMAs run.  Everything that shapes the
 // inner code (head-dim blocks, state width, chunk length) is a template parameter.
+// OWN: the tile's decays are worked out here from dt (wave 0, between the tile's first two barriers) instead of being read from
+// stage 1's output, and with own.fold the entering state from the chunks' own states (see OwnDecays).
 // y leaves in 16-byte pieces: the two lanes that hold one output column swap halves of their
 // values (v_permlane32_swap) so that each stores 8 consecutive head-dim elements.
 #pragma once
@@ -34,10 +36,10 @@
 
 namespace ssd {
 
-template <typename T, typename TO, int PB, int NK, int QB>  // Ppad = 32*PB >= P, N = 16*NK, Q = 32*QB
+template <typename T, typename TO, int PB, int NK, int QB, bool OWN>  // Ppad = 32*PB >= P, N = 16*NK, Q = 32*QB
 __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >= 4) ? 3 : 2) void chunk_scan_kernel(
     const T *__restrict__ x, const T *__restrict__ Bm, const T *__restrict__ Cm, const float *__restrict__ dtcs,
-    const float *__restrict__ prev, const float *__restrict__ D, TO *__restrict__ y, ScanShape s) {
+    OwnDecays own, const float *__restrict__ prev, const float *__restrict__ D, TO *__restrict__ y, ScanShape s) {
     constexpr int VEC = Vec16<T>::N;
     constexpr int PARTS = Split<T>::PARTS;
     constexpr int N = NK * 16, Ppad = PB * 32, Q = QB * 32, nthr = 64 * QB, nblk = QB;
@@ -70,14 +72,72 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
     const int htotal = s.P * hcpr;
 
     // ---- registers holding the next tile's inputs ----
-    float a3[2];
+    float a3[OWN ? 1 : 2];
+    ChunkSteps<T, Q> steps;  // OWN: dt and restarts (wave 0)
     Vec16<T> bv[UB], xv[UX];
     float4 hv[UH];
+    // own.fold: `prev` holds what every chunk adds to the state, and a tile works out the state entering its chunk by the
+    // recurrence over the chunks before it (the float operations of state_passing_kernel in their order); the tile of the
+    // last chunk goes one chunk further, to the final state.  This thread's pieces idx0, idx0 + nthr, ...
+    auto enter = [&](const Tile &t, int idx0, float4(&st)[UH]) __attribute__((always_inline)) {
+        const size_t bh = (size_t)t.b * s.H + t.h;
+        const bool fresh = s.fresh != nullptr && s.fresh[(size_t)t.b * s.L] != 0;  // restarts before its first step
+        const float4 *ip = own.init != nullptr && !fresh ? reinterpret_cast<const float4 *>(own.init) + bh * htotal : nullptr;
+        unsigned at[UH];
+#pragma unroll
+        for (int u = 0; u < UH; ++u) {
+            at[u] = (unsigned)min(idx0 + u * nthr, htotal - 1);  // (pieces past the state are read as its last one and not used)
+            st[u] = ip != nullptr ? ip[at[u]] : make_float4(0, 0, 0, 0);
+        }
+        const float4 *hp = reinterpret_cast<const float4 *>(prev) + ((size_t)t.b * s.nc * s.H + t.h) * htotal;
+        const size_t cstep = (size_t)s.H * htotal;
+        const float *ae = own.alpha_end + bh * s.nc;
+        auto fold = [&](int j0, auto count) __attribute__((always_inline)) {  // chunks j0 .. j0 + count - 1, all of their loads in flight at once
+            constexpr int CN = decltype(count)::value;
+            float4 sv[CN][UH];
+#pragma unroll
+            for (int j = 0; j < CN; ++j) {
+#pragma unroll
+                for (int u = 0; u < UH; ++u) sv[j][u] = hp[(size_t)(j0 + j) * cstep + at[u]];
+            }
+#pragma unroll
+            for (int j = 0; j < CN; ++j) {
+                const float dec = exp2_hw(ae[j0 + j]);
+#pragma unroll
+                for (int u = 0; u < UH; ++u) {
+                    st[u].x = dec * st[u].x + sv[j][u].x;
+                    st[u].y = dec * st[u].y + sv[j][u].y;
+                    st[u].z = dec * st[u].z + sv[j][u].z;
+                    st[u].w = dec * st[u].w + sv[j][u].w;
+                }
+            }
+        };
+        int j = 0;
+        constexpr int BATCH = UH <= 2 ? 4 : 2;
+        for (; j + BATCH <= t.c; j += BATCH) fold(j, std::integral_constant<int, BATCH>{});
+        for (; j < t.c; ++j) fold(j, std::integral_constant<int, 1>{});
+        if (t.c == s.nc - 1 && own.final_states != nullptr) {
+            float4 keep[UH];
+#pragma unroll
+            for (int u = 0; u < UH; ++u) keep[u] = st[u];
+            fold(t.c, std::integral_constant<int, 1>{});
+            float4 *fp = reinterpret_cast<float4 *>(own.final_states) + bh * htotal;
+#pragma unroll
+            for (int u = 0; u < UH; ++u) {
+                if (idx0 + u * nthr < htotal) fp[idx0 + u * nthr] = st[u];
+                st[u] = keep[u];
+            }
+        }
+    };
     auto prefetch = [&](int logical) {
         const Tile t = decode_tile(logical, s);
-        const float *arow = dtcs + ((((size_t)t.b * s.H + t.h) * s.nc + t.c) * 4) * Q;
-        a3[0] = (tid < 3 * Q) ? arow[tid] : 0.f;
-        a3[1] = (tid + nthr < 3 * Q) ? arow[tid + nthr] : 0.f;
+        if constexpr (OWN) {
+            if (wave == 0) steps.load(static_cast<const T *>(own.dt), own.reset, t, s, lane);
+        } else {
+            const float *arow = dtcs + ((((size_t)t.b * s.H + t.h) * s.nc + t.c) * 4) * Q;
+            a3[0] = (tid < 3 * Q) ? arow[tid] : 0.f;
+            a3[1] = (tid + nthr < 3 * Q) ? arow[tid + nthr] : 0.f;
+        }
         const int rows = min(Q, s.L - t.t0);  // valid rows of a ragged last chunk
         const T *bb = Bm + (((size_t)t.b * s.L + t.t0) * s.G + t.g) * N;
         const T *xb = x + (((size_t)t.b * s.L + t.t0) * s.H + t.h) * s.P;
@@ -94,6 +154,7 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
             for (int u = 0; u < UX; ++u)
                 xv[u] = (xslot && xl0 + u * xrpp < rows) ? load_vec16(xb + xoff0 + u * xstep) : zero_vec16<T>();
         }
+        if (OWN && own.fold) return;
         const float4 *hp = reinterpret_cast<const float4 *>(prev + ((((size_t)t.b * s.nc + t.c) * s.H + t.h) * s.P) * N);
 #pragma unroll
         for (int u = 0; u < UH; ++u) {
@@ -132,6 +193,18 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
         const int rows = min(Q, s.L - t.t0);
         const int lb = (wave + logical) % nblk;  // this wave's column block
         const int l = lb * 32 + r;
+        block_sync_lds();  // the previous tile's LDS reads are done (and the zero fill is visible)
+        if (OWN && own.fold) {
+            // (here rather than in the prefetch, and ahead of the loads of C: across the products below or beside C, the chunks in
+            // flight would not fit the registers)
+            for (int idx = tid; idx < htotal; idx += UH * nthr) {
+                float4 h4[UH];
+                enter(t, idx, h4);
+#pragma unroll
+                for (int u = 0; u < UH; ++u)
+                    if (idx + u * nthr < htotal) put_state(idx + u * nthr, h4[u]);
+            }
+        }
         // C fragments straight from global: column l of the tile, K = n
         Frag<T> Cf[NK];
         {
@@ -144,11 +217,25 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
                 for (int kk = 0; kk < NK; ++kk) Cf[kk] = (l < rows) ? load_frag(crow + kk * 16) : zero_frag<T>();
             }
         }
-
-        block_sync_lds();  // the previous tile's LDS reads are done (and the zero fill is visible)
         // ---- registers -> LDS ----
-        if (tid < 3 * Q) al_s[tid] = a3[0];
-        if (tid + nthr < 3 * Q) al_s[tid + nthr] = a3[1];
+        if constexpr (OWN) {
+            if (wave == 0) {
+                constexpr int EPL = ChunkScan<Q>::EPL;
+                float dtv[EPL], drop[EPL];
+                steps.values(t, s, lane, dtv, drop);
+                const ChunkScan<Q> sc(dtv, drop, (double)own.A[t.h]);
+                if (lane * EPL < Q) {
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) {
+                        sc.alpha(e, al_s[lane * EPL + e], al_s[Q + lane * EPL + e]);
+                        al_s[2 * Q + lane * EPL + e] = dtv[e];
+                    }
+                }
+            }
+        } else {
+            if (tid < 3 * Q) al_s[tid] = a3[0];
+            if (tid + nthr < 3 * Q) al_s[tid + nthr] = a3[OWN ? 0 : 1];
+        }
 #pragma unroll
         for (int u = 0; u < UB; ++u)
             *reinterpret_cast<uint4 *>(Bs + (bl0 + u * brpp) * ldb + bch * VEC) = bv[u].u;
@@ -162,14 +249,16 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
                 for (int i = 0; i < VEC; ++i) xs[(xch * VEC + i) * ldx + sr] = xv[u].e[i];
             }
         }
+        if (!(OWN && own.fold)) {
 #pragma unroll
-        for (int u = 0; u < UH; ++u) {
-            const int idx = u * nthr + tid;
-            if (idx < htotal) put_state(idx, hv[u]);
-        }
-        if constexpr (UHfull > UH) {  // the part of the entering state the register batch does not hold
-            const float4 *hp = reinterpret_cast<const float4 *>(prev + ((((size_t)t.b * s.nc + t.c) * s.H + t.h) * s.P) * N);
-            for (int idx = UH * nthr + tid; idx < htotal; idx += nthr) put_state(idx, hp[idx]);
+            for (int u = 0; u < UH; ++u) {
+                const int idx = u * nthr + tid;
+                if (idx < htotal) put_state(idx, hv[u]);
+            }
+            if constexpr (UHfull > UH) {  // the part of the entering state the register batch does not hold
+                const float4 *hp = reinterpret_cast<const float4 *>(prev + ((((size_t)t.b * s.nc + t.c) * s.H + t.h) * s.P) * N);
+                for (int idx = UH * nthr + tid; idx < htotal; idx += nthr) put_state(idx, hp[idx]);
+            }
         }
         block_sync_lds();  // alpha and dt are visible
         // decay table: row k holds F_k[s] for the rows at or below column block k
@@ -308,52 +397,52 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
 // ------------------------------------------------------------------------------------------
 // Launchers (one translation unit per input/output type pair instantiates scan_dispatch)
 // ------------------------------------------------------------------------------------------
-template <typename T, typename TO, int PB, int NK, int QB>
+template <typename T, typename TO, int PB, int NK, int QB, bool OWN>
 static hipError_t scan_launch(const ScanShape &s, const void *x, const void *Bm, const void *Cm,
-                              const float *dtcs, const float *prev, const float *D, void *y, hipStream_t st) {
+                              const float *dtcs, const OwnDecays &own, const float *prev, const float *D, void *y, hipStream_t st) {
     const size_t lds = chunk_scan_lds_bytes(s, sizeof(T));
-    hipError_t e = allow_lds(chunk_scan_kernel<T, TO, PB, NK, QB>, lds);
+    hipError_t e = allow_lds(chunk_scan_kernel<T, TO, PB, NK, QB, OWN>, lds);
     if (e != hipSuccess) return e;
     int grid = 1;
-    e = persistent_grid(chunk_scan_kernel<T, TO, PB, NK, QB>, 64 * QB, lds, s.B * s.nc * s.H, &grid);
+    e = persistent_grid(chunk_scan_kernel<T, TO, PB, NK, QB, OWN>, 64 * QB, lds, s.B * s.nc * s.H, &grid);
     if (e != hipSuccess) return e;
-    chunk_scan_kernel<T, TO, PB, NK, QB><<<dim3(grid), dim3(64 * QB), lds, st>>>(
-        static_cast<const T *>(x), static_cast<const T *>(Bm), static_cast<const T *>(Cm), dtcs, prev, D,
+    chunk_scan_kernel<T, TO, PB, NK, QB, OWN><<<dim3(grid), dim3(64 * QB), lds, st>>>(
+        static_cast<const T *>(x), static_cast<const T *>(Bm), static_cast<const T *>(Cm), dtcs, own, prev, D,
         static_cast<TO *>(y), s);
     return hipGetLastError();
 }
 
-template <typename T, typename TO, int PB, int NK>
+template <typename T, typename TO, int PB, int NK, bool OWN>
 static hipError_t scan_dispatch_q(const ScanShape &s, const void *x, const void *Bm, const void *Cm,
-                                  const float *dtcs, const float *prev, const float *D, void *y,
+                                  const float *dtcs, const OwnDecays &own, const float *prev, const float *D, void *y,
                                   hipStream_t st) {
     switch (s.Q) {
-        case 32: return scan_launch<T, TO, PB, NK, 1>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 64: return scan_launch<T, TO, PB, NK, 2>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 128: return scan_launch<T, TO, PB, NK, 4>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 256: return scan_launch<T, TO, PB, NK, 8>(s, x, Bm, Cm, dtcs, prev, D, y, st);
+        case 32: return scan_launch<T, TO, PB, NK, 1, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 64: return scan_launch<T, TO, PB, NK, 2, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 128: return scan_launch<T, TO, PB, NK, 4, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 256: return scan_launch<T, TO, PB, NK, 8, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <typename T, typename TO, int PB>
+template <typename T, typename TO, int PB, bool OWN>
 static hipError_t scan_dispatch_n(const ScanShape &s, const void *x, const void *Bm, const void *Cm,
-                                  const float *dtcs, const float *prev, const float *D, void *y,
+                                  const float *dtcs, const OwnDecays &own, const float *prev, const float *D, void *y,
                                   hipStream_t st) {
     switch (s.N) {
-        case 16: return scan_dispatch_q<T, TO, PB, 1>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 32: return scan_dispatch_q<T, TO, PB, 2>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 64: return scan_dispatch_q<T, TO, PB, 4>(s, x, Bm, Cm, dtcs, prev, D, y, st);
-        case 128: return scan_dispatch_q<T, TO, PB, 8>(s, x, Bm, Cm, dtcs, prev, D, y, st);
+        case 16: return scan_dispatch_q<T, TO, PB, 1, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 32: return scan_dispatch_q<T, TO, PB, 2, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 64: return scan_dispatch_q<T, TO, PB, 4, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
+        case 128: return scan_dispatch_q<T, TO, PB, 8, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <typename T, typename TO>
-hipError_t scan_dispatch(const ScanShape &s, const void *x, const void *Bm, const void *Cm, const float *dtcs,
+template <typename T, typename TO, bool OWN = false>
+hipError_t scan_dispatch(const ScanShape &s, const void *x, const void *Bm, const void *Cm, const float *dtcs, const OwnDecays &own,
                          const float *prev, const float *D, void *y, hipStream_t st) {
-    return (s.P <= 32) ? scan_dispatch_n<T, TO, 1>(s, x, Bm, Cm, dtcs, prev, D, y, st)
-                       : scan_dispatch_n<T, TO, 2>(s, x, Bm, Cm, dtcs, prev, D, y, st);
+    return (s.P <= 32) ? scan_dispatch_n<T, TO, 1, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st)
+                       : scan_dispatch_n<T, TO, 2, OWN>(s, x, Bm, Cm, dtcs, own, prev, D, y, st);
 }
 
 }  // namespace ssd

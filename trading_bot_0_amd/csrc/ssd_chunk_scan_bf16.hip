@@ -5,7 +5,12 @@ namespace ssd {
 
 hipError_t launch_chunk_scan_bf16(const ScanShape &s, const void *x, const void *Bm, const void *Cm,
                                   const float *dtcs, const float *prev, const float *D, void *y, hipStream_t st) {
-    return scan_dispatch<__bf16, __bf16>(s, x, Bm, Cm, dtcs, prev, D, y, st);
+    return scan_dispatch<__bf16, __bf16>(s, x, Bm, Cm, dtcs, OwnDecays{}, prev, D, y, st);
+}
+
+hipError_t launch_chunk_scan_own_bf16(const ScanShape &s, const void *x, const void *Bm, const void *Cm, const OwnDecays &own,
+                                  const float *prev, const float *D, void *y, hipStream_t st) {
+    return scan_dispatch<__bf16, __bf16, true>(s, x, Bm, Cm, nullptr, own, prev, D, y, st);
 }
 
 size_t chunk_scan_lds_bytes(const ScanShape &s, int eb) {
@@ -26,6 +31,20 @@ hipError_t launch_chunk_scan(const ScanShape &s, int dtype, const void *x, const
         case 0: return launch_chunk_scan_f32(s, x, Bm, Cm, dtcs, prev, D, y, st);
         case 1: return launch_chunk_scan_bf16(s, x, Bm, Cm, dtcs, prev, D, y, st);
         default: return launch_chunk_scan_bf16_y32(s, x, Bm, Cm, dtcs, prev, D, y, st);
+    }
+}
+
+hipError_t launch_chunk_scan_own_f32(const ScanShape &, const void *, const void *, const void *, const OwnDecays &, const float *,
+                                     const float *, void *, hipStream_t);
+hipError_t launch_chunk_scan_own_bf16_y32(const ScanShape &, const void *, const void *, const void *, const OwnDecays &,
+                                          const float *, const float *, void *, hipStream_t);
+
+hipError_t launch_chunk_scan_own(const ScanShape &s, int dtype, const void *x, const void *Bm, const void *Cm, const OwnDecays &own,
+                                 const float *prev, const float *D, void *y, hipStream_t st) {
+    switch (dtype) {
+        case 0: return launch_chunk_scan_own_f32(s, x, Bm, Cm, own, prev, D, y, st);
+        case 1: return launch_chunk_scan_own_bf16(s, x, Bm, Cm, own, prev, D, y, st);
+        default: return launch_chunk_scan_own_bf16_y32(s, x, Bm, Cm, own, prev, D, y, st);
     }
 }
 

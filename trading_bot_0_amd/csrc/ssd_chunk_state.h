@@ -15,6 +15,9 @@
 // Both operands have K = l as their slow axis in memory: bf16 tiles are stored row-major and
 // transposed by the LDS transpose read; float tiles are transposed on their way into LDS.
 //
+// OWN: the chunk's weights are worked out here from dt (wave 0, ahead of the tile's first barrier) instead of being read from
+// stage 1's output, and its total decay is left for stage 3 or 4 (see OwnDecays).
+//
 // Persistent and software-pipelined: a workgroup holds the next TWO tiles' x, B and w in
 // registers (two register sets used alternately), so a tile's loads are issued two tile
 // iterations before they are needed.  Everything that shapes the inner code
@@ -25,9 +28,9 @@
 
 namespace ssd {
 
-template <typename T, int PB, int NK, int QB, bool SCAN>  // Ppad = 32*PB >= P, N = 16*NK, Q = 32*QB
+template <typename T, int PB, int NK, int QB, bool SCAN, bool OWN>  // Ppad = 32*PB >= P, N = 16*NK, Q = 32*QB
 __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
-    const T *__restrict__ x, const T *__restrict__ Bm, const float *__restrict__ dtcs,
+    const T *__restrict__ x, const T *__restrict__ Bm, const float *__restrict__ dtcs, OwnDecays own,
     const float *init, float *__restrict__ states, float *final_states, ScanShape s) {
     constexpr int VEC = Vec16<T>::N;
     constexpr int PARTS = Split<T>::PARTS;
@@ -44,6 +47,7 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     T *xs = reinterpret_cast<T *>(smem);  // bf16: [PARTS][Q][Ppad] row-major; float: [Ppad][ldq]
     T *bs = xs + (is_bf16<T> ? PARTS * Q * Ppad : Ppad * ldq);  // bf16: [Q][Npad]; float: [Npad][ldq]
+    float *w_s = reinterpret_cast<float *>(bs + (is_bf16<T> ? Q * Npad : Npad * ldq));  // OWN: [Q] weights, the chunk's alpha
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -57,18 +61,24 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
 
     struct TileRegs {
         Vec16<T> xv[UX], bv[UB];
-        float wv[UX];
+        float wv[OWN ? 1 : UX];
         float a_end;  // SCAN: alpha at the end of the chunk (its total log2-decay)
+        ChunkSteps<T, Q> steps;  // OWN: the chunk's dt and restarts (wave 0)
     };
     // two sets when they are small enough to stay in registers, else one
     constexpr int DEPTH = (UX * 5 + UB * 4 <= 64) ? 2 : 1;
+    const T *dt = static_cast<const T *>(own.dt);
     TileRegs regs[DEPTH];
-    auto prefetch = [&](const Tile &t, TileRegs &R) {
+    auto prefetch = [&](const Tile &t, TileRegs &R) __attribute__((always_inline)) {
         Vec16<T>(&xv)[UX] = R.xv;
         Vec16<T>(&bv)[UB] = R.bv;
-        float(&wv)[UX] = R.wv;
-        const float *wrow = dtcs + ((((size_t)t.b * s.H + t.h) * s.nc + t.c) * 4 + 3) * Q;
-        if (SCAN) R.a_end = wrow[-2 * Q - 1];  // row 0 (alpha hi), element Q-1
+        auto &wv = R.wv;
+        const float *wrow = OWN ? nullptr : dtcs + ((((size_t)t.b * s.H + t.h) * s.nc + t.c) * 4 + 3) * Q;
+        if constexpr (OWN) {
+            if (wave == 0) R.steps.load(dt, own.reset, t, s, lane);
+        } else if (SCAN) {
+            R.a_end = wrow[-2 * Q - 1];  // row 0 (alpha hi), element Q-1
+        }
         const T *xb = x + (((size_t)t.b * s.L + t.t0) * s.H + t.h) * s.P;
         const T *bb = Bm + (((size_t)t.b * s.L + t.t0) * s.G + t.g) * N;
         const int rows = min(Q, s.L - t.t0);  // valid rows of a ragged last chunk
@@ -78,7 +88,7 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
                 const int l = xl0 + u * xrpp;
                 const bool in = xslot && (xrows_exact || l < Q);
                 xv[u] = in ? load_vec16(xb + xoff0 + u * xstep) : zero_vec16<T>();
-                wv[u] = wrow[(xrows_exact || l < Q) ? l : 0];
+                if constexpr (!OWN) wv[u] = wrow[(xrows_exact || l < Q) ? l : 0];
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
@@ -90,7 +100,7 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
             for (int u = 0; u < UX; ++u) {
                 const int l = xl0 + u * xrpp;
                 xv[u] = (xslot && l < rows) ? load_vec16(xb + xoff0 + u * xstep) : zero_vec16<T>();
-                wv[u] = wrow[l < Q ? l : 0];
+                if constexpr (!OWN) wv[u] = wrow[l < Q ? l : 0];
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
@@ -132,21 +142,40 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
     // One tile: its inputs are in R; when R has been copied to LDS it is refilled with the tile DEPTH
     // steps ahead.
     f32x16 acc = {0};  // SCAN: the running state block of this wave, carried from chunk to chunk
-    auto do_tile = [&](int k, TileRegs &R) {
+    // (inlined by hand: called twice, the compiler makes a function of it, whose arguments and captures live in memory)
+    auto do_tile = [&](int k, TileRegs &R) __attribute__((always_inline)) {
         const Tile t = tile_at(k);
-        const float a_end = R.a_end;
+        if constexpr (OWN) {
+            // the weights of this chunk; the previous tile's were read before its second barrier
+            if (wave == 0) {
+                constexpr int EPL = ChunkScan<Q>::EPL;
+                float dtv[EPL], drop[EPL];
+                R.steps.values(t, s, lane, dtv, drop);
+                const ChunkScan<Q> sc(dtv, drop, (double)own.A[t.h]);
+                if (lane * EPL < Q) {
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) w_s[lane * EPL + e] = sc.to_end(e) * dtv[e];
+                }
+                if (lane == 0) {
+                    w_s[Q] = sc.alpha_end();
+                    own.alpha_end[((size_t)t.b * s.H + t.h) * s.nc + t.c] = sc.alpha_end();
+                }
+            }
+        }
         block_sync_lds();  // the previous tile's operand reads are done (and the zero fill is visible)
+        const float a_end = OWN ? w_s[Q] : R.a_end;
         // ---- registers -> LDS: weighted x (hi/lo in bf16 mode), B as is ----
 #pragma unroll
         for (int u = 0; u < UX; ++u) {
             const int l = xl0 + u * xrpp;
             if (xrows_exact || l < Q) {
+                const float wl = OWN ? w_s[l] : R.wv[OWN ? 0 : u];
                 if constexpr (is_bf16<T>) {
                     Vec16<T> hi, lo;
                     unsigned hw[4], lw[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        split_pair((float)R.xv[u].e[2 * i], R.wv[u], (float)R.xv[u].e[2 * i + 1], R.wv[u], hw[i], lw[i]);
+                        split_pair((float)R.xv[u].e[2 * i], wl, (float)R.xv[u].e[2 * i + 1], wl, hw[i], lw[i]);
                     hi.u = make_uint4(hw[0], hw[1], hw[2], hw[3]);
                     lo.u = make_uint4(lw[0], lw[1], lw[2], lw[3]);
                     const int o = XT::off(l, xch * VEC);
@@ -154,7 +183,7 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
                     *reinterpret_cast<uint4 *>(xs + Q * Ppad + o) = lo.u;
                 } else {
 #pragma unroll
-                    for (int i = 0; i < VEC; ++i) xs[(xch * VEC + i) * ldq + l] = R.wv[u] * R.xv[u].e[i];
+                    for (int i = 0; i < VEC; ++i) xs[(xch * VEC + i) * ldq + l] = wl * R.xv[u].e[i];
                 }
             }
         }
@@ -236,54 +265,54 @@ __global__ __launch_bounds__(64 * PB * ((NK + 1) / 2)) void chunk_state_kernel(
 // ------------------------------------------------------------------------------------------
 // Launchers (one translation unit per mode instantiates state_dispatch)
 // ------------------------------------------------------------------------------------------
-template <typename T, int PB, int NK, int QB, bool SCAN>
-static hipError_t state_launch(const ScanShape &s, const void *x, const void *Bm, const float *dtcs,
+template <typename T, int PB, int NK, int QB, bool SCAN, bool OWN>
+static hipError_t state_launch(const ScanShape &s, const void *x, const void *Bm, const float *dtcs, const OwnDecays &own,
                                const float *init, float *states, float *final_states, hipStream_t st) {
     constexpr int block = 64 * PB * ((NK + 1) / 2);
-    const size_t lds = chunk_state_lds_bytes(s, sizeof(T));
-    hipError_t e = allow_lds(chunk_state_kernel<T, PB, NK, QB, SCAN>, lds);
+    const size_t lds = chunk_state_lds_bytes(s, sizeof(T)) + (OWN ? (s.Q + 4) * sizeof(float) : 0);
+    hipError_t e = allow_lds(chunk_state_kernel<T, PB, NK, QB, SCAN, OWN>, lds);
     if (e != hipSuccess) return e;
     int grid = 1;
-    e = persistent_grid(chunk_state_kernel<T, PB, NK, QB, SCAN>, block, lds, SCAN ? s.B * s.H : s.B * s.nc * s.H,
+    e = persistent_grid(chunk_state_kernel<T, PB, NK, QB, SCAN, OWN>, block, lds, SCAN ? s.B * s.H : s.B * s.nc * s.H,
                         &grid);
     if (e != hipSuccess) return e;
-    chunk_state_kernel<T, PB, NK, QB, SCAN><<<dim3(grid), dim3(block), lds, st>>>(
-        static_cast<const T *>(x), static_cast<const T *>(Bm), dtcs, init, states, final_states, s);
+    chunk_state_kernel<T, PB, NK, QB, SCAN, OWN><<<dim3(grid), dim3(block), lds, st>>>(
+        static_cast<const T *>(x), static_cast<const T *>(Bm), dtcs, own, init, states, final_states, s);
     return hipGetLastError();
 }
 
-template <typename T, int PB, int NK, bool SCAN>
-static hipError_t state_dispatch_q(const ScanShape &s, const void *x, const void *Bm, const float *dtcs,
+template <typename T, int PB, int NK, bool SCAN, bool OWN>
+static hipError_t state_dispatch_q(const ScanShape &s, const void *x, const void *Bm, const float *dtcs, const OwnDecays &own,
                                    const float *init, float *states, float *final_states, hipStream_t st) {
     switch (s.Q) {
-        case 32: return state_launch<T, PB, NK, 1, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 64: return state_launch<T, PB, NK, 2, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 128: return state_launch<T, PB, NK, 4, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 256: return state_launch<T, PB, NK, 8, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
+        case 32: return state_launch<T, PB, NK, 1, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 64: return state_launch<T, PB, NK, 2, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 128: return state_launch<T, PB, NK, 4, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 256: return state_launch<T, PB, NK, 8, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <typename T, int PB, bool SCAN>
-static hipError_t state_dispatch_n(const ScanShape &s, const void *x, const void *Bm, const float *dtcs,
+template <typename T, int PB, bool SCAN, bool OWN>
+static hipError_t state_dispatch_n(const ScanShape &s, const void *x, const void *Bm, const float *dtcs, const OwnDecays &own,
                                    const float *init, float *states, float *final_states, hipStream_t st) {
     switch (s.N) {
-        case 16: return state_dispatch_q<T, PB, 1, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 32: return state_dispatch_q<T, PB, 2, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 64: return state_dispatch_q<T, PB, 4, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-        case 128: return state_dispatch_q<T, PB, 8, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
+        case 16: return state_dispatch_q<T, PB, 1, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 32: return state_dispatch_q<T, PB, 2, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 64: return state_dispatch_q<T, PB, 4, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+        case 128: return state_dispatch_q<T, PB, 8, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <bool SCAN>
-hipError_t state_dispatch(const ScanShape &s, int dtype, const void *x, const void *Bm, const float *dtcs,
+template <bool SCAN, bool OWN = false>
+hipError_t state_dispatch(const ScanShape &s, int dtype, const void *x, const void *Bm, const float *dtcs, const OwnDecays &own,
                           const float *init, float *states, float *final_states, hipStream_t st) {
     if (dtype)
-        return (s.P <= 32) ? state_dispatch_n<__bf16, 1, SCAN>(s, x, Bm, dtcs, init, states, final_states, st)
-                           : state_dispatch_n<__bf16, 2, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
-    return (s.P <= 32) ? state_dispatch_n<float, 1, SCAN>(s, x, Bm, dtcs, init, states, final_states, st)
-                       : state_dispatch_n<float, 2, SCAN>(s, x, Bm, dtcs, init, states, final_states, st);
+        return (s.P <= 32) ? state_dispatch_n<__bf16, 1, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st)
+                           : state_dispatch_n<__bf16, 2, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
+    return (s.P <= 32) ? state_dispatch_n<float, 1, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st)
+                       : state_dispatch_n<float, 2, SCAN, OWN>(s, x, Bm, dtcs, own, init, states, final_states, st);
 }
 
 }  // namespace ssd

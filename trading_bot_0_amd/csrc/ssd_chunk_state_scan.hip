@@ -5,7 +5,7 @@ namespace ssd {
 
 hipError_t launch_chunk_state_scan(const ScanShape &s, int dtype, const void *x, const void *Bm, const float *dtcs,
                                    const float *init, float *prev, float *final_states, hipStream_t st) {
-    return state_dispatch<true>(s, dtype, x, Bm, dtcs, init, prev, final_states, st);
+    return state_dispatch<true>(s, dtype, x, Bm, dtcs, OwnDecays{}, init, prev, final_states, st);
 }
 
 }  // namespace ssd

@@ -219,6 +219,39 @@ __device__ inline double wave_inclusive_scan(double v) {
     return v;
 }
 
+// The decays of one chunk of Q steps of one (b, h), worked out by one wave: a lane holds EPL consecutive steps, and the
+// cumulative sum of dt A runs over the lanes in float64 (see chunk_cumsum_kernel for why).
+template <int Q> struct ChunkScan {
+    static constexpr int EPL = Q <= 64 ? 1 : Q / 64;
+    double cum[EPL], total;  // natural logarithms: up to and with each step; of the whole chunk
+    // dtv and drop (kResetDrop where the state restarts before a step, else 0) of the steps lane * EPL + e; zero past Q
+    __device__ inline ChunkScan(const float (&dtv)[EPL], const float (&drop)[EPL], double a) {
+        double run = 0.0;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            run += (double)dtv[e] * a - (double)drop[e];
+            cum[e] = run;
+        }
+        const double incl = wave_inclusive_scan(run);
+        const double excl = incl - run;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) cum[e] += excl;
+        // chunk total = the last lane's inclusive sum (lanes past Q carry zeros)
+        total = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(incl), 63),
+                                 __builtin_amdgcn_readlane(__double2loint(incl), 63));
+    }
+    static constexpr double kLog2e = 1.4426950408889634;
+    // log2-decay up to step e as an unevaluated pair hi + lo
+    __device__ inline void alpha(int e, float &hi, float &lo) const {
+        const double al = cum[e] * kLog2e;
+        hi = (float)al;
+        lo = (float)(al - (double)hi);
+    }
+    __device__ inline float alpha_end() const { return (float)(total * kLog2e); }
+    // decay from step e to the end of the chunk
+    __device__ inline float to_end(int e) const { return exp2_hw(fminf((float)((total - cum[e]) * kLog2e), 0.f)); }
+};
+
 // Sum of v over aligned groups of NL consecutive lanes (NL = 4, 8, 16, 32 or 64), left in every lane of the group.
 // Inside a row of 16 lanes the data moves by DPP (quads, then the mirrored half row, then the mirrored row: no trip
 // through the LDS crossbar); wider groups take one lane exchange per doubling on top.
@@ -505,6 +538,34 @@ __device__ inline Tile decode_tile(int logical, const ScanShape &s) {
     t.t0 = t.c * s.Q;
     return t;
 }
+
+// dt and the restart marks of one chunk as a wave of the staged kernels holds them while they are on their way from memory
+// (every load unconditional: steps past the sequence's end are read as its last step and dropped in dtv())
+template <typename T, int Q> struct ChunkSteps {
+    static constexpr int EPL = ChunkScan<Q>::EPL;
+    T raw[EPL];
+    unsigned char mark[EPL];
+    __device__ inline void load(const T *dt, const unsigned char *reset, const Tile &t, const ScanShape &s, int lane) {
+        const T *row = dt + ((size_t)t.b * s.L) * s.H + t.h;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) raw[e] = row[(size_t)min(t.t0 + lane * EPL + e, s.L - 1) * s.H];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) mark[e] = 0;
+        if (reset != nullptr) {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) mark[e] = reset[(size_t)t.b * s.L + min(t.t0 + lane * EPL + e, s.L - 1)];
+        }
+    }
+    __device__ inline void values(const Tile &t, const ScanShape &s, int lane, float (&dtv)[EPL], float (&drop)[EPL]) const {
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            const int l = lane * EPL + e;
+            const bool in = l < Q && t.t0 + l < s.L;
+            dtv[e] = in ? (float)raw[e] : 0.f;
+            drop[e] = in && mark[e] != 0 ? (float)kResetDrop : 0.f;
+        }
+    }
+};
 
 
 // ------------------------------------------------------------------------------------------

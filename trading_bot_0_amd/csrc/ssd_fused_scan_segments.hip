@@ -14,35 +14,56 @@ namespace {
 constexpr int kSegmentMinTiles = 4;        // shorter segments are mostly prologue
 constexpr int kSegmentTargetGroups = 192;  // workgroups to aim for (256 CUs; the last quarter gains little)
 
-constexpr double kFloatTileUs = 7.5;
-
 int tiles_of(const ScanShape &s) { return (s.L + kOnePassTile - 1) / kOnePassTile; }
+int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1) / fused_scan_f32_tile(); }
+
+// Estimates in microseconds, from measurements on MI355X, of the three ways a forward can run; `groups` workgroups fill a
+// CU each (eight units of 32 columns; four of a 128-wide state).  As used against measured:
+// staged kernels (every tile of 64 steps of every unit side by side): 8 heads of 32, state 64, 16 x 512 steps 18 / 17,
+// 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128, 8 x 1 000 55 / 47,
+// 8 x 4 000 189 / 172, 16 x 4 000 368 / 369; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000 63 / 67, 10 x 3 000 87 / 86.
+double staged_us(const ScanShape &s, int dtype, long long groups) {
+    const int full = dtype != 0 && s.N == 128 ? 4 : 8;
+    const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
+    if (dtype == 0) return 12.0 + 1310.0 * units;
+    return 10.0 + 518.0 * units * (s.N == 128 ? 1.4 : 1.0);
+}
+// the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
+// 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 4 000 277 / 266; float32 tiles of 32 steps, 70 x 100 26 / 27
+double whole_us(const ScanShape &s, int dtype, long long groups) {
+    const double rounds = (double)((groups + 255) / 256);
+    if (dtype == 0) return 5.0 + 5.3 * float_tiles_of(s) * rounds;
+    const double fill = groups < 256 ? (double)groups / 256.0 : 1.0;
+    return 6.0 + tiles_of(s) * rounds * (s.N == 128 ? 4.1 + 0.5 * fill : 4.1 + 1.5 * fill);
+}
+// ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 37 / 36, 16 x 1 024
+// on 4 40 / 40, 16 x 2 048 on 8 48 / 50, 48 x 2 048 on 4 65 / 70, 24 x 4 096 on 8 73 / 76, 64 x 4 096 on 4 115 / 124; float32
+// 96 x 1 999 on 2 253 / 247, 30 x 1 000 on 4 72 / 74
+double segments_us(int dtype, long long groups, int segments, int seg_tiles) {
+    const double rounds = (double)((groups * segments + 255) / 256);
+    if (dtype == 0) return 10.0 + 7.7 * seg_tiles * rounds;
+    return 8.0 + 1.9 * segments + 6.2 * seg_tiles * rounds;
+}
 
 }  // namespace
 
 // Which way a forward runs fastest: 0 = staged kernels, 1 = the one-pass kernel, 2 = the one-pass kernel on
-// *segments segments.  Estimates in microseconds from measurements on MI355X: a workgroup walks a tile of 64 steps
-// in about 6.5 (states only: 0.4 of that) and a CU holds one workgroup, so the one-pass kernel takes that times
-// the tiles of a sequence (or segment) times the rounds of 256 workgroups; the staged kernels run every tile of
-// every sequence side by side, about 510 per 2048 units x 32 tiles; a launch costs about 5.
+// *segments segments.
 int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     *segments = 1;
     if (dtype == 0) {
-        // float inputs: the one-pass kernel on three bf16 terms per operand walks a tile of 32 steps in about
-        // kFloatTileUs (states only: 0.45 of that); the staged float kernels take about 1345 per 2048 units x 32
-        // tiles of 64
+        // float inputs: the one-pass kernel on three bf16 terms per operand, tiles of 32 steps
         if (fused_scan_f32_waves(s) == 0) return 0;
         const long long groups = (long long)s.B * s.G * ((s.H / s.G) * (s.P / 32) / 8);
-        const int nc = (s.L + fused_scan_f32_tile() - 1) / fused_scan_f32_tile();
-        const double staged = 20.0 + 1345.0 * ((double)groups * 8 * tiles_of(s)) / (2048.0 * 32.0);
-        const double whole = 5.0 + kFloatTileUs * nc * (double)((groups + 255) / 256);
+        const int nc = float_tiles_of(s);
+        const double staged = staged_us(s, 0, groups), whole = whole_us(s, 0, groups);
         double cut = 1e30;
         int S = 1;
         while (groups * S < kSegmentTargetGroups && nc / (2 * S) >= 2 * kSegmentMinTiles) S *= 2;
         if (S >= 2) {
             const int seg_tiles = (nc + S - 1) / S;
             S = (nc + seg_tiles - 1) / seg_tiles;
-            cut = 10.0 + 1.45 * kFloatTileUs * seg_tiles * (double)((groups * S + 255) / 256);
+            cut = segments_us(0, groups, S, seg_tiles);
         }
         if (cut < whole && cut < staged) {
             *segments = S;
@@ -59,7 +80,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
         // segments (the states-only instance is the eight-wave one).
         const long long groups = (long long)s.B * s.G * ((s.H / s.G) * (s.P / 32) / 4);
         const int nc = tiles_of(s);
-        const double staged = 20.0 + 510.0 * ((double)groups * 4 * nc) / (2048.0 * 32.0);
+        const double staged = 10.0 + 518.0 * ((double)groups * 4 * nc) / (2048.0 * 32.0);
         const long long rounds = groups / 512, rest = groups % 512;
         const double per_tile = 7.0 * rounds + (rest == 0 ? 0.0 : rest <= 256 ? 4.2 : 4.2 + 2.8 * (double)(rest - 256) / 256.0);
         return 5.0 + per_tile * nc < staged ? 1 : 0;
@@ -68,8 +89,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     if (waves != full) return 0;
     const long long groups = (long long)s.B * s.G * ((s.H / s.G) * (s.P / 32) / full);
     const int nc = tiles_of(s);
-    const double staged = 20.0 + 510.0 * ((double)groups * full * nc) / (2048.0 * 32.0) * (s.N == 128 ? 2.0 : 1.0);
-    const double whole = 5.0 + 6.5 * nc * (double)((groups + 255) / 256);
+    const double staged = staged_us(s, dtype, groups), whole = whole_us(s, dtype, groups);
     double cut = 1e30;
     int S = 1;
     if (s.N != 128) {
@@ -77,7 +97,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
         if (S >= 2) {
             const int seg_tiles = (nc + S - 1) / S;
             S = (nc + seg_tiles - 1) / seg_tiles;
-            cut = 15.0 + 1.4 * 6.5 * seg_tiles * (double)((groups * S + 255) / 256);
+            cut = segments_us(dtype, groups, S, seg_tiles);
         }
     }
     if (cut < whole && cut < staged) {
@@ -103,26 +123,10 @@ int fused_scan_tail_rows(const ScanShape &s, int dtype) {
     tail.B = rest / per_row;
     const int tail_plan = fused_scan_plan(tail, dtype, &segments);
     if (tail_plan == 1) return 0;  // it would run as a round of the one-pass kernel anyway
-    double cost, round;  // of the remainder as its own batch, as fused_scan_plan estimates it; of one more round
-    if (dtype == 0) {
-        const int nc = (s.L + fused_scan_f32_tile() - 1) / fused_scan_f32_tile();
-        round = kFloatTileUs * nc;
-        if (tail_plan == 2) {
-            const int seg_tiles = (nc + segments - 1) / segments;
-            cost = 10.0 + 1.45 * kFloatTileUs * seg_tiles * (double)(((long long)rest * segments + 255) / 256);
-        } else {
-            cost = 20.0 + 1345.0 * ((double)rest * 8 * tiles_of(s)) / (2048.0 * 32.0);
-        }
-    } else {
-        const int nc = tiles_of(s);
-        round = 6.5 * nc;
-        if (tail_plan == 2) {
-            const int seg_tiles = (nc + segments - 1) / segments;
-            cost = 15.0 + 1.4 * 6.5 * seg_tiles * (double)(((long long)rest * segments + 255) / 256);
-        } else {
-            cost = 20.0 + 510.0 * ((double)rest * full * nc) / (2048.0 * 32.0) * (s.N == 128 ? 2.0 : 1.0);
-        }
-    }
+    // the remainder as its own batch against one more round
+    const int nc = dtype == 0 ? float_tiles_of(s) : tiles_of(s);
+    const double round = whole_us(s, dtype, 256) - whole_us(s, dtype, 0);
+    const double cost = tail_plan == 2 ? segments_us(dtype, rest, segments, (nc + segments - 1) / segments) : staged_us(tail, dtype, rest);
     return cost < round ? tail.B : 0;
 }
 

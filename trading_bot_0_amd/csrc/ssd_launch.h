@@ -63,13 +63,32 @@ hipError_t launch_chunk_cumsum(const ScanShape &s, int dtype, const void *dt, co
                                int dt_len = 0);
 hipError_t launch_chunk_state(const ScanShape &s, int dtype, const void *x, const void *Bm,
                               const float *dtcs, float *states, hipStream_t stream);
+// Stages 2 and 4 that work out a chunk's decays themselves, from dt (as the scan's inputs), A and the restart mask, instead of
+// reading stage 1's output (the same values, bit for bit; the forward's mode only).  Stage 2 then leaves every chunk's
+// total log2-decay in alpha_end [B, H, nc]; stage 4 with `fold` takes the chunk states as stage 2 left them and runs the
+// recurrence over the chunks before its own (from init [B, H, P, N] or zero), the last chunk's tile up to final_states.
+struct OwnDecays {
+    const void *dt = nullptr;
+    const float *A = nullptr;
+    const unsigned char *reset = nullptr;
+    float *alpha_end = nullptr;
+    bool fold = false;
+    const float *init = nullptr;
+    float *final_states = nullptr;
+};
+// whether stage 2 fits its LDS with the decays in it
+bool own_decays_supported(const ScanShape &s, int elem_bytes);
+hipError_t launch_chunk_state_own(const ScanShape &s, int dtype, const void *x, const void *Bm, const OwnDecays &own, float *states,
+                                  hipStream_t stream);
+hipError_t launch_chunk_scan_own(const ScanShape &s, int dtype, const void *x, const void *Bm, const void *Cm, const OwnDecays &own,
+                                 const float *prev, const float *D, void *y, hipStream_t stream);
 // stages 2+3 in one pass: writes the state entering each chunk into `prev` and the final state
 hipError_t launch_chunk_state_scan(const ScanShape &s, int dtype, const void *x, const void *Bm,
                                    const float *dtcs, const float *init, float *prev, float *final_states,
                                    hipStream_t stream);
-hipError_t launch_state_passing(const ScanShape &s, const float *states, const float *dtcs,
-                                const float *init, float *prev, float *final_states,
-                                hipStream_t stream);
+// a_end: the chunks' total log2-decays, sequence (b, h) chunk c at [((b * H + h) * nc + c) * a_stride]
+hipError_t launch_state_passing(const ScanShape &s, const float *states, const float *a_end, int a_stride, const float *init,
+                                float *prev, float *final_states, hipStream_t stream);
 hipError_t launch_chunk_scan(const ScanShape &s, int dtype, const void *x, const void *Bm,
                              const void *Cm, const float *dtcs, const float *prev, const float *D,
                              void *y, hipStream_t stream);
