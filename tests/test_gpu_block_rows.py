@@ -1,0 +1,56 @@
+"""The block's kernels for few rows at the lines of their dispatch."""
+import pytest
+import torch
+
+from trading_bot_0_amd import block_post, block_post_proj, block_proj
+
+pytestmark = pytest.mark.gpu
+
+H, N, G = 8, 64, 1
+
+
+def inputs(rows, di, n, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    y = torch.randn(1, rows, H, di // H, generator=g, device="cuda").to(torch.bfloat16)
+    z = torch.randn(1, rows, 2 * di + 2 * G * N + H, generator=g, device="cuda").to(torch.bfloat16)
+    nw = 1 + 0.2 * torch.randn(di, generator=g, device="cuda")
+    w = (torch.randn(n, di, generator=g, device="cuda") / di ** 0.5).to(torch.bfloat16)
+    return y, z, nw, w
+
+
+@pytest.mark.parametrize("di,n", [(256, 256), (256, 72), (128, 200), (128, 8)])
+def test_fused_out_projection_of_few_rows_is_the_one_of_many(di, n):
+    """Workgroups of 32 rows (up to a round of them), of 64 (up to two) and the kernel of many rows give a row the same bits: slices
+    of 40 000 rows, with last tiles that are whole, of one row and one short, against the whole."""
+    y, z, nw, w = inputs(40000, di, n, di + n)
+    whole = block_post_proj(y, z, nw, w, H, di // H, N, G)
+    for rows in (1, 31, 32, 33, 600, 8191, 8192, 8193, 12000, 16385, 32767, 32768, 32769):
+        for at in (0, 40000 - rows):
+            part = block_post_proj(y[:, at:at + rows].contiguous(), z[:, at:at + rows].contiguous(), nw, w, H, di // H, N, G)
+            assert torch.equal(part, whole[:, at:at + rows]), (rows, at)
+
+
+def test_fused_out_projection_of_few_rows_next_to_the_two_stages():
+    """Against float64 on the same inputs: no further off than the post stage and the projection one after the other."""
+    y, z, nw, w = inputs(700, 256, 256, 3)
+    v = y.double().view(1, 700, 256) * torch.nn.functional.silu(z[..., :256].double())
+    exact = (v * torch.rsqrt((v * v).mean(-1, keepdim=True) + 1e-5) * nw.double()) @ w.double().t().contiguous()
+    err = lambda o: ((o.double() - exact).norm() / exact.norm()).item()
+    one, two = err(block_post_proj(y, z, nw, w, H, 32, N, G)), err(block_proj(block_post(y, z, nw, H, 32, N, G), w))
+    assert one <= 1.02 * two, f"{one:.3e} against the two stages' {two:.3e}"
+
+
+def test_fused_out_projection_writes_nothing_past_its_rows_and_columns():
+    y, z, nw, w = inputs(45, 256, 72, 5)
+    out = block_post_proj(y, z, nw, w, H, 32, N, G)
+    big = torch.full((64, 256), 7.0, dtype=torch.bfloat16, device="cuda")
+    from ctypes import byref, c_float
+
+    from trading_bot_0_amd import ssd
+    from trading_bot_0_amd.block import SsdBlockDims, _lib
+    lib = _lib()
+    ssd._check(lib, lib.ssd_block_post_proj_fwd(byref(SsdBlockDims(1, 45, H, 32, N, G, 4, 0)), ssd.SSD_DTYPE_BF16, y.data_ptr(),
+                                                z.data_ptr(), nw.data_ptr(), c_float(1e-5), w.data_ptr(), 72, 256, big.data_ptr(),
+                                                ssd._stream_ptr(y)))
+    torch.cuda.synchronize()
+    assert torch.equal(big[:45, :72], out[0]) and bool((big[45:] == 7).all()) and bool((big[:, 72:] == 7).all())

@@ -505,9 +505,8 @@ class Mamba2Block:
             raise ValueError("backward through a window that continues a carried state is not supported")
         if block_post_proj_supported(y, w_out):
             # gate, norm and out-projection as one kernel: the normalised rows never reach memory (the backward pass
-            # needs them for one weight gradient only, and has its post stage write them on the way: yn=None).  Of few rows it
-            # saves the host's time, not the GPU's (256 -> 256 in us, one kernel / two, and called one by one: 512 rows 13.3 / 7.1
-            # and 13 / 30, 8 191 rows 14.8 / 11.0 and 15 / 29)
+            # needs them for one weight gradient only, and has its post stage write them on the way: yn=None).  256 -> 256 in us, one
+            # kernel / two: 512 rows 6.8 / 7.1, 8 191 rows 7.5 / 11.0
             out = block_post_proj(y, zxbcdt, self.norm_w, w_out, self.H, self.P, self.N, self.G, self.eps)
             yn = None
         else:

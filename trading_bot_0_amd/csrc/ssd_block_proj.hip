@@ -176,16 +176,15 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_proj_kernel(const __bf1
 // weights folded into w instead, which rounds the weights once more, the result's error against float64 was 2.88e-3 where
 // it is 2.35e-3, at scales spread by 0.2 around one; 256 -> 256 in us, folded / here: 16 384 rows 17.5 / 16.7, 131 072 rows
 // 42 / 45, 524 288 rows 176 / 176).  v takes the registers of the pieces of y and z it is formed from; the norm's weights are
-// in LDS.  A workgroup takes all out_features (at most 256) columns where rows are many, so that the prologue runs once
-// per row: its rows of w fill 132 KB of LDS, and a wave's output tile covers 16 rows at a time to fit beside them; where rows
-// are few the columns are cut as well and each block of columns gates its rows anew (launch_block_post_proj).
+// in LDS.  A workgroup takes all out_features (at most 256) columns, so that the prologue runs once per row: its rows of w fill
+// 132 KB of LDS, and a wave's output tile covers 16 rows at a time to fit beside them.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kPostProjMaxCols = 256;
 
 template <int KS, int CH>  // K = 16 * KS inner channels, CH chunks of 32 output columns
 __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     const __bf16 *__restrict__ y, const __bf16 *__restrict__ zxbcdt, const float *__restrict__ norm_w, float eps,
-    const __bf16 *__restrict__ w, __bf16 *__restrict__ out, long long M, int N, int ld_z, int ldo, int tiles, int col_blocks) {
+    const __bf16 *__restrict__ w, __bf16 *__restrict__ out, long long M, int N, int ld_z, int ldo, int tiles) {
     constexpr int K = 16 * KS, NTHR = 64 * kProjWaves, PPR = K / 8;  // 16-byte pieces per row of w
     constexpr int ROWB = K * 2 + 16;  // a staged row of w: 16 bytes of padding shift the banks from row to row
     constexpr int kTileRowB = 64 * 2 + 16;
@@ -193,11 +192,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     __shared__ __attribute__((aligned(16))) unsigned char otile[kProjWaves][16 * kTileRowB];
     __shared__ __attribute__((aligned(16))) float nw_s[K];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // (the column blocks of a range of rows are consecutive workgroups of one XCD, as in block_proj_kernel)
-    const int xcd = blockIdx.x % 8, within = blockIdx.x / 8;
-    const int n0 = (within % col_blocks) * (CH * kProjChunk);  // this workgroup's first column
-    const long long row0 = ((long long)(within / col_blocks) * 8 + xcd) * tiles * (32LL * kProjWaves);  // tiles: 32-row tiles per wave, 1 .. kProjTiles
-    if (row0 >= M) return;  // the grid is padded to whole rounds of XCDs
+    const long long row0 = (long long)blockIdx.x * tiles * (32LL * kProjWaves);  // tiles: 32-row tiles per wave, 1 .. kProjTiles
     const int r = lane & 31, half = lane >> 5;
     // this lane's K elements are 16 ks + 8 half .. + 7 for every K step
     auto tile_row0 = [&](int t) { return row0 + (long long)t * (32 * kProjWaves) + wave * 32; };
@@ -218,7 +213,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     };
     load_y(0);  // in flight while w is staged
     const float nw_q = norm_w[min(tid, K - 1)];
-    {   // rows n0 .. n0 + 32 CH - 1 of w (rows past N repeat the last one: never stored)
+    {   // rows 0 .. 32 CH - 1 of w (rows past N repeat the last one: never stored)
         constexpr int PIECES = CH * kProjChunk * PPR;
         constexpr int FILL = (PIECES + NTHR - 1) / NTHR;
 #pragma unroll 4
@@ -226,7 +221,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
             const int p = min(tid + i * NTHR, PIECES - 1);
             const int row = p / PPR, piece = p % PPR;
             *reinterpret_cast<uint4 *>(wsm + row * ROWB + piece * 16) =
-                *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + row, N - 1) * K + piece * 8);
+                *reinterpret_cast<const uint4 *>(w + (size_t)min(row, N - 1) * K + piece * 8);
         }
     }
     if (tid < K) nw_s[tid] = nw_q;
@@ -238,16 +233,20 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
     for (int t = 0; t < tiles; ++t) {
         // ---- prologue: this tile's rows of y and z -> fragments of the normalised rows ----
         load_z(t);
+        // (the row's squares: each eight channels' own sum, those of a half in order; block_post_proj_rows_kernel adds them up the
+        // same way, so that a row's result is the same bits from either)
         float v[KS][8];
         float ss = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const Pack8<__bf16> yy{yq[ks]}, zz{zq[ks]};
+            float piece = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 v[ks][i] = yy.get(i) * silu(zz.get(i));
-                ss += v[ks][i] * v[ks][i];
+                piece += v[ks][i] * v[ks][i];
             }
+            ss += piece;
         }
         ss += __shfl_xor(ss, 32, 64);
         const float rstd = rsqrtf(ss * inv_k + eps);
@@ -314,10 +313,10 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int pass = 0; pass < 2; ++pass) {
-                    const int trw = pass * 8 + (lane >> 3), row = rh * 16 + trw, lcol = c0 * kProjChunk + (lane & 7) * 8, col = n0 + lcol;
+                    const int trw = pass * 8 + (lane >> 3), row = rh * 16 + trw, col = c0 * kProjChunk + (lane & 7) * 8;
                     const u32x4 q = *reinterpret_cast<const u32x4 *>(tile + trw * kTileRowB + (lane & 7) * 16);
                     const u32x4 v = (pass & 1) ? u32x4{q.z, q.w, q.x, q.y} : q;  // (halves swapped in rows 8 .. 15)
-                    const bool ok = m0 + row < M && lcol < CH * kProjChunk && col < N;
+                    const bool ok = m0 + row < M && col < N;
                     const unsigned off = ((trow + (unsigned)row) * (unsigned)ldo + (unsigned)col) * 2u;
                     __builtin_amdgcn_raw_buffer_store_b128(v, obuf, ok ? off : kBufferDropOffset, 0, 0);
                 }
@@ -325,6 +324,108 @@ __global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_kernel(
                 __builtin_amdgcn_wave_barrier();
             }
         }
+    }
+}
+
+// The same for few rows.  There the kernel above leaves the gate to few waves -- one gates 32 rows, 128 silu per lane, six
+// microseconds of vector instructions -- and each block of columns gates its rows anew.  Here a workgroup owns 32 RT rows and all
+// columns: its eight waves gate four RT rows each (sixteen lanes a row), put the rows into
+// LDS, and then multiply 32 columns each, their weights requested straight into operand fragments ahead of the gate.  Every
+// workgroup reads all of w (128 KB at 256 x 256) from its XCD's L2, which is what bounds it and why many rows are better off above.
+// 256 -> 256 in us, the kernel above (with its columns cut in up to eight blocks below 32 768 rows) / 32 rows per workgroup / 64:
+// 600 rows 13.8 / 6.8 / 8.3, 8 192 14.7 / 7.5 / 8.9, 16 384 15.8 / 12.2 / 9.6, 32 768 18.7 / 22.6 / 16.4, 49 152 22.3 / 32 / 24.6;
+// 128 channels: 600 rows 8.5 / 4.7 / 5.4, 16 384 10.1 / 8.2 / 6.8, 32 768 12.2 / 13.9 / 10.8, 49 152 14.8 / 20 / 15.1.
+template <int KS, int RT>
+__global__ __launch_bounds__(64 * kProjWaves) void block_post_proj_rows_kernel(
+    const __bf16 *__restrict__ y, const __bf16 *__restrict__ zxbcdt, const float *__restrict__ norm_w, float eps,
+    const __bf16 *__restrict__ w, __bf16 *__restrict__ out, long long M, int N, int ld_z, int ldo) {
+    constexpr int K = 16 * KS, PPL = KS / 8;  // 16-byte pieces of a row per lane
+    constexpr int ROWB = K * 2 + 16;          // bytes of a staged row: 16 bytes of padding shift the banks
+    __shared__ __attribute__((aligned(16))) unsigned char rows_s[RT * 32 * ROWB];
+    __shared__ __attribute__((aligned(16))) float squares[32][K / 8 + 4];  // of a row's pieces of eight channels
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 31, half = lane >> 5;
+    const long long row0 = (long long)blockIdx.x * (32 * RT);
+    const int lrow = tid >> 4, l16 = tid & 15;
+    Pack8<__bf16> yv[RT][PPL], zv[RT][PPL];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const size_t row = (size_t)min(row0 + t * 32 + lrow, M - 1);  // rows past M repeat the last row; never stored
+#pragma unroll
+        for (int p = 0; p < PPL; ++p) {
+            yv[t][p] = Pack8<__bf16>::load(y + row * K + (p * 16 + l16) * 8);
+            zv[t][p] = Pack8<__bf16>::load(zxbcdt + row * ld_z + (p * 16 + l16) * 8);
+        }
+    }
+    float4 na[PPL], nb[PPL];
+#pragma unroll
+    for (int p = 0; p < PPL; ++p) {
+        na[p] = *reinterpret_cast<const float4 *>(norm_w + (p * 16 + l16) * 8);
+        nb[p] = *reinterpret_cast<const float4 *>(norm_w + (p * 16 + l16) * 8 + 4);
+    }
+    Frag<__bf16> wf[KS];  // this wave's 32 columns (columns past N repeat the last one; never stored)
+    const __bf16 *wr = w + (size_t)min(wave * 32 + r, N - 1) * K + 8 * half;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) wf[ks].v = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(wr + 16 * ks));
+    __builtin_amdgcn_sched_barrier(0);  // (all of it in flight before the first is waited for)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        float v[PPL][8];
+#pragma unroll
+        for (int p = 0; p < PPL; ++p) {
+            float piece = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                v[p][i] = yv[t][p].get(i) * silu(zv[t][p].get(i));
+                piece += v[p][i] * v[p][i];
+            }
+            squares[lrow][p * 16 + l16] = piece;
+        }
+        // (a row's lanes belong to one wave, whose LDS requests are worked off in order: only the compiler has to keep it)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        float s0 = 0.f, s1 = 0.f;  // pieces of even and of odd index, as the two halves of the kernel above hold them
+#pragma unroll
+        for (int q = 0; q < K / 8; q += 4) {
+            const float4 p4 = *reinterpret_cast<const float4 *>(&squares[lrow][q]);
+            s0 += p4.x;
+            s1 += p4.y;
+            s0 += p4.z;
+            s1 += p4.w;
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        const float rstd = rsqrtf((s0 + s1) * (1.f / (float)K) + eps);
+#pragma unroll
+        for (int p = 0; p < PPL; ++p) {
+            uint4 o;
+            o.x = pack_bf16x2(v[p][0] * rstd * na[p].x, v[p][1] * rstd * na[p].y);
+            o.y = pack_bf16x2(v[p][2] * rstd * na[p].z, v[p][3] * rstd * na[p].w);
+            o.z = pack_bf16x2(v[p][4] * rstd * nb[p].x, v[p][5] * rstd * nb[p].y);
+            o.w = pack_bf16x2(v[p][6] * rstd * nb[p].z, v[p][7] * rstd * nb[p].w);
+            *reinterpret_cast<uint4 *>(rows_s + (t * 32 + lrow) * ROWB + (p * 16 + l16) * 16) = o;
+        }
+    }
+    block_sync_lds();
+    const int n0 = wave * 32;
+    if (n0 >= N) return;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const unsigned char *ur = rows_s + (t * 32 + r) * ROWB + half * 16;
+        f32x16 acc = {0}, acc_odd = {0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks += 2) {
+            Frag<__bf16> u0, u1;
+            u0.v = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ur + ks * 32));
+            u1.v = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ur + ks * 32 + 32));
+            acc = mma32(wf[ks], u0, acc);
+            acc_odd = mma32(wf[ks + 1], u1, acc_odd);
+        }
+        float o[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = acc[i] + acc_odd[i];
+        const long long row = row0 + t * 32 + r;
+        store_column<__bf16>(out + (size_t)min(row, M - 1) * ldo + n0, o, half, N - n0, row < M);
     }
 }
 
@@ -440,31 +541,39 @@ hipError_t launch_block_post_proj(const BlockShape &s, const void *y, const void
     if (!block_post_proj_supported(s, out_features) || out_ld < out_features || out_ld % 8 != 0) return hipErrorInvalidValue;
     const int K = s.H * s.P;
     const long long rows = (long long)s.B * s.L;
-    // rows per workgroup: as many tiles of 32 rows per wave, up to kProjTiles, as make one round of workgroups (each
-    // workgroup stages all of w, as much as 256 of its rows; rounded down instead, 67 423 rows were two rounds of one tile:
-    // 44 us against 36 with two, 180 001 rows 79 against 61)
     int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = device_cu_count(dev, &cus);
     if (e != hipSuccess) return e;
-    const long long per_tile = 32LL * kProjWaves;
-    const int tiles = (int)std::max<long long>(1, std::min<long long>(kProjTiles, (rows + per_tile * cus - 1) / (per_tile * cus)));
-    // Where one tile per wave still leaves compute units idle, the columns are cut too, in up to eight blocks of 32 (each
-    // gates its rows anew; staging w and the products shrink): 16 384 rows, 256 -> 256, in us with 1, 2, 4, 8 blocks:
-    // 20.7, 17.5, 17.0, 26.3 (256 workgroups are a round); 8 192 rows 19.6, 16.4, 15.7, 14.1.
-    int col_blocks = 1;
-    const int chunks = (out_features + kProjChunk - 1) / kProjChunk;
-    while (col_blocks < 8 && 2 * col_blocks <= chunks && (rows + per_tile - 1) / per_tile * (2 * col_blocks) <= cus) col_blocks *= 2;
-    const long long rows_per_group = per_tile * tiles;
-    const long long groups = ((rows + rows_per_group - 1) / rows_per_group + 7) / 8 * 8 * col_blocks;
-    if (groups > 0x7fffffffLL || (unsigned long long)rows_per_group * out_ld * 2 > 0x7fffffffULL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)groups), block(64 * kProjWaves);
     const __bf16 *yy = static_cast<const __bf16 *>(y), *zz = static_cast<const __bf16 *>(zxbcdt), *ww = static_cast<const __bf16 *>(w);
     __bf16 *oo = static_cast<__bf16 *>(out);
-    const int ch = (chunks + col_blocks - 1) / col_blocks;
+    const dim3 block(64 * kProjWaves);
+    // Few rows: a workgroup per 32 rows up to one round of workgroups, then per 64 up to two (above, at the line, in the comment
+    // of the kernel: both sides).
+    if (rows <= 128LL * cus) {
+        const int rt = rows <= 32LL * cus ? 1 : 2;
+        const dim3 grid((unsigned)((rows + 32 * rt - 1) / (32 * rt)));
+#define SSD_POST_PROJ_ROWS(KSv, RTv)                                                                                                     \
+    if (K == 16 * KSv && rt == RTv) {                                                                                                    \
+        block_post_proj_rows_kernel<KSv, RTv><<<grid, block, 0, st>>>(yy, zz, norm_w, eps, ww, oo, rows, out_features, s.ld, out_ld);    \
+        return hipGetLastError();                                                                                                        \
+    }
+        SSD_POST_PROJ_ROWS(8, 1) SSD_POST_PROJ_ROWS(8, 2) SSD_POST_PROJ_ROWS(16, 1) SSD_POST_PROJ_ROWS(16, 2)
+#undef SSD_POST_PROJ_ROWS
+    }
+    // rows per workgroup: as many tiles of 32 rows per wave, up to kProjTiles, as make one round of workgroups (each
+    // workgroup stages all of w, as much as 256 of its rows; rounded down instead, 67 423 rows were two rounds of one tile:
+    // 44 us against 36 with two, 180 001 rows 79 against 61)
+    const long long per_tile = 32LL * kProjWaves;
+    const int tiles = (int)std::max<long long>(1, std::min<long long>(kProjTiles, (rows + per_tile * cus - 1) / (per_tile * cus)));
+    const long long rows_per_group = per_tile * tiles;
+    const long long groups = (rows + rows_per_group - 1) / rows_per_group;
+    if (groups > 0x7fffffffLL || (unsigned long long)rows_per_group * out_ld * 2 > 0x7fffffffULL) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)groups);
+    const int ch = (out_features + kProjChunk - 1) / kProjChunk;
 #define SSD_POST_PROJ_CASE(KSv, CHv)                                                                                   \
     if (K == 16 * KSv && ch == CHv) {                                                                                  \
-        block_post_proj_kernel<KSv, CHv><<<grid, block, 0, st>>>(yy, zz, norm_w, eps, ww, oo, rows, out_features, s.ld, out_ld, tiles, col_blocks); \
+        block_post_proj_kernel<KSv, CHv><<<grid, block, 0, st>>>(yy, zz, norm_w, eps, ww, oo, rows, out_features, s.ld, out_ld, tiles); \
         return hipGetLastError();                                                                                      \
     }
     SSD_POST_PROJ_CASE(8, 1) SSD_POST_PROJ_CASE(8, 2) SSD_POST_PROJ_CASE(8, 3) SSD_POST_PROJ_CASE(8, 4)
