@@ -54,3 +54,54 @@ def test_fused_out_projection_writes_nothing_past_its_rows_and_columns():
                                                 ssd._stream_ptr(y)))
     torch.cuda.synchronize()
     assert torch.equal(big[:45, :72], out[0]) and bool((big[45:] == 7).all()) and bool((big[:, 72:] == 7).all())
+
+
+def block_inputs(B, L, dtype, seed, P=32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    C, E = H * P + 2 * G * N, 2 * H * P + 2 * G * N + H
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    z = rnd(B, L, E).to(dtype)
+    reset = (torch.rand(B, L, generator=g, device="cuda") < 0.05).to(torch.uint8)
+    return z, rnd(C, 4) / 2, rnd(C) * 0.1, rnd(H), reset, rnd
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L", [(40, 1111), (700, 33), (2000, 9), (6000, 3)])
+def test_pre_stage_runs_of_four_and_of_eight(B, L, dtype):
+    """Many rows walk runs of 8 timesteps, few of 4, with last runs of 1 to 3: single sequences, carried state and restarts among
+    them, are bit for bit the batch's."""
+    from trading_bot_0_amd import block_pre
+    z, w, b, bias, reset, rnd = block_inputs(B, L, dtype, L)
+    state = rnd(B, 3, w.shape[0]).to(dtype)
+    whole = block_pre(z, w, b, bias, H, 32, N, G, conv_state=state, return_conv_state=True, reset=reset)
+    for i in (0, 1, B // 2, B - 1):
+        one = block_pre(z[i:i + 1].contiguous(), w, b, bias, H, 32, N, G, conv_state=state[i:i + 1].contiguous(),
+                        return_conv_state=True, reset=reset[i:i + 1].contiguous())
+        assert all(torch.equal(a, c[i:i + 1]) for a, c in zip(one, whole)), i
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,restarts", [(5, 4111, False), (5, 4111, True), (700, 33, True), (1, 1, True), (1, 130, False), (9, 31, True)])
+def test_pre_stage_backward_runs_of_eight_and_of_thirty_two(B, L, restarts, dtype):
+    """Beyond 20 480 rows the conv's backward walks runs of 32 timesteps, below of 8: a batch's rows of dzxbcdt against those of its
+    sequences alone, bit for bit, and the parameter gradients, float32 sums over B L terms in other orders, within 1e-5 of the
+    terms' norm (the sequences' own sums added in float64)."""
+    from trading_bot_0_amd.block import block_pre_bwd
+    z, w, b, bias, reset, rnd = block_inputs(B, L, dtype, B + L)
+    reset = reset if restarts else None
+    dx, dB, dC, ddt = (rnd(*s).to(dtype) for s in ((B, L, H, 32), (B, L, G, N), (B, L, G, N), (B, L, H)))
+
+    def run(i, j):
+        part = lambda t: None if t is None else t[i:j].contiguous()
+        dz = torch.zeros_like(part(z))
+        out = block_pre_bwd(part(z), w, b, bias, part(dx), part(dB), part(dC), part(ddt), dz, H, 32, N, G, reset=part(reset))
+        return dz, out[:3]
+
+    dz, sums = run(0, B)
+    each = [run(i, i + 1) for i in range(B if B < 20 else 20)]
+    for i, (d, _) in enumerate(each):
+        assert torch.equal(d, dz[i:i + 1]), i
+    if B < 20:
+        for k, s in enumerate(sums):
+            ref = sum(e[1][k].double() for e in each)
+            assert (s.double() - ref).norm() <= 1e-5 * (B * L) ** 0.5 * max(1.0, ref.norm().item() / (B * L) ** 0.5), k

@@ -14,7 +14,6 @@ namespace ssd {
 
 namespace {
 
-constexpr int kBwdSteps = 32;    // timesteps per thread of the conv backward
 constexpr int kBwdCh = 4;            // channels per thread of the conv backward (eight would take 290 registers)
 constexpr int kPiecesPerBlock = 32;  // channel pieces (of kBwdCh) per workgroup of the conv backward
 constexpr int kRunsPerBlock = 8;
@@ -184,43 +183,124 @@ __global__ __launch_bounds__(256) void block_post_bwd_kernel(const TY *__restric
     }
 }
 
-// out[c] = sum over parts of part[p][c] (columns = channels), in a fixed order: a workgroup is 64 columns x 4 slices
-// of its share of the parts (blockIdx.y of gridDim.y shares); a slice adds every fourth part of the share in order,
-// the four slices are added in order, and the shares' sums [gridDim.y][cols] go through the same kernel once more.
-constexpr int kSumShares = 32;
-__global__ __launch_bounds__(256) void column_sums_kernel(const float *__restrict__ part, int nparts, int cols,
-                                                          float *__restrict__ out) {
-    __shared__ float sm[4][64];
+// The sums over the workgroups' partial sums: of part[p][c] over p, for every column c, in a fixed order.  A workgroup is 64
+// columns x kSumSlices slices of its share of the parts (blockIdx.y of gridDim.y shares); a slice adds every kSumSlices-th part of
+// the share in order, and the slices are added in order.  One launch sums all there is to sum behind a kernel (two jobs: the
+// workgroups of the first come first); up to kSumWholeParts parts in one share, more as kSumShares shares whose sums go through the
+// same kernel once more.
+constexpr int kSumShares = 32, kSumSlices = 16, kSumWholeParts = 1024;
+
+struct ColumnSums {
+    const float *part = nullptr;
+    int nparts = 0, cols = 0;
+    float *out = nullptr;   // [gridDim.y][cols], or with split > 0 ...
+    float *last = nullptr;  // ... column c = split i + k: k < split - 1 to out[i (split - 1) + k], the last k to last[i]
+    int split = 0;
+    int blocks() const { return (cols + 63) / 64; }
+};
+
+__global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums first, ColumnSums second, int first_blocks) {
+    __shared__ float sm[kSumSlices][64];
+    const bool one = (int)blockIdx.x < first_blocks;
+    const ColumnSums &j = one ? first : second;
     const int cl = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + cl;
-    const int per = (nparts + gridDim.y - 1) / gridDim.y;
-    const int p0 = blockIdx.y * per, p1 = min(nparts, p0 + per);
+    const int c = ((int)blockIdx.x - (one ? 0 : first_blocks)) * 64 + cl;
+    const int per = (j.nparts + gridDim.y - 1) / gridDim.y;
+    const int p0 = blockIdx.y * per, p1 = min(j.nparts, p0 + per);
     float acc = 0.f;
-    if (c < cols) {
-#pragma unroll 4
-        for (int p = p0 + q; p < p1; p += 4) acc += part[(size_t)p * cols + c];
+    if (c < j.cols) {
+#pragma unroll 8
+        for (int p = p0 + q; p < p1; p += kSumSlices) acc += j.part[(size_t)p * j.cols + c];
     }
     sm[q][cl] = acc;
     __syncthreads();
-    if (q == 0 && c < cols) out[(size_t)blockIdx.y * cols + c] = ((sm[0][cl] + sm[1][cl]) + sm[2][cl]) + sm[3][cl];
+    if (q != 0 || c >= j.cols) return;
+    float sum = sm[0][cl];
+#pragma unroll
+    for (int i = 1; i < kSumSlices; ++i) sum += sm[i][cl];
+    if (j.split == 0) {
+        j.out[(size_t)blockIdx.y * j.cols + c] = sum;
+    } else {
+        const int i = c / j.split, k = c % j.split;
+        if (k == j.split - 1) j.last[i] = sum;
+        else j.out[(size_t)i * (j.split - 1) + k] = sum;
+    }
 }
 
-// sums of nparts rows of `cols` floats into out[cols]; tmp holds kSumShares * cols floats
-static hipError_t launch_column_sums(const float *part, int nparts, int cols, float *tmp, float *out, hipStream_t st) {
-    const dim3 blocks((cols + 63) / 64, nparts >= 4 * kSumShares ? kSumShares : 1);
-    if (blocks.y == 1) {
-        column_sums_kernel<<<blocks, dim3(256), 0, st>>>(part, nparts, cols, out);
-        return hipGetLastError();
+// Sums `job` (tmp holds kSumShares * job.cols floats) and, in the last of its launches, `other` (at most kSumWholeParts parts).
+static hipError_t launch_column_sums(const ColumnSums &job, float *tmp, const ColumnSums &other, hipStream_t st) {
+    ColumnSums last = job;
+    if (job.nparts > kSumWholeParts) {
+        ColumnSums shares = job;
+        shares.out = tmp;
+        shares.split = 0;
+        column_sums_kernel<<<dim3(job.blocks(), kSumShares), dim3(64 * kSumSlices), 0, st>>>(shares, shares, job.blocks());
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        last.part = tmp;
+        last.nparts = kSumShares;
     }
-    column_sums_kernel<<<blocks, dim3(256), 0, st>>>(part, nparts, cols, tmp);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    column_sums_kernel<<<dim3(blocks.x, 1), dim3(256), 0, st>>>(tmp, kSumShares, cols, out);
+    column_sums_kernel<<<dim3(last.blocks() + other.blocks(), 1), dim3(64 * kSumSlices), 0, st>>>(last, other, last.blocks());
     return hipGetLastError();
 }
 
+// ---- dt ----------------------------------------------------------------------------------------------------
+// ddt_raw = ddt sigmoid(dt_raw + dt_bias) into the dt channels of dzxbcdt; per workgroup the sums over its rows
+// (workgroups of the conv backward's launch, the first of them: on their own they were 36 us at 524 288 rows x 8 heads, a line of
+// zxbcdt and of dzxbcdt per row, and a launch; beside the conv's they are hidden: the whole call, 131 072 rows 80 -> 67 us, 600 rows, four launches fewer, 24.4 -> 16.4)
+template <typename T>
+__device__ inline void dt_bwd_rows(int block, int blocks, float (&red)[256], const T *__restrict__ zxbcdt,
+                                   const float *__restrict__ dt_bias, const T *__restrict__ ddt, T *__restrict__ dzxbcdt,
+                                   float *__restrict__ part, const BlockShape &s) {
+    const int DI = s.H * s.P, GN = s.G * s.N, off = 2 * DI + 2 * GN;
+    const long long rows = (long long)s.B * s.L;
+    for (int h0 = 0; h0 < s.H; h0 += 256) {
+        // thread = (row slot, head): heads fastest so that a row's heads are adjacent
+        const int hpt = min(s.H - h0, 256);          // heads handled in this pass
+        const int slots = 256 / hpt;                 // rows per pass
+        const int h = h0 + threadIdx.x % hpt, slot = threadIdx.x / hpt;
+        float acc = 0.f;
+        if (slot < slots) {
+            const float bias = dt_bias[h];
+            // four rows per round, their loads requested together and without a condition (a row past the tensor
+            // reads the last row and is not stored): one trip to memory per round instead of one per row
+            constexpr int kRound = 4;
+            const long long stride = (long long)blocks * slots;
+            for (long long row0 = (long long)block * slots + slot; row0 < rows; row0 += kRound * stride) {
+                T raw_q[kRound], ddt_q[kRound];
+#pragma unroll
+                for (int u = 0; u < kRound; ++u) {
+                    const size_t row = (size_t)min(row0 + u * stride, rows - 1);
+                    raw_q[u] = zxbcdt[row * s.ld + off + h];
+                    ddt_q[u] = ddt[row * s.H + h];
+                }
+#pragma unroll
+                for (int u = 0; u < kRound; ++u) {
+                    const long long row = row0 + u * stride;
+                    const float g = (float)ddt_q[u] * sigmoidf((float)raw_q[u] + bias);
+                    if (row < rows) {
+                        dzxbcdt[(size_t)row * s.ld + off + h] = (T)g;
+                        acc += g;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        red[threadIdx.x] = acc;
+        __syncthreads();
+        if ((int)threadIdx.x < hpt) {
+            float sum = 0.f;
+            for (int q = 0; q < slots; ++q) sum += red[q * hpt + threadIdx.x];
+            part[(size_t)block * s.H + h0 + threadIdx.x] = sum;
+        }
+    }
+}
+
+// (at 128 rows, one round of loads, and up: fewer leave the long walk of many rows to few workgroups)
+constexpr int kDtBlocks = 512, kDtRows = 128;
+
 // ---- pre -----------------------------------------------------------------------------------------------------
-// One thread per (run of kBwdSteps timesteps, kBwdCh channels of x | B | C).  pre[t] = b + sum_k w[k] in[t-(K-1)+k]
+// One thread per (run of STEPS timesteps, kBwdCh channels of x | B | C).  pre[t] = b + sum_k w[k] in[t-(K-1)+k]
 // (taps before the latest restart at or before t cut: the window's older rows are zeroed at a restart, as in the
 // forward), out = silu(pre); with dpre[t] = dout[t] silu'(pre[t]):
 //   din[s]  = sum_{q=0..K-1} w[K-1-q] dpre[s+q]      over the q whose output s+q exists and lies before any restart
@@ -234,21 +314,33 @@ static hipError_t launch_column_sums(const float *part, int nparts, int cols, fl
 // are requested K steps before they are used, into the ring slot the step K before has just emptied: a conditional
 // load is a branch at which the compiler waits for every earlier load and store, which made each step wait for the
 // store of the step before.  RS: the call has a reset mask.
-template <typename T, int K, bool RS>
+template <typename T, int K, bool RS, int STEPS>
 __global__ __launch_bounds__(256) void block_pre_bwd_kernel(const T *__restrict__ zxbcdt, const float *__restrict__ conv_w,
                                                             const float *__restrict__ conv_b, const T *__restrict__ state_in,
                                                             const unsigned char *__restrict__ reset, const T *__restrict__ dx,
                                                             const T *__restrict__ dB, const T *__restrict__ dC,
                                                             const T *__restrict__ dstate_out, T *__restrict__ dzxbcdt,
-                                                            float *__restrict__ part, BlockShape s) {
+                                                            float *__restrict__ part, const float *__restrict__ dt_bias,
+                                                            const T *__restrict__ ddt, float *__restrict__ dt_part, int dt_blocks,
+                                                            BlockShape s) {
+    __shared__ union {
+        float conv[256 * (K + 1)];
+        float dt[256];
+    } lds;
+    if ((int)blockIdx.x < dt_blocks) {
+        dt_bwd_rows<T>(blockIdx.x, dt_blocks, lds.dt, zxbcdt, dt_bias, ddt, dzxbcdt, dt_part, s);
+        return;
+    }
+    float(&red)[256 * (K + 1)] = lds.conv;
+    const unsigned conv_block = blockIdx.x - dt_blocks;
     const int DI = s.H * s.P, GN = s.G * s.N, C = DI + 2 * GN;
     const int CP = C / kBwdCh;
-    const int runs = (s.L + kBwdSteps - 1) / kBwdSteps;
+    const int runs = (s.L + STEPS - 1) / STEPS;
     const int pl = threadIdx.x % kPiecesPerBlock, rl = threadIdx.x / kPiecesPerBlock;
     // one linear grid, piece blocks fastest (the grid's second dimension stops at 65 535 run blocks)
     const unsigned piece_blocks = (CP + kPiecesPerBlock - 1) / kPiecesPerBlock;
-    const unsigned run_block = blockIdx.x / piece_blocks;
-    const int piece = (blockIdx.x % piece_blocks) * kPiecesPerBlock + pl;
+    const unsigned run_block = conv_block / piece_blocks;
+    const int piece = (conv_block % piece_blocks) * kPiecesPerBlock + pl;
     const long long br = (long long)run_block * kRunsPerBlock + rl;
     const bool active = piece < CP && br < (long long)s.B * runs;
     float dwacc[kBwdCh][K], dbacc[kBwdCh];
@@ -259,8 +351,8 @@ __global__ __launch_bounds__(256) void block_pre_bwd_kernel(const T *__restrict_
         for (int k = 0; k < K; ++k) dwacc[i][k] = 0.f;
     }
     if (active) {
-        const int t0 = (int)(br % runs) * kBwdSteps, b = (int)(br / runs);
-        const int t1 = min(t0 + kBwdSteps, s.L);
+        const int t0 = (int)(br % runs) * STEPS, b = (int)(br / runs);
+        const int t1 = min(t0 + STEPS, s.L);
         const int c0 = piece * kBwdCh;
         const T *row0 = zxbcdt + ((size_t)b * s.L) * s.ld + DI + c0;
         const unsigned char *rs = RS ? reset + (size_t)b * s.L : nullptr;
@@ -354,7 +446,7 @@ __global__ __launch_bounds__(256) void block_pre_bwd_kernel(const T *__restrict_
             }
         }
         T *drow = dzxbcdt + ((size_t)b * s.L) * s.ld + DI + c0;
-        constexpr int NT = kBwdSteps + K - 1;
+        constexpr int NT = STEPS + K - 1;
 #pragma unroll 1
         for (int jb = 0; jb < NT; jb += K) {
 #pragma unroll
@@ -424,7 +516,6 @@ __global__ __launch_bounds__(256) void block_pre_bwd_kernel(const T *__restrict_
         }
     }
     // the workgroup's partial sums: per channel piece, its kRunsPerBlock threads added in order
-    __shared__ float red[256 * (K + 1)];
     const int cols = C * (K + 1);
 #pragma unroll
     for (int i = 0; i < kBwdCh; ++i) {
@@ -528,74 +619,22 @@ __global__ __launch_bounds__(256) void block_pre_bwd_state_kernel(const T *__res
     }
 }
 
-// ddt_raw = ddt sigmoid(dt_raw + dt_bias) into the dt channels of dzxbcdt; per workgroup the sums over its rows
-template <typename T>
-__global__ __launch_bounds__(256) void block_dt_bwd_kernel(const T *__restrict__ zxbcdt, const float *__restrict__ dt_bias,
-                                                           const T *__restrict__ ddt, T *__restrict__ dzxbcdt,
-                                                           float *__restrict__ part, BlockShape s) {
-    const int DI = s.H * s.P, GN = s.G * s.N, off = 2 * DI + 2 * GN;
-    const long long rows = (long long)s.B * s.L;
-    __shared__ float red[256];
-    for (int h0 = 0; h0 < s.H; h0 += 256) {
-        // thread = (row slot, head): heads fastest so that a row's heads are adjacent
-        const int hpt = min(s.H - h0, 256);          // heads handled in this pass
-        const int slots = 256 / hpt;                 // rows per pass
-        const int h = h0 + threadIdx.x % hpt, slot = threadIdx.x / hpt;
-        float acc = 0.f;
-        if (slot < slots) {
-            const float bias = dt_bias[h];
-            // four rows per round, their loads requested together and without a condition (a row past the tensor
-            // reads the last row and is not stored): one trip to memory per round instead of one per row
-            constexpr int kRound = 4;
-            const long long stride = (long long)gridDim.x * slots;
-            for (long long row0 = (long long)blockIdx.x * slots + slot; row0 < rows; row0 += kRound * stride) {
-                T raw_q[kRound], ddt_q[kRound];
-#pragma unroll
-                for (int u = 0; u < kRound; ++u) {
-                    const size_t row = (size_t)min(row0 + u * stride, rows - 1);
-                    raw_q[u] = zxbcdt[row * s.ld + off + h];
-                    ddt_q[u] = ddt[row * s.H + h];
-                }
-#pragma unroll
-                for (int u = 0; u < kRound; ++u) {
-                    const long long row = row0 + u * stride;
-                    const float g = (float)ddt_q[u] * sigmoidf((float)raw_q[u] + bias);
-                    if (row < rows) {
-                        dzxbcdt[(size_t)row * s.ld + off + h] = (T)g;
-                        acc += g;
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        red[threadIdx.x] = acc;
-        __syncthreads();
-        if ((int)threadIdx.x < hpt) {
-            float sum = 0.f;
-            for (int q = 0; q < slots; ++q) sum += red[q * hpt + threadIdx.x];
-            part[(size_t)blockIdx.x * s.H + h0 + threadIdx.x] = sum;
-        }
-    }
-}
-
-constexpr int kDtBlocks = 512;
-
-// [C][K+1] sums -> dconv_w [C][K], dconv_b [C]
-__global__ __launch_bounds__(256) void split_conv_sums_kernel(const float *__restrict__ sums, int C, int K,
-                                                              float *__restrict__ dw, float *__restrict__ db) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    for (int k = 0; k < K; ++k) dw[(size_t)c * K + k] = sums[(size_t)c * (K + 1) + k];
-    db[c] = sums[(size_t)c * (K + 1) + K];
-}
-
 }  // namespace
+
+// Workgroups along the runs of `steps` timesteps of the conv backward.
+static long long bwd_run_blocks(const BlockShape &s, int steps) {
+    return ((long long)s.B * ((s.L + steps - 1) / steps) + kRunsPerBlock - 1) / kRunsPerBlock;
+}
+// Runs of 8 timesteps (11 with the K - 1 beyond them, where runs of 32 take 35: a serial chain of 15 us however few rows there are)
+// up to that many such workgroups, 20 480 rows.  8 heads of 32, state 64, d_conv 4, the whole call, runs of 32 / 8 in us: 600 rows
+// 16.4 / 9.3, 4 000 18.0 / 10.8, 8 192 18.1 / 13.0, 16 384 19.2 / 16.7, 32 768 24.0 / 26.4, 262 144 158 / 179.  (The workspace is sized
+// for either: it grows with batch and length.)
+constexpr long long kShortRunBlocks = 320;
 
 // workspace: the partial sums of post_bwd, or those of pre_bwd (conv, their column sums, dt)
 size_t block_bwd_workspace_bytes(const BlockShape &s) {
     const size_t DI = (size_t)s.H * s.P, C = DI + 2 * (size_t)s.G * s.N;
-    const size_t runs = (s.L + kBwdSteps - 1) / kBwdSteps;
-    const size_t run_blocks = ((size_t)s.B * runs + kRunsPerBlock - 1) / kRunsPerBlock;
+    const size_t run_blocks = std::max(bwd_run_blocks(s, 32), std::min<long long>(bwd_run_blocks(s, 8), kShortRunBlocks));
     const size_t post = (size_t)(kPostBlocks + kSumShares) * DI;
     const size_t pre = (run_blocks + 1 + kSumShares) * C * (s.d_conv + 1) + (size_t)(kDtBlocks + kSumShares) * s.H;
     return sizeof(float) * (post > pre ? post : pre);  // the two stages run one after the other and share it
@@ -630,7 +669,7 @@ static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const vo
     if (!launched) return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_column_sums(part, blocks, DI, part + (size_t)kPostBlocks * DI, dnorm_w, st);
+    return launch_column_sums(ColumnSums{part, blocks, DI, dnorm_w}, part + (size_t)kPostBlocks * DI, ColumnSums{}, st);
 }
 
 hipError_t launch_block_post_bwd(const BlockShape &s, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
@@ -651,55 +690,42 @@ static hipError_t pre_bwd_dispatch(const BlockShape &s, const void *zxbcdt, cons
                                    float *dconv_w, float *dconv_b, float *ddt_bias, void *dstate_in, float *part,
                                    hipStream_t st) {
     const int DI = s.H * s.P, C = DI + 2 * s.G * s.N, CP = C / kBwdCh, K = s.d_conv;
-    const long long runs = (s.L + kBwdSteps - 1) / kBwdSteps;
-    const long long run_blocks = ((long long)s.B * runs + kRunsPerBlock - 1) / kRunsPerBlock;
+    const int steps = bwd_run_blocks(s, 8) <= kShortRunBlocks ? 8 : 32;
+    const long long run_blocks = bwd_run_blocks(s, steps);
     const long long piece_blocks = (CP + kPiecesPerBlock - 1) / kPiecesPerBlock;
-    if (run_blocks * piece_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(run_blocks * piece_blocks));
+    const int cols = C * (K + 1);
+    float *tmp = part + (size_t)run_blocks * cols;  // (behind the partials: the shares' sums, then dt's partials)
+    float *dt_part = tmp + (size_t)kSumShares * cols;
+    const int dt_blocks = (int)std::min<long long>(kDtBlocks, ((long long)s.B * s.L + kDtRows - 1) / kDtRows);
+    if (run_blocks * piece_blocks + dt_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(run_blocks * piece_blocks + dt_blocks));
     const T *in = static_cast<const T *>(zxbcdt), *si = static_cast<const T *>(state_in);
     const T *gx = static_cast<const T *>(dx), *gb = static_cast<const T *>(dB), *gc = static_cast<const T *>(dC);
-    const T *gso = static_cast<const T *>(dstate_out);
+    const T *gso = static_cast<const T *>(dstate_out), *gt = static_cast<const T *>(ddt);
     T *out = static_cast<T *>(dzxbcdt), *gsi = static_cast<T *>(dstate_in);
     const dim3 sgrid((unsigned)(((long long)s.B * (C / 8) + 255) / 256));
-    switch (K) {
-        case 2:
-            if (reset != nullptr)
-                block_pre_bwd_kernel<T, 2, true><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            else
-                block_pre_bwd_kernel<T, 2, false><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            if (gsi) block_pre_bwd_state_kernel<T, 2><<<sgrid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, gsi, s);
-            break;
-        case 3:
-            if (reset != nullptr)
-                block_pre_bwd_kernel<T, 3, true><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            else
-                block_pre_bwd_kernel<T, 3, false><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            if (gsi) block_pre_bwd_state_kernel<T, 3><<<sgrid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, gsi, s);
-            break;
-        case 4:
-            if (reset != nullptr)
-                block_pre_bwd_kernel<T, 4, true><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            else
-                block_pre_bwd_kernel<T, 4, false><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, s);
-            if (gsi) block_pre_bwd_state_kernel<T, 4><<<sgrid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, gsi, s);
-            break;
-        default: return hipErrorInvalidValue;
+    bool launched = false;
+#define SSD_PRE_BWD_CASE(Kv, RSv, Sv)                                                                                             \
+    if (K == Kv && (reset != nullptr) == RSv && steps == Sv) {                                                                    \
+        block_pre_bwd_kernel<T, Kv, RSv, Sv><<<grid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, out, part, \
+                                                                         dt_bias, gt, dt_part, dt_blocks, s);                     \
+        launched = true;                                                                                                          \
     }
+#define SSD_PRE_BWD_FILTER(Kv)                                                                                                    \
+    SSD_PRE_BWD_CASE(Kv, false, 8) SSD_PRE_BWD_CASE(Kv, true, 8) SSD_PRE_BWD_CASE(Kv, false, 32) SSD_PRE_BWD_CASE(Kv, true, 32)   \
+    if (K == Kv && gsi)                                                                                                           \
+        block_pre_bwd_state_kernel<T, Kv><<<sgrid, dim3(256), 0, st>>>(in, conv_w, conv_b, si, reset, gx, gb, gc, gso, gsi, s);
+    SSD_PRE_BWD_FILTER(2)
+    SSD_PRE_BWD_FILTER(3)
+    SSD_PRE_BWD_FILTER(4)
+#undef SSD_PRE_BWD_FILTER
+#undef SSD_PRE_BWD_CASE
+    if (!launched) return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // the partials hold, per run block, [C][K+1] = (dw[0..K-1], db): sum the columns, then split them
-    const int cols = C * (K + 1);
-    float *sums = part + (size_t)run_blocks * cols;  // (behind the partials: cols floats, then the shares' sums)
-    float *tmp = sums + cols;
-    if ((e = launch_column_sums(part, (int)run_blocks, cols, tmp, sums, st)) != hipSuccess) return e;
-    float *dt_part = tmp + (size_t)kSumShares * cols;
-    const long long rows = (long long)s.B * s.L;
-    const int dt_blocks = (int)std::min<long long>(kDtBlocks, rows);
-    block_dt_bwd_kernel<T><<<dim3(dt_blocks), dim3(256), 0, st>>>(in, dt_bias, static_cast<const T *>(ddt), out, dt_part, s);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = launch_column_sums(dt_part, dt_blocks, s.H, dt_part + (size_t)kDtBlocks * s.H, ddt_bias, st)) != hipSuccess) return e;
-    split_conv_sums_kernel<<<dim3((C + 255) / 256), dim3(256), 0, st>>>(sums, C, K, dconv_w, dconv_b);
-    return hipGetLastError();
+    // the conv's partials hold, per run block, [C][K+1] = (dw[0..K-1], db)
+    return launch_column_sums(ColumnSums{part, (int)run_blocks, cols, dconv_w, dconv_b, K + 1}, tmp,
+                              ColumnSums{dt_part, dt_blocks, s.H, ddt_bias}, st);
 }
 
 hipError_t launch_block_pre_bwd(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w, const float *conv_b,

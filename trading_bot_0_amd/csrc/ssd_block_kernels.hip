@@ -10,7 +10,7 @@
 
 namespace ssd {
 
-// One thread per (run of kPreSteps timesteps, 8 channels of x | B | C): the filter taps of its channels are
+// One thread per (run of STEPS timesteps, 8 channels of x | B | C): the filter taps of its channels are
 // loaded once and the d_conv-1 previous input rows slide through registers, so every input row is read once
 // per run.  The dt channels are done by the threads after those, one (timestep, 8 heads) each, so that no
 // wave mixes the two code paths.  History
@@ -18,9 +18,7 @@ namespace ssd {
 // zero; state_out receives the last d_conv-1 input rows.  reset [B, L] bytes or NULL: a non-zero reset[b,t] cuts
 // the filter's history before timestep t (an episode boundary: the rows before t count as zeros from t on, in the
 // outputs and in state_out), which is what zeroing the conv state between two calls does at a window boundary.
-constexpr int kPreSteps = 16;
-
-template <typename T, int DCONV>
+template <typename T, int DCONV, int STEPS>
 __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zxbcdt, const float *__restrict__ conv_w,
                                                         const float *__restrict__ conv_b, const float *__restrict__ dt_bias,
                                                         const T *state_in, T *state_out,
@@ -29,7 +27,7 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
                                                         T *__restrict__ dt, BlockShape s) {
     const int DI = s.H * s.P, GN = s.G * s.N, C = DI + 2 * GN;
     const int CP = C / 8, HP8 = (s.H + 7) / 8;
-    const int runs = (s.L + kPreSteps - 1) / kPreSteps;
+    const int runs = (s.L + STEPS - 1) / STEPS;
     const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long conv_total = (long long)s.B * runs * CP;
     if (gid >= conv_total) {
@@ -54,17 +52,17 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
     }
     const int piece = (int)(gid % CP);
     const long long br = gid / CP;
-    const int t0 = (int)(br % runs) * kPreSteps, b = (int)(br / runs);
-    const int t1 = min(t0 + kPreSteps, s.L);
+    const int t0 = (int)(br % runs) * STEPS, b = (int)(br / runs);
+    const int t1 = min(t0 + STEPS, s.L);
     const T *row0 = zxbcdt + ((size_t)b * s.L) * s.ld;  // this batch row's first timestep
     const int c0 = piece * 8;  // channel within [x | B | C]
     // Every load of the thread is issued before the first is used and none is under a condition (a conditional load
     // is a branch, and the compiler waits for all earlier loads -- and stores -- at every one): rows outside the
     // sequence read a row inside it and are replaced by zeros or never stored.
     // the run's input rows
-    Pack8<T> in[kPreSteps];
+    Pack8<T> in[STEPS];
 #pragma unroll
-    for (int j = 0; j < kPreSteps; ++j) in[j] = Pack8<T>::load(row0 + (size_t)min(t0 + j, s.L - 1) * s.ld + DI + c0);
+    for (int j = 0; j < STEPS; ++j) in[j] = Pack8<T>::load(row0 + (size_t)min(t0 + j, s.L - 1) * s.ld + DI + c0);
     // the d_conv-1 rows before the run: rows of this call, of state_in, or zeros
     Pack8<T> hist[DCONV - 1];
 #pragma unroll
@@ -78,11 +76,11 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
     const unsigned char *rs = reset ? reset + (size_t)b * s.L : nullptr;
     unsigned flags = 0;
     if (rs != nullptr) {
-        unsigned char rv[kPreSteps + DCONV - 2];
+        unsigned char rv[STEPS + DCONV - 2];
 #pragma unroll
-        for (int j = 0; j < kPreSteps + DCONV - 2; ++j) rv[j] = rs[min(max(t0 - (DCONV - 2) + j, 0), s.L - 1)];
+        for (int j = 0; j < STEPS + DCONV - 2; ++j) rv[j] = rs[min(max(t0 - (DCONV - 2) + j, 0), s.L - 1)];
 #pragma unroll
-        for (int j = 0; j < kPreSteps + DCONV - 2; ++j) {
+        for (int j = 0; j < STEPS + DCONV - 2; ++j) {
             const int ts = t0 - (DCONV - 2) + j;
             flags |= (ts >= 0 && ts < s.L && rv[j] != 0) ? (1u << j) : 0u;
         }
@@ -138,7 +136,7 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
         dst_stride = GN;
     }
 #pragma unroll
-    for (int j = 0; j < kPreSteps; ++j) {
+    for (int j = 0; j < STEPS; ++j) {
         const int t = t0 + j;
         if (t >= t1) break;
         const Pack8<T> v = in[j];
@@ -168,7 +166,7 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
     // Streaming state: the d_conv-1 input rows before timestep L.  After the run that ends the sequence the window
     // registers hold exactly those rows -- rows of this call, or, where the call brought fewer than d_conv-1 new
     // rows, the tail of state_in, which was loaded before anything was stored: state_in and state_out may be the
-    // same memory whenever one thread both reads and writes a channel piece's state (seqlen <= kPreSteps).
+    // same memory whenever one thread both reads and writes a channel piece's state (seqlen <= STEPS).
     if (state_out != nullptr && t1 == s.L) {
 #pragma unroll
         for (int k = 0; k < DCONV - 1; ++k) Pack8<T>::store(state_out + ((size_t)b * (DCONV - 1) + k) * C + c0, win[k]);
@@ -247,19 +245,30 @@ template <typename T>
 static hipError_t pre_dispatch(const BlockShape &s, const void *zxbcdt, const float *conv_w, const float *conv_b,
                                const float *dt_bias, const void *state_in, void *state_out,
                                const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t st) {
-    const long long total = (long long)s.B * ((s.L + kPreSteps - 1) / kPreSteps) * ((s.H * s.P + 2 * s.G * s.N) / 8) +
-                            (long long)s.B * s.L * ((s.H + 7) / 8);
+    // Runs of 4 steps while those leave the chip a wave per SIMD or less -- a run of 16 is six microseconds of vector
+    // instructions for its wave, however few there are -- then of 8.  8 heads of 32, state 64, runs of 16 / 8 / 4 in us: 600 rows
+    // 7.3 / 7.1 / 6.1, 4 000 7.6 / 5.5 / 4.8, 8 192 8.1 / 6.0 / 6.2, 16 384 9.3 / 8.8 / 10.2, 131 072 40.6 / 38.8 / 42.5, 262 144
+    // 86.6 / 86.0 / 94.4.
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = device_cu_count(dev, &cus);
+    if (e != hipSuccess) return e;
+    const long long pieces = (s.H * s.P + 2 * s.G * s.N) / 8;
+    const int steps = (long long)s.B * ((s.L + 3) / 4) * pieces <= 256LL * cus ? 4 : 8;
+    const long long total = (long long)s.B * ((s.L + steps - 1) / steps) * pieces + (long long)s.B * s.L * ((s.H + 7) / 8);
     const dim3 grid((unsigned)((total + 255) / 256)), block(256);
     const T *in = static_cast<const T *>(zxbcdt), *si = static_cast<const T *>(state_in);
     T *so = static_cast<T *>(state_out), *xx = static_cast<T *>(x), *bb = static_cast<T *>(Bm), *cc = static_cast<T *>(Cm),
       *dd = static_cast<T *>(dt);
-    switch (s.d_conv) {
-        case 2: block_pre_kernel<T, 2><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, s); break;
-        case 3: block_pre_kernel<T, 3><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, s); break;
-        case 4: block_pre_kernel<T, 4><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, s); break;
-        default: return hipErrorInvalidValue;
+#define SSD_PRE_CASE(Kv, Sv)                                                                                                     \
+    if (s.d_conv == Kv && steps == Sv) {                                                                                         \
+        block_pre_kernel<T, Kv, Sv><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, s);      \
+        return hipGetLastError();                                                                                                \
     }
-    return hipGetLastError();
+    SSD_PRE_CASE(2, 4) SSD_PRE_CASE(3, 4) SSD_PRE_CASE(4, 4)
+    SSD_PRE_CASE(2, 8) SSD_PRE_CASE(3, 8) SSD_PRE_CASE(4, 8)
+#undef SSD_PRE_CASE
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_block_pre(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w,
