@@ -75,18 +75,19 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(const T *__restrict__
 }
 
 // ------------------------------------------------------------------------------------------
-// Stage 3: state_passing.  A thread holds one float4 of the [P,N] state of one (b,h) over a run of kPassRun consecutive
+// Stage 3: state_passing.  A thread holds one float4 of the [P,N] state of one (b,h) over a run of RUN consecutive
 // chunks, whose loads are all in flight at once; the kPassSegs runs of a workgroup follow one another.  Every run is
 // first folded from a zero state, the runs' results meet in LDS, every thread folds those before its own into the
 // state entering its run and writes the states entering its chunks from the registers.  So 64 chunks cost one trip to
 // memory (a thread per piece that walked the chunks eight at a time made a trip for every eight: 8 heads, state
-// 32 x 64: 4 sequences of 32 chunks 8.6 -> 5.5 us, 2 of 71 16.8 -> 9.1; 16 heads, 64 x 128, 4 of 16 chunks 12.6 -> 14.7).
+// 32 x 64: 4 sequences of 32 chunks 8.6 -> 5.5 us, 2 of 71 16.8 -> 9.1; 16 heads, 64 x 128, 4 of 16 chunks 12.6 -> 13.1).
 // a_end: alpha at the end of chunk c of sequence bh at [bh * nc + c] * a_stride.
 // prev may alias states: a thread reads its chunks before it writes them, and no other thread touches them;
 // final_states may alias init: it is written behind a barrier that all of the workgroup's reads of init precede.
 // ------------------------------------------------------------------------------------------
-constexpr int kPassSegs = 8, kPassRun = 8, kPassPieces = 32;  // P * N / 4 is a multiple of 32 (P of 8, N of 16)
+constexpr int kPassSegs = 8, kPassPieces = 32;  // P * N / 4 is a multiple of 32 (P of 8, N of 16)
 
+template <int RUN>  // 1, 2, 4 or 8
 __global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(const float *states, const float *__restrict__ a_end,
                                                                                int a_stride, const float *init, float *prev,
                                                                                float *final_states, ScanShape s) {
@@ -108,24 +109,22 @@ __global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(c
         v.z = dec * v.z + add.z;
         v.w = dec * v.w + add.w;
     };
-    // chunks per run: as few as cover the sequence, so that a short one is spread over all runs
-    const int run = min(kPassRun, (s.nc + kPassSegs - 1) / kPassSegs);
-    for (int c0 = 0, buf = 0; c0 < s.nc; c0 += run * kPassSegs, buf ^= 1) {
-        const int c = c0 + seg * run;
-        float4 sv[kPassRun];
-        float dec[kPassRun];
+    for (int c0 = 0, buf = 0; c0 < s.nc; c0 += RUN * kPassSegs, buf ^= 1) {
+        const int c = c0 + seg * RUN;
+        float4 sv[RUN];
+        float dec[RUN];
 #pragma unroll
-        for (int i = 0; i < kPassRun; ++i) {  // (past the run or the sequence: read as the last chunk and not used)
-            const int ci = min(c + min(i, run - 1), s.nc - 1);
+        for (int i = 0; i < RUN; ++i) {  // (past the sequence: read as the last chunk and not used)
+            const int ci = min(c + i, s.nc - 1);
             sv[i] = src[(size_t)ci * chunk_stride];
             dec[i] = ae[(size_t)ci * a_stride];
         }
         float4 local = make_float4(0, 0, 0, 0);
         float decay = 1.f;
 #pragma unroll
-        for (int i = 0; i < kPassRun; ++i) {
+        for (int i = 0; i < RUN; ++i) {
             dec[i] = exp2_hw(dec[i]);
-            if (i < run && c + i < s.nc) {
+            if (c + i < s.nc) {
                 step(local, dec[i], sv[i]);
                 decay *= dec[i];
             }
@@ -140,8 +139,8 @@ __global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(c
             step(st, run_decay[buf][k], run_state[buf][k][piece]);
         }
 #pragma unroll
-        for (int i = 0; i < kPassRun; ++i) {
-            if (i < run && c + i < s.nc) {
+        for (int i = 0; i < RUN; ++i) {
+            if (c + i < s.nc) {
                 dst[(size_t)(c + i) * chunk_stride] = enter;
                 step(enter, dec[i], sv[i]);
             }
@@ -347,8 +346,12 @@ hipError_t launch_state_passing(const ScanShape &s, const float *states, const f
                                 float *prev, float *final_states, hipStream_t st) {
     const long long blocks = (long long)s.B * s.H * (s.P * s.N / 4 / kPassPieces);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    state_passing_kernel<<<dim3((unsigned)blocks), dim3(kPassSegs * kPassPieces), 0, st>>>(states, a_end, a_stride, init, prev,
-                                                                                            final_states, s);
+    const dim3 grid((unsigned)blocks), block(kPassSegs * kPassPieces);
+    // as short runs as cover the sequence in one round, where eight do
+    if (s.nc <= kPassSegs) state_passing_kernel<1><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
+    else if (s.nc <= 2 * kPassSegs) state_passing_kernel<2><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
+    else if (s.nc <= 4 * kPassSegs) state_passing_kernel<4><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
+    else state_passing_kernel<8><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
     return hipGetLastError();
 }
 
