@@ -112,6 +112,10 @@ extern "C" {
         dt: *mut c_void, hip_stream: *mut c_void) -> c_int;
     pub fn ssd_block_proj_fwd(rows: i64, in_features: i64, out_features: i64, out_ld: i64, dtype: c_int,
         u: *const c_void, w: *const c_void, out: *mut c_void, hip_stream: *mut c_void) -> c_int;
+    pub fn ssd_block_dproj(rows: i64, a_features: i64, out_features: i64, a_ld: i64, w_ld: i64, dtype: c_int, a: *const c_void,
+        w_t: *const c_void, out: *mut c_void, hip_stream: *mut c_void) -> c_int;
+    pub fn ssd_block_weights(in_features: i64, d_model: i64, d_inner: i64, in_proj: *const f32, out_proj: *const f32, w_in: *mut c_void,
+        w_in_t: *mut c_void, w_out: *mut c_void, w_out_t: *mut c_void, hip_stream: *mut c_void) -> c_int;
     pub fn ssd_block_wgrad_workspace_bytes(rows: i64, a_features: i64, b_features: i64, out_bytes: *mut usize) -> c_int;
     pub fn ssd_block_wgrad(rows: i64, a_features: i64, b_features: i64, a_ld: i64, dtype: c_int, a: *const c_void,
         b: *const c_void, out: *mut f32, workspace: *mut c_void, workspace_bytes: usize, hip_stream: *mut c_void) -> c_int;

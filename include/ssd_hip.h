@@ -276,6 +276,20 @@ int ssd_block_pre_reset_fwd(const ssd_block_dims *dims, int dtype, const void *z
 int ssd_block_proj_fwd(int64_t rows, int64_t in_features, int64_t out_features, int64_t out_ld, int dtype, const void *u,
                        const void *w, void *out, void *hip_stream);
 
+/* Gradient of a projection's input: out [rows, out_features] = a [rows, a_features] . w_t [out_features, w_ld]^T, bfloat16 in and out
+ * (dtype 1), float32 accumulation; for out = u . w^T it is du with a = dout and w_t = w^T.  a's rows are a_ld elements apart (0 =
+ * a_features, else at least that and a multiple of 8; what follows a row's a_features elements is not used).  w_t is padded with
+ * zeros from column a_features to the next multiple of 16: w_ld is at least that and a multiple of 8.  Both features must be
+ * multiples of 8 and 32 rows of a fit 160 KiB (SSD_ERR_UNSUPPORTED otherwise: use the caller's BLAS). */
+int ssd_block_dproj(int64_t rows, int64_t a_features, int64_t out_features, int64_t a_ld, int64_t w_ld, int dtype, const void *a,
+                    const void *w_t, void *out, void *hip_stream);
+
+/* The block's projections in bfloat16, as the entry points around take them, from float32: in_proj [in_features, d_model] as it is
+ * (w_in) and turned with zeros up to a multiple of 16 columns (w_in_t, for ssd_block_dproj), out_proj [d_model, d_inner] as it is
+ * (w_out) and turned (w_out_t [d_inner, d_model]).  Rounded to nearest even, one launch. */
+int ssd_block_weights(int64_t in_features, int64_t d_model, int64_t d_inner, const float *in_proj, const float *out_proj, void *w_in,
+                      void *w_in_t, void *w_out, void *w_out_t, void *hip_stream);
+
 /* Weight gradient of a projection: out [a_features, b_features] (float32) = sum over rows of a[r]^T b[r], with
  * a [rows, a_features] (rows a_ld elements apart: 0 = a_features, else at least that and a multiple of 8) and
  * b [rows, b_features], bfloat16 (dtype 1), float32 accumulation in a fixed order; for out = u . w^T it is dw with

@@ -105,3 +105,35 @@ def test_pre_stage_backward_runs_of_eight_and_of_thirty_two(B, L, restarts, dtyp
         for k, s in enumerate(sums):
             ref = sum(e[1][k].double() for e in each)
             assert (s.double() - ref).norm() <= 1e-5 * (B * L) ** 0.5 * max(1.0, ref.norm().item() / (B * L) ** 0.5), k
+
+
+@pytest.mark.parametrize("E,D", [(648, 256), (392, 128), (8, 8), (136, 72), (1024, 200), (2544, 16)])
+@pytest.mark.parametrize("rows", [1, 31, 33, 64, 700, 8193, 20000])
+def test_input_gradient_of_a_projection(rows, E, D):
+    """a . w against float64, at the workgroups' sizes (32 x 128, 64 x 128, 64 x 256), features off the steps of 16 and columns off the
+    blocks; a is the first columns of longer rows whose rest is not a number.  The bound is rounding alone: one of the result, and
+    float32 sums of E terms."""
+    from trading_bot_0_amd.block import block_dproj, turned_weight
+    g = torch.Generator(device="cuda").manual_seed(rows + E)
+    buf = torch.full((rows, (E + 63) // 64 * 64), float("nan"), dtype=torch.bfloat16, device="cuda")
+    buf[:, :E] = torch.randn(rows, E, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(E, D, generator=g, device="cuda") / E ** 0.5).to(torch.bfloat16)
+    out = block_dproj(buf[:, :E], turned_weight(w))
+    ref, mag = buf[:, :E].double() @ w.double(), buf[:, :E].double().abs() @ w.double().abs()
+    assert out.shape == (rows, D) and ((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + E * 2.0 ** -24 * mag).all()
+    assert torch.equal(block_dproj(buf[:, :E].contiguous(), turned_weight(w)), out)
+
+
+@pytest.mark.parametrize("shape", [(256, 8, 32, 64, 1), (72, 8, 16, 16, 2), (128, 4, 40, 32, 1)])
+def test_weights_converted_in_one_launch(shape):
+    """The bf16 copies are torch's own rounding, the turned ones their transposes, padded with zeros; again after an update in place."""
+    from trading_bot_0_amd import Mamba2Block
+    from trading_bot_0_amd.block import turned_weight
+    d_model, heads, P, ns, groups = shape
+    blk = Mamba2Block(d_model, heads, P, ns, groups, seed=1)
+    for _ in range(2):
+        _, w_in, w_out, w_out_t, _, w_in_t = blk._converted(torch.bfloat16)
+        assert torch.equal(w_in, blk.in_proj.to(torch.bfloat16)) and torch.equal(w_out, blk.out_proj.to(torch.bfloat16))
+        assert torch.equal(w_out_t, w_out.t()) and torch.equal(w_in_t, turned_weight(w_in))
+        blk.in_proj.mul_(1.5)
+        blk.out_proj.add_(0.25)

@@ -36,6 +36,8 @@ def _lib():
         lib.ssd_block_pre_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, P, P, P, P, P, P, P, P]
         lib.ssd_block_post_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, P]
         lib.ssd_block_proj_fwd.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int, P, P, P, P]
+        lib.ssd_block_dproj.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int64, c_int, P, P, P, P]
+        lib.ssd_block_weights.argtypes = [c_int64, c_int64, c_int64, P, P, P, P, P, P, P]
         lib.ssd_block_wgrad_workspace_bytes.argtypes = [c_int64, c_int64, c_int64, POINTER(c_size_t)]
         lib.ssd_block_wgrad.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int, P, P, P, P, c_size_t, P]
         lib.ssd_block_post_proj_fwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, c_int64, c_int64, P, P]
@@ -79,6 +81,39 @@ def block_wgrad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     ssd._check(lib, lib.ssd_block_wgrad(rows, E, D, a.stride(0), ssd.SSD_DTYPE_BF16, a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                         ssd._ptr(ws), need.value, ssd._stream_ptr(a)))
     return out
+
+
+def turned_weight(weight: torch.Tensor) -> torch.Tensor:
+    """weight [a_features, out_features] as `block_dproj` takes it: transposed, a_features padded with zeros to a multiple of 16."""
+    E, D = weight.shape
+    t = weight.new_zeros((D, (E + 15) // 16 * 16))
+    t[:, :E] = weight.t()
+    return t
+
+
+def block_dproj_supported(a: torch.Tensor, w_t: torch.Tensor) -> bool:
+    """Whether `block_dproj` takes these tensors (else the caller's BLAS does it)."""
+    return (a.is_cuda and a.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16 and a.shape[1] % 8 == 0 and 0 < a.shape[1] <= 2544
+            and w_t.shape[0] % 8 == 0 and 0 < a.shape[0] < 2 ** 31 and a.stride(1) == 1 and a.stride(0) % 8 == 0
+            and a.stride(0) >= a.shape[1] and a.data_ptr() % 16 == 0 and w_t.is_contiguous() and w_t.data_ptr() % 16 == 0)
+
+
+def block_dproj(a: torch.Tensor, w_t: torch.Tensor) -> torch.Tensor:
+    """a . w [rows, out_features] (bf16) for a [rows, a_features] (rows dense or evenly padded) and w_t = turned_weight(w): the
+    gradient of a projection's input (a = the gradient of its output)."""
+    lib = _lib()
+    if a.dim() != 2 or w_t.dim() != 2 or w_t.shape[1] != (a.shape[1] + 15) // 16 * 16 or a.device != w_t.device \
+            or not block_dproj_supported(a, w_t):
+        raise ValueError(f"block_dproj does not take {tuple(a.shape)} {a.dtype} (strides {a.stride()}) and {tuple(w_t.shape)} {w_t.dtype}")
+    out = a.new_empty((a.shape[0], w_t.shape[0]))
+    ssd._check(lib, lib.ssd_block_dproj(a.shape[0], a.shape[1], w_t.shape[0], a.stride(0), w_t.shape[1], ssd.SSD_DTYPE_BF16,
+                                        a.data_ptr(), w_t.data_ptr(), out.data_ptr(), ssd._stream_ptr(a)))
+    return out
+
+
+# rows and features up to which the library's kernel forms a projection's input gradient: 648 -> 256 in us, library / BLAS, 4 000 rows
+# 8.1 / 9.5, 16 384 14.2 / 16.2, 24 000 26 / 21; 1 288 -> 256 at 800 rows 12.4 / 10.1 (and 4 / 20 of the host's time)
+DPROJ_MAX_ROWS, DPROJ_MAX_FEATURES = 16384, 1024
 
 
 def _wgrad_slab_limit(E: int, D: int) -> int:
@@ -544,7 +579,11 @@ class Mamba2Block:
                                                       g["dC"], g["ddt"], dzx, self.H, self.P, self.N, self.G, reset=reset,
                                                       workspace=ws)
         dz2 = dbuf.view(Bsz * L, ld)[:, :E]
-        du = torch.matmul(dz2, w_in).view(Bsz, L, self.d_model)
+        w_in_t = self._converted(act)[5]
+        if Bsz * L <= DPROJ_MAX_ROWS and E <= DPROJ_MAX_FEATURES and w_in_t is not None and block_dproj_supported(dz2, w_in_t):
+            du = block_dproj(dz2, w_in_t).view(Bsz, L, self.d_model)
+        else:
+            du = torch.matmul(dz2, w_in).view(Bsz, L, self.d_model)
         din_proj = _weight_gradient(dz2, u.reshape(Bsz * L, self.d_model))
         return dict(du=du, din_proj=din_proj, dconv_w=dconv_w, dconv_b=dconv_b, ddt_bias=ddt_bias, dA=g["dA"],
                     dA_log=g["dA"] * A, dD=g["dD"], dnorm_w=dnorm_w, dout_proj=dout_proj)
@@ -561,17 +600,34 @@ class Mamba2Block:
         return torch.matmul(u, w.t()).contiguous()
 
     def _converted(self, dtype: torch.dtype):
-        """(key, in_proj, out_proj, out_proj^T, step limit) in the activation dtype, converted once per dtype (and again when a
-        master copy has been modified in place)."""
+        """(key, in_proj, out_proj, out_proj^T, step limit, in_proj turned as `block_dproj` takes it) in the activation dtype, converted
+        once per dtype (and again when a master copy has been modified in place)."""
         key = (dtype, self.in_proj._version, self.out_proj._version, self.in_proj.data_ptr(), self.out_proj.data_ptr())
         cached = getattr(self, "_weights_cache", None)
         if cached is None or cached[0] != key:
-            w_in, w_out = self.in_proj.to(dtype).contiguous(), self.out_proj.to(dtype).contiguous()
+            w_in, w_out, w_out_t, w_in_t = self._convert(dtype)
             # (with them: the batch up to which a step is one launch, whose kernel reads both 16 bytes at a time)
             limit = self._step_limit if dtype in _STEP_DTYPES and (w_in.data_ptr() | w_out.data_ptr()) % 16 == 0 else 0
-            cached = (key, w_in, w_out, w_out.t().contiguous(), limit)
+            cached = (key, w_in, w_out, w_out_t, limit, w_in_t)
             self._weights_cache = cached
         return cached
+
+    def _convert(self, dtype: torch.dtype):
+        """in_proj, out_proj, out_proj^T and in_proj turned (bf16 only, else None) in `dtype`: one launch where the masters are float32
+        and bf16 is asked for, as after every update of the weights."""
+        wi, wo = self.in_proj, self.out_proj
+        if (dtype == torch.bfloat16 and wi.is_cuda and wo.device == wi.device and wi.dtype == wo.dtype == torch.float32
+                and wi.is_contiguous() and wo.is_contiguous() and wi.dim() == wo.dim() == 2 and wi.shape[1] == wo.shape[0]
+                and wi.numel() and wo.numel() and (wi.data_ptr() | wo.data_ptr()) % 16 == 0):
+            lib = _lib()
+            (E, D), DI = wi.shape, wo.shape[1]
+            new = lambda *shape: wi.new_empty(shape, dtype=dtype)
+            w_in, w_out, w_out_t, w_in_t = new(E, D), new(D, DI), new(DI, D), new(D, (E + 15) // 16 * 16)
+            ssd._check(lib, lib.ssd_block_weights(E, D, DI, wi.data_ptr(), wo.data_ptr(), w_in.data_ptr(), w_in_t.data_ptr(),
+                                                  w_out.data_ptr(), w_out_t.data_ptr(), ssd._stream_ptr(wi)))
+            return w_in, w_out, w_out_t, w_in_t
+        w_in, w_out = wi.to(dtype).contiguous(), wo.to(dtype).contiguous()
+        return w_in, w_out, w_out.t().contiguous(), turned_weight(w_in) if dtype == torch.bfloat16 else None
 
     def _weights(self, dtype: torch.dtype):
         """The two projection matrices in the activation dtype."""
@@ -598,7 +654,7 @@ class Mamba2Block:
         if u_t.dim() != 2 or u_t.shape[1] != self.d_model:
             raise ValueError(f"block step input must be [batch, {self.d_model}], got {tuple(u_t.shape)}")
         batch = u_t.shape[0]
-        _, w_in, w_out, _, limit = self._converted(u_t.dtype)
+        _, w_in, w_out, _, limit, _ = self._converted(u_t.dtype)
         if fused is None:
             fused = batch <= limit and u_t.is_cuda and u_t.data_ptr() % 16 == 0
         if fused:   # the whole step as one launch: what a step costs at a few streams is issuing its launches

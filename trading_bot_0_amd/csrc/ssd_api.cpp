@@ -1038,6 +1038,50 @@ int ssd_block_proj_fwd(int64_t rows, int64_t in_features, int64_t out_features, 
     return e == hipSuccess ? SSD_OK : hip_fail(e, "block projection launch");
 }
 
+int ssd_block_dproj(int64_t rows, int64_t a_features, int64_t out_features, int64_t a_ld, int64_t w_ld, int dtype, const void *a,
+                    const void *w_t, void *out, void *hip_stream) {
+    if (dtype != SSD_DTYPE_BF16)
+        return fail(SSD_ERR_UNSUPPORTED, "ssd: the projection's input gradient takes dtype 1 (bfloat16), got %d", dtype);
+    if (rows <= 0 || a_features <= 0 || out_features <= 0)
+        return fail(SSD_ERR_INVALID, "ssd: projection sizes must be positive, got %lld x %lld -> %lld", (long long)rows,
+                    (long long)a_features, (long long)out_features);
+    if (rows > 0x7fffffff || a_features > 0x7fffffff || out_features > 0x7fffffff ||
+        !ssd::block_dproj_supported(rows, (int)a_features, (int)out_features))
+        return fail(SSD_ERR_UNSUPPORTED,
+                    "ssd: the projection's input gradient needs features that are multiples of 8, a_features whose 32 rows fit 160 KiB "
+                    "and fewer than 2^31 rows, got %lld, %lld and %lld",
+                    (long long)a_features, (long long)out_features, (long long)rows);
+    if (a_ld == 0) a_ld = a_features;
+    if (a_ld < a_features || a_ld > 0x7fffffff || a_ld % 8 != 0)
+        return fail(SSD_ERR_INVALID, "ssd: a_ld must be 0 or at least a_features (%lld) and a multiple of 8, got %lld",
+                    (long long)a_features, (long long)a_ld);
+    if (w_ld < (a_features + 15) / 16 * 16 || w_ld > 0x7fffffff || w_ld % 8 != 0)
+        return fail(SSD_ERR_INVALID, "ssd: w_ld must be a multiple of 8 and at least a_features (%lld) rounded up to 16, got %lld",
+                    (long long)a_features, (long long)w_ld);
+    REQUIRE_PTR(a);
+    REQUIRE_PTR(w_t);
+    REQUIRE_PTR(out);
+    hipError_t e = ssd::launch_block_dproj(rows, (int)a_features, (int)out_features, (int)a_ld, (int)w_ld, a, w_t, out,
+                                           (hipStream_t)hip_stream);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "projection input gradient launch");
+}
+
+int ssd_block_weights(int64_t in_features, int64_t d_model, int64_t d_inner, const float *in_proj, const float *out_proj, void *w_in,
+                      void *w_in_t, void *w_out, void *w_out_t, void *hip_stream) {
+    if (in_features <= 0 || d_model <= 0 || d_inner <= 0 || in_features > 0xfffffff || d_model > 0xfffffff || d_inner > 0xfffffff)
+        return fail(SSD_ERR_INVALID, "ssd: weight sizes must be positive and below 2^28, got %lld, %lld and %lld", (long long)in_features,
+                    (long long)d_model, (long long)d_inner);
+    REQUIRE_PTR(in_proj);
+    REQUIRE_PTR(out_proj);
+    REQUIRE_PTR(w_in);
+    REQUIRE_PTR(w_in_t);
+    REQUIRE_PTR(w_out);
+    REQUIRE_PTR(w_out_t);
+    hipError_t e = ssd::launch_block_weights((int)in_features, (int)d_model, (int)d_inner, in_proj, out_proj, w_in, w_in_t, w_out, w_out_t,
+                                             (hipStream_t)hip_stream);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "block weights launch");
+}
+
 static int check_wgrad(int64_t rows, int64_t a_features, int64_t b_features) {
     if (rows <= 0 || a_features <= 0 || b_features <= 0)
         return fail(SSD_ERR_INVALID, "ssd: weight gradient sizes must be positive, got %lld rows of %lld and %lld", (long long)rows,

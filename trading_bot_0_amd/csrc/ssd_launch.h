@@ -148,6 +148,14 @@ bool block_supported(const BlockShape &s);
 bool block_proj_supported(long long rows, int in_features, int out_features);
 hipError_t launch_block_proj(long long rows, int in_features, int out_features, int out_ld, const void *u, const void *w,
                              void *out, hipStream_t st);
+// The gradient of a projection's input: out [rows, N] (dense) = a [rows, K] . wt [N, ldw]^T in bf16, float32 accumulation; a's rows lda
+// apart, wt zero from column K to the next multiple of 16 (ldw at least that).  K and N multiples of 8.
+bool block_dproj_supported(long long rows, int K, int N);
+hipError_t launch_block_dproj(long long rows, int K, int N, int lda, int ldw, const void *a, const void *wt, void *out, hipStream_t st);
+// The block's weights (float32: in_proj [E, D], out_proj [D, DI]) in bf16: w_in [E, D] and w_in_t [D, E to the next multiple of 16]
+// (zeros past E), w_out [D, DI] and w_out_t [DI, D].
+hipError_t launch_block_weights(int E, int D, int DI, const float *in_proj, const float *out_proj, void *w_in, void *w_in_t, void *w_out,
+                                void *w_out_t, hipStream_t st);
 // The projections' weight gradients: out [E, N] (float32) = a^T b over all rows, a [rows, E] (rows lda elements apart, a
 // multiple of 8) and b [rows, N] in bf16; E a multiple of 8, N 128 or 256.  workspace: the partial sums.
 bool block_wgrad_supported(long long rows, int E, int N);

@@ -45,6 +45,8 @@ EXPORTED_SYMBOLS = (
     "ssd_block_pre_fwd",
     "ssd_block_post_fwd",
     "ssd_block_proj_fwd",
+    "ssd_block_dproj",
+    "ssd_block_weights",
     "ssd_block_wgrad_workspace_bytes",
     "ssd_block_wgrad",
     "ssd_chunk_scan_bwd_workspace_bytes",
