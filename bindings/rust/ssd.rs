@@ -128,6 +128,23 @@ extern "C" {
         conv_w: *const f32, conv_b: *const f32, dt_bias: *const f32, a: *const f32, d: *const f32, norm_w: *const f32,
         eps: f32, w_out: *const c_void, conv_state: *mut c_void, ssm_state: *mut f32, out: *mut c_void,
         hip_stream: *mut c_void) -> c_int;
+    pub fn ssd_block_forward_workspace_bytes(dims: *const SsdBlockDims, dtype: c_int, d_model: i64, chunk: i64,
+        out_bytes: *mut usize) -> c_int;
+    pub fn ssd_block_forward(dims: *const SsdBlockDims, dtype: c_int, d_model: i64, chunk: i64, u: *const c_void,
+        w_in: *const c_void, conv_w: *const f32, conv_b: *const f32, dt_bias: *const f32, a_log: *const f32, d: *const f32,
+        norm_w: *const f32, eps: f32, w_out: *const c_void, reset: *const u8, conv_state_in: *const c_void,
+        conv_state_out: *mut c_void, initial_states: *const f32, final_states: *mut f32, zxbcdt: *mut c_void, x: *mut c_void,
+        bm: *mut c_void, cm: *mut c_void, dt: *mut c_void, y: *mut c_void, out: *mut c_void, workspace: *mut c_void,
+        workspace_bytes: usize, hip_stream: *mut c_void) -> c_int;
+    pub fn ssd_block_grad_workspace_bytes(dims: *const SsdBlockDims, dtype: c_int, d_model: i64, chunk: i64,
+        out_bytes: *mut usize) -> c_int;
+    pub fn ssd_block_grad(dims: *const SsdBlockDims, dtype: c_int, d_model: i64, chunk: i64, u: *const c_void,
+        w_in_t: *const c_void, w_in_t_ld: i64, w_out_t: *const c_void, conv_w: *const f32, conv_b: *const f32,
+        dt_bias: *const f32, a_log: *const f32, d: *const f32, norm_w: *const f32, eps: f32, reset: *const u8,
+        zxbcdt: *const c_void, x: *const c_void, bm: *const c_void, cm: *const c_void, dt: *const c_void, y: *const c_void,
+        dout: *const c_void, du: *mut c_void, din_proj: *mut f32, dconv_w: *mut f32, dconv_b: *mut f32, ddt_bias: *mut f32,
+        da: *mut f32, da_log: *mut f32, dd: *mut f32, dnorm_w: *mut f32, dout_proj: *mut f32, dzxbcdt: *mut c_void,
+        workspace: *mut c_void, workspace_bytes: usize, hip_stream: *mut c_void) -> c_int;
     pub fn ssd_block_bwd_workspace_bytes(dims: *const SsdBlockDims, dtype: c_int, out_bytes: *mut usize) -> c_int;
     pub fn ssd_block_post_bwd(dims: *const SsdBlockDims, dtype: c_int, y: *const c_void, zxbcdt: *const c_void,
         norm_w: *const f32, eps: f32, dout: *const c_void, dy: *mut c_void, dzxbcdt: *mut c_void, dnorm_w: *mut f32,

@@ -364,6 +364,30 @@ int ssd_block_pre_bwd(const ssd_block_dims *dims, int dtype, const void *zxbcdt,
                       float *dconv_b, float *ddt_bias, void *dconv_state_in, void *workspace, size_t workspace_bytes,
                       void *hip_stream);
 
+/* The whole block's forward in one call, bfloat16 (dtype 1): in-projection, pre, scan, gate + norm + out-projection on the library's own
+ * kernels (d_model and nheads*headdim of 128 or 256; SSD_ERR_UNSUPPORTED otherwise: the stages one by one, with the caller's BLAS).
+ * u [B,L,d_model], w_in [E,d_model], w_out [d_model,H*P] (ssd_block_weights makes them), A = -exp(A_log) [H] float32, the other
+ * parameters, reset and the states as for the stages; zxbcdt (rows of dims->zxbcdt_ld), x, Bm, Cm, dt and y receive what the stages
+ * hand on (ssd_block_grad takes them), out [B,L,d_model] the result.  chunk as for ssd_chunk_scan_fwd. */
+int ssd_block_forward_workspace_bytes(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, size_t *out_bytes);
+int ssd_block_forward(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, const void *u, const void *w_in,
+                      const float *conv_w, const float *conv_b, const float *dt_bias, const float *A_log, const float *D,
+                      const float *norm_w, float eps, const void *w_out, const uint8_t *reset, const void *conv_state_in,
+                      void *conv_state_out, const float *initial_states, float *final_states, void *zxbcdt, void *x, void *Bm,
+                      void *Cm, void *dt, void *y, void *out, void *workspace, size_t workspace_bytes, void *hip_stream);
+
+/* Its backward in one call, for a window without a carried state, from what the forward handed on: the gradients of sum(out * dout).
+ * w_out_t [H*P,d_model] and w_in_t [d_model,w_in_t_ld] as ssd_block_weights turns them.  du [B,L,d_model] may be NULL (the caller's BLAS
+ * forms it from dzxbcdt, the gradient of zxbcdt with its row stride, which is always written), dD NULL without D; the parameters'
+ * gradients are float32, dA_log = dA * A. */
+int ssd_block_grad_workspace_bytes(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, size_t *out_bytes);
+int ssd_block_grad(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, const void *u, const void *w_in_t,
+                   int64_t w_in_t_ld, const void *w_out_t, const float *conv_w, const float *conv_b, const float *dt_bias,
+                   const float *A_log, const float *D, const float *norm_w, float eps, const uint8_t *reset, const void *zxbcdt,
+                   const void *x, const void *Bm, const void *Cm, const void *dt, const void *y, const void *dout, void *du,
+                   float *din_proj, float *dconv_w, float *dconv_b, float *ddt_bias, float *dA, float *dA_log, float *dD,
+                   float *dnorm_w, float *dout_proj, void *dzxbcdt, void *workspace, size_t workspace_bytes, void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

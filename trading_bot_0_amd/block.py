@@ -50,6 +50,10 @@ def _lib():
         lib.ssd_block_post_bwd.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, P, P, P, P, c_size_t, P]
         lib.ssd_block_post_bwd_yn.argtypes = [POINTER(SsdBlockDims), c_int, P, P, P, c_float, P, P, P, P, P, P, c_size_t, P]
         lib.ssd_block_pre_bwd.argtypes = [POINTER(SsdBlockDims), c_int] + [P] * 17 + [c_size_t, P]
+        D, I = POINTER(SsdBlockDims), c_int64
+        lib.ssd_block_forward_workspace_bytes.argtypes = lib.ssd_block_grad_workspace_bytes.argtypes = [D, c_int, I, I, POINTER(c_size_t)]
+        lib.ssd_block_forward.argtypes = [D, c_int, I, I] + [P] * 8 + [c_float] + [P] * 14 + [c_size_t, P]
+        lib.ssd_block_grad.argtypes = [D, c_int, I, I, P, P, I] + [P] * 7 + [c_float] + [P] * 20 + [c_size_t, P]
         for name in ("ssd_block_bwd_workspace_bytes", "ssd_block_post_bwd", "ssd_block_post_bwd_yn", "ssd_block_pre_bwd"):
             getattr(lib, name).restype = c_int
         lib.ssd_block_pre_fwd.restype = c_int
@@ -128,6 +132,14 @@ def _wgrad_slab_limit(E: int, D: int) -> int:
     return 32 if 384 < E <= 512 or (E <= 128 and D == 256) else 64
 
 
+def _wgrad_slabs(rows: int) -> int:
+    """The equal slabs of 4 096 rows or more that a row count makes, a power of two."""
+    slabs = 1
+    while slabs < 128 and rows % (2 * slabs) == 0 and rows // (2 * slabs) >= 4096:
+        slabs *= 2
+    return slabs
+
+
 def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T b in float32 for tall a [rows, E] (its rows may be a view into wider ones) and b [rows, D]: a sum over all
     rows of the batch and the sequence.  bf16 with D 128 or 256 runs on the library's kernel (72 828 rows, 648 x 256 outputs:
@@ -138,9 +150,7 @@ def _weight_gradient(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     524 288 rows: 648 x 256 outputs 1 333 -> 232 us, 256 x 256 outputs 1 059 -> 129 us; the float32 partial products also
     make the result more accurate than the single GEMM's bf16 output)."""
     rows = a.shape[0]
-    slabs = 1
-    while slabs < 128 and rows % (2 * slabs) == 0 and rows // (2 * slabs) >= 4096:
-        slabs *= 2
+    slabs = _wgrad_slabs(rows)
     if slabs < _wgrad_slab_limit(a.shape[1], b.shape[1]) and block_wgrad_supported(a, b):
         return block_wgrad(a, b)
     if slabs == 1 or a.dtype == torch.float32:
@@ -524,6 +534,11 @@ class Mamba2Block:
             raise ValueError(f"block input must be [batch, seqlen, {self.d_model}], got {tuple(u.shape)}")
         if reset is not None and state is not None:
             raise ValueError("restarts inside the window and a carried conv state cannot be combined")
+        if save_for_backward and state is not None:
+            raise ValueError("backward through a window that continues a carried state is not supported")
+        weights = self._converted(u.dtype)
+        if self._one_call(u, weights):
+            return self._forward_in_one_call(u, weights, state, reset, save_for_backward)
         zxbcdt = self._project(u, self._weights(u.dtype)[0], pad_rows=True)  # internal to the block: rows of whole lines
         if state is None:
             x, Bm, Cm, dt = block_pre(zxbcdt, self.conv_w, self.conv_b, self.dt_bias, self.H, self.P, self.N, self.G,
@@ -536,8 +551,6 @@ class Mamba2Block:
             state.conv = conv
             y = state.ssm.init_from_prefix(x, dt, self.A, Bm, Cm, self.D, chunk=self.chunk)
         w_out = self._weights(u.dtype)[1]
-        if save_for_backward and state is not None:
-            raise ValueError("backward through a window that continues a carried state is not supported")
         if block_post_proj_supported(y, w_out):
             # gate, norm and out-projection as one kernel: the normalised rows never reach memory (the backward pass
             # needs them for one weight gradient only, and has its post stage write them on the way: yn=None).  256 -> 256 in us, one
@@ -551,6 +564,122 @@ class Mamba2Block:
             return out, dict(u=u, zxbcdt=zxbcdt, x=x, Bm=Bm, Cm=Cm, dt=dt, y=y, yn=yn, reset=reset)
         return out
 
+    def _one_call(self, u: torch.Tensor, weights) -> bool:
+        """Whether the library runs the whole pass as one call (else the stages one by one): what each of its kernels asks for."""
+        return (u.dtype == torch.bfloat16 and self.d_inner in (128, 256) and self.d_model in (128, 256)
+                and weights[1].shape == (in_proj_width(self.H, self.P, self.N, self.G), self.d_model)
+                and weights[2].shape == (self.d_model, self.d_inner) and u.device == weights[1].device == weights[2].device
+                and block_proj_supported(u, weights[1]) and weights[2].data_ptr() % 16 == 0
+                and self.A_log.dtype == torch.float32 and self.A_log.is_contiguous() and self.A_log.data_ptr() % 16 == 0)
+
+    def _parameters_checked(self):
+        """The float32 parameters between the projections, looked at as the stages do; D or None."""
+        for name, t, shape in (("conv_w", self.conv_w, (self.conv_dim, self.d_conv)), ("conv_b", self.conv_b, (self.conv_dim,)),
+                               ("dt_bias", self.dt_bias, (self.H,)), ("A_log", self.A_log, (self.H,)),
+                               ("norm_w", self.norm_w, (self.d_inner,))):
+            ssd._require(t, name, shape, torch.float32)
+        if self.D is not None:
+            ssd._require(self.D, "D", (self.H,), torch.float32)
+
+    def _forward_in_one_call(self, u, weights, state, reset, save_for_backward):
+        """`forward` as one call of the library: seven launches at a few rows, for which the stages' calls took the host longer than
+        the GPU (4 x 4 096: 85 us of the host, 71 of the GPU)."""
+        lib = _lib()
+        Bsz, L, _ = u.shape
+        H, P, N, G = self.H, self.P, self.N, self.G
+        self._parameters_checked()
+        u_in, u = u, u.contiguous()
+        E = in_proj_width(H, P, N, G)
+        ld = (E + 63) // 64 * 64    # rows of whole lines: internal to the block
+        dims = SsdBlockDims(Bsz, L, H, P, N, G, self.d_conv, ld)
+        conv = conv_out = init = final = None
+        if state is not None:
+            ssd._require(state.conv, "conv_state", (Bsz, self.d_conv - 1, self.conv_dim), u.dtype)
+            if state.ssm.batch != Bsz:
+                raise ValueError(f"stream state batch size mismatch: state has {state.ssm.batch}, input has {Bsz}")
+            final = state.ssm.state
+            ssd._require(final, "final_out", (Bsz, H, P, N), torch.float32)
+            if state.ssm.initialized:
+                init = final
+            conv, conv_out = state.conv, torch.empty_like(state.conv)
+        if reset is not None:
+            if reset.dtype == torch.bool:
+                reset = reset.view(torch.uint8)
+            ssd._require(reset, "reset", (Bsz, L), torch.uint8)
+        need = c_size_t(0)
+        ssd._check(lib, lib.ssd_block_forward_workspace_bytes(byref(dims), ssd.SSD_DTYPE_BF16, self.d_model, self.chunk, byref(need)))
+        rows, DI, GN = Bsz * L, self.d_inner, G * N
+        out = u.new_empty((Bsz, L, self.d_model))
+        if save_for_backward:
+            buf = u.new_empty((Bsz, L, ld))
+            x, Bm, Cm, dt, y = (u.new_empty((Bsz, L) + s) for s in ((H, P), (G, N), (G, N), (H,), (H, P)))
+            ws = u.new_empty(need.value, dtype=torch.uint8)
+            inner = [t.data_ptr() for t in (buf, x, Bm, Cm, dt, y, ws)]
+        else:   # one buffer for all that is not kept
+            sizes = [2 * rows * ld, 2 * rows * DI, 2 * rows * GN, 2 * rows * GN, 2 * rows * H, 2 * rows * DI]
+            at, inner = 0, []
+            for n in sizes:
+                inner.append(at)
+                at += (n + 255) // 256 * 256
+            ws = u.new_empty(at + need.value, dtype=torch.uint8)
+            base = ws.data_ptr()
+            inner = [base + i for i in inner] + [base + at]
+        ssd._check(lib, lib.ssd_block_forward(
+            byref(dims), ssd.SSD_DTYPE_BF16, self.d_model, self.chunk, u.data_ptr(), weights[1].data_ptr(), self.conv_w.data_ptr(),
+            self.conv_b.data_ptr(), self.dt_bias.data_ptr(), self.A_log.data_ptr(), ssd._ptr(self.D), self.norm_w.data_ptr(), self.eps,
+            weights[2].data_ptr(), ssd._ptr(reset), ssd._ptr(conv), ssd._ptr(conv_out), ssd._ptr(init), ssd._ptr(final), *inner[:6],
+            out.data_ptr(), inner[6], need.value, ssd._stream_ptr(u)))
+        if state is not None:
+            state.conv = conv_out
+            state.ssm.initialized = True
+        if save_for_backward:
+            zxbcdt = buf[..., :E] if ld != E else buf
+            return out, dict(u=u_in, zxbcdt=zxbcdt, x=x, Bm=Bm, Cm=Cm, dt=dt, y=y, yn=None, reset=reset)
+        return out
+
+    def _backward_in_one_call(self, ctx, dout, weights):
+        """`backward` as one call of the library, where its kernels take both projections' weight gradients (None otherwise)."""
+        u, zxbcdt, y, reset, x, Bm, Cm, dt = (ctx[k] for k in ("u", "zxbcdt", "y", "reset", "x", "Bm", "Cm", "dt"))
+        Bsz, L, _ = u.shape
+        H, P, N, G = self.H, self.P, self.N, self.G
+        rows, E, DI, DM = Bsz * L, in_proj_width(H, P, N, G), self.d_inner, self.d_model
+        slabs = _wgrad_slabs(rows)
+        if (ctx["yn"] is not None or not self._one_call(u, weights) or not u.is_contiguous() or dout.dtype != u.dtype
+                or tuple(dout.shape) != (Bsz, L, DM) or dout.device != u.device or not dout.is_contiguous() or dout.data_ptr() % 16
+                or slabs >= _wgrad_slab_limit(E, DM) or slabs >= _wgrad_slab_limit(DM, DI) or E > 8192 or weights[5] is None):
+            return None
+        lib = _lib()
+        self._parameters_checked()
+        if tuple(zxbcdt.shape) != (Bsz, L, E) or zxbcdt.dtype != u.dtype or not zxbcdt.is_cuda:
+            return None
+        ld = _row_stride(zxbcdt)
+        for name, t, shape in (("x", x, (Bsz, L, H, P)), ("B", Bm, (Bsz, L, G, N)), ("C", Cm, (Bsz, L, G, N)), ("dt", dt, (Bsz, L, H)),
+                               ("y", y, (Bsz, L, H, P))):
+            ssd._require(t, name, shape, u.dtype)
+        if reset is not None:
+            if reset.dtype == torch.bool:
+                reset = reset.view(torch.uint8)
+            ssd._require(reset, "reset", (Bsz, L), torch.uint8)
+        dims = SsdBlockDims(Bsz, L, H, P, N, G, self.d_conv, ld)
+        need = c_size_t(0)
+        ssd._check(lib, lib.ssd_block_grad_workspace_bytes(byref(dims), ssd.SSD_DTYPE_BF16, DM, self.chunk, byref(need)))
+        ws = u.new_empty(need.value, dtype=torch.uint8)
+        dbuf = u.new_empty((Bsz, L, ld))
+        f32 = lambda *shape: u.new_empty(shape, dtype=torch.float32)
+        own_du = rows <= DPROJ_MAX_ROWS and E <= DPROJ_MAX_FEATURES
+        g = dict(du=u.new_empty((Bsz, L, DM)) if own_du else None, din_proj=f32(E, DM), dconv_w=f32(self.conv_dim, self.d_conv),
+                 dconv_b=f32(self.conv_dim), ddt_bias=f32(H), dA=f32(H), dA_log=f32(H), dD=None if self.D is None else f32(H),
+                 dnorm_w=f32(DI), dout_proj=f32(DM, DI))
+        ssd._check(lib, lib.ssd_block_grad(
+            byref(dims), ssd.SSD_DTYPE_BF16, DM, self.chunk, u.data_ptr(), weights[5].data_ptr(), weights[5].shape[1],
+            weights[3].data_ptr(), self.conv_w.data_ptr(), self.conv_b.data_ptr(), self.dt_bias.data_ptr(), self.A_log.data_ptr(),
+            ssd._ptr(self.D), self.norm_w.data_ptr(), self.eps, ssd._ptr(reset), zxbcdt.data_ptr(), x.data_ptr(), Bm.data_ptr(),
+            Cm.data_ptr(), dt.data_ptr(), y.data_ptr(), dout.data_ptr(), *[ssd._ptr(t) for t in g.values()], dbuf.data_ptr(),
+            ws.data_ptr(), need.value, ssd._stream_ptr(u)))
+        if not own_du:
+            g["du"] = torch.matmul(dbuf.view(rows, ld)[:, :E], weights[1]).view(Bsz, L, DM)
+        return g
+
     def backward(self, ctx: dict, dout: torch.Tensor) -> dict:
         """Gradients of sum(out * dout) with respect to the input and every parameter, from the tensors `forward`
         kept: two products per projection, the library's post, scan and pre backward kernels between them.
@@ -560,7 +689,11 @@ class Mamba2Block:
         Bsz, L, _ = u.shape
         act = u.dtype
         E = in_proj_width(self.H, self.P, self.N, self.G)
-        w_in, w_out = self._weights(act)
+        weights = self._converted(act)
+        grads = self._backward_in_one_call(ctx, dout, weights)
+        if grads is not None:
+            return grads
+        w_in = weights[1]
         A = self.A
         dout2 = dout.reshape(Bsz * L, self.d_model)
         dyn = self._project(dout2, self._out_proj_transposed(act)).view(Bsz, L, self.d_inner)

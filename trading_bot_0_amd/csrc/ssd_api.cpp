@@ -637,10 +637,12 @@ int ssd_chunk_scan_bwd_workspace_bytes(const ssd_dims *dims, int dtype, size_t *
     return SSD_OK;
 }
 
-int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
+// The backward pass; with dA_log given A is -exp(A_log) and its gradient is wanted as well.
+static int scan_backward(const ssd_dims *dims, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
                        const void *Cm, const float *D, const float *initial_states, const uint8_t *reset, const void *dy,
                        const float *dfinal_states, void *dx, void *ddt, float *dA, void *dB, void *dC, float *dD,
-                       float *dinitial_states, void *workspace, size_t workspace_bytes, void *hip_stream) {
+                       float *dinitial_states, void *workspace, size_t workspace_bytes, void *hip_stream,
+                         float *dA_log = nullptr) {
     ssd::ScanShape s, sT;
     if (int rc = make_bwd_shapes(dims, dtype, &s, &sT)) return rc;
     REQUIRE_PTR(x);
@@ -843,11 +845,19 @@ int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const voi
                                    rows_in_scan ? atf(w.parts) : nullptr, s.N / 32, reset, sum_on_chip ? s.N / 32 : 0,
                                    plan.anchor_stride),
                "backward ddt");
-    BWD_LAUNCH(ssd::launch_bwd_head_sums(s, da_part, dd_part, dA, dD, st), "backward head sums");
+    BWD_LAUNCH(ssd::launch_bwd_head_sums(s, da_part, dd_part, dA, dD, st, A, dA_log), "backward head sums");
     if (dinitial_states != nullptr)
         BWD_LAUNCH(ssd::launch_bwd_dinit(s, el, dt, A, atf(w.gfin), reset, dinitial_states, st), "backward dinit");
 #undef BWD_LAUNCH
     return SSD_OK;
+}
+
+int ssd_chunk_scan_bwd(const ssd_dims *dims, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
+                       const void *Cm, const float *D, const float *initial_states, const uint8_t *reset, const void *dy,
+                       const float *dfinal_states, void *dx, void *ddt, float *dA, void *dB, void *dC, float *dD,
+                       float *dinitial_states, void *workspace, size_t workspace_bytes, void *hip_stream) {
+    return scan_backward(dims, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, dy, dfinal_states, dx, ddt, dA, dB, dC, dD,
+                         dinitial_states, workspace, workspace_bytes, hip_stream);
 }
 
 int ssd_chunk_scan_is_onepass(const ssd_dims *dims, int dtype, int *is_onepass) {
@@ -1262,6 +1272,215 @@ int ssd_block_step_fwd(const ssd_block_dims *dims, int dtype, int64_t d_model, c
     hipError_t e = ssd::launch_block_step(s, dtype == SSD_DTYPE_F32 ? 0 : 1, (int)d_model, u, w_in, conv_w, conv_b, dt_bias,
                                           A, D, norm_w, eps, w_out, conv_state, ssm_state, out, (hipStream_t)hip_stream);
     return e == hipSuccess ? SSD_OK : hip_fail(e, "fused block step launch");
+}
+
+// ---- the whole block ----
+
+// The shapes and the scratch of a whole block's passes: bf16, projections and gate on the library's own kernels.
+static int make_whole_block(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, ssd::BlockShape *s, ssd_dims *scan,
+                            int *width) {
+    if (int rc = make_block_shape(dims, dtype, s)) return rc;
+    *width = 2 * s->H * s->P + 2 * s->G * s->N + s->H;
+    if (dtype != SSD_DTYPE_BF16)
+        return fail(SSD_ERR_UNSUPPORTED, "ssd: the whole block takes dtype 1 (bfloat16), got %d", dtype);
+    if (d_model <= 0 || d_model > 0x7fffffff || !ssd::block_proj_supported((long long)s->B * s->L, (int)d_model, *width) ||
+        !ssd::block_post_proj_supported(*s, (int)d_model))
+        return fail(SSD_ERR_UNSUPPORTED,
+                    "ssd: the whole block needs d_model and nheads*headdim of 128 or 256 and a timestep's channels in whole 16-byte "
+                    "pieces, got d_model %lld, nheads*headdim %d", (long long)d_model, s->H * s->P);
+    *scan = ssd_dims{s->B, s->L, s->H, s->P, s->N, s->G, chunk};
+    return SSD_OK;
+}
+
+// Hands out 256-byte pieces of a buffer, or only counts them (base NULL).
+struct Carver {
+    char *base;
+    size_t used = 0;
+    void *take(size_t bytes) {
+        char *p = base == nullptr ? nullptr : base + used;
+        used += align_up(bytes, 256);
+        return p;
+    }
+};
+
+int ssd_block_forward_workspace_bytes(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, size_t *out_bytes) {
+    if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
+    ssd::BlockShape s;
+    ssd_dims scan;
+    ssd::ScanShape sc;
+    int width;
+    if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
+    if (int rc = make_shape(&scan, dtype, &sc)) return rc;
+    *out_bytes = align_up((size_t)s.H * sizeof(float), 256) + align_up(scan_scratch_bytes(sc, dtype), 256);
+    return SSD_OK;
+}
+
+int ssd_block_forward(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, const void *u, const void *w_in,
+                      const float *conv_w, const float *conv_b, const float *dt_bias, const float *A_log, const float *D,
+                      const float *norm_w, float eps, const void *w_out, const uint8_t *reset, const void *conv_state_in,
+                      void *conv_state_out, const float *initial_states, float *final_states, void *zxbcdt, void *x, void *Bm,
+                      void *Cm, void *dt, void *y, void *out, void *workspace, size_t workspace_bytes, void *hip_stream) {
+    ssd::BlockShape s;
+    ssd_dims scan;
+    ssd::ScanShape sc;
+    int width;
+    if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
+    if (int rc = make_shape(&scan, dtype, &sc)) return rc;
+    REQUIRE_PTR(u);
+    REQUIRE_PTR(w_in);
+    REQUIRE_PTR(conv_w);
+    REQUIRE_PTR(conv_b);
+    REQUIRE_PTR(dt_bias);
+    REQUIRE_PTR(A_log);
+    OPTIONAL_PTR(D);
+    REQUIRE_PTR(norm_w);
+    REQUIRE_PTR(w_out);
+    OPTIONAL_PTR(conv_state_in);
+    OPTIONAL_PTR(conv_state_out);
+    OPTIONAL_PTR(initial_states);
+    OPTIONAL_PTR(final_states);
+    REQUIRE_PTR(zxbcdt);
+    REQUIRE_PTR(x);
+    REQUIRE_PTR(Bm);
+    REQUIRE_PTR(Cm);
+    REQUIRE_PTR(dt);
+    REQUIRE_PTR(y);
+    REQUIRE_PTR(out);
+    REQUIRE_PTR(workspace);
+    if (!(eps > 0.f)) return fail(SSD_ERR_INVALID, "ssd: eps must be positive");
+    if (conv_state_in != nullptr && conv_state_in == conv_state_out && s.L > 1)
+        return fail(SSD_ERR_INVALID, "ssd: conv_state_in and conv_state_out may alias only for seqlen 1");
+    Carver c{static_cast<char *>(workspace)};
+    float *A = static_cast<float *>(c.take((size_t)s.H * sizeof(float)));
+    const size_t scratch_bytes = scan_scratch_bytes(sc, dtype);
+    void *scratch = c.take(scratch_bytes);
+    if (workspace_bytes < c.used)
+        return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, c.used);
+    hipStream_t st = (hipStream_t)hip_stream;
+    const long long rows = (long long)s.B * s.L;
+    hipError_t e = ssd::launch_block_proj(rows, (int)d_model, width, s.ld, u, w_in, zxbcdt, st);
+    if (e != hipSuccess) return hip_fail(e, "block projection launch");
+    e = ssd::launch_block_pre(s, 1, zxbcdt, conv_w, conv_b, dt_bias, conv_state_in, conv_state_out, reset, x, Bm, Cm, dt, st, A_log, A);
+    if (e != hipSuccess) return hip_fail(e, "block pre-scan launch");
+    if (int rc = scan_forward(sc, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, scratch_bytes, st)) return rc;
+    e = ssd::launch_block_post_proj(s, y, zxbcdt, norm_w, eps, w_out, (int)d_model, (int)d_model, out, st);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "block post-scan + out-projection launch");
+}
+
+namespace {
+
+// What a block's backward pass keeps between its launches.
+struct GradScratch {
+    void *dyn, *yn, *dy, *dx, *dB, *dC, *ddt, *sums, *wgrad, *scan;
+    float *A;
+    size_t sums_bytes, wgrad_bytes, scan_bytes;
+};
+
+int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_model, int width, Carver *c, GradScratch *g) {
+    const size_t rows = (size_t)s.B * s.L, DI = (size_t)s.H * s.P, GN = (size_t)s.G * s.N;
+    if (int rc = ssd_chunk_scan_bwd_workspace_bytes(&scan, SSD_DTYPE_BF16, &g->scan_bytes)) return rc;
+    if (int rc = check_wgrad((int64_t)rows, width, d_model)) return rc;
+    if (int rc = check_wgrad((int64_t)rows, d_model, (int64_t)DI)) return rc;
+    g->sums_bytes = ssd::block_bwd_workspace_bytes(s);
+    g->wgrad_bytes = std::max(ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model),
+                              ssd::block_wgrad_workspace_bytes((long long)rows, (int)d_model, (int)DI));
+    g->A = static_cast<float *>(c->take((size_t)s.H * sizeof(float)));
+    g->dyn = c->take(rows * DI * 2);
+    g->yn = c->take(rows * DI * 2);
+    g->dy = c->take(rows * DI * 2);
+    g->dx = c->take(rows * DI * 2);
+    g->dB = c->take(rows * GN * 2);
+    g->dC = c->take(rows * GN * 2);
+    g->ddt = c->take(rows * s.H * 2);
+    g->sums = c->take(g->sums_bytes);
+    g->wgrad = c->take(g->wgrad_bytes);
+    g->scan = c->take(g->scan_bytes);
+    return SSD_OK;
+}
+
+}  // namespace
+
+int ssd_block_grad_workspace_bytes(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, size_t *out_bytes) {
+    if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
+    ssd::BlockShape s;
+    ssd_dims scan;
+    int width;
+    if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
+    Carver c{nullptr};
+    GradScratch g;
+    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g)) return rc;
+    *out_bytes = c.used;
+    return SSD_OK;
+}
+
+int ssd_block_grad(const ssd_block_dims *dims, int dtype, int64_t d_model, int64_t chunk, const void *u, const void *w_in_t,
+                   int64_t w_in_t_ld, const void *w_out_t, const float *conv_w, const float *conv_b, const float *dt_bias,
+                   const float *A_log, const float *D, const float *norm_w, float eps, const uint8_t *reset, const void *zxbcdt,
+                   const void *x, const void *Bm, const void *Cm, const void *dt, const void *y, const void *dout, void *du,
+                   float *din_proj, float *dconv_w, float *dconv_b, float *ddt_bias, float *dA, float *dA_log, float *dD,
+                   float *dnorm_w, float *dout_proj, void *dzxbcdt, void *workspace, size_t workspace_bytes, void *hip_stream) {
+    ssd::BlockShape s;
+    ssd_dims scan;
+    int width;
+    if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
+    REQUIRE_PTR(u);
+    OPTIONAL_PTR(w_in_t);
+    REQUIRE_PTR(w_out_t);
+    REQUIRE_PTR(conv_w);
+    REQUIRE_PTR(conv_b);
+    REQUIRE_PTR(dt_bias);
+    REQUIRE_PTR(A_log);
+    OPTIONAL_PTR(D);
+    REQUIRE_PTR(norm_w);
+    REQUIRE_PTR(zxbcdt);
+    REQUIRE_PTR(x);
+    REQUIRE_PTR(Bm);
+    REQUIRE_PTR(Cm);
+    REQUIRE_PTR(dt);
+    REQUIRE_PTR(y);
+    REQUIRE_PTR(dout);
+    OPTIONAL_PTR(du);
+    REQUIRE_PTR(din_proj);
+    REQUIRE_PTR(dconv_w);
+    REQUIRE_PTR(dconv_b);
+    REQUIRE_PTR(ddt_bias);
+    REQUIRE_PTR(dA);
+    REQUIRE_PTR(dA_log);
+    OPTIONAL_PTR(dD);
+    REQUIRE_PTR(dnorm_w);
+    REQUIRE_PTR(dout_proj);
+    REQUIRE_PTR(dzxbcdt);
+    REQUIRE_PTR(workspace);
+    if (!(eps > 0.f)) return fail(SSD_ERR_INVALID, "ssd: eps must be positive");
+    const long long rows = (long long)s.B * s.L;
+    if (du != nullptr && (w_in_t == nullptr || w_in_t_ld < (width + 15) / 16 * 16 || w_in_t_ld > 0x7fffffff || w_in_t_ld % 8 != 0 ||
+                          !ssd::block_dproj_supported(rows, width, (int)d_model)))
+        return fail(SSD_ERR_INVALID, "ssd: du needs w_in_t with rows of at least the %d channels rounded up to 16", width);
+    Carver c{static_cast<char *>(workspace)};
+    GradScratch g;
+    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g)) return rc;
+    if (workspace_bytes < c.used)
+        return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, c.used);
+    hipStream_t st = (hipStream_t)hip_stream;
+    const int DI = s.H * s.P;
+    hipError_t e = ssd::launch_block_proj(rows, (int)d_model, DI, DI, dout, w_out_t, g.dyn, st);
+    if (e != hipSuccess) return hip_fail(e, "block projection launch");
+    e = ssd::launch_block_post_bwd(s, SSD_DTYPE_BF16, y, zxbcdt, norm_w, eps, g.dyn, g.dy, dzxbcdt, dnorm_w, g.sums, st, g.yn, A_log, g.A);
+    if (e != hipSuccess) return hip_fail(e, "block post-scan backward launch");
+    e = ssd::launch_block_wgrad(rows, (int)d_model, DI, (int)d_model, dout, g.yn, dout_proj, g.wgrad, st);
+    if (e != hipSuccess) return hip_fail(e, "weight gradient launch");
+    if (int rc = scan_backward(&scan, SSD_DTYPE_BF16, x, dt, g.A, Bm, Cm, D, nullptr, reset, g.dy, nullptr, g.dx, g.ddt, dA, g.dB, g.dC, dD,
+                               nullptr, g.scan, g.scan_bytes, hip_stream, dA_log))
+        return rc;
+    e = ssd::launch_block_pre_bwd(s, 1, zxbcdt, conv_w, conv_b, dt_bias, nullptr, reset, g.dx, g.dB, g.dC, g.ddt, nullptr, dzxbcdt, dconv_w,
+                                  dconv_b, ddt_bias, nullptr, g.sums, st);
+    if (e != hipSuccess) return hip_fail(e, "block pre-scan backward launch");
+    if (du != nullptr) {
+        e = ssd::launch_block_dproj(rows, width, (int)d_model, s.ld, (int)w_in_t_ld, dzxbcdt, w_in_t, du, st);
+        if (e != hipSuccess) return hip_fail(e, "projection input gradient launch");
+    }
+    e = ssd::launch_block_wgrad(rows, width, (int)d_model, s.ld, dzxbcdt, u, din_proj, g.wgrad, st);
+    return e == hipSuccess ? SSD_OK : hip_fail(e, "weight gradient launch");
 }
 
 }  // extern "C"

@@ -549,7 +549,8 @@ __global__ __launch_bounds__(64 * kDdtMaxStride) void bwd_ddt_heads_kernel(
 
 // One workgroup per head: dA[h] = the sum over (b, c) of dA_part[h,b,c], dD[h] likewise (float64 sums).
 __global__ __launch_bounds__(256) void bwd_head_sums_kernel(const double *__restrict__ dA_part, const double *__restrict__ dD_part,
-                                                            float *__restrict__ dA, float *__restrict__ dD, ScanShape s) {
+                                                            float *__restrict__ dA, float *__restrict__ dD,
+                                                            const float *__restrict__ A, float *__restrict__ dA_log, ScanShape s) {
     __shared__ double red[2][256];
     const int h = blockIdx.x;
     double sa = 0.0, sd = 0.0;
@@ -583,6 +584,7 @@ __global__ __launch_bounds__(256) void bwd_head_sums_kernel(const double *__rest
     }
     if (threadIdx.x == 0) {
         dA[h] = (float)red[0][0];
+        if (dA_log != nullptr) dA_log[h] = (float)red[0][0] * A[h];
         if (dD != nullptr) dD[h] = (float)red[1][0];
     }
 }
@@ -775,8 +777,8 @@ hipError_t launch_bwd_ddt(const ScanShape &s, int dtype, const void *dt, const f
 }
 
 hipError_t launch_bwd_head_sums(const ScanShape &s, const double *dA_part, const double *dD_part, float *dA, float *dD,
-                                hipStream_t st) {
-    bwd_head_sums_kernel<<<dim3(s.H), dim3(256), 0, st>>>(dA_part, dD_part, dA, dD, s);
+                                hipStream_t st, const float *A, float *dA_log) {
+    bwd_head_sums_kernel<<<dim3(s.H), dim3(256), 0, st>>>(dA_part, dD_part, dA, dD, A, dA_log, s);
     return hipGetLastError();
 }
 

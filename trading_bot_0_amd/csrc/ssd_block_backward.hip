@@ -55,7 +55,8 @@ __global__ __launch_bounds__(256) void block_post_bwd_kernel(const TY *__restric
                                                              const float *__restrict__ norm_w, float eps,
                                                              const T *__restrict__ dout, T *__restrict__ dy,
                                                              T *__restrict__ dzxbcdt, float *__restrict__ dw_part,
-                                                             T *__restrict__ yn, BlockShape s) {
+                                                             T *__restrict__ yn, DecayRates rates, BlockShape s) {
+    form_decay_rates(rates);
     const int DI = s.H * s.P;
     const int lane = threadIdx.x & (LPR - 1);
     constexpr int MAXP = PPL;
@@ -643,7 +644,7 @@ size_t block_bwd_workspace_bytes(const BlockShape &s) {
 template <typename T, typename TY>
 static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const void *zxbcdt, const float *norm_w, float eps,
                                     const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, float *part, void *yn,
-                                    hipStream_t st) {
+                                    const DecayRates &rates, hipStream_t st) {
     const int DI = s.H * s.P, pieces = DI / 8;
     const long long rows = (long long)s.B * s.L;
     const TY *yy = static_cast<const TY *>(y);
@@ -657,9 +658,9 @@ static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const vo
 #define SSD_POST_BWD_CASE(LPRv, PPLv)                                                                                       \
     if (lpr == LPRv && ppl == PPLv) {                                                                                       \
         if (pieces == LPRv * PPLv)                                                                                          \
-            block_post_bwd_kernel<T, TY, LPRv, PPLv, true><<<dim3(blocks), dim3(256), 0, st>>>(yy, zz, norm_w, eps, dd, oy, oz, part, on, s); \
+            block_post_bwd_kernel<T, TY, LPRv, PPLv, true><<<dim3(blocks), dim3(256), 0, st>>>(yy, zz, norm_w, eps, dd, oy, oz, part, on, rates, s); \
         else                                                                                                                \
-            block_post_bwd_kernel<T, TY, LPRv, PPLv, false><<<dim3(blocks), dim3(256), 0, st>>>(yy, zz, norm_w, eps, dd, oy, oz, part, on, s); \
+            block_post_bwd_kernel<T, TY, LPRv, PPLv, false><<<dim3(blocks), dim3(256), 0, st>>>(yy, zz, norm_w, eps, dd, oy, oz, part, on, rates, s); \
         launched = true;                                                                                                    \
     }
     SSD_POST_BWD_CASE(16, 1) SSD_POST_BWD_CASE(16, 2) SSD_POST_BWD_CASE(16, 3) SSD_POST_BWD_CASE(16, 4)
@@ -674,12 +675,13 @@ static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const vo
 
 hipError_t launch_block_post_bwd(const BlockShape &s, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
                                  float eps, const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, void *workspace,
-                                 hipStream_t st, void *yn) {
+                                 hipStream_t st, void *yn, const float *A_log, float *A) {
+    const DecayRates rates{A_log, A, s.H};
     float *part = static_cast<float *>(workspace);
     switch (dtype) {
-        case 0: return post_bwd_dispatch<float, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, st);
-        case 1: return post_bwd_dispatch<__bf16, __bf16>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, st);
-        default: return post_bwd_dispatch<__bf16, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, st);
+        case 0: return post_bwd_dispatch<float, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
+        case 1: return post_bwd_dispatch<__bf16, __bf16>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
+        default: return post_bwd_dispatch<__bf16, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
     }
 }
 

@@ -37,6 +37,17 @@ template <> struct Pack8<float> {
     }
 };
 
+// A = -exp(A_log) of a pass, formed by the first workgroup of a launch that runs ahead of the scan
+struct DecayRates {
+    const float *A_log = nullptr;
+    float *A = nullptr;
+    int heads = 0;
+};
+__device__ inline void form_decay_rates(const DecayRates &r) {
+    if (r.A == nullptr || blockIdx.x != 0) return;
+    for (int h = threadIdx.x; h < r.heads; h += blockDim.x) r.A[h] = -expf(r.A_log[h]);
+}
+
 // derivative of silu: s (1 + v (1 - s)), s = sigmoid(v)
 __device__ inline float dsilu(float v) {
     const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-v));

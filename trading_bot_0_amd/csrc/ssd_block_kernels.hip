@@ -24,7 +24,8 @@ __global__ __launch_bounds__(256) void block_pre_kernel(const T *__restrict__ zx
                                                         const T *state_in, T *state_out,
                                                         const unsigned char *__restrict__ reset,
                                                         T *__restrict__ x, T *__restrict__ Bm, T *__restrict__ Cm,
-                                                        T *__restrict__ dt, BlockShape s) {
+                                                        T *__restrict__ dt, DecayRates rates, BlockShape s) {
+    form_decay_rates(rates);
     const int DI = s.H * s.P, GN = s.G * s.N, C = DI + 2 * GN;
     const int CP = C / 8, HP8 = (s.H + 7) / 8;
     const int runs = (s.L + STEPS - 1) / STEPS;
@@ -244,7 +245,7 @@ bool block_supported(const BlockShape &s) {
 template <typename T>
 static hipError_t pre_dispatch(const BlockShape &s, const void *zxbcdt, const float *conv_w, const float *conv_b,
                                const float *dt_bias, const void *state_in, void *state_out,
-                               const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t st) {
+                               const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, const DecayRates &rates, hipStream_t st) {
     // Runs of 4 steps while those leave the chip a wave per SIMD or less -- a run of 16 is six microseconds of vector
     // instructions for its wave, however few there are -- then of 8.  8 heads of 32, state 64, runs of 16 / 8 / 4 in us: 600 rows
     // 7.3 / 7.1 / 6.1, 4 000 7.6 / 5.5 / 4.8, 8 192 8.1 / 6.0 / 6.2, 16 384 9.3 / 8.8 / 10.2, 131 072 40.6 / 38.8 / 42.5, 262 144
@@ -262,7 +263,7 @@ static hipError_t pre_dispatch(const BlockShape &s, const void *zxbcdt, const fl
       *dd = static_cast<T *>(dt);
 #define SSD_PRE_CASE(Kv, Sv)                                                                                                     \
     if (s.d_conv == Kv && steps == Sv) {                                                                                         \
-        block_pre_kernel<T, Kv, Sv><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, s);      \
+        block_pre_kernel<T, Kv, Sv><<<grid, block, 0, st>>>(in, conv_w, conv_b, dt_bias, si, so, reset, xx, bb, cc, dd, rates, s);      \
         return hipGetLastError();                                                                                                \
     }
     SSD_PRE_CASE(2, 4) SSD_PRE_CASE(3, 4) SSD_PRE_CASE(4, 4)
@@ -273,9 +274,11 @@ static hipError_t pre_dispatch(const BlockShape &s, const void *zxbcdt, const fl
 
 hipError_t launch_block_pre(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w,
                             const float *conv_b, const float *dt_bias, const void *state_in, void *state_out,
-                            const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t st) {
-    return dtype ? pre_dispatch<__bf16>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, state_out, reset, x, Bm, Cm, dt, st)
-                 : pre_dispatch<float>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, state_out, reset, x, Bm, Cm, dt, st);
+                            const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t st, const float *A_log,
+                            float *A) {
+    const DecayRates rates{A_log, A, s.H};
+    return dtype ? pre_dispatch<__bf16>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, state_out, reset, x, Bm, Cm, dt, rates, st)
+                 : pre_dispatch<float>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, state_out, reset, x, Bm, Cm, dt, rates, st);
 }
 
 template <typename T, typename TY>

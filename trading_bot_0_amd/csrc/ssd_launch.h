@@ -164,7 +164,8 @@ hipError_t launch_block_wgrad(long long rows, int E, int N, int lda, const void 
                               hipStream_t st);
 hipError_t launch_block_pre(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w,
                             const float *conv_b, const float *dt_bias, const void *state_in, void *state_out,
-                            const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t stream);
+                            const unsigned char *reset, void *x, void *Bm, void *Cm, void *dt, hipStream_t stream,
+                            const float *A_log = nullptr, float *A = nullptr);  // (given: A [H] = -exp(A_log) as well)
 bool block_step_supported(const BlockShape &s, int d_model);
 hipError_t launch_block_step(const BlockShape &s, int dtype, int d_model, const void *u, const void *w_in, const float *conv_w,
                              const float *conv_b, const float *dt_bias, const float *A, const float *D, const float *norm_w,
@@ -183,7 +184,7 @@ hipError_t launch_block_post(const BlockShape &s, int dtype, const void *y, cons
 size_t block_bwd_workspace_bytes(const BlockShape &s);
 hipError_t launch_block_post_bwd(const BlockShape &s, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
                                  float eps, const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, void *workspace,
-                                 hipStream_t stream, void *yn = nullptr);
+                                 hipStream_t stream, void *yn = nullptr, const float *A_log = nullptr, float *A = nullptr);
 hipError_t launch_block_pre_bwd(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w, const float *conv_b,
                                 const float *dt_bias, const void *state_in, const unsigned char *reset, const void *dx,
                                 const void *dB, const void *dC, const void *ddt, const void *dstate_out, void *dzxbcdt,
@@ -294,8 +295,9 @@ hipError_t launch_bwd_ddt(const ScanShape &s, int dtype, const void *dt, const f
                           hipStream_t stream, const float *parts = nullptr, int nparts = 0,
                           const unsigned char *reset = nullptr, int raw_anchors = 0, int anchor_stride = 1);
 // dA[h], dD[h] (NULL allowed) = the sums over batch and chunks of the parts
+// and with dA_log given, dA_log[h] = dA[h] A[h] (A = -exp(A_log))
 hipError_t launch_bwd_head_sums(const ScanShape &s, const double *dA_part, const double *dD_part, float *dA, float *dD,
-                                hipStream_t stream);
+                                hipStream_t stream, const float *A = nullptr, float *dA_log = nullptr);
 hipError_t launch_bwd_dinit(const ScanShape &s, int dtype, const void *dt, const float *A, const float *gfin,
                             const unsigned char *reset, float *dinit, hipStream_t stream);
 

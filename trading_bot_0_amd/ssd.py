@@ -59,6 +59,10 @@ EXPORTED_SYMBOLS = (
     "ssd_block_pre_bwd",
     "ssd_block_post_proj_fwd",
     "ssd_block_step_fwd",
+    "ssd_block_forward_workspace_bytes",
+    "ssd_block_forward",
+    "ssd_block_grad_workspace_bytes",
+    "ssd_block_grad",
 )
 
 
