@@ -144,7 +144,8 @@ def test_weights_converted_in_one_launch(shape):
 @pytest.mark.parametrize("kind", ["plain", "reset", "state", "no D"])
 def test_whole_passes_in_one_call_are_the_stages(dims, B, L, kind):
     """Forward (with what it keeps, or with a carried state) and backward as one call each against the same stages called one by
-    one: the same kernels, so the same bits."""
+    one: the same kernels, so the same bits -- but for the two weight gradients, whose launch in common cuts the rows elsewhere: float32
+    sums of up to B L terms in another order, within 1e-5 of their norm."""
     from trading_bot_0_amd import Mamba2Block
     blk = Mamba2Block(*dims, seed=2)
     blk.norm_w.add_(torch.randn(blk.norm_w.shape, device="cuda"), alpha=0.2)
@@ -170,7 +171,10 @@ def test_whole_passes_in_one_call_are_the_stages(dims, B, L, kind):
     two = passes()
     assert one.keys() == two.keys()
     for k in one:
-        assert (one[k] is None and two[k] is None) or torch.equal(one[k], two[k]), k
+        if k in ("din_proj", "dout_proj"):
+            assert (one[k].double() - two[k].double()).norm() <= 1e-5 * two[k].double().norm(), k
+        else:
+            assert (one[k] is None and two[k] is None) or torch.equal(one[k], two[k]), k
 
 
 def test_whole_pass_captured_reads_the_parameters_at_replay():

@@ -1371,9 +1371,10 @@ namespace {
 
 // What a block's backward pass keeps between its launches.
 struct GradScratch {
-    void *dyn, *yn, *dy, *dx, *dB, *dC, *ddt, *sums, *wgrad, *scan;
+    void *dyn, *yn, *dy, *dx, *dB, *dC, *ddt, *norm, *sums, *wgrad, *scan;
     float *A;
-    size_t sums_bytes, wgrad_bytes, scan_bytes;
+    size_t scan_bytes;
+    bool pair;  // both weight gradients in one launch
 };
 
 int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_model, int width, Carver *c, GradScratch *g) {
@@ -1381,9 +1382,10 @@ int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_m
     if (int rc = ssd_chunk_scan_bwd_workspace_bytes(&scan, SSD_DTYPE_BF16, &g->scan_bytes)) return rc;
     if (int rc = check_wgrad((int64_t)rows, width, d_model)) return rc;
     if (int rc = check_wgrad((int64_t)rows, d_model, (int64_t)DI)) return rc;
-    g->sums_bytes = ssd::block_bwd_workspace_bytes(s);
-    g->wgrad_bytes = std::max(ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model),
-                              ssd::block_wgrad_workspace_bytes((long long)rows, (int)d_model, (int)DI));
+    g->pair = d_model == (int64_t)DI;
+    const size_t wgrad_bytes = g->pair ? ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model, (int)d_model)
+                                       : std::max(ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model),
+                                                  ssd::block_wgrad_workspace_bytes((long long)rows, (int)d_model, (int)DI));
     g->A = static_cast<float *>(c->take((size_t)s.H * sizeof(float)));
     g->dyn = c->take(rows * DI * 2);
     g->yn = c->take(rows * DI * 2);
@@ -1392,8 +1394,9 @@ int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_m
     g->dB = c->take(rows * GN * 2);
     g->dC = c->take(rows * GN * 2);
     g->ddt = c->take(rows * s.H * 2);
-    g->sums = c->take(g->sums_bytes);
-    g->wgrad = c->take(g->wgrad_bytes);
+    g->norm = c->take(ssd::block_norm_sums_bytes(s));
+    g->sums = c->take(ssd::block_bwd_workspace_bytes(s));
+    g->wgrad = c->take(wgrad_bytes);
     g->scan = c->take(g->scan_bytes);
     return SSD_OK;
 }
@@ -1463,23 +1466,27 @@ int ssd_block_grad(const ssd_block_dims *dims, int dtype, int64_t d_model, int64
         return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, c.used);
     hipStream_t st = (hipStream_t)hip_stream;
     const int DI = s.H * s.P;
+    ssd::NormSums norm;
     hipError_t e = ssd::launch_block_proj(rows, (int)d_model, DI, DI, dout, w_out_t, g.dyn, st);
     if (e != hipSuccess) return hip_fail(e, "block projection launch");
-    e = ssd::launch_block_post_bwd(s, SSD_DTYPE_BF16, y, zxbcdt, norm_w, eps, g.dyn, g.dy, dzxbcdt, dnorm_w, g.sums, st, g.yn, A_log, g.A);
+    e = ssd::launch_block_post_bwd(s, SSD_DTYPE_BF16, y, zxbcdt, norm_w, eps, g.dyn, g.dy, dzxbcdt, dnorm_w, g.norm, st, g.yn, A_log, g.A, &norm);
     if (e != hipSuccess) return hip_fail(e, "block post-scan backward launch");
-    e = ssd::launch_block_wgrad(rows, (int)d_model, DI, (int)d_model, dout, g.yn, dout_proj, g.wgrad, st);
-    if (e != hipSuccess) return hip_fail(e, "weight gradient launch");
+    const ssd::WgradArgs of_out{dout, g.yn, dout_proj, (int)d_model, (int)d_model}, of_in{dzxbcdt, u, din_proj, width, s.ld};
+    if (!g.pair) {
+        e = ssd::launch_block_wgrad2(rows, DI, of_out, ssd::WgradArgs{}, g.wgrad, st);
+        if (e != hipSuccess) return hip_fail(e, "weight gradient launch");
+    }
     if (int rc = scan_backward(&scan, SSD_DTYPE_BF16, x, dt, g.A, Bm, Cm, D, nullptr, reset, g.dy, nullptr, g.dx, g.ddt, dA, g.dB, g.dC, dD,
                                nullptr, g.scan, g.scan_bytes, hip_stream, dA_log))
         return rc;
     e = ssd::launch_block_pre_bwd(s, 1, zxbcdt, conv_w, conv_b, dt_bias, nullptr, reset, g.dx, g.dB, g.dC, g.ddt, nullptr, dzxbcdt, dconv_w,
-                                  dconv_b, ddt_bias, nullptr, g.sums, st);
+                                  dconv_b, ddt_bias, nullptr, g.sums, st, norm);
     if (e != hipSuccess) return hip_fail(e, "block pre-scan backward launch");
     if (du != nullptr) {
         e = ssd::launch_block_dproj(rows, width, (int)d_model, s.ld, (int)w_in_t_ld, dzxbcdt, w_in_t, du, st);
         if (e != hipSuccess) return hip_fail(e, "projection input gradient launch");
     }
-    e = ssd::launch_block_wgrad(rows, width, (int)d_model, s.ld, dzxbcdt, u, din_proj, g.wgrad, st);
+    e = ssd::launch_block_wgrad2(rows, (int)d_model, of_in, g.pair ? of_out : ssd::WgradArgs{}, g.wgrad, st);
     return e == hipSuccess ? SSD_OK : hip_fail(e, "weight gradient launch");
 }
 

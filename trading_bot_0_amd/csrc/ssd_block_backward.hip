@@ -200,12 +200,14 @@ struct ColumnSums {
     int blocks() const { return (cols + 63) / 64; }
 };
 
-__global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums first, ColumnSums second, int first_blocks) {
+__global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums first, ColumnSums second, ColumnSums third,
+                                                                      int first_blocks, int second_blocks) {
     __shared__ float sm[kSumSlices][64];
-    const bool one = (int)blockIdx.x < first_blocks;
-    const ColumnSums &j = one ? first : second;
+    const int at = (int)blockIdx.x;
+    const int job = at < first_blocks ? 0 : at < first_blocks + second_blocks ? 1 : 2;
+    const ColumnSums &j = job == 0 ? first : job == 1 ? second : third;
     const int cl = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int c = ((int)blockIdx.x - (one ? 0 : first_blocks)) * 64 + cl;
+    const int c = (at - (job == 0 ? 0 : job == 1 ? first_blocks : first_blocks + second_blocks)) * 64 + cl;
     const int per = (j.nparts + gridDim.y - 1) / gridDim.y;
     const int p0 = blockIdx.y * per, p1 = min(j.nparts, p0 + per);
     float acc = 0.f;
@@ -228,20 +230,22 @@ __global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums
     }
 }
 
-// Sums `job` (tmp holds kSumShares * job.cols floats) and, in the last of its launches, `other` (at most kSumWholeParts parts).
-static hipError_t launch_column_sums(const ColumnSums &job, float *tmp, const ColumnSums &other, hipStream_t st) {
+// Sums `job` (tmp holds kSumShares * job.cols floats) and, in the last of its launches, `other` and `third` (at most kSumWholeParts
+// parts each).
+static hipError_t launch_column_sums(const ColumnSums &job, float *tmp, const ColumnSums &other, const ColumnSums &third, hipStream_t st) {
     ColumnSums last = job;
     if (job.nparts > kSumWholeParts) {
         ColumnSums shares = job;
         shares.out = tmp;
         shares.split = 0;
-        column_sums_kernel<<<dim3(job.blocks(), kSumShares), dim3(64 * kSumSlices), 0, st>>>(shares, shares, job.blocks());
+        column_sums_kernel<<<dim3(job.blocks(), kSumShares), dim3(64 * kSumSlices), 0, st>>>(shares, ColumnSums{}, ColumnSums{}, job.blocks(), 0);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         last.part = tmp;
         last.nparts = kSumShares;
     }
-    column_sums_kernel<<<dim3(last.blocks() + other.blocks(), 1), dim3(64 * kSumSlices), 0, st>>>(last, other, last.blocks());
+    column_sums_kernel<<<dim3(last.blocks() + other.blocks() + third.blocks(), 1), dim3(64 * kSumSlices), 0, st>>>(
+        last, other, third, last.blocks(), other.blocks());
     return hipGetLastError();
 }
 
@@ -632,6 +636,8 @@ static long long bwd_run_blocks(const BlockShape &s, int steps) {
 // for either: it grows with batch and length.)
 constexpr long long kShortRunBlocks = 320;
 
+size_t block_norm_sums_bytes(const BlockShape &s) { return (size_t)kPostBlocks * s.H * s.P * sizeof(float); }
+
 // workspace: the partial sums of post_bwd, or those of pre_bwd (conv, their column sums, dt)
 size_t block_bwd_workspace_bytes(const BlockShape &s) {
     const size_t DI = (size_t)s.H * s.P, C = DI + 2 * (size_t)s.G * s.N;
@@ -644,7 +650,7 @@ size_t block_bwd_workspace_bytes(const BlockShape &s) {
 template <typename T, typename TY>
 static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const void *zxbcdt, const float *norm_w, float eps,
                                     const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, float *part, void *yn,
-                                    const DecayRates &rates, hipStream_t st) {
+                                    const DecayRates &rates, NormSums *later, hipStream_t st) {
     const int DI = s.H * s.P, pieces = DI / 8;
     const long long rows = (long long)s.B * s.L;
     const TY *yy = static_cast<const TY *>(y);
@@ -670,18 +676,22 @@ static hipError_t post_bwd_dispatch(const BlockShape &s, const void *y, const vo
     if (!launched) return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_column_sums(ColumnSums{part, blocks, DI, dnorm_w}, part + (size_t)kPostBlocks * DI, ColumnSums{}, st);
+    if (later != nullptr) {
+        *later = NormSums{part, blocks, dnorm_w};
+        return hipSuccess;
+    }
+    return launch_column_sums(ColumnSums{part, blocks, DI, dnorm_w}, part + (size_t)kPostBlocks * DI, ColumnSums{}, ColumnSums{}, st);
 }
 
 hipError_t launch_block_post_bwd(const BlockShape &s, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
                                  float eps, const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, void *workspace,
-                                 hipStream_t st, void *yn, const float *A_log, float *A) {
+                                 hipStream_t st, void *yn, const float *A_log, float *A, NormSums *later) {
     const DecayRates rates{A_log, A, s.H};
     float *part = static_cast<float *>(workspace);
     switch (dtype) {
-        case 0: return post_bwd_dispatch<float, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
-        case 1: return post_bwd_dispatch<__bf16, __bf16>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
-        default: return post_bwd_dispatch<__bf16, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, st);
+        case 0: return post_bwd_dispatch<float, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, later, st);
+        case 1: return post_bwd_dispatch<__bf16, __bf16>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, later, st);
+        default: return post_bwd_dispatch<__bf16, float>(s, y, zxbcdt, norm_w, eps, dout, dy, dzxbcdt, dnorm_w, part, yn, rates, later, st);
     }
 }
 
@@ -690,7 +700,7 @@ static hipError_t pre_bwd_dispatch(const BlockShape &s, const void *zxbcdt, cons
                                    const float *dt_bias, const void *state_in, const unsigned char *reset, const void *dx,
                                    const void *dB, const void *dC, const void *ddt, const void *dstate_out, void *dzxbcdt,
                                    float *dconv_w, float *dconv_b, float *ddt_bias, void *dstate_in, float *part,
-                                   hipStream_t st) {
+                                   const NormSums &norm, hipStream_t st) {
     const int DI = s.H * s.P, C = DI + 2 * s.G * s.N, CP = C / kBwdCh, K = s.d_conv;
     const int steps = bwd_run_blocks(s, 8) <= kShortRunBlocks ? 8 : 32;
     const long long run_blocks = bwd_run_blocks(s, steps);
@@ -727,21 +737,22 @@ static hipError_t pre_bwd_dispatch(const BlockShape &s, const void *zxbcdt, cons
     if (e != hipSuccess) return e;
     // the conv's partials hold, per run block, [C][K+1] = (dw[0..K-1], db)
     return launch_column_sums(ColumnSums{part, (int)run_blocks, cols, dconv_w, dconv_b, K + 1}, tmp,
-                              ColumnSums{dt_part, dt_blocks, s.H, ddt_bias}, st);
+                              ColumnSums{dt_part, dt_blocks, s.H, ddt_bias},
+                              norm.part != nullptr ? ColumnSums{norm.part, norm.parts, DI, norm.out} : ColumnSums{}, st);
 }
 
 hipError_t launch_block_pre_bwd(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w, const float *conv_b,
                                 const float *dt_bias, const void *state_in, const unsigned char *reset, const void *dx,
                                 const void *dB, const void *dC, const void *ddt, const void *dstate_out, void *dzxbcdt,
                                 float *dconv_w, float *dconv_b, float *ddt_bias, void *dstate_in, void *workspace,
-                                hipStream_t st) {
+                                hipStream_t st, const NormSums &norm) {
     // the post partials occupy the front of the workspace (the two stages of one backward pass share it: post runs
     // first and has added its partials up before pre starts on the same stream)
     float *part = static_cast<float *>(workspace);
     return dtype ? pre_bwd_dispatch<__bf16>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, reset, dx, dB, dC, ddt, dstate_out,
-                                            dzxbcdt, dconv_w, dconv_b, ddt_bias, dstate_in, part, st)
+                                            dzxbcdt, dconv_w, dconv_b, ddt_bias, dstate_in, part, norm, st)
                  : pre_bwd_dispatch<float>(s, zxbcdt, conv_w, conv_b, dt_bias, state_in, reset, dx, dB, dC, ddt, dstate_out,
-                                           dzxbcdt, dconv_w, dconv_b, ddt_bias, dstate_in, part, st);
+                                           dzxbcdt, dconv_w, dconv_b, ddt_bias, dstate_in, part, norm, st);
 }
 
 }  // namespace ssd

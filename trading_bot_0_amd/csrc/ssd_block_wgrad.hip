@@ -29,10 +29,24 @@ constexpr int kWgradThreads = 512;
 constexpr int kFlushSteps = 64;
 constexpr int kWgradMinRows = 256;  // per split: shorter ones are mostly the partial block's way out
 
+// One weight gradient of a launch: its operands and where its splits' blocks go ([splits, E, N]).
+struct WgradJob {
+    const __bf16 *a, *b;
+    float *part;
+    int E, lda, blocks;
+};
+
+// (two jobs over the same rows, of which the second may have no blocks: the workgroups of the first come first)
 template <int NB>  // N = 128 NB
-__global__ __launch_bounds__(kWgradThreads) void block_wgrad_kernel(const __bf16 *__restrict__ a, const __bf16 *__restrict__ b,
-                                                                    float *__restrict__ part, long long rows, int E, int lda,
-                                                                    int blocks, int splits, long long split_rows) {
+__global__ __launch_bounds__(kWgradThreads) void block_wgrad_kernel(WgradJob first, WgradJob second, int first_groups, long long rows,
+                                                                    int splits, long long split_rows) {
+    const bool one = (int)blockIdx.x < first_groups;
+    const WgradJob &job = one ? first : second;
+    const int group = (int)blockIdx.x - (one ? 0 : first_groups);  // (a multiple of 8: the XCD is the block's)
+    const __bf16 *__restrict__ a = job.a;
+    const __bf16 *__restrict__ b = job.b;
+    float *__restrict__ part = job.part;
+    const int E = job.E, lda = job.lda, blocks = job.blocks;
     using T = ChunkTile<128>;
     constexpr int N = 128 * NB, TILE = kWgradRows * 128;
     constexpr int WN = N / 64, WM = 8 / WN, MI = kWgradCols / WM / 32, NI = 2;  // a wave: MI x NI tiles of 32 x 32
@@ -40,7 +54,7 @@ __global__ __launch_bounds__(kWgradThreads) void block_wgrad_kernel(const __bf16
     __shared__ __attribute__((aligned(16))) __bf16 sm[2][TILE * (1 + NB)];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN;
-    const int xcd = blockIdx.x % 8, within = blockIdx.x / 8;
+    const int xcd = group % 8, within = group / 8;
     const int split = (within / blocks) * 8 + xcd, m0 = (within % blocks) * kWgradCols;
     if (split >= splits) return;  // (the grid is padded to whole rounds of XCDs)
     const long long begin = split * split_rows, end = min(rows, begin + split_rows);
@@ -132,11 +146,16 @@ __global__ __launch_bounds__(kWgradThreads) void block_wgrad_kernel(const __bf16
     }
 }
 
-// out = the splits' blocks added in order; four elements per thread, eight splits' requested at a time
-__global__ __launch_bounds__(256) void block_wgrad_sum_kernel(const float4 *__restrict__ part, float4 *__restrict__ out, int splits,
-                                                              int pieces) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= pieces) return;
+// out = the splits' blocks added in order; four elements per thread, eight splits' requested at a time (two jobs, as above)
+__global__ __launch_bounds__(256) void block_wgrad_sum_kernel(const float4 *__restrict__ part0, float4 *__restrict__ out0, int pieces0,
+                                                              const float4 *__restrict__ part1, float4 *__restrict__ out1, int pieces1,
+                                                              int splits) {
+    int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces0 + pieces1) return;
+    const bool one = i < pieces0;
+    const int pieces = one ? pieces0 : pieces1;
+    const float4 *part = one ? part0 : part1;
+    if (!one) i -= pieces0;
     float4 sum = make_float4(0, 0, 0, 0);
     for (int s0 = 0; s0 < splits; s0 += 8) {
         float4 q[8];
@@ -151,20 +170,21 @@ __global__ __launch_bounds__(256) void block_wgrad_sum_kernel(const float4 *__re
             sum.w += w != 0.f ? q[u].w : 0.f;
         }
     }
-    out[i] = sum;
+    (one ? out0 : out1)[i] = sum;
 }
 
 struct WgradPlan {
-    int blocks, splits;
+    int splits;
     long long split_rows;
 };
 
+int wgrad_blocks(int E) { return (E + kWgradCols - 1) / kWgradCols; }
+
 // Splits: one round of workgroups (a compute unit holds one), whole XCDs, none below kWgradMinRows rows.  (256 compute units are
 // a constant here: the workspace is laid out by the splits, and the order of the sums, so the bits, do not depend on the device.)
-WgradPlan wgrad_plan(long long rows, int E) {
+WgradPlan wgrad_plan(long long rows, int blocks) {
     WgradPlan p;
-    p.blocks = (E + kWgradCols - 1) / kWgradCols;
-    const long long fill = std::max(1, 256 / 8 / p.blocks) * 8;
+    const long long fill = std::max(1, 256 / 8 / blocks) * 8;
     const long long most = std::max<long long>(1, std::min(fill, rows / kWgradMinRows));
     p.split_rows = ((rows + most - 1) / most + kWgradRows - 1) / kWgradRows * kWgradRows;
     p.splits = (int)((rows + p.split_rows - 1) / p.split_rows);
@@ -177,28 +197,43 @@ bool block_wgrad_supported(long long rows, int E, int N) {
     return rows > 0 && rows <= 0x7fffffffLL && E >= 8 && E % 8 == 0 && E <= 8192 && (N == 128 || N == 256);
 }
 
-size_t block_wgrad_workspace_bytes(long long rows, int E, int N) {
-    const WgradPlan p = wgrad_plan(rows, E);
-    return p.splits > 1 ? (size_t)p.splits * E * N * sizeof(float) : 0;
+size_t block_wgrad_workspace_bytes(long long rows, int E, int N, int E2) {
+    const WgradPlan p = wgrad_plan(rows, wgrad_blocks(E) + (E2 > 0 ? wgrad_blocks(E2) : 0));
+    return p.splits > 1 ? (size_t)p.splits * (E + E2) * N * sizeof(float) : 0;
+}
+
+// Both weight gradients of a block in one launch: the blocks of both share one round of workgroups, and a few rows' partial
+// blocks one launch for their sums (the two on their own, 648 x 256 and 256 x 256 outputs in us: 800 rows 12 + 4 + 11 + 4 -> 12.2 + 4,
+// 16 384 rows 17.5 + 5 + 12.7 + 5.9 -> 20.2 + 6).
+hipError_t launch_block_wgrad2(long long rows, int N, const WgradArgs &x, const WgradArgs &y, void *workspace, hipStream_t st) {
+    if (!block_wgrad_supported(rows, x.E, N) || x.lda < x.E || x.lda % 8 != 0) return hipErrorInvalidValue;
+    const bool two = y.E > 0;
+    if (two && (!block_wgrad_supported(rows, y.E, N) || y.lda < y.E || y.lda % 8 != 0)) return hipErrorInvalidValue;
+    const int blocks0 = wgrad_blocks(x.E), blocks1 = two ? wgrad_blocks(y.E) : 0;
+    const WgradPlan p = wgrad_plan(rows, blocks0 + blocks1);
+    float *part0 = p.splits > 1 ? static_cast<float *>(workspace) : x.out;
+    float *part1 = p.splits > 1 ? part0 + (size_t)p.splits * x.E * N : y.out;
+    auto job = [](const WgradArgs &g, float *part, int blocks) {
+        return WgradJob{static_cast<const __bf16 *>(g.a), static_cast<const __bf16 *>(g.b), part, g.E, g.lda, blocks};
+    };
+    const int per_block = (p.splits + 7) / 8 * 8, groups0 = per_block * blocks0;
+    const dim3 grid((unsigned)(groups0 + per_block * blocks1)), block(kWgradThreads);
+    if (N == 256)
+        block_wgrad_kernel<2><<<grid, block, 0, st>>>(job(x, part0, blocks0), job(y, part1, blocks1), groups0, rows, p.splits, p.split_rows);
+    else
+        block_wgrad_kernel<1><<<grid, block, 0, st>>>(job(x, part0, blocks0), job(y, part1, blocks1), groups0, rows, p.splits, p.split_rows);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.splits == 1) return e;
+    const int pieces0 = x.E * N / 4, pieces1 = two ? y.E * N / 4 : 0;
+    block_wgrad_sum_kernel<<<dim3((pieces0 + pieces1 + 255) / 256), dim3(256), 0, st>>>(
+        reinterpret_cast<const float4 *>(part0), reinterpret_cast<float4 *>(x.out), pieces0, reinterpret_cast<const float4 *>(part1),
+        reinterpret_cast<float4 *>(y.out), pieces1, p.splits);
+    return hipGetLastError();
 }
 
 hipError_t launch_block_wgrad(long long rows, int E, int N, int lda, const void *a, const void *b, float *out, void *workspace,
                               hipStream_t st) {
-    if (!block_wgrad_supported(rows, E, N) || lda < E || lda % 8 != 0) return hipErrorInvalidValue;
-    const WgradPlan p = wgrad_plan(rows, E);
-    float *part = p.splits > 1 ? static_cast<float *>(workspace) : out;
-    const dim3 grid((unsigned)((p.splits + 7) / 8 * 8 * p.blocks)), block(kWgradThreads);
-    const __bf16 *aa = static_cast<const __bf16 *>(a), *bb = static_cast<const __bf16 *>(b);
-    if (N == 256)
-        block_wgrad_kernel<2><<<grid, block, 0, st>>>(aa, bb, part, rows, E, lda, p.blocks, p.splits, p.split_rows);
-    else
-        block_wgrad_kernel<1><<<grid, block, 0, st>>>(aa, bb, part, rows, E, lda, p.blocks, p.splits, p.split_rows);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.splits == 1) return e;
-    const int pieces = E * N / 4;
-    block_wgrad_sum_kernel<<<dim3((pieces + 255) / 256), dim3(256), 0, st>>>(reinterpret_cast<const float4 *>(part),
-                                                                             reinterpret_cast<float4 *>(out), p.splits, pieces);
-    return hipGetLastError();
+    return launch_block_wgrad2(rows, N, WgradArgs{a, b, out, E, lda}, WgradArgs{}, workspace, st);
 }
 
 }  // namespace ssd

@@ -159,7 +159,14 @@ hipError_t launch_block_weights(int E, int D, int DI, const float *in_proj, cons
 // The projections' weight gradients: out [E, N] (float32) = a^T b over all rows, a [rows, E] (rows lda elements apart, a
 // multiple of 8) and b [rows, N] in bf16; E a multiple of 8, N 128 or 256.  workspace: the partial sums.
 bool block_wgrad_supported(long long rows, int E, int N);
-size_t block_wgrad_workspace_bytes(long long rows, int E, int N);
+size_t block_wgrad_workspace_bytes(long long rows, int E, int N, int E2 = 0);
+// two over the same rows in one launch (with E2 in the workspace's size; the second's E may be 0)
+struct WgradArgs {
+    const void *a = nullptr, *b = nullptr;
+    float *out = nullptr;
+    int E = 0, lda = 0;
+};
+hipError_t launch_block_wgrad2(long long rows, int N, const WgradArgs &x, const WgradArgs &y, void *workspace, hipStream_t st);
 hipError_t launch_block_wgrad(long long rows, int E, int N, int lda, const void *a, const void *b, float *out, void *workspace,
                               hipStream_t st);
 hipError_t launch_block_pre(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w,
@@ -182,14 +189,23 @@ hipError_t launch_block_post(const BlockShape &s, int dtype, const void *y, cons
 // ([B,L,H*P], the activation type) post_bwd also writes the forward's normalised rows, bit for bit what
 // launch_block_post writes, for a forward that did not keep them.
 size_t block_bwd_workspace_bytes(const BlockShape &s);
+// dnorm_w's partial sums for a caller that has launch_block_pre_bwd add them up with its own: post_bwd then only leaves them in its
+// workspace (block_norm_sums_bytes, not pre_bwd's) and names them here.
+struct NormSums {
+    const float *part = nullptr;
+    int parts = 0;
+    float *out = nullptr;
+};
+size_t block_norm_sums_bytes(const BlockShape &s);
 hipError_t launch_block_post_bwd(const BlockShape &s, int dtype, const void *y, const void *zxbcdt, const float *norm_w,
                                  float eps, const void *dout, void *dy, void *dzxbcdt, float *dnorm_w, void *workspace,
-                                 hipStream_t stream, void *yn = nullptr, const float *A_log = nullptr, float *A = nullptr);
+                                 hipStream_t stream, void *yn = nullptr, const float *A_log = nullptr, float *A = nullptr,
+                                 NormSums *later = nullptr);
 hipError_t launch_block_pre_bwd(const BlockShape &s, int dtype, const void *zxbcdt, const float *conv_w, const float *conv_b,
                                 const float *dt_bias, const void *state_in, const unsigned char *reset, const void *dx,
                                 const void *dB, const void *dC, const void *ddt, const void *dstate_out, void *dzxbcdt,
                                 float *dconv_w, float *dconv_b, float *ddt_bias, void *dstate_in, void *workspace,
-                                hipStream_t stream);
+                                hipStream_t stream, const NormSums &norm = NormSums{});
 
 // The backward pass's two scans of the transposed state with the sum over a group's heads taken on chip (bf16,
 // headdim 32, eight heads per group; sT is the transposed shape: P = dstate, N = 32, G = H; sT.mode / dt_len as
