@@ -72,12 +72,12 @@ def c_oracle_reset(cpu, mask):
     return y, fin
 
 
-@pytest.mark.parametrize("seqlen", [100, 400, 2000])
+@pytest.mark.parametrize("batch,seqlen", [(3, 100), (3, 400), (3, 2000), (90, 1024), (60, 1000)])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-def test_final_state_written_over_the_initial_state(seqlen, dtype):
+def test_final_state_written_over_the_initial_state(batch, seqlen, dtype):
     """A stream's prefix that continues a state in place: the same buffer as initial and final state, at lengths whose separate
-    buffers would take the recurrence inside stage 4."""
-    w = Workload("inplace", 3, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
+    buffers would take the recurrence inside stage 4, or on segments, inside their prologues."""
+    w = Workload("inplace", batch, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
     cpu = make_inputs(w, seed=3)
     dev = to_dev(cpu)
     yr, fr = oracle_scan(cpu)
@@ -111,3 +111,25 @@ def test_state_passing_runs(nc):
         prev, fin = ssd.state_passing(S.cuda(), dtcs, init.cuda(), in_place=in_place)
         assert (prev.cpu().double() - ref).abs().max() <= 1e-5 * ref.abs().max()
         assert (fin.cpu().double() - st).abs().max() <= 1e-5 * st.abs().max()
+
+
+@pytest.mark.parametrize("batch,seqlen,dtype", [(24, 2100, "bf16"), (16, 4100, "bf16"), (90, 1030, "bf16"), (90, 2500, "bf16"), (20, 4000, "f32"),
+                                                (96, 1999, "f32"), (60, 1001, "f32")])
+def test_forward_on_segments(batch, seqlen, dtype):
+    """Cuts into a few segments (states entering them worked out in the prologues), into eight and more (in a launch of their own) and
+    over two rounds of workgroups, with restarts, a row whose initial state is not read, and ragged last segments."""
+    w = Workload("segments", batch, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
+    assert ssd.chunk_scan_segments(batch, seqlen, 8, 32, 64, 1, 128, w.torch_dtype) > 1
+    cpu = make_inputs(w, seed=seqlen)
+    dev = to_dev(cpu)
+    mask = torch.rand(batch, seqlen, generator=torch.Generator().manual_seed(5)) < 0.002
+    mask[0, 0] = True
+    dev["init"][0] = float("nan")
+    rows = [0, batch // 2, batch - 1]
+    y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=128, initial_states=dev["init"],
+                          reset=mask.cuda(), y_dtype=torch.float32)
+    sub = {k: (v if k in ("A", "D") else v[rows].clone()) for k, v in cpu.items()}
+    sub["init"][0] = 0.0
+    yr, fr = c_oracle_reset(sub, mask[rows])
+    assert_close(y[rows], yr, w.torch_dtype, "y")
+    assert_close(f[rows], fr, w.torch_dtype, "final")

@@ -187,9 +187,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fused_scan_f32_kernel(
     f32x16 st[NB];
     {
         const bool folded = !STATES_ONLY && s.seg_local != nullptr;
-        const bool fresh = rsb != nullptr && rsb[0] != 0;  // a restart before the first step: init is not read
+        // (segments that are given the state they start from have one each, [B, S, H, P, N])
+        const bool entered = !STATES_ONLY && S > 1 && !folded;
+        // a restart before the first step: init is not read
+        const bool fresh = rsb != nullptr && rsb[0] != 0 && !(entered && seg > 0);
         const size_t lane_off = (size_t)(pb * 32 + r) * N + 4 * half;
-        const float *ib = !STATES_ONLY && init && !fresh ? init + ((size_t)b * s.H + h) * s.P * N + lane_off : nullptr;
+        const float *ib = !STATES_ONLY && init && !fresh
+                              ? init + ((entered ? (size_t)b * S + seg : (size_t)b) * s.H + h) * s.P * N + lane_off : nullptr;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -471,7 +475,7 @@ hipError_t launch_fused_scan_f32(const ScanShape &s, const void *x, const void *
     if (fused_scan_f32_waves(s) != 8) return hipErrorInvalidValue;
     const int nc = (s.L + kFloatTile - 1) / kFloatTile;
     const int segments = s.seg_tiles > 0 ? (nc + s.seg_tiles - 1) / s.seg_tiles : 1;
-    if ((segments > 1) != (s.seg_local != nullptr)) return hipErrorInvalidValue;
+    if (segments > 1 ? s.seg_local == nullptr && init == nullptr : s.seg_local != nullptr) return hipErrorInvalidValue;
     const int grid = s.B * s.G * ((s.H / s.G) * (s.P / 32) / 8) * segments;
     const float *xx = static_cast<const float *>(x), *dd = static_cast<const float *>(dt);
     const float *bb = static_cast<const float *>(Bm), *cc = static_cast<const float *>(Cm);
@@ -489,7 +493,7 @@ int fused_scan_f32_tile() { return kFloatTile; }
 hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, const void *x, const void *dt, const float *A,
                                            const void *Bm, const void *Cm, const float *D, const float *init,
                                            const unsigned char *reset, void *y, float *final_states, float *seg_states,
-                                           float *seg_decay, hipStream_t st) {
+                                           float *seg_decay, bool passed, hipStream_t st) {
     if (segments < 2 || fused_scan_f32_waves(s) != 8) return hipErrorInvalidValue;
     const int nc = (s.L + kFloatTile - 1) / kFloatTile;
     ScanShape t = s;
@@ -504,6 +508,10 @@ hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, con
         fused_scan_f32_kernel<2, 8, true><<<dim3(grid), dim3(512), 0, st>>>(xx, dd, A, bb, bb, nullptr, nullptr, reset, nullptr, seg_states, seg_decay, t);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    if (passed) {
+        e = launch_segment_passing(t, segments, seg_states, seg_decay, init, reset, st);
+        return e != hipSuccess ? e : launch_fused_scan_f32(t, x, dt, A, Bm, Cm, D, seg_states, reset, y, final_states, st);
+    }
     t.seg_local = seg_states;
     t.seg_local_decay = seg_decay;
     return launch_fused_scan_f32(t, x, dt, A, Bm, Cm, D, init, reset, y, final_states, st);

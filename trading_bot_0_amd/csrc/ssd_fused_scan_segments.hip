@@ -11,8 +11,13 @@ namespace ssd {
 
 namespace {
 
-constexpr int kSegmentMinTiles = 4;        // shorter segments are mostly prologue
-constexpr int kSegmentTargetGroups = 192;  // workgroups to aim for (256 CUs; the last quarter gains little)
+constexpr int kSegmentMinTiles = 4;   // shorter segments are mostly prologue (and their states would not fit chunks of 256 steps)
+constexpr int kSegmentMaxGroups = 768;  // three rounds of workgroups
+// From so many segments on the states entering them are worked out by a launch of their own instead of in every workgroup's
+// prologue, which reads those of all segments before it.  One by one / in a launch, us: 16 x 4 096 on 16 67 / 50, 24 x 4 096 on 8
+// 76 / 71, 24 x 2 048 on 8 51 / 46; 48 x 4 096 on 5 99 / 105, 61 x 3 999 on 4 120 / 127; float32 20 x 4 000 on 8 134 / 133, 60 x 1 000 on
+// 4 79 / 87.
+constexpr int kPassMinSegments = 8;
 
 int tiles_of(const ScanShape &s) { return (s.L + kOnePassTile - 1) / kOnePassTile; }
 int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1) / fused_scan_f32_tile(); }
@@ -36,13 +41,29 @@ double whole_us(const ScanShape &s, int dtype, long long groups) {
     const double fill = groups < 256 ? (double)groups / 256.0 : 1.0;
     return 6.0 + tiles_of(s) * rounds * (s.N == 128 ? 4.1 + 0.5 * fill : 4.1 + 1.5 * fill);
 }
-// ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 37 / 36, 16 x 1 024
-// on 4 40 / 40, 16 x 2 048 on 8 48 / 50, 48 x 2 048 on 4 65 / 70, 24 x 4 096 on 8 73 / 76, 64 x 4 096 on 4 115 / 124; float32
-// 96 x 1 999 on 2 253 / 247, 30 x 1 000 on 4 72 / 74
+// ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 40 / 36, 90 x 1 024
+// on 2 65 / 66, 61 x 3 999 on 4 117 / 120, 48 x 4 096 on 5 101 / 99, 24 x 4 096 on 8 69 / 71, 90 x 4 096 on 5 (two rounds) 198 / 198;
+// float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12 98 / 105
 double segments_us(int dtype, long long groups, int segments, int seg_tiles) {
-    const double rounds = (double)((groups * segments + 255) / 256);
-    if (dtype == 0) return 10.0 + 7.7 * seg_tiles * rounds;
-    return 8.0 + 1.9 * segments + 6.2 * seg_tiles * rounds;
+    const double rounds = (double)((groups * segments + 255) / 256), tiles = seg_tiles * rounds, more = rounds - 1.0;
+    if (dtype == 0) return 6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more;
+    return 12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more;
+}
+// the fastest cut of nc tiles into segments of min_tiles or more, by that estimate; in bf16 a power of two unless another is clearly
+// faster (the estimate is good to a few per cent, and programs size and compare by the number of segments)
+double best_segments(int dtype, long long groups, int nc, int min_tiles, int *segments) {
+    double best = 1e30;
+    *segments = 1;
+    for (int S = 2; nc >= S * min_tiles && groups * S <= kSegmentMaxGroups; ++S) {
+        const int seg_tiles = (nc + S - 1) / S;
+        if ((nc + seg_tiles - 1) / seg_tiles != S) continue;
+        const double cost = segments_us(dtype, groups, S, seg_tiles) * (dtype == 0 || (S & (S - 1)) == 0 ? 1.0 : 1.07);
+        if (cost < best) {
+            best = cost;
+            *segments = S;
+        }
+    }
+    return *segments > 1 ? segments_us(dtype, groups, *segments, (nc + *segments - 1) / *segments) : best;
 }
 
 }  // namespace
@@ -57,14 +78,8 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
         const long long groups = (long long)s.B * s.G * ((s.H / s.G) * (s.P / 32) / 8);
         const int nc = float_tiles_of(s);
         const double staged = staged_us(s, 0, groups), whole = whole_us(s, 0, groups);
-        double cut = 1e30;
-        int S = 1;
-        while (groups * S < kSegmentTargetGroups && nc / (2 * S) >= 2 * kSegmentMinTiles) S *= 2;
-        if (S >= 2) {
-            const int seg_tiles = (nc + S - 1) / S;
-            S = (nc + seg_tiles - 1) / seg_tiles;
-            cut = segments_us(0, groups, S, seg_tiles);
-        }
+        int S;
+        const double cut = best_segments(0, groups, nc, 2 * kSegmentMinTiles, &S);
         if (cut < whole && cut < staged) {
             *segments = S;
             return 2;
@@ -90,16 +105,8 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     const long long groups = (long long)s.B * s.G * ((s.H / s.G) * (s.P / 32) / full);
     const int nc = tiles_of(s);
     const double staged = staged_us(s, dtype, groups), whole = whole_us(s, dtype, groups);
-    double cut = 1e30;
     int S = 1;
-    if (s.N != 128) {
-        while (groups * S < kSegmentTargetGroups && nc / (2 * S) >= kSegmentMinTiles) S *= 2;
-        if (S >= 2) {
-            const int seg_tiles = (nc + S - 1) / S;
-            S = (nc + seg_tiles - 1) / seg_tiles;
-            cut = segments_us(dtype, groups, S, seg_tiles);
-        }
-    }
+    const double cut = s.N != 128 ? best_segments(dtype, groups, nc, kSegmentMinTiles, &S) : 1e30;
     if (cut < whole && cut < staged) {
         *segments = S;
         return 2;
@@ -134,9 +141,14 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
                                        const float *A, const void *Bm, const void *Cm, const float *D, const float *init,
                                        const unsigned char *reset, void *y, float *final_states, float *seg_states,
                                        float *seg_decay, hipStream_t st) {
+    // (a prologue reads the true initial state, which a final state written over it -- a stream's prefix continued in place --
+    // could have replaced by then: those calls have the entering states worked out ahead as well)
+    const size_t state_floats = (size_t)s.B * s.H * s.P * s.N;
+    const bool in_place = init != nullptr && final_states != nullptr && init < final_states + state_floats && final_states < init + state_floats;
+    const bool passed = segments >= kPassMinSegments || in_place;
     if (dtype == 0)
         return launch_fused_scan_f32_segmented(s, segments, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states,
-                                               seg_decay, st);
+                                               seg_decay, passed, st);
     if (segments < 2 || fused_scan_waves(s, dtype) != 8 || s.N == 128) return hipErrorInvalidValue;
     ScanShape t = s;
     t.Q = kOnePassTile;
@@ -149,6 +161,10 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
     // the forward per segment; its prologue runs the recurrence over the segment states
     ScanShape f = s;
     f.seg_tiles = t.seg_tiles;
+    if (passed) {
+        e = launch_segment_passing(s, segments, seg_states, seg_decay, init, reset, st);
+        return e != hipSuccess ? e : launch_fused_scan(f, dtype, x, dt, A, Bm, Cm, D, seg_states, reset, y, final_states, st);
+    }
     f.seg_local = seg_states;
     f.seg_local_decay = seg_decay;
     return launch_fused_scan(f, dtype, x, dt, A, Bm, Cm, D, init, reset, y, final_states, st);

@@ -89,6 +89,10 @@ hipError_t launch_chunk_state_scan(const ScanShape &s, int dtype, const void *x,
 // a_end: the chunks' total log2-decays, sequence (b, h) chunk c at [((b * H + h) * nc + c) * a_stride]
 hipError_t launch_state_passing(const ScanShape &s, const float *states, const float *a_end, int a_stride, const float *init,
                                 float *prev, float *final_states, hipStream_t stream);
+// The same over the segments of a cut sequence, in place: seg_states [B, segments, H, P, N], what each adds from zero, become the
+// states entering them (from init, or zero); seg_decay [B, segments, H] their total decays.  fresh: the restart mask or NULL.
+hipError_t launch_segment_passing(const ScanShape &s, int segments, float *seg_states, const float *seg_decay, const float *init,
+                                  const unsigned char *fresh, hipStream_t stream);
 hipError_t launch_chunk_scan(const ScanShape &s, int dtype, const void *x, const void *Bm,
                              const void *Cm, const float *dtcs, const float *prev, const float *D,
                              void *y, hipStream_t stream);
@@ -114,7 +118,7 @@ int fused_scan_f32_tile();  // time steps per tile of the float one-pass kernel
 hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, const void *x, const void *dt, const float *A,
                                            const void *Bm, const void *Cm, const float *D, const float *init,
                                            const unsigned char *reset, void *y, float *final_states, float *seg_states,
-                                           float *seg_decay, hipStream_t st);
+                                           float *seg_decay, bool passed, hipStream_t st);
 // fused_scan_plan: which way a forward of this shape runs fastest by the library's cost estimates: 0 = the
 // staged kernels, 1 = the one-pass kernel, 2 = the one-pass kernel on *segments segments.
 int fused_scan_plan(const ScanShape &s, int dtype, int *segments);

@@ -81,16 +81,21 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(const T *__restrict__
 // state entering its run and writes the states entering its chunks from the registers.  So 64 chunks cost one trip to
 // memory (a thread per piece that walked the chunks eight at a time made a trip for every eight: 8 heads, state
 // 32 x 64: 4 sequences of 32 chunks 8.6 -> 5.5 us, 2 of 71 16.8 -> 9.1; 16 heads, 64 x 128, 4 of 16 chunks 12.6 -> 13.1).
-// a_end: alpha at the end of chunk c of sequence bh at [bh * nc + c] * a_stride.
+// The chunks' total decays: log2 (alpha at the chunk's end; LOG) or the factors themselves, chunk c of sequence (b, h) at
+// a.of[b * a.b + h * a.h + c * a.c].
 // prev may alias states: a thread reads its chunks before it writes them, and no other thread touches them;
 // final_states may alias init: it is written behind a barrier that all of the workgroup's reads of init precede.
 // ------------------------------------------------------------------------------------------
 constexpr int kPassSegs = 8, kPassPieces = 32;  // P * N / 4 is a multiple of 32 (P of 8, N of 16)
 
-template <int RUN>  // 1, 2, 4 or 8
-__global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(const float *states, const float *__restrict__ a_end,
-                                                                               int a_stride, const float *init, float *prev,
-                                                                               float *final_states, ScanShape s) {
+struct PassDecays {
+    const float *of;
+    long long b, h, c;
+};
+
+template <int RUN, bool LOG>  // RUN: 1, 2, 4 or 8
+__global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(const float *states, PassDecays a, const float *init,
+                                                                               float *prev, float *final_states, ScanShape s) {
     __shared__ float4 run_state[2][kPassSegs][kPassPieces];
     __shared__ float run_decay[2][kPassSegs];
     const int pn4 = s.P * s.N / 4, blocks = pn4 / kPassPieces;
@@ -100,7 +105,7 @@ __global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(c
     const size_t chunk_stride = (size_t)s.H * pn4;  // in float4
     const float4 *src = reinterpret_cast<const float4 *>(states) + ((size_t)b * s.nc * s.H + h) * pn4 + idx;
     float4 *dst = reinterpret_cast<float4 *>(prev) + ((size_t)b * s.nc * s.H + h) * pn4 + idx;
-    const float *ae = a_end + (size_t)bh * s.nc * a_stride;
+    const float *ae = a.of + b * a.b + h * a.h;
     const bool fresh = s.fresh != nullptr && s.fresh[(size_t)b * s.L] != 0;  // restarts before its first step
     float4 st = init && !fresh ? reinterpret_cast<const float4 *>(init)[(size_t)bh * pn4 + idx] : make_float4(0, 0, 0, 0);
     auto step = [](float4 &v, float dec, const float4 &add) {
@@ -117,13 +122,13 @@ __global__ __launch_bounds__(kPassSegs *kPassPieces) void state_passing_kernel(c
         for (int i = 0; i < RUN; ++i) {  // (past the sequence: read as the last chunk and not used)
             const int ci = min(c + i, s.nc - 1);
             sv[i] = src[(size_t)ci * chunk_stride];
-            dec[i] = ae[(size_t)ci * a_stride];
+            dec[i] = ae[(size_t)ci * a.c];
         }
         float4 local = make_float4(0, 0, 0, 0);
         float decay = 1.f;
 #pragma unroll
         for (int i = 0; i < RUN; ++i) {
-            dec[i] = exp2_hw(dec[i]);
+            if constexpr (LOG) dec[i] = exp2_hw(dec[i]);
             if (c + i < s.nc) {
                 step(local, dec[i], sv[i]);
                 decay *= dec[i];
@@ -342,17 +347,31 @@ hipError_t launch_chunk_cumsum(const ScanShape &s, int dtype, const void *dt, co
                  : cumsum_dispatch<float>(s, dt, A, reset, dtcs, st, mode, dt_len);
 }
 
-hipError_t launch_state_passing(const ScanShape &s, const float *states, const float *a_end, int a_stride, const float *init,
-                                float *prev, float *final_states, hipStream_t st) {
+template <bool LOG>
+static hipError_t pass_dispatch(const ScanShape &s, const float *states, const PassDecays &a, const float *init, float *prev,
+                                float *final_states, hipStream_t st) {
     const long long blocks = (long long)s.B * s.H * (s.P * s.N / 4 / kPassPieces);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks), block(kPassSegs * kPassPieces);
     // as short runs as cover the sequence in one round, where eight do
-    if (s.nc <= kPassSegs) state_passing_kernel<1><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
-    else if (s.nc <= 2 * kPassSegs) state_passing_kernel<2><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
-    else if (s.nc <= 4 * kPassSegs) state_passing_kernel<4><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
-    else state_passing_kernel<8><<<grid, block, 0, st>>>(states, a_end, a_stride, init, prev, final_states, s);
+    if (s.nc <= kPassSegs) state_passing_kernel<1, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
+    else if (s.nc <= 2 * kPassSegs) state_passing_kernel<2, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
+    else if (s.nc <= 4 * kPassSegs) state_passing_kernel<4, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
+    else state_passing_kernel<8, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
     return hipGetLastError();
+}
+
+hipError_t launch_state_passing(const ScanShape &s, const float *states, const float *a_end, int a_stride, const float *init,
+                                float *prev, float *final_states, hipStream_t st) {
+    return pass_dispatch<true>(s, states, PassDecays{a_end, (long long)s.H * s.nc * a_stride, (long long)s.nc * a_stride, a_stride}, init, prev, final_states, st);
+}
+
+hipError_t launch_segment_passing(const ScanShape &s, int segments, float *seg_states, const float *seg_decay, const float *init,
+                                  const unsigned char *fresh, hipStream_t st) {
+    ScanShape t = s;
+    t.nc = segments;  // (what stands in the last segment's place is read, and goes nowhere)
+    t.fresh = fresh;
+    return pass_dispatch<false>(t, seg_states, PassDecays{seg_decay, (long long)segments * s.H, 1, s.H}, init, seg_states, nullptr, st);
 }
 
 template <typename T, typename TO>
