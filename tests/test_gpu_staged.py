@@ -113,20 +113,26 @@ def test_state_passing_runs(nc):
         assert (fin.cpu().double() - st).abs().max() <= 1e-5 * st.abs().max()
 
 
-@pytest.mark.parametrize("batch,seqlen,dtype", [(24, 2100, "bf16"), (16, 4100, "bf16"), (90, 1030, "bf16"), (90, 2500, "bf16"), (20, 4000, "f32"),
-                                                (96, 1999, "f32"), (60, 1001, "f32")])
-def test_forward_on_segments(batch, seqlen, dtype):
+POLICY, LONG = (8, 32, 64, 1, 128), (16, 64, 128, 2, 256)  # heads, head dimension, state, groups, chunk
+
+
+@pytest.mark.parametrize("batch,seqlen,dtype,dims", [(24, 2100, "bf16", POLICY), (16, 4100, "bf16", POLICY), (90, 1030, "bf16", POLICY),
+                                                     (90, 2500, "bf16", POLICY), (20, 4000, "f32", POLICY), (96, 1999, "f32", POLICY),
+                                                     (60, 1001, "f32", POLICY), (4, 4000, "bf16", LONG), (12, 2060, "bf16", LONG),
+                                                     (7, 4097, "bf16", LONG), (30, 2500, "bf16", (4, 32, 128, 1, 64))])
+def test_forward_on_segments(batch, seqlen, dtype, dims):
     """Cuts into a few segments (states entering them worked out in the prologues), into eight and more (in a launch of their own) and
-    over two rounds of workgroups, with restarts, a row whose initial state is not read, and ragged last segments."""
-    w = Workload("segments", batch, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
-    assert ssd.chunk_scan_segments(batch, seqlen, 8, 32, 64, 1, 128, w.torch_dtype) > 1
+    over two rounds of workgroups, a 128-wide state (two waves per unit), with restarts, a row whose initial state is not read, and
+    ragged last segments."""
+    w = Workload("segments", batch, seqlen, *dims, dtype=dtype, init_std=0.5)
+    assert ssd.chunk_scan_segments(batch, seqlen, *dims, w.torch_dtype) > 1
     cpu = make_inputs(w, seed=seqlen)
     dev = to_dev(cpu)
     mask = torch.rand(batch, seqlen, generator=torch.Generator().manual_seed(5)) < 0.002
     mask[0, 0] = True
     dev["init"][0] = float("nan")
     rows = [0, batch // 2, batch - 1]
-    y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=128, initial_states=dev["init"],
+    y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=dims[4], initial_states=dev["init"],
                           reset=mask.cuda(), y_dtype=torch.float32)
     sub = {k: (v if k in ("A", "D") else v[rows].clone()) for k, v in cpu.items()}
     sub["init"][0] = 0.0

@@ -1,4 +1,4 @@
-// One-pass forward for batches too small to fill the chip with one workgroup per 8 units: the sequence is cut
+// One-pass forward for batches too small to fill the chip with one workgroup per 8 units (4 of a 128-wide state): the sequence is cut
 // into segments that different workgroups walk side by side.
 //   1. states only (no y, no C): what every segment adds to the state, from a zero state, and its total decay;
 //   2. the forward proper per segment; each workgroup first runs the recurrence over the states of the segments
@@ -25,45 +25,48 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // Estimates in microseconds, from measurements on MI355X, of the three ways a forward can run; `groups` workgroups fill a
 // CU each (eight units of 32 columns; four of a 128-wide state).  As used against measured:
 // staged kernels (every tile of 64 steps of every unit side by side): 8 heads of 32, state 64, 16 x 512 steps 18 / 17,
-// 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128, 8 x 1 000 55 / 47,
-// 8 x 4 000 189 / 172, 16 x 4 000 368 / 369; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000 63 / 67, 10 x 3 000 87 / 86.
+// 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128 (16 heads of 64),
+// 3 x 1 000 23 / 28, 8 x 1 000 49 / 47, 2 x 4 000 54 / 54, 8 x 4 000 174 / 172; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000 63 / 67, 10 x 3 000 87 / 86.
 double staged_us(const ScanShape &s, int dtype, long long groups) {
     const int full = dtype != 0 && s.N == 128 ? 4 : 8;
     const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
     if (dtype == 0) return 12.0 + 1310.0 * units;
-    return 10.0 + 518.0 * units * (s.N == 128 ? 1.4 : 1.0);
+    return s.N == 128 ? 6.0 + 650.0 * units + 0.13 * tiles_of(s) : 10.0 + 518.0 * units;
 }
 // the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
-// 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 4 000 277 / 266; float32 tiles of 32 steps, 70 x 100 26 / 27
+// 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000 143 / 138; float32 tiles of 32 steps, 70 x 100 26 / 27
 double whole_us(const ScanShape &s, int dtype, long long groups) {
     const double rounds = (double)((groups + 255) / 256);
     if (dtype == 0) return 5.0 + 5.3 * float_tiles_of(s) * rounds;
     const double fill = groups < 256 ? (double)groups / 256.0 : 1.0;
-    return 6.0 + tiles_of(s) * rounds * (s.N == 128 ? 4.1 + 0.5 * fill : 4.1 + 1.5 * fill);
+    return 6.0 + tiles_of(s) * rounds * (s.N == 128 ? 3.9 + 0.7 * fill * fill : 4.1 + 1.5 * fill);
 }
 // ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 40 / 36, 90 x 1 024
 // on 2 65 / 66, 61 x 3 999 on 4 117 / 120, 48 x 4 096 on 5 101 / 99, 24 x 4 096 on 8 69 / 71, 90 x 4 096 on 5 (two rounds) 198 / 198;
-// float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12 98 / 105
-double segments_us(int dtype, long long groups, int segments, int seg_tiles) {
+// float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12 98 / 105; state 128 (two waves per unit, the
+// entering states always in a launch of their own), 2 x 4 000 on 13 52 / 48, 4 x 4 000 on 8 68 / 69, 8 x 4 000 on 4 121 / 119, 16 x 2 000
+// on 2 130 / 128, 4 x 16 384 on 8 212 / 218, 12 x 4 000 on 8 (three rounds) 209 / 193
+double segments_us(const ScanShape &s, int dtype, long long groups, int segments, int seg_tiles) {
     const double rounds = (double)((groups * segments + 255) / 256), tiles = seg_tiles * rounds, more = rounds - 1.0;
+    if (dtype != 0 && s.N == 128) return 16.0 + 0.14 * groups + 6.0 * tiles + 18.0 * more;
     if (dtype == 0) return 6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more;
     return 12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more;
 }
 // the fastest cut of nc tiles into segments of min_tiles or more, by that estimate; in bf16 a power of two unless another is clearly
 // faster (the estimate is good to a few per cent, and programs size and compare by the number of segments)
-double best_segments(int dtype, long long groups, int nc, int min_tiles, int *segments) {
+double best_segments(const ScanShape &s, int dtype, long long groups, int nc, int min_tiles, int *segments) {
     double best = 1e30;
     *segments = 1;
     for (int S = 2; nc >= S * min_tiles && groups * S <= kSegmentMaxGroups; ++S) {
         const int seg_tiles = (nc + S - 1) / S;
         if ((nc + seg_tiles - 1) / seg_tiles != S) continue;
-        const double cost = segments_us(dtype, groups, S, seg_tiles) * (dtype == 0 || (S & (S - 1)) == 0 ? 1.0 : 1.07);
+        const double cost = segments_us(s, dtype, groups, S, seg_tiles) * (dtype == 0 || (S & (S - 1)) == 0 ? 1.0 : 1.07);
         if (cost < best) {
             best = cost;
             *segments = S;
         }
     }
-    return *segments > 1 ? segments_us(dtype, groups, *segments, (nc + *segments - 1) / *segments) : best;
+    return *segments > 1 ? segments_us(s, dtype, groups, *segments, (nc + *segments - 1) / *segments) : best;
 }
 
 }  // namespace
@@ -79,7 +82,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
         const int nc = float_tiles_of(s);
         const double staged = staged_us(s, 0, groups), whole = whole_us(s, 0, groups);
         int S;
-        const double cut = best_segments(0, groups, nc, 2 * kSegmentMinTiles, &S);
+        const double cut = best_segments(s, 0, groups, nc, 2 * kSegmentMinTiles, &S);
         if (cut < whole && cut < staged) {
             *segments = S;
             return 2;
@@ -106,7 +109,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     const int nc = tiles_of(s);
     const double staged = staged_us(s, dtype, groups), whole = whole_us(s, dtype, groups);
     int S = 1;
-    const double cut = s.N != 128 ? best_segments(dtype, groups, nc, kSegmentMinTiles, &S) : 1e30;
+    const double cut = best_segments(s, dtype, groups, nc, kSegmentMinTiles, &S);
     if (cut < whole && cut < staged) {
         *segments = S;
         return 2;
@@ -133,7 +136,7 @@ int fused_scan_tail_rows(const ScanShape &s, int dtype) {
     // the remainder as its own batch against one more round
     const int nc = dtype == 0 ? float_tiles_of(s) : tiles_of(s);
     const double round = whole_us(s, dtype, 256) - whole_us(s, dtype, 0);
-    const double cost = tail_plan == 2 ? segments_us(dtype, rest, segments, (nc + segments - 1) / segments) : staged_us(tail, dtype, rest);
+    const double cost = tail_plan == 2 ? segments_us(s, dtype, rest, segments, (nc + segments - 1) / segments) : staged_us(tail, dtype, rest);
     return cost < round ? tail.B : 0;
 }
 
@@ -149,12 +152,14 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
     if (dtype == 0)
         return launch_fused_scan_f32_segmented(s, segments, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states,
                                                seg_decay, passed, st);
-    if (segments < 2 || fused_scan_waves(s, dtype) != 8 || s.N == 128) return hipErrorInvalidValue;
+    if (segments < 2 || fused_scan_waves(s, dtype) != (s.N == 128 ? 4 : 8)) return hipErrorInvalidValue;
     ScanShape t = s;
     t.Q = kOnePassTile;
     t.nc = tiles_of(s);
     t.seg_tiles = (t.nc + segments - 1) / segments;
     if ((t.nc + t.seg_tiles - 1) / t.seg_tiles != segments) return hipErrorInvalidValue;
+    if (s.N == 128)
+        return launch_fused_scan_wide_segmented(t, dtype, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states, seg_decay, st);
     hipError_t e = t.N == 32 ? fused_launch_states<2, kOnePassTile / 32, 8>(t, x, dt, A, Bm, nullptr, reset, seg_states, seg_decay, st)
                              : fused_launch_states<4, kOnePassTile / 32, 8>(t, x, dt, A, Bm, nullptr, reset, seg_states, seg_decay, st);
     if (e != hipSuccess) return e;

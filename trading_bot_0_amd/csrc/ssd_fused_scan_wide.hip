@@ -18,6 +18,11 @@
 // sharing the B and C tiles of their (batch, group) as before.  The scan of dt*A and the decay tables of a unit are
 // computed by its first wave for both (250 vector instructions, about what the second wave's extra score block costs).
 //
+// A batch too small to fill the chip runs on segments of the sequence: the states each segment adds (an instance without C, scores and
+// outputs: 124 registers), the states entering them (state_passing over the segments), the forward from those.  16 heads of 64 in 2
+// groups, us against the staged kernels (or the uncut walk): 2 x 4 000 48 (54), 4 x 4 000 69 (100), 8 x 4 000 119 (172), 4 x 16 384 218
+// (357), 12 x 16 384 637 (978, uncut).
+//
 // Everything else -- tiling of time by 64 steps whatever chunk length the caller names, the separable decay factors
 // with the exact path for blocks that decay by more than 2^-120, hi + lo operands for everything the kernel
 // manufactures, restarts as a drop of the cumulative log-decay, ragged last tiles, swizzled LDS tiles read with the
@@ -42,12 +47,16 @@ constexpr size_t kWideLdsBytes = (size_t)2 * kWideQ * kWideN * 2 + (size_t)kWide
                                  (size_t)kWideUnits * 2 * 32 * 32 * 4 + (size_t)kWideUnits * kWideTableFloats * 4 +
                                  (size_t)3 * 32 * 32 * 4;
 
-template <typename TO>
+// KIND 0: the whole sequence.  1: a segment of s.seg_tiles tiles, from a state of its own (init [B, S, H, P, N]).  2: the same without
+// outputs: what every segment but the last adds to the state from zero, into final_states [B, S, H, P, N], and its total decay,
+// into seg_decay [B, S, H] (no C is read and no scores are formed).
+template <typename TO, int KIND>
 __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
     const __bf16 *__restrict__ x, const __bf16 *__restrict__ dt, const float *__restrict__ A,
     const __bf16 *__restrict__ Bm, const __bf16 *__restrict__ Cm, const float *__restrict__ D, const float *init,
-    const unsigned char *__restrict__ reset, TO *__restrict__ y, float *final_states, ScanShape s) {
+    const unsigned char *__restrict__ reset, TO *__restrict__ y, float *final_states, float *seg_decay, ScanShape s) {
     using T = __bf16;
+    constexpr bool STATES = KIND == 2;
     constexpr int N = kWideN, NK = kWideNK, Q = kWideQ, QB = kWideQB, nthr = 64 * kWideWaves, UNITS = kWideUnits;
     constexpr int HNB = 2;                     // 32-column blocks of this wave's half of the state
     constexpr int BPR = N / 8;                 // 16-byte pieces per B (or C) row
@@ -80,7 +89,11 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
     // ---- which units this workgroup owns ----
     const int PBn = s.P / 32, HG = s.H / s.G;
     const int UW = (HG * PBn) / UNITS;  // workgroups per (batch, group)
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int slot = xcd_remap(blockIdx.x, gridDim.x);
+    const int S = KIND == 0 ? 1 : (s.nc + s.seg_tiles - 1) / s.seg_tiles, seg = KIND == 0 ? 0 : slot % S;
+    const int logical = KIND == 0 ? slot : slot / S;
+    const int c_first = KIND == 0 ? 0 : seg * s.seg_tiles, c_end = KIND == 0 ? s.nc : min(s.nc, c_first + s.seg_tiles);
+    if (STATES && seg == S - 1) return;  // (nobody asks what the last segment adds)
     const int b = logical / (s.G * UW), g = (logical / UW) % s.G;
     const int unit0 = (logical % UW) * UNITS, unit = unit0 + ul;
     const int h = g * HG + unit / PBn, pb = unit % PBn;
@@ -118,7 +131,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
 #pragma unroll
             for (int u = 0; u < UBC; ++u) {
                 bq[u] = *reinterpret_cast<const uint4 *>(bp + (size_t)u * BRP * s.G * N + bc_off0);
-                cq[u] = *reinterpret_cast<const uint4 *>(cp + (size_t)u * BRP * s.G * N + bc_off0);
+                if constexpr (!STATES) cq[u] = *reinterpret_cast<const uint4 *>(cp + (size_t)u * BRP * s.G * N + bc_off0);
             }
 #pragma unroll
             for (int u = 0; u < UX; ++u) xq[u] = *reinterpret_cast<const uint4 *>(xp + (size_t)u * XRP * HP + x_off0);
@@ -129,7 +142,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
             for (int u = 0; u < UBC; ++u) {
                 const bool ok = bc_row0 + u * BRP < rows;
                 bq[u] = ld16(bp + (size_t)u * BRP * s.G * N + bc_off0, ok);
-                cq[u] = ld16(cp + (size_t)u * BRP * s.G * N + bc_off0, ok);
+                if constexpr (!STATES) cq[u] = ld16(cp + (size_t)u * BRP * s.G * N + bc_off0, ok);
             }
 #pragma unroll
             for (int u = 0; u < UX; ++u) xq[u] = ld16(xp + (size_t)u * XRP * HP + x_off0, x_row0 + u * XRP < rows);
@@ -142,8 +155,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
     // ---- this wave's half of the unit's running state: st[j][v] = H[p = lane % 32, n = 32 (2 role + j) + 8 (v/4) +
     // 4 (lane / 32) + v%4] ----
     f32x16 st[HNB];
-    const bool fresh = rsb != nullptr && rsb[0] != 0;  // a restart before the first step: the initial state is not read
-    prefetch(0);
+    const bool fresh = rsb != nullptr && seg == 0 && rsb[0] != 0;  // a restart before the first step: the initial state is not read
+    prefetch(c_first);
     const size_t lane_off = (size_t)(pb * 32 + (lane0 & 31)) * N + 64 * role + 4 * (lane0 >> 5);
     {
         float4 iq[HNB][4];
@@ -152,8 +165,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) iq[j][gq] = make_float4(0, 0, 0, 0);
         }
-        if (init != nullptr && !fresh) {  // (one uniform branch around all of the state's loads)
-            const float *ib = init + ((size_t)b * s.H + h) * s.P * N + lane_off;
+        if (!STATES && init != nullptr && !fresh) {  // (one uniform branch around all of the state's loads)
+            const float *ib = init + (((size_t)b * S + seg) * s.H + h) * s.P * N + lane_off;
 #pragma unroll
             for (int j = 0; j < HNB; ++j) {
 #pragma unroll
@@ -178,7 +191,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
     // along the loop's own path, where they are older than the tile's stores of y (which the wave need not see
     // acknowledged), not along the prologue's, where they are the youngest requests.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    for (int c = 0; c < s.nc; ++c) {
+    float seg_total = 1.f;
+    for (int c = c_first; c < c_end; ++c) {
         const int t0 = c * Q;
         const int rows = min(Q, s.L - t0);
         block_sync_lds();  // every wave is done reading the previous tile's tiles and operand fragments
@@ -207,8 +221,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
         for (int u = 0; u < UBC; ++u) {
             *reinterpret_cast<uint2 *>(Bs + bw[0] + u * BRP * N) = swap ? make_uint2(bq[u].z, bq[u].w) : make_uint2(bq[u].x, bq[u].y);
             *reinterpret_cast<uint2 *>(Bs + bw[1] + u * BRP * N) = swap ? make_uint2(bq[u].x, bq[u].y) : make_uint2(bq[u].z, bq[u].w);
-            *reinterpret_cast<uint2 *>(Cs + bw[0] + u * BRP * N) = swap ? make_uint2(cq[u].z, cq[u].w) : make_uint2(cq[u].x, cq[u].y);
-            *reinterpret_cast<uint2 *>(Cs + bw[1] + u * BRP * N) = swap ? make_uint2(cq[u].x, cq[u].y) : make_uint2(cq[u].z, cq[u].w);
+            if constexpr (!STATES) {
+                *reinterpret_cast<uint2 *>(Cs + bw[0] + u * BRP * N) = swap ? make_uint2(cq[u].z, cq[u].w) : make_uint2(cq[u].x, cq[u].y);
+                *reinterpret_cast<uint2 *>(Cs + bw[1] + u * BRP * N) = swap ? make_uint2(cq[u].x, cq[u].y) : make_uint2(cq[u].z, cq[u].w);
+            }
         }
 #pragma unroll
         for (int u = 0; u < UX; ++u) {
@@ -251,7 +267,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
         const float a_end = blk_s[4];  // exp2(alpha[Q-1])
         // ---- the tile's scores, once per workgroup: block g = sb + lb, (0,0), (0,1), (1,1), by the first waves of three
         // units (which have one score block to apply in phase 1 where the second waves have two) ----
-        if (wave < 3) {
+        if (!STATES && wave < 3) {
             // (the wave index hidden from the compiler: it would keep these sixteen addresses, which differ from the
             // ones every wave uses by a wave-uniform offset only, in registers of their own across the tile loop)
             int pw = wave;
@@ -268,7 +284,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
         // the next tile's inputs: requested here, in flight during both phases, stored to LDS at the top of the next tile
-        if (c + 1 < s.nc) prefetch(c + 1);
+        if (c + 1 < c_end) prefetch(c + 1);
         __builtin_amdgcn_sched_barrier(0);  // (left alone, the scheduler moves the loads down to where their values are used)
 
         // ---- phase 1: the outputs of this wave's block of 32 timesteps ----
@@ -407,13 +423,17 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
             const int yrow = t0 + l;
             store_column_buffer<TO>(ybuf, (unsigned)yrow * (unsigned)(HP * sizeof(TO)) + ycol_bytes, o, half, l < rows);
         };
-        if (role == 0)
-            phase1(std::integral_constant<int, 0>{});
-        else
-            phase1(std::integral_constant<int, 1>{});
+        if constexpr (!STATES) {
+            if (role == 0)
+                phase1(std::integral_constant<int, 0>{});
+            else
+                phase1(std::integral_constant<int, 1>{});
+        }
 
         // ---- phase 2: this half of the state leaving the tile ----
-        if (c + 1 == s.nc && final_states == nullptr) break;  // nobody reads the state the last tile leaves
+        // nobody reads the state the last tile leaves (a segment's, unless it is the sequence's last)
+        if (!STATES && c + 1 == c_end && (final_states == nullptr || seg != S - 1)) break;
+        seg_total *= a_end;
 #pragma unroll
         for (int j = 0; j < HNB; ++j) st[j] = st[j] * a_end;
         int xo[2][2], bo[2][2][HNB];
@@ -456,8 +476,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
         }
     }
 
-    if (final_states != nullptr) {
-        float *fb = final_states + ((size_t)b * s.H + h) * s.P * N + lane_off;
+    if (STATES && pb == 0 && role == 0 && lane0 == 0) seg_decay[((size_t)b * S + seg) * s.H + h] = seg_total;
+    if (STATES || (final_states != nullptr && seg == S - 1)) {
+        float *fb = final_states + ((STATES ? (size_t)b * S + seg : (size_t)b) * s.H + h) * s.P * N + lane_off;
 #pragma unroll
         for (int j = 0; j < HNB; ++j) {
 #pragma unroll
@@ -470,7 +491,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
 
 }  // namespace
 
-// Whether the two-waves-per-unit kernel takes the shape: a 128-wide state, units in fours, forward in time, uncut.
+// Whether the two-waves-per-unit kernel takes the shape: a 128-wide state, units in fours, forward in time, uncut (launch_fused_scan_wide)
+// or on segments (launch_fused_scan_wide_segmented).
 bool fused_scan_wide_supported(const ScanShape &s) {
     return s.N == kWideN && s.P % 32 == 0 && ((s.H / s.G) * (s.P / 32)) % kWideUnits == 0 && s.mode == 0 && s.x_groups == 0 &&
            s.seg_tiles == 0 && s.seg_local == nullptr && (long long)s.L * s.H * s.P * 4 < (1LL << 31);
@@ -485,11 +507,37 @@ hipError_t launch_fused_scan_wide(const ScanShape &s, int dtype, const void *x, 
     const __bf16 *xx = static_cast<const __bf16 *>(x), *dd = static_cast<const __bf16 *>(dt);
     const __bf16 *bb = static_cast<const __bf16 *>(Bm), *cc = static_cast<const __bf16 *>(Cm);
     if (dtype == 2)
-        fused_scan_wide_kernel<float><<<dim3(grid), dim3(64 * kWideWaves), 0, st>>>(xx, dd, A, bb, cc, D, init, reset,
-                                                                                   static_cast<float *>(y), final_states, s);
+        fused_scan_wide_kernel<float, 0><<<dim3(grid), dim3(64 * kWideWaves), 0, st>>>(xx, dd, A, bb, cc, D, init, reset,
+                                                                                   static_cast<float *>(y), final_states, nullptr, s);
     else
-        fused_scan_wide_kernel<__bf16><<<dim3(grid), dim3(64 * kWideWaves), 0, st>>>(xx, dd, A, bb, cc, D, init, reset,
-                                                                                    static_cast<__bf16 *>(y), final_states, s);
+        fused_scan_wide_kernel<__bf16, 0><<<dim3(grid), dim3(64 * kWideWaves), 0, st>>>(xx, dd, A, bb, cc, D, init, reset,
+                                                                                    static_cast<__bf16 *>(y), final_states, nullptr, s);
+    return hipGetLastError();
+}
+
+// On segments of t.seg_tiles tiles: what each adds to the state, the states entering them (by the recurrence over the segments), the
+// forward from those.
+hipError_t launch_fused_scan_wide_segmented(const ScanShape &t, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
+                                            const void *Cm, const float *D, const float *init, const unsigned char *reset, void *y,
+                                            float *final_states, float *seg_states, float *seg_decay, hipStream_t st) {
+    ScanShape s = t;
+    s.seg_tiles = 0;
+    const int segments = scan_segments(t);
+    if (!fused_scan_wide_supported(s) || t.Q != kWideQ || t.nc != (t.L + kWideQ - 1) / kWideQ || segments < 2) return hipErrorInvalidValue;
+    const int grid = t.B * t.G * (((t.H / t.G) * (t.P / 32)) / kWideUnits) * segments;
+    const dim3 block(64 * kWideWaves);
+    const __bf16 *xx = static_cast<const __bf16 *>(x), *dd = static_cast<const __bf16 *>(dt);
+    const __bf16 *bb = static_cast<const __bf16 *>(Bm), *cc = static_cast<const __bf16 *>(Cm);
+    fused_scan_wide_kernel<__bf16, 2><<<dim3(grid), block, 0, st>>>(xx, dd, A, bb, bb, nullptr, nullptr, reset, nullptr, seg_states, seg_decay, t);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = launch_segment_passing(t, segments, seg_states, seg_decay, init, reset, st);
+    if (e != hipSuccess) return e;
+    if (dtype == 2)
+        fused_scan_wide_kernel<float, 1><<<dim3(grid), block, 0, st>>>(xx, dd, A, bb, cc, D, seg_states, reset, static_cast<float *>(y),
+                                                                      final_states, nullptr, t);
+    else
+        fused_scan_wide_kernel<__bf16, 1><<<dim3(grid), block, 0, st>>>(xx, dd, A, bb, cc, D, seg_states, reset, static_cast<__bf16 *>(y),
+                                                                       final_states, nullptr, t);
     return hipGetLastError();
 }
 

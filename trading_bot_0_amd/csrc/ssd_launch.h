@@ -129,6 +129,10 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
                                        const float *A, const void *Bm, const void *Cm, const float *D, const float *init,
                                        const unsigned char *reset, void *y, float *final_states, float *seg_states,
                                        float *seg_decay, hipStream_t stream);
+// ... of a 128-wide state, on the kernel of two waves per unit: s.Q, s.nc and s.seg_tiles are that kernel's own tiling of time.
+hipError_t launch_fused_scan_wide_segmented(const ScanShape &s, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
+                                            const void *Cm, const float *D, const float *init, const unsigned char *reset, void *y,
+                                            float *final_states, float *seg_states, float *seg_decay, hipStream_t stream);
 hipError_t launch_step(const StepShape &s, int dtype, float *state, const void *x, const void *dt,
                        const float *A, const void *Bm, const void *Cm, const float *D, void *y,
                        hipStream_t stream);
