@@ -118,7 +118,7 @@ POLICY, LONG = (8, 32, 64, 1, 128), (16, 64, 128, 2, 256)  # heads, head dimensi
 
 @pytest.mark.parametrize("batch,seqlen,dtype,dims", [(24, 2100, "bf16", POLICY), (16, 4100, "bf16", POLICY), (90, 1030, "bf16", POLICY),
                                                      (90, 2500, "bf16", POLICY), (20, 4000, "f32", POLICY), (96, 1999, "f32", POLICY),
-                                                     (60, 1001, "f32", POLICY), (4, 4000, "bf16", LONG), (12, 2060, "bf16", LONG),
+                                                     (60, 1001, "f32", POLICY), (4, 4000, "bf16", LONG), (8, 2060, "bf16", LONG),
                                                      (7, 4097, "bf16", LONG), (30, 2500, "bf16", (4, 32, 128, 1, 64))])
 def test_forward_on_segments(batch, seqlen, dtype, dims):
     """Cuts into a few segments (states entering them worked out in the prologues), into eight and more (in a launch of their own) and

@@ -424,7 +424,9 @@ __device__ inline void split_pair(float a0, float f0, float a1, float f1, unsign
 // select that form, so it is written out; and since it does not look inside such a block, the wait the hardware needs
 // between a dot product and the next instruction that reads its result (three wait states, which the compiler inserts
 // by itself behind the two-operand form) stands at the end of the block, behind eight independent products.
-__device__ inline void split8_keep(const float (&a)[8], unsigned (&hi)[4], unsigned (&lo)[4]) {
+// rest, where given: the third bf16 term, what hi and lo leave of the value.
+__device__ inline void split8_keep(const float (&a)[8], unsigned (&hi)[4], unsigned (&lo)[4], unsigned (*rest)[4] = nullptr) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     unsigned first = 0x0000bf80u, second = 0xbf800000u;
     asm("" : "+s"(first));
     asm("" : "+s"(second));
@@ -447,6 +449,15 @@ __device__ inline void split8_keep(const float (&a)[8], unsigned (&hi)[4], unsig
     lo[1] = pack_bf16x2(l2, l3);
     lo[2] = pack_bf16x2(l4, l5);
     lo[3] = pack_bf16x2(l6, l7);
+    if (rest != nullptr) {
+        const float l[8] = {l0, l1, l2, l3, l4, l5, l6, l7};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bf16x2 p = __builtin_bit_cast(bf16x2, lo[k]);
+            (*rest)[k] = pack_bf16x2(__builtin_amdgcn_fdot2_f32_bf16(p, __builtin_bit_cast(bf16x2, first), l[2 * k], false),
+                                     __builtin_amdgcn_fdot2_f32_bf16(p, __builtin_bit_cast(bf16x2, second), l[2 * k + 1], false));
+        }
+    }
 }
 struct FragBits {  // an operand fragment as four packed pairs
     unsigned u[4];

@@ -44,11 +44,11 @@ double whole_us(const ScanShape &s, int dtype, long long groups) {
 // ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 40 / 36, 90 x 1 024
 // on 2 65 / 66, 61 x 3 999 on 4 117 / 120, 48 x 4 096 on 5 101 / 99, 24 x 4 096 on 8 69 / 71, 90 x 4 096 on 5 (two rounds) 198 / 198;
 // float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12 98 / 105; state 128 (two waves per unit, the
-// entering states always in a launch of their own), 2 x 4 000 on 13 52 / 48, 4 x 4 000 on 8 68 / 69, 8 x 4 000 on 4 121 / 119, 16 x 2 000
-// on 2 130 / 128, 4 x 16 384 on 8 212 / 218, 12 x 4 000 on 8 (three rounds) 209 / 193
+// entering states always in a launch of their own), 2 x 4 000 on 13 49 / 49, 4 x 4 000 on 8 69 / 70, 8 x 4 000 on 4 123 / 122, 16 x 2 000
+// on 2 132 / 131, 4 x 16 384 on 8 216 / 220, 12 x 4 000 on 8 (three rounds) 212 / 196
 double segments_us(const ScanShape &s, int dtype, long long groups, int segments, int seg_tiles) {
     const double rounds = (double)((groups * segments + 255) / 256), tiles = seg_tiles * rounds, more = rounds - 1.0;
-    if (dtype != 0 && s.N == 128) return 16.0 + 0.14 * groups + 6.0 * tiles + 18.0 * more;
+    if (dtype != 0 && s.N == 128) return 16.0 + 0.14 * groups + 6.1 * tiles + 18.0 * more;
     if (dtype == 0) return 6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more;
     return 12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more;
 }

@@ -20,8 +20,8 @@
 //
 // A batch too small to fill the chip runs on segments of the sequence: the states each segment adds (an instance without C, scores and
 // outputs: 124 registers), the states entering them (state_passing over the segments), the forward from those.  16 heads of 64 in 2
-// groups, us against the staged kernels (or the uncut walk): 2 x 4 000 48 (54), 4 x 4 000 69 (100), 8 x 4 000 119 (172), 4 x 16 384 218
-// (357), 12 x 16 384 637 (978, uncut).
+// groups, us against the staged kernels (or the uncut walk): 2 x 4 000 49 (54), 4 x 4 000 70 (98), 8 x 4 000 122 (172), 4 x 16 384 220
+// (357), 12 x 16 384 662 (978, uncut).
 //
 // Everything else -- tiling of time by 64 steps whatever chunk length the caller names, the separable decay factors
 // with the exact path for blocks that decay by more than 2^-120, hi + lo operands for everything the kernel
@@ -258,10 +258,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
             dt_s[l] = dtv;
             w_s[l] = exp2_hw(fminf(alpha_diff(endh[QB - 1], endl[QB - 1], hi, lo), 0.f)) * dtv;
             const float rh = blk >= 1 ? refh[1] : refh[0], rl = blk >= 1 ? refl[1] : refl[0];
-            E_s[l] = exp2_hw(fminf(alpha_diff(hi, lo, rh, rl), 0.f));
+            if constexpr (!STATES) {
+                E_s[l] = exp2_hw(fminf(alpha_diff(hi, lo, rh, rl), 0.f));
 #pragma unroll
-            for (int lb = 0; lb < QB; ++lb)
-                if (lb >= blk) F_s[lb * Q + l] = exp2_hw(fminf(alpha_diff(refh[lb], refl[lb], hi, lo), 126.f)) * dtv;
+                for (int lb = 0; lb < QB; ++lb)
+                    if (lb >= blk) F_s[lb * Q + l] = exp2_hw(fminf(alpha_diff(refh[lb], refl[lb], hi, lo), 126.f)) * dtv;
+            }
         }
         block_sync_lds();  // tiles, operand fragments and tables are visible
         const float a_end = blk_s[4];  // exp2(alpha[Q-1])
@@ -303,16 +305,24 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void fused_scan_wide_kernel(
             for (int k4 = 0; k4 < NK / 2; ++k4) {
                 const int col = 16 * (4 * role + k4) + 4 * half;
                 const Frag<T> Cown = BT::split_frag(Cs, l, col), Coth = BT::split_frag(Cs, (1 - lb) * 32 + r, col);
-                FragBits fh, fl;
+                FragBits fh, fl, fr;
                 float sv[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) sv[i] = st[k4 / 2][8 * (k4 % 2) + i];
-                split8_keep(sv, fh.u, fl.u);
+                split8_keep(sv, fh.u, fl.u, KIND == 1 ? &fr.u : nullptr);
                 const Frag<T> Hh = fh.frag(), Hl = fl.frag();
                 acc = mma32(Hh, Cown, acc);
                 oth = mma32(Hh, Coth, oth);
                 acc = mma32(Hl, Cown, acc);
                 oth = mma32(Hl, Coth, oth);
+                // on segments the state goes through a third term: more of what the tiles read reaches them through the state than
+                // on the chunks of 128 or 256 steps these batches would take, with one rounding of 2^-17 more (steep decays, against
+                // float64: 1.12e-6 of y with two terms, 0.90e-6 with three, 1.01e-6 on chunks of 256; 119, 122 and 172 us at 8 x 4 000)
+                if constexpr (KIND == 1) {
+                    const Frag<T> Hr = fr.frag();
+                    acc = mma32(Hr, Cown, acc);
+                    oth = mma32(Hr, Coth, oth);
+                }
             }
             {
                 float *pd = part_unit + role * 1024 + lane * 4;
