@@ -147,7 +147,8 @@ int ssd_chunk_scan_reset_fwd(const ssd_dims *dims, int dtype, const void *x, con
  * segmented paths need comes from an array of SSD_STATIC_SCRATCH_BYTES (64 MiB) that is part of the library's device
  * code (each GPU the library runs on holds it until the process ends).  No counterpart in the reference.  Same
  * arguments and results as ssd_chunk_scan_reset_fwd minus the workspace.  SSD_ERR_WORKSPACE when the scratch that the
- * shape's own path uses exceeds the array: all of ssd_workspace_bytes on the staged kernels, the segment states and
+ * shape's own path uses exceeds the array and the one-pass kernel, which then runs it as one launch, does not take the
+ * shape: all of ssd_workspace_bytes on the staged kernels, the segment states and
  * decays (batch * segments * nheads * (headdim * dstate + 1) floats) when the sequences run cut into segments
  * (ssd_chunk_scan_segments > 1), nothing when the shape runs as one launch of the one-pass kernel
  * (ssd_chunk_scan_is_onepass), at any size.  Calls no hipMalloc/hipFree or any other allocating

@@ -1,6 +1,8 @@
 """The staged forward in two or three launches (stages 2 and 4 work out the decays themselves; stage 4 runs the recurrence over
 the chunks where they are few) at the edges of its dispatch, against the float64 sequential oracle and against the stages
 called one by one, which share the same arithmetic up to the order of float32 sums."""
+from ctypes import byref
+
 import pytest
 import torch
 
@@ -11,6 +13,7 @@ from _util import assert_close, check_y, np64, oracle_scan, to_dev
 from oracle import c_oracle
 
 pytestmark = pytest.mark.gpu
+POLICY, LONG = (8, 32, 64, 1, 128), (16, 64, 128, 2, 256)  # heads, head dimension, state, groups, chunk
 
 
 # (batch, seqlen, heads, headdim, dstate, groups, chunk): one chunk; a batch of the recurrence and one over (2, 3, 4, 5 chunks);
@@ -72,18 +75,21 @@ def c_oracle_reset(cpu, mask):
     return y, fin
 
 
-@pytest.mark.parametrize("batch,seqlen", [(3, 100), (3, 400), (3, 2000), (90, 1024), (60, 1000)])
+@pytest.mark.parametrize("batch,seqlen,dims", [(3, 100, POLICY), (3, 400, POLICY), (3, 2000, POLICY), (90, 1024, POLICY), (60, 1000, POLICY),
+                                               (8, 2060, LONG)])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-def test_final_state_written_over_the_initial_state(batch, seqlen, dtype):
+def test_final_state_written_over_the_initial_state(batch, seqlen, dims, dtype):
     """A stream's prefix that continues a state in place: the same buffer as initial and final state, at lengths whose separate
     buffers would take the recurrence inside stage 4, or on segments, inside their prologues."""
-    w = Workload("inplace", batch, seqlen, 8, 32, 64, 1, 128, dtype=dtype, init_std=0.5)
+    if dtype == "f32" and dims is LONG:
+        dims = (16, 64, 128, 2, 64)   # (float32 tiles of the largest head sizes do not fit the LDS)
+    w = Workload("inplace", batch, seqlen, *dims, dtype=dtype, init_std=0.5)
     cpu = make_inputs(w, seed=3)
     dev = to_dev(cpu)
     yr, fr = oracle_scan(cpu)
     for _ in range(4):
         state = dev["init"].clone()
-        y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=128, initial_states=state,
+        y, f = ssd_chunk_scan(dev["x"], dev["dt"], dev["A"], dev["B"], dev["C"], dev["D"], chunk=dims[4], initial_states=state,
                               final_out=state, y_dtype=torch.float32)
         assert f.data_ptr() == state.data_ptr()
         assert_close(y, yr, w.torch_dtype, "y")
@@ -113,7 +119,24 @@ def test_state_passing_runs(nc):
         assert (fin.cpu().double() - st).abs().max() <= 1e-5 * st.abs().max()
 
 
-POLICY, LONG = (8, 32, 64, 1, 128), (16, 64, 128, 2, 256)  # heads, head dimension, state, groups, chunk
+@pytest.mark.parametrize("batch,seqlen,dims", [(44, 600, (16, 64, 128, 2, 64)), (300, 300, (8, 32, 64, 1, 64))])
+def test_forward_without_a_workspace_past_the_scratch_array(batch, seqlen, dims):
+    """Shapes whose own path (whole rounds of workgroups and a rest on the staged kernels) needs more than the library's scratch array:
+    one launch of the one-pass kernel, and so its bits."""
+    w = Workload("noalloc", batch, seqlen, *dims, init_std=0.5)
+    assert not ssd.chunk_scan_is_onepass(batch, seqlen, *dims, w.torch_dtype)
+    assert ssd.workspace_bytes(batch, seqlen, *dims) > 64 << 20
+    i = make_inputs(w, seed=7, device="cuda")
+    lib, d, code = ssd.load_library(), ssd.SsdDims(batch, seqlen, *dims), ssd.SSD_DTYPE_BF16
+    got = []
+    for entry in (lib.ssd_chunk_scan_noalloc_fwd, lib.ssd_chunk_scan_onepass_fwd):
+        y, fin = torch.empty_like(i["x"]), torch.empty_like(i["init"])
+        rc = entry(byref(d), code, i["x"].data_ptr(), i["dt"].data_ptr(), i["A"].data_ptr(), i["B"].data_ptr(), i["C"].data_ptr(),
+                   i["D"].data_ptr(), i["init"].data_ptr(), None, y.data_ptr(), fin.data_ptr(), None)
+        assert rc == 0, ssd.last_error(lib)
+        got.append((y, fin))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
 @pytest.mark.parametrize("batch,seqlen,dtype,dims", [(24, 2100, "bf16", POLICY), (16, 4100, "bf16", POLICY), (90, 1030, "bf16", POLICY),

@@ -617,12 +617,20 @@ int ssd_chunk_scan_noalloc_fwd(const ssd_dims *dims, int dtype, const void *x, c
     ssd::ScanShape s;
     if (int rc = make_shape(dims, dtype, &s)) return rc;
     const size_t need = scan_scratch_bytes(s, dtype);
-    if (need > kStaticScratchBytes)
+    // a shape whose own path needs more than the array, but which the one-pass kernel takes: as one launch, without scratch
+    const bool whole = need > kStaticScratchBytes &&
+                       (dtype == SSD_DTYPE_F32 ? ssd::fused_scan_f32_waves(s) : ssd::fused_scan_waves(s, dtype)) != 0;
+    if (need > kStaticScratchBytes && !whole)
         return fail(SSD_ERR_WORKSPACE,
                     "ssd: this shape needs %zu bytes of scratch, the library's static scratch array holds %zu; call "
                     "ssd_chunk_scan_fwd with a workspace of ssd_workspace_bytes() instead",
                     need, kStaticScratchBytes);
     SSD_SCAN_POINTER_CHECKS;
+    if (whole) {
+        const hipError_t e = ssd::launch_fused_scan(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states,
+                                                    (hipStream_t)hip_stream);
+        return e == hipSuccess ? SSD_OK : hip_fail(e, "one-pass scan launch");
+    }
     void *scratch = nullptr;
     if (int rc = static_scratch_address(&scratch)) return rc;
     return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, kStaticScratchBytes,

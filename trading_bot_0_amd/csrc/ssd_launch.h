@@ -104,7 +104,7 @@ hipError_t launch_fused_scan(const ScanShape &s, int dtype, const void *x, const
                              const void *Bm, const void *Cm, const float *D, const float *init,
                              const unsigned char *reset, void *y, float *final_states, hipStream_t stream,
                              float *tile_states = nullptr);
-// The one-pass forward with the sequence cut into segments that run side by side (bf16 inputs, dstate 32 or 64):
+// The one-pass forward with the sequence cut into segments that run side by side (float32 inputs, or bf16):
 // first every segment's own contribution to the state and its total decay (states only, no y, no C), then the
 // state entering every segment by a recurrence over the segments, then the forward proper per segment.
 // seg_states [B, segments, H, P, N] and seg_decay [B, segments, H] are scratch of the caller.
