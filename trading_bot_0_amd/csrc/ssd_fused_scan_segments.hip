@@ -26,7 +26,8 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // CU each (eight units of 32 columns; four of a 128-wide state).  As used against measured:
 // staged kernels (every tile of 64 steps of every unit side by side): 8 heads of 32, state 64, 16 x 512 steps 18 / 17,
 // 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128 (16 heads of 64),
-// 3 x 1 000 23 / 28, 8 x 1 000 49 / 47, 2 x 4 000 54 / 54, 8 x 4 000 174 / 172; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000 63 / 67, 10 x 3 000 87 / 86.
+// 3 x 1 000 23 / 28, 8 x 1 000 49 / 47, 2 x 4 000 54 / 54, 8 x 4 000 174 / 172; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000
+// 63 / 67, 10 x 3 000 87 / 86.
 double staged_us(const ScanShape &s, int dtype, long long groups) {
     const int full = dtype != 0 && s.N == 128 ? 4 : 8;
     const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
@@ -34,7 +35,8 @@ double staged_us(const ScanShape &s, int dtype, long long groups) {
     return s.N == 128 ? 6.0 + 650.0 * units + 0.13 * tiles_of(s) : 10.0 + 518.0 * units;
 }
 // the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
-// 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000 143 / 138; float32 tiles of 32 steps, 70 x 100 26 / 27
+// 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000
+// 143 / 138; float32 tiles of 32 steps, 70 x 100 26 / 27
 double whole_us(const ScanShape &s, int dtype, long long groups) {
     const double rounds = (double)((groups + 255) / 256);
     if (dtype == 0) return 5.0 + 5.3 * float_tiles_of(s) * rounds;
@@ -43,9 +45,9 @@ double whole_us(const ScanShape &s, int dtype, long long groups) {
 }
 // ... on segments, with the states-only pass and the entering states in front: 16 x 512 steps on 2 segments 40 / 36, 90 x 1 024
 // on 2 65 / 66, 61 x 3 999 on 4 117 / 120, 48 x 4 096 on 5 101 / 99, 24 x 4 096 on 8 69 / 71, 90 x 4 096 on 5 (two rounds) 198 / 198;
-// float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12 98 / 105; state 128 (two waves per unit, the
-// entering states always in a launch of their own), 2 x 4 000 on 13 49 / 49, 4 x 4 000 on 8 69 / 70, 8 x 4 000 on 4 123 / 122, 16 x 2 000
-// on 2 132 / 131, 4 x 16 384 on 8 216 / 220, 12 x 4 000 on 8 (three rounds) 212 / 196
+// float32 96 x 1 999 on 2 250 / 246, on 5 (two rounds) 234 / 232 to 246, 60 x 1 000 on 4 78 / 79, 20 x 4 000 on 8 135 / 133, on 12
+// 98 / 105; state 128 (two waves per unit, the entering states always in a launch of their own), 2 x 4 000 on 13 49 / 49, 4 x 4 000 on
+// 8 69 / 70, 8 x 4 000 on 4 123 / 122, 16 x 2 000 on 2 132 / 131, 4 x 16 384 on 8 216 / 220, 12 x 4 000 on 8 (three rounds) 212 / 196
 double segments_us(const ScanShape &s, int dtype, long long groups, int segments, int seg_tiles) {
     const double rounds = (double)((groups * segments + 255) / 256), tiles = seg_tiles * rounds, more = rounds - 1.0;
     if (dtype != 0 && s.N == 128) return 16.0 + 0.14 * groups + 6.1 * tiles + 18.0 * more;
