@@ -25,14 +25,16 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // Estimates in microseconds, from measurements on MI355X, of the three ways a forward can run; `groups` workgroups fill a
 // CU each (eight units of 32 columns; four of a 128-wide state).  As used against measured:
 // staged kernels (every tile of 64 steps of every unit side by side): 8 heads of 32, state 64, 16 x 512 steps 18 / 17,
-// 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128 (16 heads of 64),
-// 3 x 1 000 23 / 28, 8 x 1 000 49 / 47, 2 x 4 000 54 / 54, 8 x 4 000 174 / 172; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000
+// 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128 (16 heads of 64,
+// chunks of 256), 2 x 300 20 / 22, 3 x 1 000 31 / 28, 6 x 600 39 / 42, 8 x 1 000 58 / 47, 12 x 600 63 / 60, 2 x 4 000 58 / 54, 12 x 1 300
+// 112 / 111, 8 x 4 000 187 / 172, 16 x 4 000 360 / 369; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000
 // 63 / 67, 10 x 3 000 87 / 86.
 double staged_us(const ScanShape &s, int dtype, long long groups) {
     const int full = dtype != 0 && s.N == 128 ? 4 : 8;
     const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
     if (dtype == 0) return 12.0 + 1310.0 * units;
-    return s.N == 128 ? 6.0 + 650.0 * units + 0.13 * tiles_of(s) : 10.0 + 518.0 * units;
+    if (s.N != 128) return 10.0 + 518.0 * units;
+    return 15.0 + 690.0 * units * ((double)s.nc * s.Q / ((double)tiles_of(s) * kOnePassTile));  // (its chunks are whole: 600 steps 3 of 256)
 }
 // the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
 // 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000
@@ -59,6 +61,8 @@ double segments_us(const ScanShape &s, int dtype, long long groups, int segments
 double best_segments(const ScanShape &s, int dtype, long long groups, int nc, int min_tiles, int *segments) {
     double best = 1e30;
     *segments = 1;
+    // (more than a round of workgroups: whole rounds and a rest of its own, not three rounds of halves: 272 x 2 048 steps 217 us, 328)
+    if (groups > 256) return best;
     for (int S = 2; nc >= S * min_tiles && groups * S <= kSegmentMaxGroups; ++S) {
         const int seg_tiles = (nc + S - 1) / S;
         if ((nc + seg_tiles - 1) / seg_tiles != S) continue;
@@ -119,6 +123,10 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     return whole < staged ? 1 : 0;
 }
 
+// What a batch of its own costs besides: its launches start when the whole rounds have drained (300 sequences of 300 steps, 8 heads of 32:
+// 58 us with the 44 of the rest apart, 55 in two rounds; 36 of 200 steps, 16 heads of 64, state 128: 47, 43).
+constexpr double kTailLaunchUs = 6.0;
+
 // A batch whose workgroups fill the chip k >= 1 whole times plus a remainder that would be cheaper as a batch of
 // its own (by the plan's estimates) than as one more round: the rows of that remainder, else 0.
 int fused_scan_tail_rows(const ScanShape &s, int dtype) {
@@ -137,9 +145,10 @@ int fused_scan_tail_rows(const ScanShape &s, int dtype) {
     if (tail_plan == 1) return 0;  // it would run as a round of the one-pass kernel anyway
     // the remainder as its own batch against one more round
     const int nc = dtype == 0 ? float_tiles_of(s) : tiles_of(s);
-    const double round = whole_us(s, dtype, 256) - whole_us(s, dtype, 0);
+    // (a 128-wide state's round of a few workgroups is a faster one: 48 x 2 000 steps of 16 heads of 64 271 us, 279 with the last 16 apart)
+    const double round = whole_us(s, dtype, dtype != 0 && s.N == 128 ? rest : 256) - whole_us(s, dtype, 0);
     const double cost = tail_plan == 2 ? segments_us(s, dtype, rest, segments, (nc + segments - 1) / segments) : staged_us(tail, dtype, rest);
-    return cost < round ? tail.B : 0;
+    return cost + kTailLaunchUs < round ? tail.B : 0;
 }
 
 hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segments, const void *x, const void *dt,
