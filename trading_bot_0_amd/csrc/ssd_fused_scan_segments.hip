@@ -53,8 +53,11 @@ double whole_us(const ScanShape &s, int dtype, long long groups) {
 double segments_us(const ScanShape &s, int dtype, long long groups, int segments, int seg_tiles) {
     const double rounds = (double)((groups * segments + 255) / 256), tiles = seg_tiles * rounds, more = rounds - 1.0;
     if (dtype != 0 && s.N == 128) return 16.0 + 0.14 * groups + 6.1 * tiles + 18.0 * more;
-    if (dtype == 0) return 6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more;
-    return 12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more;
+    // (several rounds a tenth dearer than fitted: how they fall varies, 132 x 4 096 on 5 296 where the uncut kernel takes 287, 170 x 8 192
+    // on 3 647 / 583, float32 104 x 3 999 on 7 496, on 2 477)
+    const double fall = rounds > 1.0 ? 1.12 : 1.0;
+    if (dtype == 0) return fall * (6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more);
+    return fall * (12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more);
 }
 // the fastest cut of nc tiles into segments of min_tiles or more, by that estimate; in bf16 a power of two unless another is clearly
 // faster (the estimate is good to a few per cent, and programs size and compare by the number of segments)
@@ -62,7 +65,8 @@ double best_segments(const ScanShape &s, int dtype, long long groups, int nc, in
     double best = 1e30;
     *segments = 1;
     // (more than a round of workgroups: whole rounds and a rest of its own, not three rounds of halves: 272 x 2 048 steps 217 us, 328)
-    if (groups > 256) return best;
+    // nor, but for a 128-wide state, is more than half a round (170 x 8 192 on 3 647 us, uncut 583)
+    if (groups > (dtype != 0 && s.N == 128 ? 256 : 128)) return best;
     for (int S = 2; nc >= S * min_tiles && groups * S <= kSegmentMaxGroups; ++S) {
         const int seg_tiles = (nc + S - 1) / S;
         if ((nc + seg_tiles - 1) / seg_tiles != S) continue;
@@ -98,7 +102,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
     const int waves = fused_scan_waves(s, dtype);
     if (waves == 4 && s.N != 128) {
         // groups of four units (four heads of 32, two of 64 ...): workgroups of four waves, two to a CU.  A workgroup
-        // alone on its CU walks a tile in about 4.2 (one wave per SIMD), two sharing it in about 7.0 each; a round is 512
+        // alone on its CU walks a tile in 3.3 (100 sequences of 400 steps 28, staged 34) to 4.3 (one wave per SIMD), two sharing it in about 7.0 each; a round is 512
         // workgroups.  Measured at 2 048 steps, 4 heads of 32, state 64: 256 sequences 144 (staged 263), 512 221
         // (503), 1 024 459 (1 010); 128 sequences 125 against 124, below that the staged kernels win.  Not cut into
         // segments (the states-only instance is the eight-wave one).
@@ -106,7 +110,7 @@ int fused_scan_plan(const ScanShape &s, int dtype, int *segments) {
         const int nc = tiles_of(s);
         const double staged = 10.0 + 518.0 * ((double)groups * 4 * nc) / (2048.0 * 32.0);
         const long long rounds = groups / 512, rest = groups % 512;
-        const double per_tile = 7.0 * rounds + (rest == 0 ? 0.0 : rest <= 256 ? 4.2 : 4.2 + 2.8 * (double)(rest - 256) / 256.0);
+        const double per_tile = 7.0 * rounds + (rest == 0 ? 0.0 : rest <= 256 ? 3.2 + 1.1 * (double)rest / 256.0 : 4.3 + 2.7 * (double)(rest - 256) / 256.0);
         return 5.0 + per_tile * nc < staged ? 1 : 0;
     }
     const int full = s.N == 128 ? 4 : 8;  // waves of a workgroup that fills a CU
