@@ -205,3 +205,53 @@ def test_whole_pass_captured_reads_the_parameters_at_replay():
         torch.cuda.synchronize()
         for k in eager:
             assert torch.equal(res[k], eager[k]), (i, k)
+
+
+def conv_backward_inputs(B, L):
+    """Few channels (eight heads of 8, state 16, d_conv 2: 64 + 32 of x | B | C), so that many rows are cheap."""
+    zeros = lambda *s: torch.zeros(*s, device="cuda")
+    return (zeros(B, L, 168), zeros(96, 2), zeros(96), zeros(8), zeros(B, L, 8, 8), zeros(B, L, 1, 16), zeros(B, L, 1, 16),
+            zeros(B, L, 8))
+
+
+@pytest.mark.parametrize("B,L", [(128, 2048), (139, 2048), (3, 131072)])
+def test_partial_sums_of_the_conv_backward_keep_float32_accuracy(B, L):
+    """dconv_b over 1 024 workgroups' partial sums, as many as one launch adds, and over 1 112 and 1 536, which two launches do.  With
+    every input zero the filter's output is zero and silu' one half, so a workgroup's partial sum is half of the one output gradient
+    put into its 256 rows: 2^24 in the first sixteen, one in the others.  Adding those one by one behind a large one loses every one of
+    them; no part may go through more than 24 additions, whose roundings are at most 2^-24 of the sum each."""
+    from trading_bot_0_amd.block import block_pre_bwd
+    z, w, b, bias, dx, dB, dC, ddt = conv_backward_inputs(B, L)
+    parts = B * L // 256
+    value = torch.ones(parts, device="cuda")
+    value[:16] = 2.0 ** 24
+    dx.view(parts, 256, 64)[:, 0, :] = 2 * value[:, None]
+    db = block_pre_bwd(z, w, b, bias, dx, dB, dC, ddt, torch.zeros_like(z), 8, 8, 16, 1)[1]
+    total = value.double().sum()
+    assert ((db[:64].double() - total).abs() <= 24 * 2.0 ** -24 * total).all() and not bool(db[64:].any())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L", [(140, 2001), (700, 33), (300, 1001)])
+def test_parameter_gradients_of_the_conv_backward_over_many_rows(B, L, dtype):
+    """dconv_w, dconv_b and ddt_bias against float64 autograd: 1 103 and 1 200 workgroups' partial sums (two launches, the second of
+    shares that are not equal), and 175.  Bound: the roundings of 2^-24 in a term (8) and on its way through the sums, of the terms'
+    absolute sum: a run of 32 steps, the eight runs of a workgroup, 24 additions of the workgroups; for dt the 12 rows of a thread, the 256
+    threads of a workgroup and the same."""
+    from trading_bot_0_amd.block import block_pre_bwd
+    g = torch.Generator(device="cuda").manual_seed(B)
+    rnd = lambda t, s=1.0: torch.randn(t.shape, generator=g, device="cuda") * s
+    z, w, b, bias, dx, dB, dC, ddt = conv_backward_inputs(B, L)
+    w, b, bias = rnd(w, 0.5), rnd(b, 0.1), rnd(bias)
+    z, dx, dB, dC, ddt = (rnd(t).to(dtype) for t in (z, dx, dB, dC, ddt))
+    dw, db, dbias = block_pre_bwd(z, w, b, bias, dx, dB, dC, ddt, torch.zeros_like(z), 8, 8, 16, 1)[:3]
+    inp = z[..., 64:160].double()
+    before = torch.nn.functional.pad(inp, (0, 0, 1, 0))[:, :-1]
+    pre = b.double() + w[:, 0].double() * before + w[:, 1].double() * inp
+    sg = torch.sigmoid(pre)
+    d = torch.cat([t.reshape(B, L, -1) for t in (dx, dB, dC)], -1).double() * sg * (1 + pre * (1 - sg))
+    dt_terms = ddt.double() * torch.sigmoid(z[..., 160:].double() + bias.double())
+    for name, got, terms, roundings in (("dconv_w[0]", dw[:, 0], d * before, 72), ("dconv_w[1]", dw[:, 1], d * inp, 72),
+                                        ("dconv_b", db, d, 72), ("ddt_bias", dbias, dt_terms, 300)):
+        over = (got.double() - terms.sum((0, 1))).abs() / terms.abs().sum((0, 1)) * 2.0 ** 24
+        assert bool((over <= roundings).all()), f"{name}: {over.max().item():.1f} roundings"

@@ -185,10 +185,11 @@ __global__ __launch_bounds__(256) void block_post_bwd_kernel(const TY *__restric
 }
 
 // The sums over the workgroups' partial sums: of part[p][c] over p, for every column c, in a fixed order.  A workgroup is 64
-// columns x kSumSlices slices of its share of the parts (blockIdx.y of gridDim.y shares); a slice adds every kSumSlices-th part of
-// the share in order, and the slices are added in order.  One launch sums all there is to sum behind a kernel (two jobs: the
+// columns x kSumSlices slices of its share of the parts (blockIdx.y of gridDim.y shares); a slice takes every kSumSlices-th part of
+// the share, sixteen at a time whose loads are in flight together.  One launch sums all there is to sum behind a kernel (three jobs: the
 // workgroups of the first come first); up to kSumWholeParts parts in one share, more as kSumShares shares whose sums go through the
-// same kernel once more.
+// same kernel once more.  The sixteen parts of a slice's round, and then the slices, are added in pairs: a part goes through at most
+// 4 + 4 + 4 float32 additions at 1 024 parts, where slices and parts added one after the other make it 80.
 constexpr int kSumShares = 32, kSumSlices = 16, kSumWholeParts = 1024;
 
 struct ColumnSums {
@@ -199,6 +200,15 @@ struct ColumnSums {
     int split = 0;
     int blocks() const { return (cols + 63) / 64; }
 };
+
+template <int N> __device__ inline float sum_in_pairs(float (&v)[N]) {  // N a power of two
+#pragma unroll
+    for (int n = N / 2; n > 0; n /= 2) {
+#pragma unroll
+        for (int i = 0; i < n; ++i) v[i] += v[i + n];
+    }
+    return v[0];
+}
 
 __global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums first, ColumnSums second, ColumnSums third,
                                                                       int first_blocks, int second_blocks) {
@@ -212,15 +222,23 @@ __global__ __launch_bounds__(64 * kSumSlices) void column_sums_kernel(ColumnSums
     const int p0 = blockIdx.y * per, p1 = min(j.nparts, p0 + per);
     float acc = 0.f;
     if (c < j.cols) {
-#pragma unroll 8
-        for (int p = p0 + q; p < p1; p += kSumSlices) acc += j.part[(size_t)p * j.cols + c];
+        constexpr int kRound = 16;
+        for (int p = p0 + q; p < p1; p += kRound * kSumSlices) {
+            float v[kRound];
+#pragma unroll
+            for (int u = 0; u < kRound; ++u) v[u] = j.part[(size_t)min(p + u * kSumSlices, p1 - 1) * j.cols + c];
+#pragma unroll
+            for (int u = 0; u < kRound; ++u) v[u] = p + u * kSumSlices < p1 ? v[u] : 0.f;
+            acc += sum_in_pairs(v);
+        }
     }
     sm[q][cl] = acc;
     __syncthreads();
     if (q != 0 || c >= j.cols) return;
-    float sum = sm[0][cl];
+    float slice[kSumSlices];
 #pragma unroll
-    for (int i = 1; i < kSumSlices; ++i) sum += sm[i][cl];
+    for (int i = 0; i < kSumSlices; ++i) slice[i] = sm[i][cl];
+    const float sum = sum_in_pairs(slice);
     if (j.split == 0) {
         j.out[(size_t)blockIdx.y * j.cols + c] = sum;
     } else {
