@@ -255,3 +255,16 @@ def test_parameter_gradients_of_the_conv_backward_over_many_rows(B, L, dtype):
                                         ("dconv_b", db, d, 72), ("ddt_bias", dbias, dt_terms, 300)):
         over = (got.double() - terms.sum((0, 1))).abs() / terms.abs().sum((0, 1)) * 2.0 ** 24
         assert bool((over <= roundings).all()), f"{name}: {over.max().item():.1f} roundings"
+
+
+@pytest.mark.parametrize("rows", [8192, 60000])
+def test_weight_gradient_loses_little_behind_a_large_product(rows):
+    """One product of 2^24 and 2^-4 for every other row: sixteen of those make one, half a unit in the last place of the large one,
+    and added to it one by one every such sum is lost.  A product goes through at most 16 additions in its run of 256 rows, one per
+    run of its split (1 920 rows at 60 000: 8) and one per split (32), each with a rounding of at most 2^-24 of the sum."""
+    from trading_bot_0_amd.block import block_wgrad
+    a = torch.full((rows, 1024), 2.0 ** -4, dtype=torch.bfloat16, device="cuda")
+    a[0] = 2.0 ** 24
+    b = torch.ones(rows, 128, dtype=torch.bfloat16, device="cuda")
+    total = 2.0 ** 24 + (rows - 1) * 2.0 ** -4
+    assert bool(((block_wgrad(a, b).double() - total).abs() <= (16 + 8 + 32) * 2.0 ** -24 * total).all())

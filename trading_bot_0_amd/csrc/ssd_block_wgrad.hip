@@ -7,7 +7,11 @@
 // and walks it 64 rows at a time: both operands have the sum's index along their rows, so the tiles go to LDS as they lie in
 // memory and come out through the transposing read; two sets of tiles, one barrier a step, the next step's rows requested
 // behind it.  Partial blocks go out once per split and a second kernel adds them in order (the same bits every run).  Every
-// kFlushSteps steps the accumulators are added to a second set and cleared, so that no float32 sum is longer than 4 096 rows.
+// kFlushSteps steps the accumulators are added to a second set and cleared, so that a product goes through the 16 additions of
+// 256 rows, one per 256 rows of its split and one per split (256 x 256 outputs beside 648 x 256, error against float64 with a set
+// cleared every 4 096 rows / 512 / 256: 12 000 rows 1.65e-7 / 1.65e-7 / 1.46e-7, 16 384 1.78e-7 / 1.78e-7 / 1.51e-7, 60 000 3.01e-7 /
+// 1.83e-7 / 1.62e-7, 81 920 3.38e-7 / 1.87e-7 / 1.64e-7; 4 096 / 256 rows, us: 648 x 256 outputs at 16 384 rows 23.5 / 23.9, 72 828 55.0 / 56.9,
+// 524 288 351.8 / 354.8, both of a training pass at 16 384 rows within the runs).
 //
 // Against the BLAS, whose batched products over equal slabs of rows need a row count with a power of two in it (any other
 // ran as one product with a bf16 result at a fifth of the rate), in us, BLAS / here: 648 x 256 outputs at 16 384 rows 38 / 26,
@@ -26,7 +30,7 @@ namespace {
 constexpr int kWgradCols = 128;     // output rows (columns of a) per workgroup
 constexpr int kWgradRows = 64;      // rows per step
 constexpr int kWgradThreads = 512;
-constexpr int kFlushSteps = 64;
+constexpr int kFlushSteps = 4;     // 256 rows
 constexpr int kWgradMinRows = 256;  // per split: shorter ones are mostly the partial block's way out
 
 // One weight gradient of a launch: its operands and where its splits' blocks go ([splits, E, N]).
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(kWgradThreads) void block_wgrad_kernel(WgradJob fir
                     for (int j = 0; j < NI; ++j) acc[i][j] = mma32(fa[i], fb[j], acc[i][j]);
                 }
             }
-            if ((step + 1) % kFlushSteps == 0) {
+            if ((step + 1) % kFlushSteps == 0 && r0 + kWgradRows < end) {
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
 #pragma unroll
