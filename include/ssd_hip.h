@@ -79,8 +79,8 @@ char *ssd_get_and_reset_last_err(void);
 /* Bytes of scratch ssd_chunk_scan_fwd needs for these dims.  The reference lets ATen allocate
  * op temporaries; a capturable op cannot, so the caller owns the buffer (the Rust side would
  * hold it as a Tensor::empty, cf. the persistent rollout buffers at
- * trading_bots/src/torch/train/trainer.rs:622-944).  (A float32 forward that runs on the staged kernels uses chunks of 64
- * steps, and runs faster, if the workspace has room for them: what this function names for dims with chunk 64, where that is more.) */
+ * trading_bots/src/torch/train/trainer.rs:622-944).  (`chunk` is how the staged kernels tile time.  In float32 with headdim * dstate up
+ * to 2 048 they are a tenth to a third faster on 64 than on 128, at up to twice the workspace.) */
 int ssd_workspace_bytes(const ssd_dims *dims, size_t *out_bytes);
 
 /* Whole forward: stages 1-4 on one stream.  Fills y and, when non-NULL, final_states.
@@ -146,12 +146,12 @@ int ssd_chunk_scan_reset_fwd(const ssd_dims *dims, int dtype, const void *x, con
  * tight serving loops, harnesses that forbid hipMalloc -- and so cannot bring a workspace: the scratch the staged and
  * segmented paths need comes from an array of SSD_STATIC_SCRATCH_BYTES (64 MiB) that is part of the library's device
  * code (each GPU the library runs on holds it until the process ends).  No counterpart in the reference.  Same
- * arguments and results as ssd_chunk_scan_reset_fwd minus the workspace.  SSD_ERR_WORKSPACE when the scratch that the
- * shape's own path uses exceeds the array and the one-pass kernel, which then runs it as one launch, does not take the
- * shape: all of ssd_workspace_bytes on the staged kernels, the segment states and
+ * arguments as ssd_chunk_scan_reset_fwd minus the workspace, and the same results, bit for bit, where the scratch that the
+ * shape's own path uses fits the array: all of ssd_workspace_bytes on the staged kernels, the segment states and
  * decays (batch * segments * nheads * (headdim * dstate + 1) floats) when the sequences run cut into segments
  * (ssd_chunk_scan_segments > 1), nothing when the shape runs as one launch of the one-pass kernel
- * (ssd_chunk_scan_is_onepass), at any size.  Calls no hipMalloc/hipFree or any other allocating
+ * (ssd_chunk_scan_is_onepass), at any size.  Where it does not fit, the shape runs as one launch of the one-pass kernel (the
+ * bits of ssd_chunk_scan_onepass_fwd), or, if that does not take it, the call is refused with SSD_ERR_WORKSPACE.  Calls no hipMalloc/hipFree or any other allocating
  * routine.  Every call on a GPU shares that GPU's array: calls that overlap in time on one GPU (different streams or
  * threads) race on it; calls on one stream are ordered and safe.  Nothing in the array has to start at zero (every
  * kernel writes what it later reads), so it is not cleared between calls.

@@ -162,3 +162,29 @@ def test_forward_on_segments(batch, seqlen, dtype, dims):
     yr, fr = c_oracle_reset(sub, mask[rows])
     assert_close(y[rows], yr, w.torch_dtype, "y")
     assert_close(f[rows], fr, w.torch_dtype, "final")
+
+
+@pytest.mark.parametrize("batch,seqlen,dims", [(3, 300, POLICY), (20, 1000, POLICY), (3, 300, (8, 16, 16, 1, 256)), (2, 700, (8, 64, 64, 1, 128))])
+def test_float32_result_does_not_depend_on_the_scratch(batch, seqlen, dims):
+    """Float32 on the staged kernels: the same bits without a workspace, with one of the size the library names for the sizes as they
+    are, with one of the size it uses and with a larger one; a smaller one is refused."""
+    w = Workload("scratch", batch, seqlen, *dims, dtype="f32", init_std=0.5)
+    i = make_inputs(w, seed=1, device="cuda")
+    assert ssd.chunk_scan_segments(batch, seqlen, *dims, torch.float32) == 1
+
+    def call(workspace):
+        return ssd_chunk_scan(i["x"], i["dt"], i["A"], i["B"], i["C"], i["D"], chunk=dims[4], initial_states=i["init"], workspace=workspace)
+
+    y, f = call(None)
+    least, used = ssd.workspace_bytes(batch, seqlen, *dims), ssd.workspace_bytes(batch, seqlen, *dims, dtype=torch.float32)
+    assert least <= used
+    for size in (least, used, 4 * used):
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        y2, f2 = call(ws)
+        assert torch.equal(y, y2) and torch.equal(f, f2), size
+        p = ssd.PreparedChunkScan(i["x"], i["dt"], i["A"], i["B"], i["C"], i["D"], chunk=dims[4], initial_states=i["init"], workspace=ws)
+        y2, f2 = p()
+        assert torch.equal(y, y2) and torch.equal(f, f2), size
+    with pytest.raises(ssd.SsdError, match="workspace") as e:
+        call(torch.empty(least - 256, dtype=torch.uint8, device="cuda"))
+    assert e.value.code == 3

@@ -1,6 +1,7 @@
 """ssd_chunk_scan_noalloc_fwd -- the forward for callers that cannot allocate device memory -- through the C ABI,
 against ssd_chunk_scan_reset_fwd with a caller-owned workspace: the same kernels on a different scratch buffer, so
-y and the final states must be equal bit for bit.  Each case makes two calls in a row on the library's static
+y and the final states must be equal bit for bit, where the shape's scratch fits the array (the others run as one launch of
+the one-pass kernel: tests/test_gpu_staged.py compares them with that entry point).  Each case makes two calls in a row on the library's static
 scratch array, the second with a smaller input (the array still holds the first call's intermediates), and checks
 that the device's free memory does not move across the calls.
 
@@ -167,3 +168,13 @@ def test_noalloc_forward_captured_in_a_graph(name, batch, seqlen):
         torch.cuda.synchronize()
         assert not torch.isnan(y_new.float()).any()
         assert torch.equal(y_new, y_ref) and torch.equal(f_new, f_ref), f"replay {replay}"
+
+
+def test_noalloc_forward_of_float32_on_long_chunks_equals_the_workspace_forward():
+    """Staged float32 with chunks of 128 in policy heads: the chunk is the caller's, however much scratch there is."""
+    lib = ssd.load_library()
+    torch.cuda.set_device(0)
+    prime(lib)
+    w = WORKLOADS["policy_bf16"].with_dtype("f32")
+    for i, (batch, seqlen) in enumerate(((10, 300), (3, 300))):
+        assert run_pair(lib, w.with_batch(batch), seqlen, with_reset=(i == 0), with_init=(i == 1)) <= (64 << 20)

@@ -124,19 +124,6 @@ Workspace carve(const ssd::ScanShape &s) {
     return w;
 }
 
-// The chunk the staged forward runs on.  In float32 a chunk's scores cost a quarter of the time they take in bf16 as states would:
-// chunks of 64 instead of the caller's 128 (8 heads of 32, state 64: 3 x 300 steps 21 -> 17 us, 10 x 3 000 102 -> 86, 60 x 300
-// 76 -> 61, 5 x 1 500 as fast), where the scratch holds their states: ssd_workspace_bytes of the caller's own chunk does not, that
-// of chunk 64 does.  (Wider states go the other way: heads of 64, state 128,
-// 4 x 2 000 172 -> 219.)
-ssd::ScanShape staged_shape(const ssd::ScanShape &s, int dtype, size_t scratch_bytes) {
-    ssd::ScanShape f = s;
-    f.Q = 64;
-    f.nc = (s.L + 63) / 64;
-    if (dtype != SSD_DTYPE_F32 || s.Q <= 64 || s.P * s.N > 2048 || (int64_t)f.B * f.nc * f.H > 0x7fffffff) return s;
-    return carve(f).total <= scratch_bytes ? f : s;
-}
-
 bool takes_one_pass(const ssd::ScanShape &s, int dtype) {
     int segments;
     return ssd::fused_scan_plan(s, dtype, &segments) == 1;
@@ -528,12 +515,15 @@ size_t scan_scratch_bytes(const ssd::ScanShape &s, int dtype) {
     return carve(s).total;
 }
 
-// The forward proper, arguments checked: the way the plan says for this shape, with `workspace` (carve(s).total bytes or
-// more, or anything at all when scan_scratch_bytes says the shape needs none) as scratch.
+// The forward proper, arguments checked: the way the plan says for this shape, with `workspace` (carve(s).total bytes,
+// or anything at all when scan_scratch_bytes says the shape needs none) as scratch.
 static int scan_forward(const ssd::ScanShape &s, int dtype, const void *x, const void *dt, const float *A, const void *Bm,
                         const void *Cm, const float *D, const float *initial_states, const uint8_t *reset, void *y,
-                        float *final_states, void *workspace, size_t workspace_bytes, hipStream_t st) {
+                        float *final_states, void *workspace, hipStream_t st) {
+    const Workspace w = carve(s);
     char *base = static_cast<char *>(workspace);
+    float *dtcs = reinterpret_cast<float *>(base + w.dtcs_off);
+    float *states = reinterpret_cast<float *>(base + w.st_off);
     // One batch of sequences, the way the plan says.  The workspace is carved for the whole batch and so holds any
     // part of it.
     auto forward = [&](const ssd::ScanShape &part, const void *px, const void *pdt, const void *pb, const void *pc,
@@ -555,10 +545,7 @@ static int scan_forward(const ssd::ScanShape &s, int dtype, const void *x, const
                                                  seg_states, seg_decay, st);
             return e == hipSuccess ? SSD_OK : hip_fail(e, "segmented one-pass scan launch");
         }
-        const ssd::ScanShape on = staged_shape(part, dtype, workspace_bytes);
-        const Workspace w = carve(on);
-        return run_staged(on, dtype, px, pdt, A, pb, pc, D, pinit, preset, 0, py, pfinal, reinterpret_cast<float *>(base + w.dtcs_off),
-                          reinterpret_cast<float *>(base + w.st_off), st);
+        return run_staged(part, dtype, px, pdt, A, pb, pc, D, pinit, preset, 0, py, pfinal, dtcs, states, st);
     };
     // A batch that fills the chip some whole number of times and a bit: the whole rounds run as one launch of the
     // one-pass kernel, the rest as a batch of its own (cut into segments or staged, as the plan says for it) -- a
@@ -607,7 +594,7 @@ int ssd_chunk_scan_reset_fwd(const ssd_dims *dims, int dtype, const void *x, con
     const Workspace w = carve(s);
     if (workspace_bytes < w.total)
         return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, w.total);
-    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, workspace, workspace_bytes,
+    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, workspace,
                         (hipStream_t)hip_stream);
 }
 
@@ -633,7 +620,7 @@ int ssd_chunk_scan_noalloc_fwd(const ssd_dims *dims, int dtype, const void *x, c
     }
     void *scratch = nullptr;
     if (int rc = static_scratch_address(&scratch)) return rc;
-    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, kStaticScratchBytes,
+    return scan_forward(s, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch,
                         (hipStream_t)hip_stream);
 }
 
@@ -1370,7 +1357,7 @@ int ssd_block_forward(const ssd_block_dims *dims, int dtype, int64_t d_model, in
     if (e != hipSuccess) return hip_fail(e, "block projection launch");
     e = ssd::launch_block_pre(s, 1, zxbcdt, conv_w, conv_b, dt_bias, conv_state_in, conv_state_out, reset, x, Bm, Cm, dt, st, A_log, A);
     if (e != hipSuccess) return hip_fail(e, "block pre-scan launch");
-    if (int rc = scan_forward(sc, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, scratch_bytes, st)) return rc;
+    if (int rc = scan_forward(sc, dtype, x, dt, A, Bm, Cm, D, initial_states, reset, y, final_states, scratch, st)) return rc;
     e = ssd::launch_block_post_proj(s, y, zxbcdt, norm_w, eps, w_out, (int)d_model, (int)d_model, out, st);
     return e == hipSuccess ? SSD_OK : hip_fail(e, "block post-scan + out-projection launch");
 }

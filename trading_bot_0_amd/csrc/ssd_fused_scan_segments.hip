@@ -27,14 +27,19 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // staged kernels (every tile of 64 steps of every unit side by side): 8 heads of 32, state 64, 16 x 512 steps 18 / 17,
 // 32 x 512 26 / 24, 64 x 512 42 / 40, 8 x 2 048 26 / 24, 16 x 2 048 42 / 42, 64 x 2 048 140 / 123; state 128 (16 heads of 64,
 // chunks of 256), 2 x 300 20 / 22, 3 x 1 000 31 / 28, 6 x 600 39 / 42, 8 x 1 000 58 / 47, 12 x 600 63 / 60, 2 x 4 000 58 / 54, 12 x 1 300
-// 112 / 111, 8 x 4 000 187 / 172, 16 x 4 000 360 / 369; float32 (chunks of 64) 3 x 300 14 / 17, 20 x 1 000
-// 63 / 67, 10 x 3 000 87 / 86.
+// 112 / 111, 8 x 4 000 187 / 172, 16 x 4 000 360 / 369; float32 on chunks of 64, 3 x 300 14 / 18, 2 x 9 000 57 / 60, 20 x 1 000 63 / 65,
+// 10 x 3 000 87 / 86, of 128, 3 x 300 16 / 22, 2 x 9 000 63 / 72, 20 x 1 000 69 / 72, 10 x 3 000 97 / 102, 100 x 300 118 / 117, of 256, 3 x 300
+// 36 / 40, 2 x 9 000 99 / 111, 10 x 3 000 144 / 145.
 double staged_us(const ScanShape &s, int dtype, long long groups) {
     const int full = dtype != 0 && s.N == 128 ? 4 : 8;
     const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
-    if (dtype == 0) return 12.0 + 1310.0 * units;
+    const double whole_chunks = (double)s.nc * s.Q / ((double)tiles_of(s) * kOnePassTile);  // (a chunk runs whole: 600 steps 3 of 256)
+    if (dtype == 0) {
+        if (s.Q <= 64) return 12.0 + 1310.0 * units;
+        return s.Q == 128 ? 13.0 + 1430.0 * units * whole_chunks : 30.0 + 1950.0 * units * whole_chunks;
+    }
     if (s.N != 128) return 10.0 + 518.0 * units;
-    return 15.0 + 690.0 * units * ((double)s.nc * s.Q / ((double)tiles_of(s) * kOnePassTile));  // (its chunks are whole: 600 steps 3 of 256)
+    return 15.0 + 690.0 * units * whole_chunks;
 }
 // the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
 // 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000

@@ -213,30 +213,56 @@ def num_chunks(seqlen: int, chunk: int) -> int:
     return -(-seqlen // chunk)
 
 
-def workspace_bytes(batch, seqlen, nheads, headdim, dstate, ngroups, chunk) -> int:
+def workspace_bytes(batch, seqlen, nheads, headdim, dstate, ngroups, chunk, dtype=None) -> int:
+    """Bytes of `workspace` that a forward of these sizes takes; with dtype torch.float32 as many as it uses, which may be more
+    (see `_scan_tiling`; it allocates the difference itself)."""
     lib = load_library()
-    out = c_size_t(0)
-    _check(lib, lib.ssd_workspace_bytes(byref(SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk)),
-                                        byref(out)))
-    return out.value
+    dims = SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk)
+    need = _workspace_need(lib, dims)
+    return max(need, _workspace_need(lib, _scan_tiling(lib, dims, SSD_DTYPE_F32))) if dtype == torch.float32 else need
 
 
-def _scan_workspace(lib, dims: SsdDims, x: torch.Tensor, workspace: Optional[torch.Tensor]) -> torch.Tensor:
-    """The forward's scratch: the caller's, or a new one of ssd_workspace_bytes -- for float32 also of chunks of 64, with
-    which the library runs short batches on such chunks (8 heads of 32, state 64, 10 x 3 000 steps: 86 us, on 128 102)."""
+def _workspace_need(lib, dims: SsdDims) -> int:
+    need = c_size_t(0)
+    _check(lib, lib.ssd_workspace_bytes(byref(dims), byref(need)))
+    return need.value
+
+
+def _plan(lib, dims: SsdDims, code: int) -> Tuple[bool, int]:
+    """Whether the library runs these dims as one launch of the one-pass kernel, and on how many segments."""
+    flag, segments = c_int(0), c_int(0)
+    _check(lib, lib.ssd_chunk_scan_is_onepass(byref(dims), code, byref(flag)))
+    _check(lib, lib.ssd_chunk_scan_segments(byref(dims), code, byref(segments)))
+    return bool(flag.value), segments.value
+
+
+def _scan_tiling(lib, dims: SsdDims, code: int) -> SsdDims:
+    """The dims the library is given: a float32 forward on its staged kernels runs on chunks of 64 where longer ones were asked for.
+    In float32 a chunk's scores cost four times what they do in bf16 beside its states (8 heads of 32, state 64, chunks of 128 / 64 in us:
+    3 x 300 steps 22.4 / 17.8, 2 x 9 000 71.8 / 59.9, 40 x 700 100.4 / 83.9, 16 x 2 000 104 / 90; state 32, 30 x 600 46.9 / 41.4; heads
+    of 64 and state 128 the other way, 4 x 2 000 172 / 219).  A function of sizes and type alone, so that a result does not depend on the
+    scratch that a caller brings."""
+    if code != SSD_DTYPE_F32 or dims.chunk <= 64 or dims.headdim * dims.dstate > 2048:
+        return dims
+    tiled = SsdDims(dims.batch, dims.seqlen, dims.nheads, dims.headdim, dims.dstate, dims.ngroups, 64)
+    _workspace_need(lib, dims)   # (sizes that are refused are refused as they were named)
+    return tiled if _plan(lib, tiled, code) == (False, 1) else dims
+
+
+def _scan_workspace(lib, asked: SsdDims, dims: SsdDims, x: torch.Tensor, workspace: Optional[torch.Tensor]):
+    """(dims, scratch) of a forward of the dims `asked` for that runs on `dims`: the caller's scratch, or a new one where there is none
+    or where it holds what was asked for but not what is run; one too small for either goes to the library, which refuses it."""
     if workspace is None:
-        need = c_size_t(0)
-        _check(lib, lib.ssd_workspace_bytes(byref(dims), byref(need)))
-        size = need.value
-        if x.dtype == torch.float32 and dims.chunk > 64 and dims.headdim * dims.dstate <= 2048 \
-                and dims.batch * dims.seqlen * dims.nheads <= 1 << 21:   # (larger batches run on the one-pass kernel, without any)
-            small = SsdDims(dims.batch, dims.seqlen, dims.nheads, dims.headdim, dims.dstate, dims.ngroups, 64)
-            _check(lib, lib.ssd_workspace_bytes(byref(small), byref(need)))
-            size = max(size, need.value)
-        return x.new_empty(size, dtype=torch.uint8)
+        return dims, x.new_empty(_workspace_need(lib, dims), dtype=torch.uint8)
     if (not workspace.is_cuda) or workspace.dtype != torch.uint8 or not workspace.is_contiguous():
         raise ValueError("SSD workspace must be a contiguous uint8 GPU tensor")
-    return workspace
+    if dims is not asked:
+        if workspace.numel() < _workspace_need(lib, asked):
+            return asked, workspace
+        need = _workspace_need(lib, dims)
+        if workspace.numel() < need:
+            return dims, x.new_empty(need, dtype=torch.uint8)
+    return dims, workspace
 
 
 def _validate_scan_inputs(x, dt, A, Bm, Cm, D, initial_states, dims: SsdDims):
@@ -281,7 +307,7 @@ def ssd_chunk_scan(
     `reset` [B,L] (uint8 or bool): a non-zero entry restarts that batch row's state from zero before the
     timestep (episode boundaries inside a window).
 
-    `workspace` (uint8, >= workspace_bytes(...)), `out` and `final_out` let a caller that runs
+    `workspace` (uint8, >= workspace_bytes(...), for float32 with its dtype), `out` and `final_out` let a caller that runs
     under stream capture or in a tight loop avoid any allocation.  `y_dtype=torch.float32` with
     bf16 inputs writes y without the output rounding."""
     lib = load_library()
@@ -295,7 +321,7 @@ def ssd_chunk_scan(
         shape = (dims.batch, dims.nheads, dims.headdim, dims.dstate)
         final = x.new_empty(shape, dtype=torch.float32) if final_out is None else final_out
         _require(final, "final_out", shape, torch.float32)
-    workspace = _scan_workspace(lib, dims, x, workspace)
+    dims, workspace = _scan_workspace(lib, dims, _scan_tiling(lib, dims, code), x, workspace)
     reset = _reset_mask(reset, dims)
     rc = lib.ssd_chunk_scan_reset_fwd(byref(dims), code, x.data_ptr(), dt.data_ptr(), A.data_ptr(),
                                       Bm.data_ptr(), Cm.data_ptr(), _ptr(D), _ptr(initial_states), _ptr(reset),
@@ -368,7 +394,8 @@ class PreparedChunkScan:
             shape = (dims.batch, dims.nheads, dims.headdim, dims.dstate)
             self.final = torch.empty(shape, dtype=torch.float32, device=x.device) if final_out is None else final_out
             _require(self.final, "final_out", shape, torch.float32)
-        workspace = _scan_workspace(self._lib, dims, x, workspace)
+        dims, workspace = _scan_workspace(self._lib, dims, _scan_tiling(self._lib, dims, self._code), x, workspace)
+        self._dims = dims
         reset = _reset_mask(reset, dims)
         self._keep = (x, dt, A, Bm, Cm, D, initial_states, workspace, reset)
         self._device = x.device
@@ -387,22 +414,16 @@ class PreparedChunkScan:
 def chunk_scan_is_onepass(batch, seqlen, nheads, headdim, dstate, ngroups, chunk, dtype=torch.bfloat16) -> bool:
     """Whether ssd_chunk_scan runs this shape as the one-pass kernel (True) or as the staged kernels."""
     lib = load_library()
-    dims = SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk)
-    flag = c_int(0)
     code = SSD_DTYPE_BF16 if dtype == torch.bfloat16 else SSD_DTYPE_F32
-    _check(lib, lib.ssd_chunk_scan_is_onepass(byref(dims), code, byref(flag)))
-    return bool(flag.value)
+    return _plan(lib, _scan_tiling(lib, SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk), code), code)[0]
 
 
 def chunk_scan_segments(batch, seqlen, nheads, headdim, dstate, ngroups, chunk, dtype=torch.bfloat16) -> int:
     """Into how many segments ssd_chunk_scan cuts the sequences of this shape to run them on the one-pass kernel
     side by side (1 = not cut)."""
     lib = load_library()
-    dims = SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk)
-    n = c_int(0)
     code = SSD_DTYPE_BF16 if dtype == torch.bfloat16 else SSD_DTYPE_F32
-    _check(lib, lib.ssd_chunk_scan_segments(byref(dims), code, byref(n)))
-    return n.value
+    return _plan(lib, _scan_tiling(lib, SsdDims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk), code), code)[1]
 
 
 def ssd_chunk_scan_onepass(
