@@ -76,6 +76,9 @@ int ssd_version(void);
  * (vendor/torch-sys-0.25.0/libtch/torch_api.h:33, torch_api.cpp:84-88). */
 char *ssd_get_and_reset_last_err(void);
 
+/* The sizes that the ..._workspace_bytes queries name grow with batch, length and rows: a workspace sized for the largest of a program's
+ * calls holds the others. */
+
 /* Bytes of scratch ssd_chunk_scan_fwd needs for these dims.  The reference lets ATen allocate
  * op temporaries; a capturable op cannot, so the caller owns the buffer (the Rust side would
  * hold it as a Tensor::empty, cf. the persistent rollout buffers at

@@ -156,8 +156,7 @@ def dims(**kw):
 @pytest.mark.parametrize("layout", [dict(nheads=8, dstate=64), dict(nheads=8, dstate=32), dict(nheads=24, dstate=64, ngroups=3)])
 def test_backward_workspace_of_few_sequences_holds_smaller_calls(lib, layout):
     """Where the backward pass runs on segments, what it asks for grows with the batch and with the length, although the number
-    of segments does not: a workspace sized for the largest call of a program holds the others.  (From 96 groups of eight heads on
-    the pass runs on other kernels, which ask for less.)"""
+    of segments does not: a workspace sized for the largest call of a program holds the others."""
     def need(batch, seqlen):
         out = c_size_t(0)
         d = ssd.SsdDims(batch, seqlen, layout["nheads"], 32, layout["dstate"], layout.get("ngroups", 1), 64)
@@ -169,6 +168,35 @@ def test_backward_workspace_of_few_sequences_holds_smaller_calls(lib, layout):
     sizes = [[need(batch, seqlen) for batch in range(1, most + 1)] for seqlen in lengths]
     assert all(a <= b for row in sizes for a, b in zip(row, row[1:])), "a larger batch asks for less"
     assert all(a <= b for col in zip(*sizes) for a, b in zip(col, col[1:])), "a longer sequence asks for less"
+
+
+@pytest.mark.parametrize("layout", [(8, 32, 64, 1), (8, 16, 16, 1), (8, 32, 32, 2), (8, 32, 128, 1), (16, 16, 64, 2), (4, 32, 32, 1), (4, 64, 128, 1)])
+@pytest.mark.parametrize("query", ["scan", "scan backward", "block forward", "block backward", "weight gradient"])
+def test_workspace_of_the_largest_call_holds_the_others(query, layout):
+    """What a query asks for grows with the batch and with the length, across every line at which the kernels behind it change."""
+    from trading_bot_0_amd.block import SsdBlockDims, _lib
+    lib = _lib()
+    H, P, N, G = layout
+    out = c_size_t(0)
+    if query.startswith("block") and H % 8:
+        pytest.skip("not the block's heads")
+
+    def need(B, L):
+        scan, block = ssd.SsdDims(B, L, H, P, N, G, 128), SsdBlockDims(B, L, H, P, N, G, 4, 0)
+        rc = {"scan": lambda: lib.ssd_workspace_bytes(byref(scan), byref(out)),
+              "scan backward": lambda: lib.ssd_chunk_scan_bwd_workspace_bytes(byref(scan), 1, byref(out)),
+              "block forward": lambda: lib.ssd_block_forward_workspace_bytes(byref(block), 1, 256, 128, byref(out)),
+              "block backward": lambda: lib.ssd_block_grad_workspace_bytes(byref(block), 1, 256, 128, byref(out)),
+              "weight gradient": lambda: lib.ssd_block_wgrad_workspace_bytes(B * L, 2 * H * P + 2 * G * N + H // 8 * 8, 256, byref(out))}[query]()
+        assert rc == 0, ssd.last_error(lib)
+        return out.value
+
+    for L in (1, 64, 300, 700, 2048, 4100):
+        sizes = [need(B, L) for B in range(1, 420)]
+        assert all(a <= b for a, b in zip(sizes, sizes[1:])), f"a larger batch of {L} steps asks for less"
+    for B in (1, 8, 33, 60, 97, 200):
+        sizes = [need(B, L) for L in range(1, 4200, 13)]
+        assert all(a <= b for a, b in zip(sizes, sizes[1:])), f"longer sequences, {B} of them, ask for less"
 
 
 def test_workspace_bytes_formula(lib):

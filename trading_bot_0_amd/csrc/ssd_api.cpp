@@ -399,6 +399,29 @@ int make_bwd_shapes(const ssd_dims *dims, int dtype, ssd::ScanShape *s, ssd::Sca
     return make_shape(&t, dtype, sT);
 }
 
+// What the backward pass of these shapes is asked to be given: no less than for a smaller batch or a shorter sequence, so that a
+// workspace sized for the largest of a program's calls holds the others.  A plan asks for more the larger the batch, but the kernels
+// of large batches need less than those of small ones: the largest batch below each line of plan_bwd counts too.
+size_t bwd_workspace_bound(const ssd::ScanShape &s, const ssd::ScanShape &sT, int dtype) {
+    const int eb = dtype == SSD_DTYPE_F32 ? 4 : 2, inner = dtype == SSD_DTYPE_F32 ? SSD_DTYPE_F32 : SSD_DTYPE_BF16_Y32;
+    auto need = [&](int batch) {
+        ssd::ScanShape a = s, b = sT;
+        a.B = b.B = batch;
+        return carve_bwd(a, b, eb, plan_bwd(a, b, dtype)).total;
+    };
+    size_t most = need(s.B);
+    auto line = [&](int64_t groups_per_row, int64_t from) {
+        const int64_t below = groups_per_row > 0 ? (from - 1) / groups_per_row : 0;
+        if (below >= 1 && below < s.B) most = std::max(most, need((int)below));
+    };
+    for (const ssd::ScanShape &t : {s, sT}) {
+        const int waves = ssd::fused_scan_waves(t, inner);
+        if (waves != 0) line((int64_t)t.G * ((t.H / t.G) * (t.P / 32) / waves), waves == 8 ? kOnePassMinWorkgroups : 4 * kOnePassMinWorkgroups);
+    }
+    line((int64_t)(s.H / 8) * (s.N / 32), kOnePassMinWorkgroups);
+    return most;
+}
+
 }  // namespace
 
 extern "C" {
@@ -628,7 +651,7 @@ int ssd_chunk_scan_bwd_workspace_bytes(const ssd_dims *dims, int dtype, size_t *
     if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
     ssd::ScanShape s, sT;
     if (int rc = make_bwd_shapes(dims, dtype, &s, &sT)) return rc;
-    *out_bytes = carve_bwd(s, sT, dtype == SSD_DTYPE_F32 ? 4 : 2, plan_bwd(s, sT, dtype)).total;
+    *out_bytes = bwd_workspace_bound(s, sT, dtype);
     return SSD_OK;
 }
 
@@ -1103,7 +1126,7 @@ static int check_wgrad(int64_t rows, int64_t a_features, int64_t b_features) {
 int ssd_block_wgrad_workspace_bytes(int64_t rows, int64_t a_features, int64_t b_features, size_t *out_bytes) {
     if (out_bytes == nullptr) return fail(SSD_ERR_INVALID, "ssd: out_bytes must not be NULL");
     if (int rc = check_wgrad(rows, a_features, b_features)) return rc;
-    *out_bytes = ssd::block_wgrad_workspace_bytes(rows, (int)a_features, (int)b_features);
+    *out_bytes = ssd::block_wgrad_workspace_bound(rows, (int)a_features, (int)b_features);
     return SSD_OK;
 }
 
@@ -1306,7 +1329,9 @@ int ssd_block_forward_workspace_bytes(const ssd_block_dims *dims, int dtype, int
     int width;
     if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
     if (int rc = make_shape(&scan, dtype, &sc)) return rc;
-    *out_bytes = align_up((size_t)s.H * sizeof(float), 256) + align_up(scan_scratch_bytes(sc, dtype), 256);
+    // (what the scan's own query names: it grows with batch and length, which what the scan of this size uses, checked by
+    // ssd_block_forward, does not)
+    *out_bytes = align_up((size_t)s.H * sizeof(float), 256) + align_up(carve(sc).total, 256);
     return SSD_OK;
 }
 
@@ -1372,15 +1397,19 @@ struct GradScratch {
     bool pair;  // both weight gradients in one launch
 };
 
-int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_model, int width, Carver *c, GradScratch *g) {
+// bound: what the caller is asked for, which grows with batch and length; else what the pass uses
+int carve_block_grad(const ssd::BlockShape &s, const ssd_dims &scan, int64_t d_model, int width, Carver *c, GradScratch *g, bool bound) {
     const size_t rows = (size_t)s.B * s.L, DI = (size_t)s.H * s.P, GN = (size_t)s.G * s.N;
-    if (int rc = ssd_chunk_scan_bwd_workspace_bytes(&scan, SSD_DTYPE_BF16, &g->scan_bytes)) return rc;
+    ssd::ScanShape fwd, bwd;
+    if (int rc = make_bwd_shapes(&scan, SSD_DTYPE_BF16, &fwd, &bwd)) return rc;
+    g->scan_bytes = bound ? bwd_workspace_bound(fwd, bwd, SSD_DTYPE_BF16) : carve_bwd(fwd, bwd, 2, plan_bwd(fwd, bwd, SSD_DTYPE_BF16)).total;
     if (int rc = check_wgrad((int64_t)rows, width, d_model)) return rc;
     if (int rc = check_wgrad((int64_t)rows, d_model, (int64_t)DI)) return rc;
     g->pair = d_model == (int64_t)DI;
-    const size_t wgrad_bytes = g->pair ? ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model, (int)d_model)
-                                       : std::max(ssd::block_wgrad_workspace_bytes((long long)rows, width, (int)d_model),
-                                                  ssd::block_wgrad_workspace_bytes((long long)rows, (int)d_model, (int)DI));
+    const auto wgrad = bound ? ssd::block_wgrad_workspace_bound : ssd::block_wgrad_workspace_bytes;
+    const size_t wgrad_bytes = g->pair ? wgrad((long long)rows, width, (int)d_model, (int)d_model)
+                                       : std::max(wgrad((long long)rows, width, (int)d_model, 0),
+                                                  wgrad((long long)rows, (int)d_model, (int)DI, 0));
     g->A = static_cast<float *>(c->take((size_t)s.H * sizeof(float)));
     g->dyn = c->take(rows * DI * 2);
     g->yn = c->take(rows * DI * 2);
@@ -1406,7 +1435,7 @@ int ssd_block_grad_workspace_bytes(const ssd_block_dims *dims, int dtype, int64_
     if (int rc = make_whole_block(dims, dtype, d_model, chunk, &s, &scan, &width)) return rc;
     Carver c{nullptr};
     GradScratch g;
-    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g)) return rc;
+    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g, true)) return rc;
     *out_bytes = c.used;
     return SSD_OK;
 }
@@ -1456,7 +1485,7 @@ int ssd_block_grad(const ssd_block_dims *dims, int dtype, int64_t d_model, int64
         return fail(SSD_ERR_INVALID, "ssd: du needs w_in_t with rows of at least the %d channels rounded up to 16", width);
     Carver c{static_cast<char *>(workspace)};
     GradScratch g;
-    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g)) return rc;
+    if (int rc = carve_block_grad(s, scan, d_model, width, &c, &g, false)) return rc;
     if (workspace_bytes < c.used)
         return fail(SSD_ERR_WORKSPACE, "ssd: workspace has %zu bytes, %zu needed", workspace_bytes, c.used);
     hipStream_t st = (hipStream_t)hip_stream;

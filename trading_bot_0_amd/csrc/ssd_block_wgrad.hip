@@ -186,10 +186,14 @@ int wgrad_blocks(int E) { return (E + kWgradCols - 1) / kWgradCols; }
 
 // Splits: one round of workgroups (a compute unit holds one), whole XCDs, none below kWgradMinRows rows.  (256 compute units are
 // a constant here: the workspace is laid out by the splits, and the order of the sums, so the bits, do not depend on the device.)
+long long wgrad_most_splits(long long rows, int blocks) {
+    const long long fill = std::max(1, 256 / 8 / blocks) * 8;
+    return std::max<long long>(1, std::min(fill, rows / kWgradMinRows));
+}
+
 WgradPlan wgrad_plan(long long rows, int blocks) {
     WgradPlan p;
-    const long long fill = std::max(1, 256 / 8 / blocks) * 8;
-    const long long most = std::max<long long>(1, std::min(fill, rows / kWgradMinRows));
+    const long long most = wgrad_most_splits(rows, blocks);
     p.split_rows = ((rows + most - 1) / most + kWgradRows - 1) / kWgradRows * kWgradRows;
     p.splits = (int)((rows + p.split_rows - 1) / p.split_rows);
     return p;
@@ -204,6 +208,11 @@ bool block_wgrad_supported(long long rows, int E, int N) {
 size_t block_wgrad_workspace_bytes(long long rows, int E, int N, int E2) {
     const WgradPlan p = wgrad_plan(rows, wgrad_blocks(E) + (E2 > 0 ? wgrad_blocks(E2) : 0));
     return p.splits > 1 ? (size_t)p.splits * (E + E2) * N * sizeof(float) : 0;
+}
+
+size_t block_wgrad_workspace_bound(long long rows, int E, int N, int E2) {
+    const long long most = wgrad_most_splits(rows, wgrad_blocks(E) + (E2 > 0 ? wgrad_blocks(E2) : 0));
+    return most > 1 ? (size_t)most * (E + E2) * N * sizeof(float) : 0;
 }
 
 // Both weight gradients of a block in one launch: the blocks of both share one round of workgroups, and a few rows' partial

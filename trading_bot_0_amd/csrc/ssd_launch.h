@@ -168,6 +168,8 @@ hipError_t launch_block_weights(int E, int D, int DI, const float *in_proj, cons
 // multiple of 8) and b [rows, N] in bf16; E a multiple of 8, N 128 or 256.  workspace: the partial sums.
 bool block_wgrad_supported(long long rows, int E, int N);
 size_t block_wgrad_workspace_bytes(long long rows, int E, int N, int E2 = 0);
+// what the caller is asked for: no less for more rows (rounded to whole steps, the rows of a split make fewer splits now and then)
+size_t block_wgrad_workspace_bound(long long rows, int E, int N, int E2 = 0);
 // two over the same rows in one launch (with E2 in the workspace's size; the second's E may be 0)
 struct WgradArgs {
     const void *a = nullptr, *b = nullptr;
