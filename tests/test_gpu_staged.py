@@ -188,3 +188,16 @@ def test_float32_result_does_not_depend_on_the_scratch(batch, seqlen, dims):
     with pytest.raises(ssd.SsdError, match="workspace") as e:
         call(torch.empty(least - 256, dtype=torch.uint8, device="cuda"))
     assert e.value.code == 3
+
+
+def test_state_passing_over_more_threads_than_one_dimension_of_a_launch():
+    """2^31 state elements of one chunk each, and a few more: as many threads as a launch may not have along one dimension.  Without
+    decay the state entering is the initial one and the final one the sum, one number per sequence."""
+    B, H, P, N = 2 ** 15 + 3, 8, 64, 128
+    number = torch.arange(B, device="cuda", dtype=torch.float32)
+    S, init = (torch.empty(B, 1, H, P, N, device="cuda").copy_((f * number).view(B, 1, 1, 1, 1)) for f in (1.0, 0.5))
+    prev, fin = ssd.state_passing(S, torch.zeros(B, H, 1, 4, 32, device="cuda"), init[:, 0], in_place=True)
+    assert prev.data_ptr() == S.data_ptr()
+    for got, f in ((prev, 0.5), (fin, 1.5)):
+        rows = got.view(B, -1)
+        assert torch.equal(rows.amax(1), f * number) and torch.equal(rows.amin(1), f * number)

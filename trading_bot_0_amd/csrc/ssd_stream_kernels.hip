@@ -350,9 +350,24 @@ hipError_t launch_chunk_cumsum(const ScanShape &s, int dtype, const void *dt, co
 template <bool LOG>
 static hipError_t pass_dispatch(const ScanShape &s, const float *states, const PassDecays &a, const float *init, float *prev,
                                 float *final_states, hipStream_t st) {
-    const long long blocks = (long long)s.B * s.H * (s.P * s.N / 4 / kPassPieces);
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)blocks), block(kPassSegs * kPassPieces);
+    // A launch takes fewer than 2^32 threads along a dimension, which 2^31 state elements are (8.6 GB: 32 768 sequences of 8 heads of 64
+    // with a state of 128): more sequences than make 2^22 workgroups run in parts.
+    const int per_sequence = s.H * (s.P * s.N / 4 / kPassPieces), most = std::max(1, (1 << 22) / per_sequence);
+    if (s.B > most) {
+        const long long state = (long long)s.H * s.P * s.N;
+        for (int b0 = 0; b0 < s.B; b0 += most) {
+            ScanShape part = s;
+            part.B = std::min(most, s.B - b0);
+            if (s.fresh != nullptr) part.fresh = s.fresh + (size_t)b0 * s.L;
+            PassDecays pa = a;
+            pa.of += b0 * a.b;
+            const hipError_t e = pass_dispatch<LOG>(part, states + b0 * s.nc * state, pa, init ? init + b0 * state : nullptr,
+                                                    prev + b0 * s.nc * state, final_states ? final_states + b0 * state : nullptr, st);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    const dim3 grid((unsigned)(s.B * per_sequence)), block(kPassSegs * kPassPieces);
     // as short runs as cover the sequence in one round, where eight do
     if (s.nc <= kPassSegs) state_passing_kernel<1, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
     else if (s.nc <= 2 * kPassSegs) state_passing_kernel<2, LOG><<<grid, block, 0, st>>>(states, a, init, prev, final_states, s);
