@@ -322,3 +322,24 @@ def test_groups_of_four_units_take_the_one_pass_kernel(heads):
     assert_close(y32[rows], yr, torch.bfloat16, "four-wave one-pass y (float32 y)")
     assert_close(final[rows], fr, torch.bfloat16, "four-wave one-pass final")
     assert_stored_bf16_close(y16[rows], yr, "four-wave one-pass stored y")
+
+
+@pytest.mark.parametrize("dstate", [32, 64])
+def test_float32_state_takes_few_roundings_a_tile(dstate):
+    """A state between one and two that does not decay, to which every step adds little of either sign: each float32 addition onto it is a
+    rounding of at most 2^-24, with a root mean square of 2^-24 / sqrt(3).  A tile of 32 steps may round five times (what the leading
+    terms leave, then two matrix instructions of sixteen steps, each of which accumulates eight products at a time), so the error after n
+    tiles has a root mean square of sqrt(5 n) of that; a tenth is left for the products' own error.  (All twelve instructions of a tile accumulated onto the state make it sqrt(24 n).)"""
+    B, L, H, P = 8, 8192, 8, 32
+    g = torch.Generator(device="cuda").manual_seed(dstate)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, Bm, Cm = rnd(B, L, H, P), 2e-4 * rnd(B, L, 1, dstate), rnd(B, L, 1, dstate)
+    dt, A = torch.ones(B, L, H, device="cuda"), torch.full((H,), -1e-30, device="cuda")
+    init = 1.25 + 0.5 * torch.rand(B, H, P, dstate, generator=g, device="cuda")
+    _, final = ssd_chunk_scan_onepass(x, dt, A, Bm, Cm, None, chunk=64, initial_states=init)
+    ref = init.double() + torch.matmul(x.double().permute(0, 2, 3, 1).contiguous(), Bm.double()[:, :, 0].unsqueeze(1))
+    assert bool((ref > 1).all()) and bool((ref < 2).all())
+    rms = (final.double() - ref).square().mean().sqrt().item()
+    bound = 1.1 * (5 * L / 32) ** 0.5 * 2.0 ** -24 / 3 ** 0.5
+    print(f"{rms / bound:.2f} of the bound")
+    assert rms <= bound

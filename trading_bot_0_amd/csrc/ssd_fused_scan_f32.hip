@@ -86,15 +86,19 @@ struct Bits3 {
 };
 
 // c += a . b to float precision; the small products first
-__device__ inline f32x16 mma6(const Frag3 &a, const Frag3 &b, f32x16 c) {
+__device__ inline f32x16 mma5(const Frag3 &a, const Frag3 &b, f32x16 c) {  // all but the product of the leading terms
     c = mma32(a.t[2], b.t[0], c);
     c = mma32(a.t[0], b.t[2], c);
     c = mma32(a.t[1], b.t[1], c);
     c = mma32(a.t[1], b.t[0], c);
     c = mma32(a.t[0], b.t[1], c);
-    c = mma32(a.t[0], b.t[0], c);
     return c;
 }
+__device__ inline f32x16 mma6(const Frag3 &a, const Frag3 &b, f32x16 c) { return mma32(a.t[0], b.t[0], mma5(a, b, c)); }
+
+// Keeps the registers of v from being given to what is computed from it just before (a sum that is wanted in the registers of its other
+// operand, from one iteration of a loop to the next: else 32 moves per tile take it back).
+__device__ inline void still_in_use(const f32x16 &v) { asm volatile("" ::"v"(v)); }
 
 // STATES_ONLY: no outputs, no C: the state a segment of the sequence leaves behind from a zero state, into
 // final_states [B, segments, H, P, N], and the segment's total decay into seg_decay [B, segments, H] -- for sequences
@@ -413,11 +417,17 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fused_scan_f32_kernel(
         // (the forward's last tile of a segment other than the last, or of a call that asks for no final state)
         if (!STATES_ONLY && c + 1 == c_end && !(final_states != nullptr && seg == S - 1)) break;
         seg_total *= a_end;
+        // What the tile adds but for the products of the leading terms is summed from zero and added to the decayed state, then those two:
+        // an instruction rounds after every eight products, so five roundings of the state's size, where all twelve accumulated onto the
+        // state make 24 (96 x 1 999 steps, 8 heads of 32, state 64, steep decays, against float64: final state 1.62e-7 -> 1.02e-7, y
+        // 1.19e-7 -> 0.97e-7; 248 us either way, with the sum of one half of the columns beside the products of the other, else 251).
+        f32x16 add[NB];
+        Frag<T> xw_lead[Q / 16], b_lead[Q / 16][NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) st[nb] = st[nb] * a_end;
+        for (int nb = 0; nb < NB; ++nb) add[nb] = f32x16{0};
 #pragma unroll
-        for (int ks = 0; ks < Q; ks += 16) {
-            const int k0 = ks + 8 * half;
+        for (int k = 0; k < Q / 16; ++k) {
+            const int k0 = 16 * k + 8 * half;
             // (w o x)[l = k0 .. k0+7, p = r]
             const float4 wa = *reinterpret_cast<const float4 *>(w_s + k0);
             const float4 wb = *reinterpret_cast<const float4 *>(w_s + k0 + 4);
@@ -428,16 +438,23 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fused_scan_f32_kernel(
                 split3_pair(xf[xfloat_off(k0 + 2 * i, r)] * wv[2 * i], xf[xfloat_off(k0 + 2 * i + 1, r)] * wv[2 * i + 1],
                             xw.t[0].u[i], xw.t[1].u[i], xw.t[2].u[i]);
             const Frag3 xwf = xw.frags();
+            xw_lead[k] = xwf.t[0];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 Frag3 bf;  // B^T[n = 32 nb + r, l = k0 .. k0+7]
 #pragma unroll
                 for (int t = 0; t < 3; ++t) {
-                    const bf16x4 lo4 = BT::tr_read(Bs + t * TB + BT::tr_off(ks + 8 * half, nb * 32, lane));
-                    const bf16x4 hi4 = BT::tr_read(Bs + t * TB + BT::tr_off(ks + 8 * half + 4, nb * 32, lane));
+                    const bf16x4 lo4 = BT::tr_read(Bs + t * TB + BT::tr_off(k0, nb * 32, lane));
+                    const bf16x4 hi4 = BT::tr_read(Bs + t * TB + BT::tr_off(k0 + 4, nb * 32, lane));
                     bf.t[t].v = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
                 }
-                st[nb] = mma6(bf, xwf, st[nb]);
+                add[nb] = mma5(bf, xwf, add[nb]);
+                b_lead[k][nb] = bf.t[0];
+                if (k + 1 < Q / 16) continue;
+                st[nb] = st[nb] * a_end + add[nb];  // (beside the products of the next 32 columns)
+                still_in_use(add[nb]);
+#pragma unroll
+                for (int i = 0; i < Q / 16; ++i) st[nb] = mma32(b_lead[i][nb], xw_lead[i], st[nb]);
             }
         }
     }
