@@ -140,7 +140,8 @@ def test_weights_converted_in_one_launch(shape):
 
 
 @pytest.mark.parametrize("dims,B,L", [((256, 8, 32, 64, 1), 3, 77), ((256, 8, 32, 64, 1), 9, 2100), ((128, 8, 16, 16, 2), 2, 300),
-                                      ((256, 16, 16, 32, 1), 1, 1)])
+                                      ((256, 16, 16, 32, 1), 1, 1), ((128, 8, 32, 64, 1), 2, 300), ((256, 8, 16, 16, 1), 3, 700),
+                                      ((256, 8, 16, 16, 1), 4, 4096)])  # (d_model unlike nheads headdim: a launch per weight gradient)
 @pytest.mark.parametrize("kind", ["plain", "reset", "state", "no D"])
 def test_whole_passes_in_one_call_are_the_stages(dims, B, L, kind):
     """Forward (with what it keeps, or with a carried state) and backward as one call each against the same stages called one by
