@@ -5,7 +5,8 @@ The model's constants are measurements that every kernel change moves; this test
 cross-overs, the plan's choice beside the alternatives a caller can force -- the one-pass kernel
 (ssd_chunk_scan_onepass_fwd), the staged kernels through their own entry points, and a batch of more than a round of
 workgroups as two calls, its whole rounds as one launch and the rest as the plan says for it -- and asserts that what the
-plan picked is within a quarter of the fastest of them (a wrong side of a cross-over costs a factor of about two).
+plan picked is within a quarter of the fastest of them, but for 5 us of launches in all but the shortest calls (a wrong side of a
+cross-over costs a factor of about two).
 
 Timing: the best of three means over twenty calls, HIP events on the launch stream, after a spin of the same work."""
 from ctypes import byref
@@ -39,6 +40,10 @@ SHAPES = [
     # (nheads, headdim, dstate, ngroups, seqlen, batches either side of the cross-overs)
     (8, 32, 64, 1, 2048, "bf16", (4, 16, 32, 64, 128, 160, 256, 272)),   # staged | segments | one launch | whole rounds + a rest
     (8, 32, 64, 1, 512, "bf16", (16, 64, 128, 256)),
+    (8, 32, 64, 1, 64, "bf16", (1, 16, 40)),                             # as short as the launches themselves
+    (4, 32, 64, 1, 96, "bf16", (1, 16, 40)),
+    (8, 32, 32, 1, 128, "bf16", (1, 16, 40)),
+    (8, 32, 32, 1, 64, "f32", (1, 16, 40)),
     (8, 32, 64, 1, 8192, "bf16", (24, 130, 170, 250)),                   # more than half a round of long sequences: uncut
     (4, 32, 64, 1, 2048, "bf16", (32, 64, 128, 192, 256, 512)),          # four units per group: staged | four-wave one-pass
     (16, 64, 128, 2, 4096, "bf16", (1, 4, 8, 16)),                       # 128-wide state
@@ -96,6 +101,6 @@ def test_plan_picks_a_path_within_a_quarter_of_the_fastest(H, P, N, G, L, dtype,
         one = ssd.chunk_scan_is_onepass(Bsz, L, H, P, N, G, w.chunk, td)
         chosen = "one launch" if one else (f"{segs} segments" if segs > 1 else "staged / split")
         report.append(f"batch {Bsz}: plan ({chosen}) {t_plan:.0f} us; " + ", ".join(f"{k} {v:.0f}" for k, v in times.items()))
-        assert t_plan <= 1.25 * fastest + 5.0, "\n".join(report)
+        assert t_plan <= 1.25 * fastest + (5.0 if L > 128 else 1.0), "\n".join(report)
         del plan, inp, x, dt, Bm, Cm, y, fin, dtcs, prev
     print("\n".join(report))
