@@ -18,11 +18,13 @@ POLICY, LONG = (8, 32, 64, 1, 128), (16, 64, 128, 2, 256)  # heads, head dimensi
 
 # (batch, seqlen, heads, headdim, dstate, groups, chunk): one chunk; a batch of the recurrence and one over (2, 3, 4, 5 chunks);
 # the last chunk of one step; heads of 8, 24 and 64; every state width; more chunks than are folded (33), than one round of the
-# separate recurrence holds (65) and a run of it that is cut short (18); more tiles, and more bytes, than are folded
+# separate recurrence holds (65) and a run of it that is cut short (18); more tiles, and more bytes, than are folded; one sequence's chunks
+# one after the other as fast as a launch (4 and 6 of 16 KB) and slower (7 and 12)
 SHAPES = [(1, 1, 1, 8, 16, 1, 32), (3, 70, 4, 24, 16, 1, 128), (2, 129, 2, 64, 128, 1, 64), (2, 161, 8, 32, 64, 1, 32),
           (2, 320, 4, 16, 32, 2, 64), (1, 130, 3, 40, 128, 3, 128), (2, 33 * 32, 2, 16, 16, 1, 32), (1, 65 * 32 - 5, 2, 32, 64, 1, 32),
           (2, 18 * 64 - 63, 2, 8, 64, 2, 64), (70, 8 * 64, 8, 16, 16, 1, 64), (3, 256 * 3 + 1, 16, 64, 128, 2, 256),
-          (3, 290, 8, 32, 64, 1, 128)]
+          (3, 290, 8, 32, 64, 1, 128), (1, 250, 8, 64, 64, 1, 64), (1, 380, 8, 64, 64, 1, 64), (1, 400, 8, 64, 64, 1, 64),
+          (1, 12 * 64, 8, 64, 64, 1, 64)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)

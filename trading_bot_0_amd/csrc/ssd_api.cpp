@@ -161,12 +161,19 @@ int static_scratch_address(void **out) {
 // against separate (us of the GPU): 8 heads of 32, state 64, 3 x 300 steps 13.1 / 16, 8 x 2 048 (64 MB of reads) 24.1 / 30.3, 20 x 1 000
 // 29.2 / 37.2, 4 x 4 096 (134 MB) 31.7 / 29.9; 4 heads of 16, state 16, 20 x 2 000 (32 chunks) 31.2 / 32.6, 100 x 1 000 (6 400 tiles)
 // 66.2 / 62.5; 16 heads of 64, state 128, 4 x 2 000 (67 MB) 51.7 / 59.5, 2 x 4 000 (134 MB) 62.2 / 57.4.
+// The last chunk's tile reads one chunk's state after the other, 36 KB per us (45 in float32 on chunks of 128 and more): where few
+// sequences have many chunks or wide states that takes longer than the launch does, about 2 us and its own reads and writes at 1 MB
+// per us.  Folded against separate, one sequence of 8 heads of 64, state 64, 6 chunks 17.4 / 17.0, 12 22.2 / 17.9, 28 33.4 / 20.5, four
+// sequences 12 23.5 / 26.1, float32 one 8 28.6 / 28.6, 16 31.9 / 30.0, two 16 32.5 / 33.2; 8 heads of 32, one sequence 8 15.4 / 15.6, 16
+// 17.3 / 16.0, 32 21.5 / 17.2, two 16 17.0 / 17.2, 32 23.5 / 21.7, four 24 23.7 / 26.0; 16 heads of 64, state 128, one 4 26.0 / 26.8, 5 26.2 /
+// 28.1, 8 32.6 / 29.3, 16 40.5 / 34.9; 4 heads of 16, state 16, one 32 13.9 / 14.1.
 constexpr int kFoldMaxChunks = 32, kFoldMaxTiles = 4096;
 constexpr int64_t kFoldMaxBytes = (int64_t)72 << 20;
 
-bool fold_states(const ssd::ScanShape &s) {
-    const int64_t tiles = (int64_t)s.B * s.H * s.nc;
-    return s.nc <= kFoldMaxChunks && tiles <= kFoldMaxTiles && tiles * (s.nc / 2) * s.P * s.N * 4 <= kFoldMaxBytes;
+bool fold_states(const ssd::ScanShape &s, int dtype) {
+    const int64_t tiles = (int64_t)s.B * s.H * s.nc, state_bytes = (int64_t)s.P * s.N * 4;
+    if (s.nc > kFoldMaxChunks || tiles > kFoldMaxTiles || tiles * (s.nc / 2) * state_bytes > kFoldMaxBytes) return false;
+    return s.nc * state_bytes / (dtype == SSD_DTYPE_F32 && s.Q >= 128 ? 45e3 : 36e3) <= 2.0 + tiles * state_bytes / 1e6;
 }
 
 // The forward in two or three launches, stages 2 and 4 working out the decays themselves (short batches are bound by launches,
@@ -193,7 +200,7 @@ int run_staged_own(const ssd::ScanShape &s, int dtype, const void *x, const void
     const size_t state_floats = (size_t)s.B * s.H * s.P * s.N;
     const bool in_place = initial_states != nullptr && final_states != nullptr && initial_states < final_states + state_floats &&
                           final_states < initial_states + state_floats;
-    own.fold = !keep_prev && !in_place && fold_states(s);
+    own.fold = !keep_prev && !in_place && fold_states(s, dtype);
     own.init = initial_states;
     own.final_states = final_states;
     if (!own.fold) {

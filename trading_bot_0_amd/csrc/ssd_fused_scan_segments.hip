@@ -31,11 +31,12 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // 10 x 3 000 87 / 86, of 128, 3 x 300 16 / 22, 2 x 9 000 63 / 72, 20 x 1 000 69 / 72, 10 x 3 000 97 / 102, 100 x 300 118 / 117, of 256, 3 x 300
 // 36 / 40, 2 x 9 000 99 / 111, 10 x 3 000 144 / 145.
 // However little there is to do, their launches take 12.4 to 16 us (128-wide state 21).  What stands here is a little above the estimate for
-// as many of the one-pass kernel's tiles as take no longer: two of 64 steps, or of 32 in float32, and four of a 128-wide state.  One sequence,
-// staged / one-pass: 8 heads of 32, state 64, 64 steps 12.7 / 9, 128 steps 13.0 / 13.0, 160 12.8 / 17.2; state 32, 128 steps 12.6 / 10.7, 160
+// as many of the one-pass kernel's tiles as are faster: one of 64 steps, two of state 32, of workgroups of four waves and, of 32 steps, in
+// float32, four of a 128-wide state.  One sequence, staged / one-pass: 8 heads of 32, state 64, 64 steps 12.7 / 9, 128 steps 13.0 / 13.0 (from
+// a carried state 13.0 / 14.8); state 32, 128 steps 12.6 / 10.7, 160
 // 12.5 / 14.7; 4 heads, 128 steps 12.0 / 10.0, 160 12.8 / 13.5; 16 heads of 64, state 128, 192 steps 22.0 / 16.7, 256 22.2 / 20.6, 320 22.1 /
 // 24.5; float32, 64 steps, state 64 16.0 / 15.0, state 32 14.1 / 11.8, 96 steps 15.9 / 20.0 and 13.8 / 15.8.
-double staged_least_us(const ScanShape &s, int dtype) { return dtype == 0 ? 15.7 : s.N == 128 ? 22.0 : s.N == 32 ? 16.0 : 14.3; }
+double staged_least_us(const ScanShape &s, int dtype) { return dtype == 0 ? 15.7 : s.N == 128 ? 22.0 : s.N == 32 ? 16.0 : 13.5; }
 
 double staged_us(const ScanShape &s, int dtype, long long groups, int full) {
     const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
