@@ -104,3 +104,19 @@ def test_plan_picks_a_path_within_a_quarter_of_the_fastest(H, P, N, G, L, dtype,
         assert t_plan <= 1.25 * fastest + (5.0 if L > 128 else 1.0), "\n".join(report)
         del plan, inp, x, dt, Bm, Cm, y, fin, dtcs, prev
     print("\n".join(report))
+
+
+@pytest.mark.parametrize("H,P,N,L,few,more", [(4, 32, 64, 320, 1, 2), (4, 64, 64, 300, 3, 4), (4, 16, 16, 290, 5, 6)])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_fewer_sequences_take_no_longer(H, P, N, L, few, more, dtype):
+    """Staged calls whose tiles all have a workgroup of their own: a number of tiles that is no multiple of the eight XCDs (12, 36 and 60 or
+    100) takes what the next one that is takes (24, 48 and 72 or 120), a tenth and half a microsecond allowed, not one more tile of 6 us."""
+    times = []
+    for Bsz in (few, more):
+        w = Workload("plan", Bsz, L, H, P, N, 1, 128 if P * N > 2048 or dtype == "bf16" and P > 16 else 64, dtype=dtype)
+        inp = make_inputs(w, seed=1, device="cuda")
+        times.append(best_of(ssd.PreparedChunkScan(*(inp[k] for k in ("x", "dt", "A", "B", "C", "D")), chunk=w.chunk)))
+        assert ssd.chunk_scan_segments(Bsz, L, H, P, N, 1, w.chunk, w.torch_dtype) == 1
+        assert not ssd.chunk_scan_is_onepass(Bsz, L, H, P, N, 1, w.chunk, w.torch_dtype)
+    print(times)
+    assert times[0] <= 1.1 * times[1] + 0.5

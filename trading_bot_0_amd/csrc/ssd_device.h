@@ -641,8 +641,9 @@ static inline hipError_t device_cu_count(int dev, int *cus) {
     return e;
 }
 
-// Workgroups of a persistent kernel: as many as stay resident on the current device, in whole
-// multiples of the 8 XCDs, never more than there are tiles.
+// Workgroups of a persistent kernel: one per tile where all of them stay resident on the current device, else as many as do, in
+// whole multiples of the 8 XCDs.  (Rounded down with few tiles, some workgroups walk two: 4 heads of 32, one sequence of 320 steps, 12
+// tiles, 19.5 us instead of 13.4.)
 template <typename K>
 static inline hipError_t persistent_grid(K kernel, int block, size_t lds, int tiles, int *grid) {
     int dev = 0, cus = 0;
@@ -666,8 +667,8 @@ static inline hipError_t persistent_grid(K kernel, int block, size_t lds, int ti
         launch_facts().keep(kp, key, per_cu);
     }
     long long g = (long long)cus * per_cu;
-    if (g > tiles) g = tiles;
-    if (g >= 8) g -= g % 8;
+    if (g >= tiles) g = tiles;
+    else if (g >= 8) g -= g % 8;
     *grid = (int)(g < 1 ? 1 : g);
     return hipSuccess;
 }
