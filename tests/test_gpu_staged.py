@@ -143,11 +143,12 @@ def test_forward_without_a_workspace_past_the_scratch_array(batch, seqlen, dims)
 
 @pytest.mark.parametrize("batch,seqlen,dtype,dims", [(24, 2100, "bf16", POLICY), (16, 4100, "bf16", POLICY), (90, 1030, "bf16", POLICY),
                                                      (90, 2500, "bf16", POLICY), (20, 4000, "f32", POLICY), (96, 1999, "f32", POLICY),
-                                                     (60, 1001, "f32", POLICY), (4, 4000, "bf16", LONG), (8, 2060, "bf16", LONG),
+                                                     (60, 1001, "f32", POLICY), (24, 2100, "f32", POLICY), (28, 2907, "f32", POLICY),
+                                                     (12, 2700, "f32", (8, 32, 32, 1, 64)), (16, 4100, "f32", (8, 32, 32, 1, 64)), (4, 4000, "bf16", LONG), (8, 2060, "bf16", LONG),
                                                      (7, 4097, "bf16", LONG), (30, 2500, "bf16", (4, 32, 128, 1, 64))])
 def test_forward_on_segments(batch, seqlen, dtype, dims):
-    """Cuts into a few segments (states entering them worked out in the prologues), into eight and more (in a launch of their own) and
-    over two rounds of workgroups, a 128-wide state (two waves per unit), with restarts, a row whose initial state is not read, and
+    """Cuts into a few segments (states entering them worked out in the prologues), into eight and more (in a launch of their own; in
+    float32 from nine, or fourteen of a 32-wide state) and over two rounds of workgroups, a 128-wide state (two waves per unit), with restarts, a row whose initial state is not read, and
     ragged last segments."""
     w = Workload("segments", batch, seqlen, *dims, dtype=dtype, init_std=0.5)
     assert ssd.chunk_scan_segments(batch, seqlen, *dims, w.torch_dtype) > 1

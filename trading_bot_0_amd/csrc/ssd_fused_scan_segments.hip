@@ -1,9 +1,11 @@
 // One-pass forward for batches too small to fill the chip with one workgroup per 8 units (4 of a 128-wide state): the sequence is cut
 // into segments that different workgroups walk side by side.
 //   1. states only (no y, no C): what every segment adds to the state, from a zero state, and its total decay;
-//   2. the forward proper per segment; each workgroup first runs the recurrence over the states of the segments
-//      before its own (a few fused multiply-adds per state element), which gives the state entering its segment.
-// Step 1 costs about 0.4 of step 2 (staging, scan and the state update, without the output phase); the two
+//   2. where segments are many, or their number is small but the state is continued in place or 128 wide: the states entering the
+//      segments, by a launch of their own (launch_segment_passing);
+//   3. the forward proper per segment, from those or, without step 2, from what each workgroup works out first: the recurrence
+//      over the states of the segments before its own (a few fused multiply-adds per state element).
+// Step 1 costs about 0.4 of step 3 (staging, scan and the state update, without the output phase); the two
 // together run S times as many workgroups as the uncut kernel.
 #include "ssd_fused_scan.h"
 
@@ -14,10 +16,11 @@ namespace {
 constexpr int kSegmentMinTiles = 4;   // shorter segments are mostly prologue (and their states would not fit chunks of 256 steps)
 constexpr int kSegmentMaxGroups = 768;  // three rounds of workgroups
 // From so many segments on the states entering them are worked out by a launch of their own instead of in every workgroup's
-// prologue, which reads those of all segments before it.  One by one / in a launch, us: 16 x 4 096 on 16 67 / 50, 24 x 4 096 on 8
-// 76 / 71, 24 x 2 048 on 8 51 / 46; 48 x 4 096 on 5 99 / 105, 61 x 3 999 on 4 120 / 127; float32 20 x 4 000 on 8 134 / 133, 60 x 1 000 on
-// 4 79 / 87.
-constexpr int kPassMinSegments = 8;
+// prologue, which reads those of all segments before it.  One by one / in a launch, us: 8 heads of 32, state 64, 16 x 8 192 on 16 90 /
+// 74, 24 x 8 192 on 8 121 / 118, 16 x 2 907 on 7 60 / 57, 32 x 2 907 on 7 65.3 / 65.1, on 6 68 / 70; state 32 16 x 8 192 on 8 98 / 96, 32 x
+// 2 907 on 7 53.5 / 54.6; float32 12 x 8 192 on 12 183 / 174, 20 x 2 907 on 9 101 / 99, 24 x 8 192 on 8 260 / 262, 32 x 2 907 on 8 113 / 116,
+// 42 x 2 907 on 6 141 / 150, state 32 16 x 8 192 on 16 124 / 121, 20 x 8 192 on 12 150 / 152, 24 x 8 192 on 10 180 / 187, 32 x 8 192 on 8 238 / 245.
+int pass_min_segments(const ScanShape &s, int dtype) { return dtype != 0 ? 8 : s.N == 32 ? 14 : 9; }
 
 int tiles_of(const ScanShape &s) { return (s.L + kOnePassTile - 1) / kOnePassTile; }
 int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1) / fused_scan_f32_tile(); }
@@ -68,8 +71,9 @@ double segments_us(const ScanShape &s, int dtype, long long groups, int segments
     // (several rounds a tenth dearer than fitted: how they fall varies, 132 x 4 096 on 5 296 where the uncut kernel takes 287, 170 x 8 192
     // on 3 647 / 583, float32 104 x 3 999 on 7 496, on 2 477)
     const double fall = rounds > 1.0 ? 1.12 : 1.0;
-    if (dtype == 0) return fall * (6.0 + (segments < kPassMinSegments ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more);
-    return fall * (12.0 + (segments < kPassMinSegments ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more);
+    const bool few = segments < 8;  // (from here on as long with the entering states in a launch, which it is from about there)
+    if (dtype == 0) return fall * (6.0 + (few ? 3.0 * segments : 10.0) + 7.45 * tiles + 19.0 * more);
+    return fall * (12.0 + (few ? 1.9 * segments : 8.0) + 6.1 * tiles + 18.0 * more);
 }
 // the fastest cut of nc tiles into segments of min_tiles or more, by that estimate; in bf16 a power of two unless another is clearly
 // faster (the estimate is good to a few per cent, and programs size and compare by the number of segments)
@@ -175,7 +179,7 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
     // could have replaced by then: those calls have the entering states worked out ahead as well)
     const size_t state_floats = (size_t)s.B * s.H * s.P * s.N;
     const bool in_place = init != nullptr && final_states != nullptr && init < final_states + state_floats && final_states < init + state_floats;
-    const bool passed = segments >= kPassMinSegments || in_place;
+    const bool passed = segments >= pass_min_segments(s, dtype) || in_place;
     if (dtype == 0)
         return launch_fused_scan_f32_segmented(s, segments, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states,
                                                seg_decay, passed, st);
