@@ -33,24 +33,28 @@ int float_tiles_of(const ScanShape &s) { return (s.L + fused_scan_f32_tile() - 1
 // 112 / 111, 8 x 4 000 187 / 172, 16 x 4 000 360 / 369; float32 on chunks of 64, 3 x 300 14 / 18, 2 x 9 000 57 / 60, 20 x 1 000 63 / 65,
 // 10 x 3 000 87 / 86, of 128, 3 x 300 16 / 22, 2 x 9 000 63 / 72, 20 x 1 000 69 / 72, 10 x 3 000 97 / 102, 100 x 300 118 / 117, of 256, 3 x 300
 // 36 / 40, 2 x 9 000 99 / 111, 10 x 3 000 144 / 145.
+double staged_work_us(const ScanShape &s, int dtype, long long groups, int full) {
+    const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
+    const double whole_chunks = (double)s.nc * s.Q / ((double)tiles_of(s) * kOnePassTile);  // (a chunk runs whole: 600 steps 3 of 256)
+    if (dtype == 0) {
+        if (s.Q <= 64) return 12.0 + 1310.0 * units;
+        return s.Q == 128 ? 13.0 + 1430.0 * units * whole_chunks : 30.0 + 1950.0 * units * whole_chunks;
+    }
+    if (s.N != 128) return 10.0 + 518.0 * units;
+    return 15.0 + 690.0 * units * whole_chunks;
+}
+
 // However little there is to do, their launches take 12.4 to 16 us (128-wide state 21).  What stands here is a little above the estimate for
 // as many of the one-pass kernel's tiles as are faster: one of 64 steps, two of state 32, of workgroups of four waves and, of 32 steps, in
 // float32, four of a 128-wide state.  One sequence, staged / one-pass: 8 heads of 32, state 64, 64 steps 12.7 / 9, 128 steps 13.0 / 13.0 (from
-// a carried state 13.0 / 14.8); state 32, 128 steps 12.6 / 10.7, 160
-// 12.5 / 14.7; 4 heads, 128 steps 12.0 / 10.0, 160 12.8 / 13.5; 16 heads of 64, state 128, 192 steps 22.0 / 16.7, 256 22.2 / 20.6, 320 22.1 /
+// a carried state 13.0 / 14.8); state 32, 128 steps 12.6 / 10.7, 160 12.5 / 14.7; 4 heads, 128 steps 12.0 / 10.0, 160 12.8 / 13.5; 16 heads of 64, state 128, 192 steps 22.0 / 16.7, 256 22.2 / 20.6, 320 22.1 /
 // 24.5; float32, 64 steps, state 64 16.0 / 15.0, state 32 14.1 / 11.8, 96 steps 15.9 / 20.0 and 13.8 / 15.8.
 double staged_least_us(const ScanShape &s, int dtype) { return dtype == 0 ? 15.7 : s.N == 128 ? 22.0 : s.N == 32 ? 16.0 : 13.5; }
 
 double staged_us(const ScanShape &s, int dtype, long long groups, int full) {
-    const double units = (double)groups * full * tiles_of(s) / (2048.0 * 32.0);
-    const double whole_chunks = (double)s.nc * s.Q / ((double)tiles_of(s) * kOnePassTile);  // (a chunk runs whole: 600 steps 3 of 256)
-    double us;
-    if (dtype == 0)
-        us = s.Q <= 64 ? 12.0 + 1310.0 * units : s.Q == 128 ? 13.0 + 1430.0 * units * whole_chunks : 30.0 + 1950.0 * units * whole_chunks;
-    else
-        us = s.N != 128 ? 10.0 + 518.0 * units : 15.0 + 690.0 * units * whole_chunks;
-    return std::max(us, staged_least_us(s, dtype));
+    return std::max(staged_work_us(s, dtype, groups, full), staged_least_us(s, dtype));
 }
+
 // the one-pass kernel: a round of 256 workgroups walks a tile in 4 (few of them) to 5.6 (at the power limit): 16 x 2 048 139 / 140,
 // 90 x 2 048 155 / 145, 256 x 2 048 187 / 185; state 128, 16 x 2 000 136 / 136, 16 x 4 000 263 / 266, 24 x 2 000
 // 143 / 138; float32 tiles of 32 steps, 70 x 100 26 / 27
@@ -163,11 +167,11 @@ int fused_scan_tail_rows(const ScanShape &s, int dtype) {
     tail.B = rest / per_row;
     const int tail_plan = fused_scan_plan(tail, dtype, &segments);
     if (tail_plan == 1) return 0;  // it would run as a round of the one-pass kernel anyway
-    // the remainder as its own batch against one more round
+    // the remainder as its own batch (its launches wait for the whole rounds anyway) against one more round
     const int nc = dtype == 0 ? float_tiles_of(s) : tiles_of(s);
     // (a 128-wide state's round of a few workgroups is a faster one: 48 x 2 000 steps of 16 heads of 64 271 us, 279 with the last 16 apart)
     const double round = whole_us(s, dtype, dtype != 0 && s.N == 128 ? rest : 256) - whole_us(s, dtype, 0);
-    const double cost = tail_plan == 2 ? segments_us(s, dtype, rest, segments, (nc + segments - 1) / segments) : staged_us(tail, dtype, rest, full);
+    const double cost = tail_plan == 2 ? segments_us(s, dtype, rest, segments, (nc + segments - 1) / segments) : staged_work_us(tail, dtype, rest, full);
     return cost + kTailLaunchUs < round ? tail.B : 0;
 }
 
