@@ -167,6 +167,28 @@ def test_forward_on_segments(batch, seqlen, dtype, dims):
     assert_close(f[rows], fr, w.torch_dtype, "final")
 
 
+@pytest.mark.parametrize("batch,seqlen,dtype,dims", [(90, 1024, "bf16", POLICY), (33, 2907, "bf16", POLICY), (50, 3001, "bf16", (16, 32, 32, 2, 128)),
+                                                     (33, 2100, "bf16", (8, 64, 64, 2, 64)), (96, 1999, "f32", POLICY), (42, 2907, "f32", POLICY),
+                                                     (33, 2907, "f32", (8, 32, 32, 1, 64)), (40, 2500, "f32", (8, 64, 64, 2, 64))])
+def test_state_continued_in_place_on_few_segments(batch, seqlen, dtype, dims):
+    """Where the prologues work out the entering states, a call that writes its final state over its initial one reads a copy of it: the
+    same bits as with separate buffers, several workgroups per sequence among them, with rows whose initial state is not read."""
+    w = Workload("inplace", batch, seqlen, *dims, dtype=dtype, init_std=0.5)
+    assert 1 < ssd.chunk_scan_segments(batch, seqlen, *dims, w.torch_dtype) < 8
+    dev = to_dev(make_inputs(w, seed=seqlen))
+    mask = torch.rand(batch, seqlen, generator=torch.Generator().manual_seed(6)) < 0.002
+    mask[0, 0] = True
+    dev["init"][0] = float("nan")
+    args = [dev[k] for k in ("x", "dt", "A", "B", "C", "D")]
+    y0, f0 = ssd_chunk_scan(*args, chunk=dims[4], initial_states=dev["init"], reset=mask.cuda())
+    assert bool(torch.isfinite(f0).all())
+    for _ in range(3):
+        state = dev["init"].clone()
+        y, f = ssd_chunk_scan(*args, chunk=dims[4], initial_states=state, final_out=state, reset=mask.cuda())
+        assert f.data_ptr() == state.data_ptr()
+        assert torch.equal(y, y0) and torch.equal(state, f0)
+
+
 @pytest.mark.parametrize("batch,seqlen,dims", [(3, 300, POLICY), (20, 1000, POLICY), (3, 300, (8, 16, 16, 1, 256)), (2, 700, (8, 64, 64, 1, 128))])
 def test_float32_result_does_not_depend_on_the_scratch(batch, seqlen, dims):
     """Float32 on the staged kernels: the same bits without a workspace, with one of the size the library names for the sizes as they

@@ -537,6 +537,19 @@ struct TileSched {
     __device__ void advance() { pos += step; }
 };
 
+// FLOATS floats from one place to another by a workgroup of THREADS, all loads in flight at once
+template <int FLOATS, int THREADS> __device__ inline void copy_state(const float *from, float *to) {
+    constexpr int PIECES = FLOATS / 4 / THREADS;
+    static_assert(PIECES * 4 * THREADS == FLOATS, "whole 16-byte pieces for every thread");
+    const float4 *f = reinterpret_cast<const float4 *>(from) + threadIdx.x;
+    float4 *t = reinterpret_cast<float4 *>(to) + threadIdx.x;
+    float4 v[PIECES];
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u) v[u] = f[u * THREADS];
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u) t[u * THREADS] = v[u];
+}
+
 struct Tile {
     int b, c, h, g, t0;
 };

@@ -248,8 +248,17 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     const int seg = slot % S, logical = slot / S;
     // states only: nothing comes after the last segment, so what it adds to the state is not needed (the final
-    // state comes from the forward over that segment) -- its workgroups leave at once
-    if (STATES_ONLY && S > 1 && seg == S - 1) return;
+    // state comes from the forward over that segment) -- its workgroups leave at once, or behind a copy of the initial state
+    if constexpr (STATES_ONLY) {
+        if (S > 1 && seg == S - 1) {
+            if (init != nullptr) {
+                const int groups = s.H * PBn / WAVES, row = logical / groups;  // (this workgroup's units: one contiguous piece)
+                const size_t piece = (size_t)(logical % groups) * (WAVES * 32) * N, states = (size_t)s.H * s.P * N;
+                copy_state<WAVES * 32 * N, 64 * WAVES>(init + row * states + piece, final_states + ((size_t)row * S + S - 1) * states + piece);
+            }
+            return;
+        }
+    }
     const int c_first = seg * (s.seg_tiles > 0 ? s.seg_tiles : s.nc);
     const int c_end = s.seg_tiles > 0 ? min(s.nc, c_first + s.seg_tiles) : s.nc;
     // transposed: the workgroup is heads h0 .. h0+7 (one per wave) on x slice pb; s.G == s.H there, and
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
         const size_t lane_off = (size_t)((pb + sl) * 32 + (lane0 & 31)) * N + 4 * (lane0 >> 5);
         // (one uniform branch around all of the state's loads: with a condition on each, the compiler waits for every
         // load before the next -- eight or sixteen trips to memory before the first tile)
-        const bool have_init = init != nullptr && !fresh;
+        const bool have_init = !STATES_ONLY && init != nullptr && !fresh;
         float4 iq[NB][4];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -448,7 +457,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 || NK == 8) ? 1 : 2) void f
             for (int gq = 0; gq < 4; ++gq) iq[nb][gq] = make_float4(0, 0, 0, 0);
         }
         if (have_init) {
-            const float *ib = init + (((size_t)b * (folded ? 1 : S) + (folded ? 0 : seg)) * s.H + h) * s.P * N + lane_off;
+            const float *ib = init + (((size_t)b * (folded ? s.seg_init_rows : S) + (folded ? 0 : seg)) * s.H + h) * s.P * N + lane_off;
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -1170,8 +1179,9 @@ static hipError_t fused_launch(const ScanShape &s, const void *x, const void *dt
     return hipGetLastError();
 }
 
-// States only (KIND 2, or 8 for the reversed-adjoint recurrence): per segment, the state it leaves behind from `init`
-// ([B,S,H,P,N] or NULL = zero) into seg_states [B,S,H,P,N] and its total decay into seg_decay [B,S,H].
+// States only (KIND 2, or 8 for the reversed-adjoint recurrence): per segment but the last, the state it leaves behind from
+// zero into seg_states [B,S,H,P,N] and its total decay into seg_decay [B,S,H].  With `init` [B,H,P,N] given, the last segment's
+// place in seg_states receives a copy of it.
 template <int NK, int QB, int WAVES, int KIND = 2>
 static hipError_t fused_launch_states(const ScanShape &s, const void *x, const void *dt, const float *A, const void *Bm,
                                       const float *init, const unsigned char *reset, float *seg_states, float *seg_decay,

@@ -141,8 +141,17 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fused_scan_f32_kernel(
     const int S = s.seg_tiles > 0 ? (nc + s.seg_tiles - 1) / s.seg_tiles : 1;
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     const int seg = slot % S, logical = slot / S;
-    // states only: nothing comes after the last segment, its workgroups leave at once
-    if (STATES_ONLY && S > 1 && seg == S - 1) return;
+    // states only: nothing comes after the last segment, its workgroups leave at once, or behind a copy of the initial state
+    if constexpr (STATES_ONLY) {
+        if (S > 1 && seg == S - 1) {
+            if (init != nullptr) {
+                const int groups = s.G * UW, row = logical / groups;  // (this workgroup's units: one contiguous piece)
+                const size_t piece = (size_t)(logical % groups) * (WAVES * 32) * N, states = (size_t)s.H * s.P * N;
+                copy_state<WAVES * 32 * N, nthr>(init + row * states + piece, final_states + ((size_t)row * S + S - 1) * states + piece);
+            }
+            return;
+        }
+    }
     const int c_first = seg * (s.seg_tiles > 0 ? s.seg_tiles : nc);
     const int c_end = s.seg_tiles > 0 ? min(nc, c_first + s.seg_tiles) : nc;
     const int b = logical / (s.G * UW), g = (logical / UW) % s.G, unit0 = (logical % UW) * WAVES;
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fused_scan_f32_kernel(
         const bool fresh = rsb != nullptr && rsb[0] != 0 && !(entered && seg > 0);
         const size_t lane_off = (size_t)(pb * 32 + r) * N + 4 * half;
         const float *ib = !STATES_ONLY && init && !fresh
-                              ? init + ((entered ? (size_t)b * S + seg : (size_t)b) * s.H + h) * s.P * N + lane_off : nullptr;
+                              ? init + ((entered ? (size_t)b * S + seg : (size_t)b * s.seg_init_rows) * s.H + h) * s.P * N + lane_off : nullptr;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -510,7 +519,7 @@ int fused_scan_f32_tile() { return kFloatTile; }
 hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, const void *x, const void *dt, const float *A,
                                            const void *Bm, const void *Cm, const float *D, const float *init,
                                            const unsigned char *reset, void *y, float *final_states, float *seg_states,
-                                           float *seg_decay, bool passed, hipStream_t st) {
+                                           float *seg_decay, bool passed, bool copied, hipStream_t st) {
     if (segments < 2 || fused_scan_f32_waves(s) != 8) return hipErrorInvalidValue;
     const int nc = (s.L + kFloatTile - 1) / kFloatTile;
     ScanShape t = s;
@@ -520,9 +529,9 @@ hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, con
     const float *xx = static_cast<const float *>(x), *dd = static_cast<const float *>(dt);
     const float *bb = static_cast<const float *>(Bm);
     if (s.N == 64)
-        fused_scan_f32_kernel<4, 8, true><<<dim3(grid), dim3(512), 0, st>>>(xx, dd, A, bb, bb, nullptr, nullptr, reset, nullptr, seg_states, seg_decay, t);
+        fused_scan_f32_kernel<4, 8, true><<<dim3(grid), dim3(512), 0, st>>>(xx, dd, A, bb, bb, nullptr, copied ? init : nullptr, reset, nullptr, seg_states, seg_decay, t);
     else
-        fused_scan_f32_kernel<2, 8, true><<<dim3(grid), dim3(512), 0, st>>>(xx, dd, A, bb, bb, nullptr, nullptr, reset, nullptr, seg_states, seg_decay, t);
+        fused_scan_f32_kernel<2, 8, true><<<dim3(grid), dim3(512), 0, st>>>(xx, dd, A, bb, bb, nullptr, copied ? init : nullptr, reset, nullptr, seg_states, seg_decay, t);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (passed) {
@@ -531,6 +540,10 @@ hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, con
     }
     t.seg_local = seg_states;
     t.seg_local_decay = seg_decay;
+    if (copied) {
+        init = seg_states + (size_t)(segments - 1) * s.H * s.P * s.N;
+        t.seg_init_rows = segments;
+    }
     return launch_fused_scan_f32(t, x, dt, A, Bm, Cm, D, init, reset, y, final_states, st);
 }
 

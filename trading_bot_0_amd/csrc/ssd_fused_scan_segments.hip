@@ -1,8 +1,8 @@
 // One-pass forward for batches too small to fill the chip with one workgroup per 8 units (4 of a 128-wide state): the sequence is cut
 // into segments that different workgroups walk side by side.
 //   1. states only (no y, no C): what every segment adds to the state, from a zero state, and its total decay;
-//   2. where segments are many, or their number is small but the state is continued in place or 128 wide: the states entering the
-//      segments, by a launch of their own (launch_segment_passing);
+//   2. where segments are many or the state is 128 wide: the states entering the segments, by a launch of their own
+//      (launch_segment_passing);
 //   3. the forward proper per segment, from those or, without step 2, from what each workgroup works out first: the recurrence
 //      over the states of the segments before its own (a few fused multiply-adds per state element).
 // Step 1 costs about 0.4 of step 3 (staging, scan and the state update, without the output phase); the two
@@ -179,14 +179,17 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
                                        const float *A, const void *Bm, const void *Cm, const float *D, const float *init,
                                        const unsigned char *reset, void *y, float *final_states, float *seg_states,
                                        float *seg_decay, hipStream_t st) {
-    // (a prologue reads the true initial state, which a final state written over it -- a stream's prefix continued in place --
-    // could have replaced by then: those calls have the entering states worked out ahead as well)
+    const bool passed = segments >= pass_min_segments(s, dtype);
+    // A prologue reads the true initial state, which a final state written over it -- a stream's prefix continued in place --
+    // could have replaced by then: there it reads a copy, which the states-only launch leaves in the last segment's place
+    // (one launch fewer than with the entering states worked out ahead, 90 x 1 024 on 2 78.2 -> 65.6 us, 128 x 2 048 on 2 141 -> 126, 48 x 4 096
+    // on 5 104.6 -> 99.1, float32 60 x 1 000 on 4 85.3 -> 77.6; separate buffers 65.5, 122.7, 99.2, 77.7).
     const size_t state_floats = (size_t)s.B * s.H * s.P * s.N;
     const bool in_place = init != nullptr && final_states != nullptr && init < final_states + state_floats && final_states < init + state_floats;
-    const bool passed = segments >= pass_min_segments(s, dtype) || in_place;
+    const bool copied = in_place && !passed;
     if (dtype == 0)
         return launch_fused_scan_f32_segmented(s, segments, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states,
-                                               seg_decay, passed, st);
+                                               seg_decay, passed, copied, st);
     if (segments < 2 || fused_scan_waves(s, dtype) != (s.N == 128 ? 4 : 8)) return hipErrorInvalidValue;
     ScanShape t = s;
     t.Q = kOnePassTile;
@@ -195,8 +198,8 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
     if ((t.nc + t.seg_tiles - 1) / t.seg_tiles != segments) return hipErrorInvalidValue;
     if (s.N == 128)
         return launch_fused_scan_wide_segmented(t, dtype, x, dt, A, Bm, Cm, D, init, reset, y, final_states, seg_states, seg_decay, st);
-    hipError_t e = t.N == 32 ? fused_launch_states<2, kOnePassTile / 32, 8>(t, x, dt, A, Bm, nullptr, reset, seg_states, seg_decay, st)
-                             : fused_launch_states<4, kOnePassTile / 32, 8>(t, x, dt, A, Bm, nullptr, reset, seg_states, seg_decay, st);
+    hipError_t e = t.N == 32 ? fused_launch_states<2, kOnePassTile / 32, 8>(t, x, dt, A, Bm, copied ? init : nullptr, reset, seg_states, seg_decay, st)
+                             : fused_launch_states<4, kOnePassTile / 32, 8>(t, x, dt, A, Bm, copied ? init : nullptr, reset, seg_states, seg_decay, st);
     if (e != hipSuccess) return e;
     // the forward per segment; its prologue runs the recurrence over the segment states
     ScanShape f = s;
@@ -207,6 +210,10 @@ hipError_t launch_fused_scan_segmented(const ScanShape &s, int dtype, int segmen
     }
     f.seg_local = seg_states;
     f.seg_local_decay = seg_decay;
+    if (copied) {
+        init = seg_states + (size_t)(segments - 1) * s.H * s.P * s.N;
+        f.seg_init_rows = segments;
+    }
     return launch_fused_scan(f, dtype, x, dt, A, Bm, Cm, D, init, reset, y, final_states, st);
 }
 

@@ -22,8 +22,10 @@ struct ScanShape {
     int seg_tiles = 0;
     // The forward on segments: what the states-only pass left, per segment but the last, [B, segments, H, P, N] (the
     // state a segment adds from zero) and [B, segments, H] (its total decay).  A workgroup's prologue runs the
-    // recurrence over the segments before its own, from the true initial state [B, H, P, N].
+    // recurrence over the segments before its own, from the true initial state [B, H, P, N], one batch row's seg_init_rows
+    // of [H, P, N] apart.
     const float *seg_local = nullptr, *seg_local_decay = nullptr;
+    int seg_init_rows = 1;
     // The staged kernels that read the initial state only: the restart mask [B, L] (or NULL).  A sequence that
     // restarts before its first step does not read its initial state at all, whatever that holds.
     const unsigned char *fresh = nullptr;
@@ -118,7 +120,7 @@ int fused_scan_f32_tile();  // time steps per tile of the float one-pass kernel
 hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, const void *x, const void *dt, const float *A,
                                            const void *Bm, const void *Cm, const float *D, const float *init,
                                            const unsigned char *reset, void *y, float *final_states, float *seg_states,
-                                           float *seg_decay, bool passed, hipStream_t st);
+                                           float *seg_decay, bool passed, bool copied, hipStream_t st);
 // fused_scan_plan: which way a forward of this shape runs fastest by the library's cost estimates: 0 = the
 // staged kernels, 1 = the one-pass kernel, 2 = the one-pass kernel on *segments segments.
 int fused_scan_plan(const ScanShape &s, int dtype, int *segments);
