@@ -77,7 +77,8 @@ __global__ __launch_bounds__(64 * QB, (is_bf16<T> && PB == 1 && NK <= 4 && QB >=
     Vec16<T> bv[UB], xv[UX];
     float4 hv[UH];
     // own.fold: `prev` holds what every chunk adds to the state, and a tile works out the state entering its chunk by the
-    // recurrence over the chunks before it (the float operations of state_passing_kernel in their order); the tile of the
+    // recurrence over the chunks before it, one after the other (up to eight chunks the float operations of state_passing_kernel in
+    // their order; with more that kernel combines runs of two and four, and the last bits differ); the tile of the
     // last chunk goes one chunk further, to the final state.  This thread's pieces idx0, idx0 + nthr, ...
     auto enter = [&](const Tile &t, int idx0, float4(&st)[UH]) __attribute__((always_inline)) {
         const size_t bh = (size_t)t.b * s.H + t.h;

@@ -83,7 +83,8 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(const T *__restrict__
 // 32 x 64: 4 sequences of 32 chunks 8.6 -> 5.5 us, 2 of 71 16.8 -> 9.1; 16 heads, 64 x 128, 4 of 16 chunks 12.6 -> 13.1).
 // The chunks' total decays: log2 (alpha at the chunk's end; LOG) or the factors themselves, chunk c of sequence (b, h) at
 // a.of[b * a.b + h * a.h + c * a.c].
-// prev may alias states: a thread reads its chunks before it writes them, and no other thread touches them;
+// prev may alias states: a thread reads its chunks before it writes them, and no other thread uses them (those past the
+// sequence read the last chunk, possibly after it has been written, and drop what they read);
 // final_states may alias init: it is written behind a barrier that all of the workgroup's reads of init precede.
 // ------------------------------------------------------------------------------------------
 constexpr int kPassSegs = 8, kPassPieces = 32;  // P * N / 4 is a multiple of 32 (P of 8, N of 16)
