@@ -102,7 +102,8 @@ __device__ inline void still_in_use(const f32x16 &v) { asm volatile("" ::"v"(v))
 
 // STATES_ONLY: no outputs, no C: the state a segment of the sequence leaves behind from a zero state, into
 // final_states [B, segments, H, P, N], and the segment's total decay into seg_decay [B, segments, H] -- for sequences
-// cut into segments of s.seg_tiles tiles (of 32 steps here) that different workgroups walk side by side.  The
+// cut into segments of s.seg_tiles tiles (of 32 steps here) that different workgroups walk side by side.  With init [B, H, P, N]
+// given, the last segment's place receives a copy of it.  The
 // forward on segments (s.seg_local set) starts every segment from the recurrence over those states, run in its
 // workgroups' prologue, as in the bf16 kernel.
 template <int NK, int WAVES, bool STATES_ONLY>  // dstate N = 16 NK

@@ -117,6 +117,8 @@ hipError_t launch_fused_scan_f32(const ScanShape &s, const void *x, const void *
                                  const void *Cm, const float *D, const float *init, const unsigned char *reset, void *y,
                                  float *final_states, hipStream_t st);
 int fused_scan_f32_tile();  // time steps per tile of the float one-pass kernel
+// passed: the states entering the segments by a launch of their own, else in the prologues; copied: those read a copy of init that the
+// states-only pass leaves in the last segment's place (final_states may then be written over init)
 hipError_t launch_fused_scan_f32_segmented(const ScanShape &s, int segments, const void *x, const void *dt, const float *A,
                                            const void *Bm, const void *Cm, const float *D, const float *init,
                                            const unsigned char *reset, void *y, float *final_states, float *seg_states,
